@@ -134,6 +134,8 @@ SIGNATURES = {
     "huv_kernels_info_get": (C.c_int, [P, C.POINTER(huv_kernels_info)]),
     "huv_kernels_copy": (C.c_int, [P, PI64, PI64, PD, PD]),
     "huv_kernels_free": (None, [P]),
+    "huv_real_fields": (C.c_int, [C.c_int, C.c_int, C.c_int64, PI64, PD, PD, C.c_int64, PD,
+                                  C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "huv_rasterize_rects": (C.c_int, [C.c_int, C.c_double, C.c_int, PD, C.c_double, C.c_double,
                                       PD]),
     "huv_ctx_create": (C.c_int, [C.c_int, C.POINTER(P)]),

@@ -24,7 +24,8 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
              "-Wno-unused-command-line-argument"]
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]
 
-HOST_SRC = ["host/optics_source.cpp", "host/linalg.cpp", "host/kernels_build.cpp"]
+HOST_SRC = ["host/optics_source.cpp", "host/linalg.cpp", "host/kernels_build.cpp",
+            "host/real_form.cpp"]
 HIP_SRC = ["hip/socs_kernels.hip", "hip/ilt_kernels.hip", "hip/unet_kernels.hip",
            "hip/mask_kernels.hip", "hip/kbuild_kernels.hip", "capi.cpp", "capi_kbuild.cpp",
            "capi_ilt.cpp", "capi_unet.cpp"]

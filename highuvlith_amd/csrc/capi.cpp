@@ -223,7 +223,7 @@ Ctx::~Ctx() {
   for (auto& kv : plane_tables) hipFree(kv.second);
   for (auto& kv : plane_packs) {
     hipFree(kv.second.kern);
-    hipFree(kv.second.lam);
+    hipFree(kv.second.tab);
   }
   for (auto& kv : graphs) drop_graph(kv.second);
   if (pin_h) hipHostFree(pin_h);
@@ -311,7 +311,7 @@ void Ctx::forget_kset(uint64_t id) {
       if (!busy) hipStreamSynchronize(stream());
       busy = true;
       hipFree(it->second.kern);
-      hipFree(it->second.lam);
+      hipFree(it->second.tab);
       it = plane_packs.erase(it);
     } else {
       ++it;
@@ -452,6 +452,19 @@ huv_status validate_rects(int nclips, int n, const RectBatch& rb) {
         return fail(HUV_INVALID_PARAMETER, "polygon values must be finite");
   }
   return HUV_OK;
+}
+
+// Whether every amplitude of a feature batch is real (its spectra are then
+// Hermitian).
+static bool features_real(int nclips, const RectBatch& rb) {
+  for (int64_t r = 0; r < rb.offsets[nclips]; ++r)
+    if (rb.rects[6 * r + 5] != 0.0) return false;
+  for (int i = 0; i < nclips; ++i)
+    if (rb.background[2 * i + 1] != 0.0) return false;
+  if (rb.polys)
+    for (int64_t j = 0; j < rb.polys->poly_offsets[nclips]; ++j)
+      if (rb.polys->values[2 * j + 1] != 0.0) return false;
+  return true;
 }
 
 namespace {
@@ -791,6 +804,39 @@ huv_status huv_kernels_copy(const huv_host_kernels* k, int64_t* support, int64_t
 
 void huv_kernels_free(huv_host_kernels* k) { delete k; }
 
+huv_status huv_real_fields(int n, int K, int64_t S, const int64_t* support, const double* eig,
+                           const double* values, int64_t capacity, double* fields, int* band,
+                           int* count) {
+  if (!support || !eig || !values || !band || !count || (capacity > 0 && !fields))
+    return fail(HUV_INVALID_PARAMETER, "null argument");
+  if (n < 2 || K < 1 || S < 1) return fail(HUV_INVALID_PARAMETER, "empty kernel set");
+  int B = 0;
+  for (int64_t t = 0; t < S; ++t) {
+    if (support[t] < 0 || support[t] >= (int64_t)n * n)
+      return fail(HUV_INVALID_PARAMETER, "support index out of range");
+    const int64_t i = support[t] / n, j = support[t] % n;
+    B = std::max<int>(B, (int)std::max(i < n / 2 ? i : n - i, j < n / 2 ? j : n - j));
+  }
+  try {
+    huv::RealFields rf;
+    huv::real_fields(n, B, K, S, support, eig, values, rf);
+    *band = B;
+    *count = rf.R;
+    const int W = 2 * B + 1;
+    for (int64_t f = 0; f < std::min<int64_t>(capacity, rf.R); ++f)
+      for (int kx = -B; kx <= B; ++kx)
+        for (int ky = -B; ky <= B; ++ky) {
+          const huv::cd v = huv::real_field_value(rf, (int)f, kx, ky);
+          double* o = fields + 2 * (((size_t)f * W + (kx + B)) * W + (ky + B));
+          o[0] = v.real();
+          o[1] = v.imag();
+        }
+    return HUV_OK;
+  } catch (const std::exception& ex) {
+    return fail(HUV_INTERNAL_ERROR, ex.what());
+  }
+}
+
 huv_status huv_rasterize_rects(int n, double pixel_nm, int nrects, const double* rects,
                                double bg_re, double bg_im, double* out) {
   if (!out || (nrects > 0 && !rects) || n < 1 || !(pixel_nm > 0.0))
@@ -982,12 +1028,62 @@ huv_status validate_planes(Ctx* c, int n, int nplanes, huv_kset* const* planes) 
   return HUV_OK;
 }
 
+// The power of two at or below x > 0: stacks carry their eigenvalues' roots in
+// units of such a scale, which is exact in FP32 over n^4, a power of two too (a
+// rounded scale would move a whole image by the same 2^-24: a resist gradient of
+// steepness 50 then moves by 1e-6).
+static double pow2_scale(double x) { return std::exp2(std::floor(std::log2(x))); }
+
+// Values of packed real field j of a set, v_{2j} + i v_{2j+1}, over the root of
+// pow2_scale(mu[0]), every packed field's eigenvalue.
+static huv::cd packed_value(const huv::RealFields& f, int j, int kx, int ky) {
+  const huv::cd a = huv::real_field_value(f, 2 * j, kx, ky);
+  const huv::cd b = 2 * j + 1 < f.R ? huv::real_field_value(f, 2 * j + 1, kx, ky) : huv::cd(0, 0);
+  return (a + huv::cd(0, 1) * b) / std::sqrt(pow2_scale(f.mu[0]));
+}
+
+huv_status kset_real(huv_kset* ks, bool boxes) {
+  if (!ks->real_done) {
+    if (huv::real_fields(ks->n, ks->B, ks->K, ks->S, ks->support.data(), ks->lam_host.data(),
+                         ks->values.data(), ks->rf)) {
+      const int kr = (ks->rf.R + 1) / 2;
+      ks->Kr = kr < ks->K ? kr : 0;
+    }
+    ks->real_done = true;
+  }
+  if (!boxes || !ks->Kr || ks->kern_r) return HUV_OK;
+  const int W = 2 * ks->BB + 1;
+  std::vector<float2> box((size_t)ks->Kr * W * W, make_float2(0.f, 0.f));
+  for (int k = 0; k < ks->Kr; ++k)
+    for (int kx = -ks->B; kx <= ks->B; ++kx)
+      for (int ky = -ks->B; ky <= ks->B; ++ky) {
+        const huv::cd v = packed_value(ks->rf, k, kx, ky);
+        box[((size_t)k * W + (kx + ks->BB)) * W + (ky + ks->BB)] =
+            make_float2((float)v.real(), (float)v.imag());
+      }
+  const std::vector<float> lam((size_t)ks->Kr,
+                               (float)(pow2_scale(ks->rf.mu[0]) / std::pow((double)ks->n, 4.0)));
+  hipError_t e = hipMalloc(&ks->lam_r, lam.size() * sizeof(float));
+  if (e == hipSuccess) e = hipMemcpy(ks->lam_r, lam.data(), lam.size() * sizeof(float), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMalloc(&ks->kern_r, box.size() * sizeof(float2));
+  if (e == hipSuccess) e = hipMemcpy(ks->kern_r, box.data(), box.size() * sizeof(float2), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    hipFree(ks->kern_r);
+    hipFree(ks->lam_r);
+    ks->kern_r = nullptr;
+    ks->lam_r = nullptr;
+    return hip_fail(e, "real-field upload");
+  }
+  return HUV_OK;
+}
+
 // Device copy of the per-plane (K, kernel pointer, eigenvalue pointer)
 // tables, uploaded once per distinct plane list.
-huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, const int** dK,
-                       const float2* const** dkern, const float* const** dlam) {
+huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, bool real_masks,
+                       const int** dK, const float2* const** dkern, const float* const** dlam) {
   std::vector<uint64_t> key;
   for (int p = 0; p < nplanes; ++p) key.push_back(planes[p]->id);
+  key.push_back((uint64_t)real_masks);
   const size_t offk = 0, offp = ((size_t)nplanes * sizeof(int) + 63) / 64 * 64;
   const size_t offl = offp + (size_t)nplanes * sizeof(void*);
   const size_t tbl = offl + (size_t)nplanes * sizeof(void*);
@@ -998,9 +1094,14 @@ huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, const int**
   } else {
     std::vector<char> host(tbl, 0);
     for (int p = 0; p < nplanes; ++p) {
-      ((int*)(host.data() + offk))[p] = planes[p]->K;
-      ((const float2**)(host.data() + offp))[p] = planes[p]->kern;
-      ((const float**)(host.data() + offl))[p] = planes[p]->lam;
+      if (real_masks) {
+        const huv_status st = kset_real(planes[p], true);
+        if (st != HUV_OK) return st;
+      }
+      const bool packed = real_masks && planes[p]->Kr;
+      ((int*)(host.data() + offk))[p] = packed ? planes[p]->Kr : planes[p]->K;
+      ((const float2**)(host.data() + offp))[p] = packed ? planes[p]->kern_r : planes[p]->kern;
+      ((const float**)(host.data() + offl))[p] = packed ? planes[p]->lam_r : planes[p]->lam;
     }
     hipError_t e = hipMalloc(&dtab, tbl);
     if (e != hipSuccess) return hip_fail(e, "plane table");
@@ -1017,29 +1118,101 @@ huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, const int**
   return HUV_OK;
 }
 
-// Kernel stacks of a plane list packed into one zero-padded buffer
-// [Q][nplanes][Kmax][W][W] for coarse grid m (W = 2 BB + 1, BB = (m - 1) / 4
-// >= every set's band, Q = m / 32; copy q multiplied by e^{2 pi i kx q / m} in
-// FP64) with eigenvalues / n^4 in [nplanes][Kmax] (0 for padding), built from
-// the host copies of the sets.
+// Kernel stacks of a plane list packed into one buffer [Q][total][W][W] for
+// coarse grid m (W = 2 BB + 1, BB = (m - 1) / 4 >= every set's band, Q = m / 32;
+// copy q multiplied by e^{2 pi i kx q / m} in FP64) and each box scaled by the root of
+// its eigenvalue (huvk::PlaneStack), built from the host copies of the sets.  For real masks a plane's
+// stack holds its packed real fields where these are fewer than its kernels,
+// and a plane whose real form equals an earlier plane's (opposite defocus under
+// a point-symmetric source, a plane listed twice) has no stack of its own.
+// Each plane's stack depends on that plane alone, so its images do not depend
+// on which other planes share the call, except through such an equality.
 huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool paired,
-                      const float2** kern, const float** lam, int* Kmax) {
+                      bool real_masks, const Ctx::PlanePack** pack) {
   const int BB = huvk::coarse_band(m), Q = huvk::coarse_classes(m);
   std::vector<uint64_t> key;
   for (int p = 0; p < nplanes; ++p) key.push_back(planes[p]->id);
   key.push_back((uint64_t)m);
   key.push_back((uint64_t)paired);
+  key.push_back((uint64_t)real_masks);
   auto it = c->plane_packs.find(key);
-  if (it == c->plane_packs.end() && c->fixed_mode)
-    return fail(HUV_INVALID_PARAMETER,
-                "kernel stacks of this plane list are not built yet: call huv_socs_images once "
-                "with the same kernel sets before the no-allocation entry point");
+  if (it == c->plane_packs.end() && c->fixed_mode) {
+    // a stack built by an earlier call for complex masks serves real ones too
+    key.back() = 0;
+    it = c->plane_packs.find(key);
+    if (it == c->plane_packs.end())
+      return fail(HUV_INVALID_PARAMETER,
+                  "kernel stacks of this plane list are not built yet: call huv_socs_images once "
+                  "with the same kernel sets before the no-allocation entry point");
+  }
   if (it == c->plane_packs.end()) {
     Ctx::PlanePack pk;
+    std::vector<int> src(nplanes), rep;  // distinct image of each plane; its plane
     for (int p = 0; p < nplanes; ++p) {
-      pk.Kmax = std::max(pk.Kmax, planes[p]->K);
       if (planes[p]->B > BB) return fail(HUV_INTERNAL_ERROR, "kernel band exceeds the packed box");
+      int u = (int)rep.size();
+      if (real_masks) {
+        const huv_status st = kset_real(planes[p], false);
+        if (st != HUV_OK) return st;
+        for (int t = 0; t < (int)rep.size() && u == (int)rep.size(); ++t)
+          if (planes[rep[t]] == planes[p] || huv::same_real_form(planes[rep[t]]->rf, planes[p]->rf))
+            u = t;
+      }
+      src[p] = u;
+      if (u == (int)rep.size()) rep.push_back(p);
     }
+    pk.nd = (int)rep.size();
+    // longest stacks first: the field work-groups of the last plane end a launch
+    auto count = [&](int t) { return real_masks && planes[t]->Kr ? planes[t]->Kr : planes[t]->K; };
+    std::vector<int> order(pk.nd), where(pk.nd);
+    for (int u = 0; u < pk.nd; ++u) order[u] = u;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int b) { return count(rep[a]) > count(rep[b]); });
+    std::vector<int> sorted(pk.nd);
+    for (int u = 0; u < pk.nd; ++u) {
+      sorted[u] = rep[order[u]];
+      where[order[u]] = u;
+    }
+    rep.swap(sorted);
+    for (int& u : src) u = where[u];
+    std::vector<int> tab;
+    std::vector<std::vector<int>> kernels(pk.nd);  // of each stack, in its order
+    std::vector<double> scale(pk.nd, 0.0);
+    for (int u = 0; u < pk.nd; ++u) {
+      const huv_kset* ks = planes[rep[u]];
+      const int cnt = count(rep[u]);
+      const double n4 = std::pow((double)ks->n, 4.0);
+      int negative = 0;
+      if (real_masks && ks->Kr) {
+        scale[u] = pow2_scale(ks->rf.mu[0]);
+      } else {
+        for (int sign : {-1, 1})
+          for (int k = 0; k < ks->K; ++k)
+            if ((ks->lam_host[k] < 0.0) == (sign < 0)) kernels[u].push_back(k);
+        for (double l : ks->lam_host) {
+          negative += l < 0.0;
+          scale[u] = std::max(scale[u], std::fabs(l));
+        }
+        if (std::isfinite(scale[u]) && scale[u] > 0.0) scale[u] = pow2_scale(scale[u]);
+      }
+      if (!(scale[u] > 0.0)) scale[u] = 1.0;
+      const float f = (float)(scale[u] / n4);
+      int bits;
+      std::memcpy(&bits, &f, sizeof bits);
+      tab.insert(tab.end(), {pk.total, cnt, negative, bits});
+      pk.total += cnt;
+      pk.Kmax = std::max(pk.Kmax, cnt);
+    }
+    const int src_at = (int)tab.size(), off_at = src_at + nplanes, list_at = off_at + pk.nd + 1;
+    tab.insert(tab.end(), src.begin(), src.end());
+    std::vector<int> list;
+    for (int u = 0; u < pk.nd; ++u) {
+      tab.push_back((int)list.size());
+      for (int p = 0; p < nplanes; ++p)
+        if (src[p] == u) list.push_back(p);
+    }
+    tab.push_back(nplanes);
+    tab.insert(tab.end(), list.begin(), list.end());
     const int W = 2 * BB + 1;
     // W x W, or column-paired (W + 1) x W: column col at [(col + 1) / 2][row][(col + 1) % 2]
     const size_t box = (size_t)(paired ? W + 1 : W) * W;
@@ -1047,43 +1220,56 @@ huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool 
       return paired ? ((size_t)((col + 1) >> 1) * W + row) * 2 + ((col + 1) & 1)
                     : (size_t)col * W + row;
     };
-    const size_t per_class = (size_t)nplanes * pk.Kmax * box;
+    std::vector<huv::cd> tw((size_t)m);  // e^{2 pi i e / m}
+    for (int e = 0; e < m; ++e)
+      tw[e] = huv::cd(std::cos(2.0 * M_PI * e / m), std::sin(2.0 * M_PI * e / m));
+    const size_t per_class = (size_t)pk.total * box;
     std::vector<float2> hk((size_t)Q * per_class, make_float2(0.f, 0.f));
-    std::vector<float> hl((size_t)nplanes * pk.Kmax, 0.f);
-    for (int p = 0; p < nplanes; ++p) {
-      const huv_kset* ks = planes[p];
+    for (int u = 0; u < pk.nd; ++u) {
+      const huv_kset* ks = planes[rep[u]];
       const int64_t n = ks->n;
-      const double n4 = std::pow((double)n, 4.0);
-      for (int k = 0; k < ks->K; ++k) {
-        hl[(size_t)p * pk.Kmax + k] = (float)(ks->lam_host[k] / n4);
+      const int first = tab[4 * u];
+      auto put = [&](int g, int64_t kx, int64_t ky, huv::cd v) {
+        for (int q = 0; q < Q; ++q) {
+          const huv::cd w = v * tw[(size_t)(((kx * q) % m + m) % m)];
+          hk[q * per_class + (size_t)g * box + at((int)kx + BB, (int)ky + BB)] =
+              make_float2((float)w.real(), (float)w.imag());
+        }
+      };
+      if (real_masks && ks->Kr) {
+        for (int k = 0; k < ks->Kr; ++k)
+          for (int kx = -ks->B; kx <= ks->B; ++kx)
+            for (int ky = -ks->B; ky <= ks->B; ++ky)
+              put(first + k, kx, ky, packed_value(ks->rf, k, kx, ky));
+        continue;
+      }
+      for (int g = 0; g < ks->K; ++g) {
+        const int k = kernels[u][g];
+        const double root = std::sqrt(std::fabs(ks->lam_host[k]) / scale[u]);
         for (int64_t t = 0; t < ks->S; ++t) {
           const int64_t i = ks->support[t] / n, j = ks->support[t] % n;
           const int64_t ky = i < n / 2 ? i : i - n, kx = j < n / 2 ? j : j - n;
-          const double re = ks->values[2 * (k * ks->S + t)], im = ks->values[2 * (k * ks->S + t) + 1];
-          for (int q = 0; q < Q; ++q) {
-            const long e = ((kx * q) % m + m) % m;  // e^{2 pi i kx q / m}
-            const double a = 2.0 * M_PI * (double)e / (double)m;
-            const double cs = std::cos(a), sn = std::sin(a);
-            hk[q * per_class + ((size_t)p * pk.Kmax + k) * box + at(kx + BB, ky + BB)] =
-                make_float2((float)(re * cs - im * sn), (float)(re * sn + im * cs));
-          }
+          put(first + g, kx, ky,
+              root * huv::cd(ks->values[2 * (k * ks->S + t)], ks->values[2 * (k * ks->S + t) + 1]));
         }
       }
     }
     hipError_t e = hipMalloc(&pk.kern, hk.size() * sizeof(float2));
-    if (e == hipSuccess) e = hipMalloc(&pk.lam, hl.size() * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&pk.tab, tab.size() * sizeof(int));
     if (e == hipSuccess) e = hipMemcpy(pk.kern, hk.data(), hk.size() * sizeof(float2), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(pk.lam, hl.data(), hl.size() * sizeof(float), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(pk.tab, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
       hipFree(pk.kern);
-      hipFree(pk.lam);
+      hipFree(pk.tab);
       return hip_fail(e, "plane pack upload");
     }
+    bool own = true;  // every plane has its own image, in order
+    for (int p = 0; p < nplanes; ++p) own = own && src[p] == p;
+    if (!own)
+      pk.map = huvk::PlaneMap{nplanes, pk.nd, pk.tab + src_at, pk.tab + off_at, pk.tab + list_at};
     it = c->plane_packs.emplace(key, pk).first;
   }
-  *kern = it->second.kern;
-  *lam = it->second.lam;
-  *Kmax = it->second.Kmax;
+  *pack = &it->second;
   return HUV_OK;
 }
 
@@ -1095,14 +1281,16 @@ size_t image_interm_bytes(int m, int B, int S) {
 
 // Default number of clip ranges: enough that one range's intermediates (the
 // coarse images and intensity bands written by one stage and read by the
-// next) stay within about 160 MB, so they are served from the device's
-// last-level cache rather than HBM, but no more than keeps at least 768
-// field work-groups per range (1.5 rounds of two per CU).
-int clip_ranges_default(int nclips, int nplanes, int m, int B, int S) {
-  const double interm = (double)nclips * nplanes * (double)image_interm_bytes(m, B, S);
-  int r = (int)std::ceil(interm / 160e6);
-  const int wgs = nclips * huvk::coarse_classes(m) * S;
-  r = std::min(r, std::max(1, wgs / 768));
+// next; nd distinct images per clip) stay within about 230 MB, near the
+// device's last-level cache, but no more than keeps at least 768 field
+// work-groups per range (1.5 rounds of two per CU).  512 clips of 1024^2 with
+// three distinct images (447 MB): one range 5.52 ms, two 5.17, three 5.27,
+// four 5.31; 512 clips with one (149 MB): one range 1.78 ms, two 1.79.
+int clip_ranges_default(int nclips, int nd, int m, int B, int S) {
+  const double interm = (double)nclips * nd * (double)image_interm_bytes(m, B, S);
+  int r = (int)std::ceil(interm / 230e6);
+  const int64_t wgs = (int64_t)nclips * huvk::coarse_classes(m) * S * nd;
+  r = (int)std::min<int64_t>(r, std::max<int64_t>(1, wgs / 768));
   return std::max(1, std::min(r, 16));
 }
 
@@ -1136,12 +1324,12 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
     Mp = (float2*)c->buf(Workspace::BAND_PAIRED, (size_t)nclips * (W + 1) * W * sizeof(float2), e);
     if (!Mp) return hip_fail(e, "workspace");
   }
-  const float2* kern;
-  const float* lam;
-  int Kmax;
-  huv_status st = plane_pack(c, nplanes, planes, m, xlanes == 2, &kern, &lam, &Kmax);
+  const Ctx::PlanePack* pack;
+  huv_status st = plane_pack(c, nplanes, planes, m, xlanes == 2, src.real_mask(), &pack);
   if (st != HUV_OK) return st;
-  int S = huvk::fields_splits(m, split_batch > 0 ? split_batch : nclips, Kmax);
+  const int Kmax = pack->Kmax;
+  const int nd = pack->nd;  // distinct images per clip, nplanes or fewer
+  int S = huvk::fields_splits(m, (split_batch > 0 ? split_batch : nclips) * nd, Kmax);
   if (max_splits > 0 && S > max_splits) {
     // every split must own at least one kernel (its partials are summed)
     const int ks = (Kmax + max_splits - 1) / max_splits;
@@ -1149,12 +1337,12 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
   }
   // Clip ranges (one for the fidelity epilogue, whose partials are indexed by
   // image, and for the no-allocation path, whose scratch is sized for one).
-  int nr = tune && tune->chunks ? tune->chunks : clip_ranges_default(nclips, nplanes, m, B, S);
+  int nr = tune && tune->chunks ? tune->chunks : clip_ranges_default(nclips, nd, m, B, S);
   if (fid || c->fixed_mode) nr = 1;
   nr = std::max(1, std::min(nr, nclips));
   const int cc = (nclips + nr - 1) / nr;  // clips per range
   nr = (nclips + cc - 1) / cc;            // ranges actually used
-  const int cimg = cc * nplanes;          // images per range
+  const int cimg = cc * nd;               // distinct images per range
   const bool raster = src.kind == MaskSource::REAL || src.kind == MaskSource::COMPLEX;
   // Feature lists and host spectra: the band of every clip at once (their
   // stages keep no per-clip rows); rasters: per range, below.
@@ -1183,7 +1371,7 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
   const size_t box_c = (size_t)(xlanes == 2 ? W + 1 : W) * W;  // band box per clip
   hipEvent_t ev;
   for (int i = 0; i < nr; ++i) {
-    const int c0 = i * cc, cn = std::min(cc, nclips - c0), ni = cn * nplanes;
+    const int c0 = i * cc, cn = std::min(cc, nclips - c0), ni = cn * nd;
     if (src.kind == MaskSource::REAL) {
       st = band_stage(c, cn, n, B, BB, src.raster + (size_t)c0 * n * n, Mq + (size_t)c0 * W * W,
                       pt, n1, Mp ? Mp + (size_t)c0 * (W + 1) * W : nullptr);
@@ -1194,8 +1382,8 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
     }
     if (st != HUV_OK) return st;
     c->stage_begin(ST_FIELDS, &ev);
-    e = huvk::launch_socs_fields(m, xnb, xlanes, cn, nplanes, Kmax, S, kern, lam,
-                                 box + (size_t)c0 * box_c, tw_m, coarse, c->stream());
+    e = huvk::launch_socs_fields(m, xnb, xlanes, cn, nd, pack->stacks(), pack->total, S,
+                                 pack->kern, box + (size_t)c0 * box_c, tw_m, coarse, c->stream());
     if (e != hipSuccess) return hip_fail(e, "socs_fields launch");
     c->stage_end(ST_FIELDS, ev);
     if (fused) {
@@ -1214,9 +1402,10 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
       c->stage_end(ST_COARSE_COLS, ev);
     }
     c->stage_begin(ST_BAND_IMAGE, &ev);
-    e = fid ? huvk::launch_band_image_fidelity(n, G, ni, Ib, tw_n, *fid, c->stream())
+    e = fid ? huvk::launch_band_image_fidelity(n, G, cn * nplanes, Ib, tw_n, pack->map, *fid,
+                                               c->stream())
             : huvk::launch_band_image(n, G, ni, Ib, tw_n, out + (size_t)c0 * nplanes * n * n,
-                                      c->stream());
+                                      pack->map, c->stream());
     if (e != hipSuccess) return hip_fail(e, "band_image launch");
     c->stage_end(ST_BAND_IMAGE, ev);
   }
@@ -1521,22 +1710,25 @@ huv_status huv_socs_images_noalloc(huv_ctx* c, int nclips, int n, const float* m
     return fail(HUV_INVALID_PARAMETER,
                 "transform tables for this grid are not built yet: call huv_socs_images once "
                 "with the same kernel sets before the no-allocation entry point");
-  int Kmax = 0;
-  for (int p = 0; p < nplanes; ++p) Kmax = std::max(Kmax, planes[p]->K);
-  // As many kernel splits as huv_socs_images would use, fewer if the scratch
-  // array is too small for their partial images.
-  int S = huvk::fields_splits(m, nclips, Kmax);
-  size_t need = 0;
-  for (;; --S) {
-    const int ks = (Kmax + S - 1) / S, s_eff = (Kmax + ks - 1) / ks;
-    need = socs_sizes(nclips, n, B, m, xlanes == 2, nplanes, s_eff, true).total();
-    if (need <= c->fixed_cap || S == 1) break;
-  }
+  size_t need = socs_sizes(nclips, n, B, m, xlanes == 2, nplanes, 1, true).total();
   if (need > c->fixed_cap)
     return fail(HUV_INVALID_PARAMETER,
                 "this batch needs " + std::to_string((need + (1 << 20) - 1) >> 20) +
                     " MiB of scratch; the no-allocation entry point has " +
                     std::to_string(c->fixed_cap >> 20) + " MiB per GPU: pass fewer clips per call");
+  c->fixed_mode = true;
+  c->fixed_used = 0;
+  const Ctx::PlanePack* pack = nullptr;
+  st = plane_pack(c, nplanes, planes, m, xlanes == 2, true, &pack);
+  c->fixed_mode = false;
+  if (st != HUV_OK) return st;
+  // As many kernel splits as huv_socs_images would use, fewer if the scratch
+  // array is too small for their partial images.
+  int S = huvk::fields_splits(m, nclips * pack->nd, pack->Kmax);
+  for (; S > 1; --S) {
+    const int ks = (pack->Kmax + S - 1) / S, s_eff = (pack->Kmax + ks - 1) / ks;
+    if (socs_sizes(nclips, n, B, m, xlanes == 2, pack->nd, s_eff, true).total() <= c->fixed_cap) break;
+  }
   const bool prof = c->profiling;
   c->profiling = false;  // per-stage timing creates events
   c->fixed_mode = true;
@@ -1570,6 +1762,7 @@ huv_status huv_socs_images_features(huv_ctx* c, int nclips, int n, double pixel_
   MaskSource src;
   src.kind = MaskSource::FEATURES;
   src.rects = &rb;
+  src.real_features = features_real(nclips, rb);
   return socs_forward(c, nclips, n, src, nplanes, planes, out, false, nullptr,
                       it != c->tuned.end() ? &it->second : nullptr);
 }

@@ -40,6 +40,10 @@ struct huv_ilt {
 namespace {
 
 constexpr int kBpi = 64;  // reduction blocks per image
+// Batch size the field kernel's split of the kernel sum is chosen for (m = 128,
+// three conditions, 32 kernels: 16 partial images instead of 32 for one target;
+// 5 targets then take 960 field work-groups of two kernels, not 1920 of one).
+constexpr int kSplitBatch = 2;
 
 struct IltBuffers {
   float *m, *t, *G, *dcdm, *reg_grad, *G0g;
@@ -53,10 +57,13 @@ struct IltBuffers {
   int KS = 1;  // adjoint work-groups per image (kernels dealt over them)
 };
 
-// One adjoint work-group per kernel of the largest condition.
+// One adjoint work-group per kernel of the largest condition (packed real
+// fields where the transmittance is real: with A = a_1 + i a_2 and K = K_1 +
+// i K_2 for two real fields, the Hermitian part of conj(K) F(G0 A), all that
+// the gradient 2 Re[.] keeps, is conj(K_1) F(G0 a_1) + conj(K_2) F(G0 a_2)).
 static int ilt_splits(const huv_ilt* p) {
   int ks = 1;
-  for (const huv_kset* k : p->conds) ks = std::max(ks, k->K);
+  for (const huv_kset* k : p->conds) ks = std::max(ks, !p->complex_abs && k->Kr ? k->Kr : k->K);
   return ks;
 }
 
@@ -130,7 +137,7 @@ huv_status ilt_filter(huv_ilt* p, int count, const float* in, float* out, IltBuf
   if (e != hipSuccess) return hip_fail(e, "ilt filter band launch");
   const float2* tw_n = c->twiddles(n, e);
   if (!tw_n) return hip_fail(e, "twiddle table");
-  e = huvk::launch_band_image(n, p->Bf, count, b.If, tw_n, out, c->stream());
+  e = huvk::launch_band_image(n, p->Bf, count, b.If, tw_n, out, huvk::PlaneMap{}, c->stream());
   return e == hipSuccess ? HUV_OK : hip_fail(e, "ilt filter image launch");
 }
 
@@ -204,7 +211,7 @@ huv_status ilt_eval(huv_ilt* p, int T, const float* targets, const int* trows,
   float2* Mq = nullptr;
   MaskSource mask = MaskSource::real(b.t);
   if (p->complex_abs) mask.kind = MaskSource::COMPLEX;
-  // The kernel sum is split as for a single target at every batch size, so a
+  // The kernel sum is split as for kSplitBatch targets at every batch size, so a
   // target's images, and with them its whole optimisation trajectory, do not
   // depend on which other targets are still live in the batch.  The images
   // are never stored: the last stage evaluates the fidelity (and G) of every
@@ -220,7 +227,7 @@ huv_status ilt_eval(huv_ilt* p, int T, const float* targets, const int* trows,
   fid.dose = p->dose_d;
   fid.G = grad ? b.G : nullptr;
   fid.partial = b.fid_part;
-  st = socs_forward(c, T, n, mask, C, p->conds.data(), nullptr, false, &Mq, nullptr, 0, 1, &fid);
+  st = socs_forward(c, T, n, mask, C, p->conds.data(), nullptr, false, &Mq, nullptr, 0, kSplitBatch, &fid);
   if (st != HUV_OK) return st;
   c->stage_begin(ST_ILT_POINTWISE, &ev);
   if (reg) {
@@ -251,7 +258,7 @@ huv_status ilt_eval(huv_ilt* p, int T, const float* targets, const int* trows,
     const int* dK;
     const float2* const* dkern;
     const float* const* dlam;
-    st = plane_table(c, C, p->conds.data(), &dK, &dkern, &dlam);
+    st = plane_table(c, C, p->conds.data(), !p->complex_abs, &dK, &dkern, &dlam);
     if (st != HUV_OK) return st;
     c->stage_begin(ST_ILT_ADJOINT, &ev);
     const double n2 = (double)n * n;
@@ -280,7 +287,7 @@ huv_status ilt_eval(huv_ilt* p, int T, const float* targets, const int* trows,
     const float2* tw_n = c->twiddles(n, e);
     if (!tw_n) return hip_fail(e, "twiddle table");
     if (filt) {
-      e = huvk::launch_band_image(n, B, T, b.H, tw_n, b.dcdm, s);
+      e = huvk::launch_band_image(n, B, T, b.H, tw_n, b.dcdm, huvk::PlaneMap{}, s);
     } else {
       // the chain rule where the image of dC/dm would be stored: the
       // gradient rows are written directly
@@ -405,6 +412,9 @@ huv_status huv_ilt_create(huv_ctx* c, int n, int ncond, huv_kset* const* conds, 
   p->filter_c = filter_c;
   std::vector<float> d(dose, dose + ncond), w(weight, weight + ncond);
   p->weight_h = w;
+  if (!p->complex_abs)
+    for (huv_kset* k : p->conds)
+      if ((st = kset_real(k, true)) != HUV_OK) return st;
   hipError_t e = hipMalloc(&p->dose_d, ncond * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&p->weight_d, ncond * sizeof(float));
   if (e == hipSuccess) e = hipMemcpy(p->dose_d, d.data(), ncond * sizeof(float), hipMemcpyHostToDevice);

@@ -52,11 +52,16 @@ struct Ctx {
   // by the ids of the kernel sets in a plane list (dropped when a set dies).
   std::map<std::vector<uint64_t>, void*> plane_tables;
   struct PlanePack {
-    float2* kern = nullptr;  // [Q][nplanes][Kmax] boxes (W x W or column-paired)
-    float* lam = nullptr;    // [nplanes][Kmax], zero-padded
-    int Kmax = 0;
+    float2* kern = nullptr;  // [Q][total] boxes (W x W or column-paired)
+    int* tab = nullptr;      // nd PlaneStacks, then map.src, map.off, map.list
+    int nd = 0;              // distinct images per clip
+    int total = 0;           // kernels of the nd stacks
+    int Kmax = 0;            // largest of their counts
+    const huvk::PlaneStack* stacks() const { return (const huvk::PlaneStack*)tab; }
+    huvk::PlaneMap map;      // src null where every plane has its own image
   };
-  // keyed by the kernel-set ids followed by the box half-width
+  // keyed by the kernel-set ids followed by the coarse size, the box layout
+  // and whether the stack is the one for real masks
   std::map<std::vector<uint64_t>, PlanePack> plane_packs;
   // Launch shapes chosen by the autotuner, keyed by (n, band, nplanes, Kmax).
   std::map<std::vector<int>, huv_socs_tuning> tuned;
@@ -162,16 +167,25 @@ struct MaskSource {
   const float* raster = nullptr;     // REAL: [nclips][n][n]; COMPLEX: interleaved pairs
   const RectBatch* rects = nullptr;  // FEATURES
   const double* spectra = nullptr;   // SPECTRUM (host)
+  bool real_features = false;        // FEATURES: every amplitude is real
   static MaskSource real(const float* p) { MaskSource s; s.raster = p; return s; }
+  bool real_mask() const { return kind == REAL || (kind == FEATURES && real_features); }
 };
 
 huv_status validate_planes(Ctx* c, int n, int nplanes, huv_kset* const* planes);
-huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, const int** dK,
-                       const float2* const** dkern, const float* const** dlam);
+// Per-plane (K, boxes, eigenvalues) device tables; real_masks: of the packed
+// real fields where the set has a shorter list of those (kset_real).
+huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, bool real_masks,
+                       const int** dK, const float2* const** dkern, const float* const** dlam);
+// The set's kernels for real masks: computes the real fields on first use and
+// uploads their packed boxes; ks->Kr == 0 where the set keeps its own kernels.
+huv_status kset_real(huv_kset* ks, bool boxes);
 // Per-class pre-twisted kernel stacks at coarse size m (column-paired boxes
-// when `paired`, for the two-lane field kernel).
+// when `paired`, for the two-lane field kernel).  real_masks: for masks with a
+// real transmittance, where a plane's kernels may be replaced by fewer packed
+// real fields and planes with the same real form share one image.
 huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool paired,
-                      const float2** kern, const float** lam, int* Kmax);
+                      bool real_masks, const Ctx::PlanePack** pack);
 // Forward images; tune = NULL uses the kernel sets' own coarse grid and the
 // default launch shapes (the ILT adjoint relies on that band layout).
 // pixel_transfer applies to rasters only.
@@ -201,8 +215,15 @@ struct huv_kset {
   std::vector<double> lam_host;
   std::vector<int64_t> support;
   std::vector<double> values;
+  // Real masks (kset_real): the set's real fields and, where they pack into
+  // Kr < K complex ones, boxes as `kern` with eigenvalues as `lam`.
+  bool real_done = false;
+  huv::RealFields rf;
+  int Kr = 0;
+  float2* kern_r = nullptr;
+  float* lam_r = nullptr;
   ~huv_kset() {
-    if (kern) hipFree(kern);
-    if (lam) hipFree(lam);
+    for (void* p : {(void*)kern, (void*)lam, (void*)kern_r, (void*)lam_r})
+      if (p) hipFree(p);
   }
 };

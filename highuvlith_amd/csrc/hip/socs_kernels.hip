@@ -207,7 +207,7 @@ __global__ __launch_bounds__(TEAMS * N2) void k_cols_band_c(
 }
 
 // ---------------------------------------------------------------------------
-// socs_fields: one work-group per (clip, x class q), all planes of the clip.
+// socs_fields: one work-group per (clip, x class q, plane).
 // Coarse grid M = 32 Q, Q = R = M / 32 classes and residues, band half-width
 // BB = (M - 1) / 4 at compile time (kernel boxes are zero beyond the set's
 // own band).  With P = K . M (untwisted band product), a field sample is
@@ -302,17 +302,34 @@ __device__ __forceinline__ c32x2 load_c32x2(__amdgpu_buffer_rsrc_t r, int voff, 
   return c32x2{c32{f.x, f.y}, c32{f.z, f.w}};
 }
 
+// Split sj of S takes the kernels [lo, hi) of a plane: a share that depends on
+// the plane's own count and S alone, empty for some splits where the count is
+// below S.
+struct KernelShare {
+  int lo, hi;
+};
+__device__ __forceinline__ KernelShare kernel_share(const PlaneStack& p, int sj, int S) {
+  return KernelShare{p.first + (int)((unsigned)p.count * (unsigned)sj / (unsigned)S),
+                     p.first + (int)((unsigned)p.count * (unsigned)(sj + 1) / (unsigned)S)};
+}
+
 // XNB: band columns per load block of the x pass (a tuning parameter).
-// kern: [Q][nplanes * Kmax][W][W], class q's copy twisted by e^{2 pi i kx q / M}.
-// S > 1 (small batches): work-group split j takes the kernels [j ks, j ks + ks)
-// of every plane (ks = ceil(Kmax / S), every split non-empty) and writes its
-// partial coarse images at coarse + j * nclips * nplanes * M^2; coarse_rows
+// kern: [Q][total][W][W], class q's copy twisted by e^{2 pi i kx q / M} and scaled
+// by the root of its eigenvalue's magnitude (relative to the plane's scale), so
+// the sum over kernels is one of plain squares and no step loads an eigenvalue.
+// The plane's kernels with negative eigenvalues come first and are subtracted.
+// S > 1 (small batches): work-group split j takes its share of every plane's
+// kernels (kernel_share) and writes its partial coarse images at
+// coarse + j * nclips * nplanes * M^2 (zeros for an empty share); coarse_rows
 // sums the S partials in split order.
+// One plane per work-group rather than all planes of a clip: a launch then ends
+// with short work-groups instead of a lone one of all planes' kernels per CU
+// (96 clips of 1024^2, 80 packed kernels in three planes: 552 -> 450 us).
 template <int M, int XNB, int XS>
 __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_waves_per_eu(4))) void k_socs_fields(
-    const float2* __restrict__ Mq, const float2* __restrict__ kern, const float* __restrict__ lam,
-    int nclips, int nplanes, int Kmax, int S, const float2* __restrict__ tw_m,
-    float* __restrict__ coarse) {
+    const float2* __restrict__ Mq, const float2* __restrict__ kern, int nclips, int nplanes,
+    const PlaneStack* __restrict__ stacks, int total, int S,
+    const float2* __restrict__ tw_m, float* __restrict__ coarse) {
   using C = CoarseCfg<M, XS>;
   constexpr int F = C::F, Q = C::Q, R = C::R, BB = C::BB, W = C::W, TP = C::TP;
   constexpr int TMIN = C::TMIN, TMAX = C::TMAX, NT = TMAX - TMIN + 1;
@@ -324,7 +341,9 @@ __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_
   const int slot = L / kXcds;
   const int q = slot % Q;
   const int sj = (slot / Q) % S;
-  const int clip = (slot / (Q * S)) * kXcds + L % kXcds;
+  const int groups = (nclips + kXcds - 1) / kXcds;
+  const int plane = slot / (Q * S * groups);
+  const int clip = (slot / (Q * S)) % groups * kXcds + L % kXcds;
   if (clip >= nclips) return;  // whole work-group, before any barrier
   const int tid = threadIdx.x;
   for (int i = tid; i < R * F; i += C::THREADS) twy[i] = tw_pos(tw_m, (i % F) * (i / F), M);
@@ -332,12 +351,6 @@ __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_
   // band spectrum box of this clip (column-paired for XS = 2)
   constexpr int BOX = XS == 1 ? W * W : (W + 1) * W;
   const __amdgpu_buffer_rsrc_t mr = box_rsrc(Mq + (size_t)clip * BOX, BOX);
-  const int steps = nplanes * Kmax;
-  // this split's kernels k0 .. k0 + kc - 1 of each plane; local step l is
-  // plane l / kc, kernel k0 + l % kc
-  const int ks = (Kmax + S - 1) / S, k0 = sj * ks, kc = min(ks, Kmax - k0);
-  const int lsteps = nplanes * kc;
-  auto gstep = [&](int l) { return (l / kc) * Kmax + k0 + l % kc; };
   const bool is_y = tid < C::YT;
   const int j = tid % F, r = tid / F;
   const int ix = tid - C::XOFF;  // x lane
@@ -348,18 +361,22 @@ __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_
 #pragma unroll
   for (int t = 0; t < NT; ++t) wf[t] = tw_pos(tw_m, (t + TMIN) * (is_y ? r : 0) * F, M);
   __syncthreads();
-  // The two groups run separate loops (wave-uniform split) with the same
-  // number of barriers, so their register live ranges do not overlap.
+  // The two groups run separate loops over the same kernels (wave-uniform
+  // split) with one barrier per kernel, so their register live ranges do not
+  // overlap: the barrier ends the x group's kernel and lets the y group take
+  // it while the x group fills the other tile.
+  int tile = 0;
+  const PlaneStack stack = stacks[plane];
+  const KernelShare ks = kernel_share(stack, sj, S);
   if (ix >= 0) {
-    for (int s = 0; s <= lsteps; ++s) {
-      if (s < lsteps && iy < W) {
-        const int sg = gstep(s);
-        c32* Tr = T + (s & 1) * W * TP + iy * TP;
+    for (int sg = ks.lo; sg < ks.hi; ++sg, tile ^= 1) {
+      if (iy < W) {
+        c32* Tr = T + tile * W * TP + iy * TP;
         if constexpr (XS == 1) {
           // Buffer loads: one VGPR offset per lane, the column offset in an SGPR.
           const int vo = iy * (int)sizeof(float2);
           const __amdgpu_buffer_rsrc_t kr =
-              box_rsrc(kern + ((size_t)q * steps + sg) * W * W, W * W);
+              box_rsrc(kern + ((size_t)q * total + sg) * W * W, W * W);
           c32 c[F];
 #pragma unroll
           for (int h = 0; h < F; ++h) c[h] = c32{0.f, 0.f};
@@ -407,7 +424,7 @@ __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_
           const int col0 = part ? C::xcol0(1) : C::xcol0(0);
           const int vo = (((col0 + 1) >> 1) * W + iy) * (int)(2 * sizeof(float2));
           const __amdgpu_buffer_rsrc_t kr =
-              box_rsrc(kern + ((size_t)q * steps + sg) * BOX, BOX);
+              box_rsrc(kern + ((size_t)q * total + sg) * BOX, BOX);
           c32 c[F / 2];  // bins 16 part + h
 #pragma unroll
           for (int h = 0; h < F / 2; ++h) c[h] = c32{0.f, 0.f};
@@ -469,14 +486,19 @@ __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_
     float acc[F];
 #pragma unroll
     for (int i = 0; i < F; ++i) acc[i] = 0.f;
-    for (int s = 0; s <= lsteps; ++s) {
-      if (is_y && s >= 1) {
-        const int sp = s - 1;
+    const int flip = stack.first + stack.negative;  // first non-negative eigenvalue
+    for (int sg = ks.lo; sg < ks.hi; ++sg, tile ^= 1) {
+      __syncthreads();
+      if (is_y) {
+        if (sg == flip) {
+#pragma unroll
+          for (int i = 0; i < F; ++i) acc[i] = -acc[i];
+        }
         // Re-read the twiddles every step rather than holding them in registers.
         int tyo = r * F;
         asm volatile("" : "+v"(tyo));
         const c32* ty = twy + tyo;
-        const c32* Tb = T + (sp & 1) * W * TP;
+        const c32* Tb = T + tile * W * TP;
         c32 d[F];
 #pragma unroll
         for (int h = 0; h < F; ++h) {
@@ -492,24 +514,21 @@ __global__ __launch_bounds__((CoarseCfg<M, XS>::THREADS)) __attribute__((amdgpu_
           d[h] = cmul(v, ty[h]);
         }
         fft_reg<+1, F>(d);
-        const float l = lam[gstep(sp)];
 #pragma unroll
-        for (int i = 0; i < F; ++i) acc[i] += l * cnorm(d[i]);
-        if (sp % kc == kc - 1) {
-          // Vector buffer stores: one VGPR offset, the row offset in an SGPR.
-          const __amdgpu_buffer_rsrc_t orc = __builtin_amdgcn_make_buffer_rsrc(
-              coarse + (((size_t)sj * nclips + clip) * nplanes + sp / kc) * M * M, (short)0,
-              M * M * (int)sizeof(float), 0x00020000);
-          const int vo = (r * M + F * q + j) * (int)sizeof(float);
-#pragma unroll
-          for (int i = 0; i < F; ++i) {
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, acc[i]), orc, vo,
-                                                  R * i * M * (int)sizeof(float), 0);
-            acc[i] = 0.f;
-          }
-        }
+        for (int i = 0; i < F; ++i) acc[i] += cnorm(d[i]);  // one rounding into the sum
       }
-      __syncthreads();
+    }
+    if (is_y) {
+      // Vector buffer stores: one VGPR offset, the row offset in an SGPR.
+      const __amdgpu_buffer_rsrc_t orc = __builtin_amdgcn_make_buffer_rsrc(
+          coarse + (((size_t)sj * nclips + clip) * nplanes + plane) * M * M, (short)0,
+          M * M * (int)sizeof(float), 0x00020000);
+      const int vo = (r * M + F * q + j) * (int)sizeof(float);
+      const float l = ks.hi <= flip ? -stack.scale : stack.scale;
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l * acc[i]), orc, vo,
+                                              R * i * M * (int)sizeof(float), 0);
     }
   }
 }
@@ -856,7 +875,8 @@ __device__ __forceinline__ void chain_task(float beta, const c32* d, int C, int 
   }
 }
 
-// MODE 0: the image.  MODE 1 (fidelity): instead of the image, the ILT
+// MODE 0: the image (with a plane map: image (clip, distinct image u) to
+// every plane that has it).  MODE 1 (fidelity): instead of the image, the ILT
 // fidelity of every pixel against the target (epi): per-work-group FP64
 // partial sums of r^2 at epi.partial[img][p] and, when epi.G is set,
 // G = dC/dI written where the image would be; image img is (target
@@ -866,8 +886,8 @@ __device__ __forceinline__ void chain_task(float beta, const c32* d, int C, int 
 template <int TMIN, int TMAX, int MODE>
 __global__ __launch_bounds__(256) void k_band_image(const float2* __restrict__ Ib, int n, int G,
                                                     int nimg, const float2* __restrict__ tw_n,
-                                                    float* __restrict__ out, FidelityEpi epi,
-                                                    ChainEpi ch) {
+                                                    float* __restrict__ out, PlaneMap map,
+                                                    FidelityEpi epi, ChainEpi ch) {
   constexpr bool FID = MODE == 1, CHAIN = MODE == 2;
   constexpr int F = 32, NT = TMAX - TMIN + 1;
   extern __shared__ c32 smem[];
@@ -881,6 +901,8 @@ __global__ __launch_bounds__(256) void k_band_image(const float2* __restrict__ I
   const int p = slot % P;
   const int img = (slot / P) * kXcds + L % kXcds;
   if (img >= nimg) return;  // whole work-group, before any barrier
+  // the band this image comes from (several conditions may share one)
+  const int ib = FID && map.src ? (img / map.nplanes) * map.nd + map.src[img % map.nplanes] : img;
   const int tid = threadIdx.x;
   // Class-indexed tables: lane c of a phase-2 wave reads consecutive entries.
   for (int i = tid; i < F * C; i += 256) twh[i] = tw_lookup<+1>(tw_n, (i / C) * (i % C));
@@ -906,7 +928,7 @@ __global__ __launch_bounds__(256) void k_band_image(const float2* __restrict__ I
     // lanes past the band fold a valid column and store nothing, so every
     // lane of a wave takes part in the swap
     const int gxa = col ? gx : G;
-    const __amdgpu_buffer_rsrc_t br = box_rsrc(Ib + (size_t)img * nk * (G + 1), nk * (G + 1));
+    const __amdgpu_buffer_rsrc_t br = box_rsrc(Ib + (size_t)ib * nk * (G + 1), nk * (G + 1));
     int vo = (gxa + H * hi * (G + 1)) * (int)sizeof(float2);
     c32 u[H];
 #pragma unroll
@@ -1061,11 +1083,23 @@ __global__ __launch_bounds__(256) void k_band_image(const float2* __restrict__ I
       if (ch.reg) chain_task<true>(ch.beta, d, C, va, vb, mrc, rrc, orc);
       else chain_task<false>(ch.beta, d, C, va, vb, mrc, rrc, orc);
     } else if constexpr (!FID) {
+      auto store = [&](__amdgpu_buffer_rsrc_t rc) {
 #pragma unroll
-      for (int i = 0; i < F; ++i) {
-        const int so = C * i * (int)sizeof(float);
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d[i].re), orc, va, so, 2);
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d[i].im), orc, vb, so, 2);
+        for (int i = 0; i < F; ++i) {
+          const int so = C * i * (int)sizeof(float);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d[i].re), rc, va, so, 2);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d[i].im), rc, vb, so, 2);
+        }
+      };
+      if (!map.src) {
+        store(orc);
+      } else {
+        // every plane with this image (map.list, by distinct image)
+        const int clip = img / map.nd, u = img % map.nd;
+        for (int t = map.off[u]; t < map.off[u + 1]; ++t)
+          store(__builtin_amdgcn_make_buffer_rsrc(
+              out + ((size_t)clip * map.nplanes + map.list[t]) * n * n, (short)0,
+              n * n * (int)sizeof(float), 0x00020000));
       }
     } else {
       // the fidelity term of each pixel instead of the pixel (G = dC/dI in
@@ -1209,8 +1243,8 @@ hipError_t launch_cols_band_c(int n, int n1, int B, int BB, int nclips, const fl
 }
 
 template <int M, int XNB, int XS = 1>
-static hipError_t fields_m(int nclips, int nplanes, int Kmax, int S, const float2* kern,
-                           const float* lam, const float2* Mq, const float2* tw_m, float* coarse,
+static hipError_t fields_m(int nclips, int nplanes, const PlaneStack* stacks, int total, int S,
+                           const float2* kern, const float2* Mq, const float2* tw_m, float* coarse,
                            hipStream_t s) {
   using C = CoarseCfg<M, XS>;
   // the two-lane x pass needs every column in [-1, W)
@@ -1222,23 +1256,24 @@ static hipError_t fields_m(int nclips, int nplanes, int Kmax, int S, const float
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   if (attr != hipSuccess) return attr;
   const int groups = (nclips + kXcds - 1) / kXcds;
-  HUV_LAUNCH(kernel, dim3(groups * kXcds * C::Q * S), dim3(C::THREADS), shmem, s, Mq, kern, lam,
-             nclips, nplanes, Kmax, S, tw_m, coarse);
+  HUV_LAUNCH(kernel, dim3(groups * kXcds * C::Q * S * nplanes), dim3(C::THREADS), shmem, s, Mq, kern,
+             nclips, nplanes, stacks, total, S, tw_m, coarse);
 }
 
 template <int M>
-static hipError_t fields_x(int xnb, int xlanes, int nclips, int nplanes, int Kmax, int S,
-                           const float2* kern, const float* lam, const float2* Mq,
+static hipError_t fields_x(int xnb, int xlanes, int nclips, int nplanes,
+                           const PlaneStack* stacks, int total, int S, const float2* kern,
+                           const float2* Mq,
                            const float2* tw_m, float* coarse, hipStream_t s) {
   if (!xlanes) xlanes = fields_lanes_default(M);
   if (!xnb) xnb = xlanes == 2 ? kFieldsXnbDefault2 : kFieldsXnbDefault;
   switch (xlanes * 100 + xnb) {
-    case 104: return fields_m<M, 4>(nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 106: return fields_m<M, 6>(nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 108: return fields_m<M, 8>(nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 204: return fields_m<M, 4, 2>(nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 206: return fields_m<M, 6, 2>(nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 208: return fields_m<M, 8, 2>(nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
+    case 104: return fields_m<M, 4>(nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 106: return fields_m<M, 6>(nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 108: return fields_m<M, 8>(nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 204: return fields_m<M, 4, 2>(nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 206: return fields_m<M, 6, 2>(nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 208: return fields_m<M, 8, 2>(nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1247,11 +1282,11 @@ int fields_lanes_default(int m) { return m >= 64 ? 2 : 1; }
 
 bool fields_lanes_supported(int m, int xlanes) { return xlanes == 1 || (xlanes == 2 && m >= 64); }
 
-int fields_splits(int m, int nclips, int Kmax) {
+int fields_splits(int m, int images, int Kmax) {
   const int Q = coarse_classes(m);
   if (Q <= 0 || Kmax <= 1) return 1;
   // small batches: deal the kernels over more work-groups (about 512 busy ones)
-  const int wgs = nclips * Q;
+  const int wgs = images * Q;
   int S = (512 + wgs - 1) / wgs;
   if (S <= 1) return 1;
   if (S > Kmax) S = Kmax;
@@ -1259,16 +1294,17 @@ int fields_splits(int m, int nclips, int Kmax) {
   return (Kmax + ks - 1) / ks;  // every split non-empty
 }
 
-hipError_t launch_socs_fields(int m, int xnb, int xlanes, int nclips, int nplanes, int Kmax, int S,
-                              const float2* kern, const float* lam, const float2* Mq,
+hipError_t launch_socs_fields(int m, int xnb, int xlanes, int nclips, int nplanes,
+                              const PlaneStack* stacks, int total, int S, const float2* kern,
+                              const float2* Mq,
                               const float2* tw_m, float* coarse, hipStream_t s) {
-  if (S < 1 || S > Kmax) return hipErrorInvalidValue;
+  if (S < 1 || total < 1 || !stacks) return hipErrorInvalidValue;
   switch (m) {
-    case 32: return fields_x<32>(xnb, xlanes, nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 64: return fields_x<64>(xnb, xlanes, nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 128: return fields_x<128>(xnb, xlanes, nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 192: return fields_x<192>(xnb, xlanes, nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
-    case 256: return fields_x<256>(xnb, xlanes, nclips, nplanes, Kmax, S, kern, lam, Mq, tw_m, coarse, s);
+    case 32: return fields_x<32>(xnb, xlanes, nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 64: return fields_x<64>(xnb, xlanes, nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 128: return fields_x<128>(xnb, xlanes, nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 192: return fields_x<192>(xnb, xlanes, nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
+    case 256: return fields_x<256>(xnb, xlanes, nclips, nplanes, stacks, total, S, kern, Mq, tw_m, coarse, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1357,8 +1393,8 @@ hipError_t launch_coarse_cols(int m, int B, int nimg, float flare, const float2*
 
 template <int TMIN, int TMAX, int MODE>
 static hipError_t band_image_t(int n, int G, int nimg, const float2* Ib, const float2* tw_n,
-                               float* out, const FidelityEpi& epi, const ChainEpi& ch,
-                               hipStream_t s) {
+                               float* out, const PlaneMap& map, const FidelityEpi& epi,
+                               const ChainEpi& ch, hipStream_t s) {
   constexpr int UP = 32 * (-TMIN) + 1, NT = TMAX - TMIN + 1;
   auto bytes = [](int nn) { return ((size_t)32 * UP + (size_t)(32 + NT) * (nn / 32)) * sizeof(c32); };
   const size_t shmem = bytes(n);
@@ -1369,38 +1405,42 @@ static hipError_t band_image_t(int n, int G, int nimg, const float2* Ib, const f
   if (attr != hipSuccess) return attr;
   const int groups = (nimg + kXcds - 1) / kXcds;
   HUV_LAUNCH(kern, dim3(groups * kXcds * (n / 32)), dim3(256), shmem, s, Ib, n, G, nimg, tw_n,
-             out, epi, ch);
+             out, map, epi, ch);
 }
 
 template <int MODE>
 static hipError_t band_image_g(int n, int G, int nimg, const float2* Ib, const float2* tw_n,
-                               float* out, const FidelityEpi& epi, const ChainEpi& ch,
-                               hipStream_t s) {
+                               float* out, const PlaneMap& map, const FidelityEpi& epi,
+                               const ChainEpi& ch, hipStream_t s) {
   if (n < 256 || n > 2048 || (n & (n - 1)) != 0 || G < 0 || G > 255 || 2 * G + 1 > n)
     return hipErrorInvalidValue;
-  if (G <= 31) return band_image_t<-1, 0, MODE>(n, G, nimg, Ib, tw_n, out, epi, ch, s);
-  if (G <= 63) return band_image_t<-2, 1, MODE>(n, G, nimg, Ib, tw_n, out, epi, ch, s);
-  if (G <= 95) return band_image_t<-3, 2, MODE>(n, G, nimg, Ib, tw_n, out, epi, ch, s);
-  if (G <= 127) return band_image_t<-4, 3, MODE>(n, G, nimg, Ib, tw_n, out, epi, ch, s);
+  if (G <= 31) return band_image_t<-1, 0, MODE>(n, G, nimg, Ib, tw_n, out, map, epi, ch, s);
+  if (G <= 63) return band_image_t<-2, 1, MODE>(n, G, nimg, Ib, tw_n, out, map, epi, ch, s);
+  if (G <= 95) return band_image_t<-3, 2, MODE>(n, G, nimg, Ib, tw_n, out, map, epi, ch, s);
+  if (G <= 127) return band_image_t<-4, 3, MODE>(n, G, nimg, Ib, tw_n, out, map, epi, ch, s);
   return hipErrorInvalidValue;
 }
 
 hipError_t launch_band_image(int n, int G, int nimg, const float2* Ib, const float2* tw_n,
-                             float* out, hipStream_t s) {
-  return band_image_g<0>(n, G, nimg, Ib, tw_n, out, FidelityEpi{}, ChainEpi{}, s);
+                             float* out, const PlaneMap& map, hipStream_t s) {
+  if (map.src && (map.nd < 1 || map.nplanes < 1 || !map.off || !map.list || nimg % map.nd != 0))
+    return hipErrorInvalidValue;
+  return band_image_g<0>(n, G, nimg, Ib, tw_n, out, map, FidelityEpi{}, ChainEpi{}, s);
 }
 
 hipError_t launch_band_image_fidelity(int n, int G, int nimg, const float2* Ib,
-                                      const float2* tw_n, const FidelityEpi& epi, hipStream_t s) {
-  if (!epi.target || !epi.dose || !epi.partial || epi.ncond < 1 || nimg % epi.ncond != 0)
+                                      const float2* tw_n, const PlaneMap& map,
+                                      const FidelityEpi& epi, hipStream_t s) {
+  if (!epi.target || !epi.dose || !epi.partial || epi.ncond < 1 || nimg % epi.ncond != 0 ||
+      (map.src && (map.nd < 1 || map.nplanes != epi.ncond)))
     return hipErrorInvalidValue;
-  return band_image_g<1>(n, G, nimg, Ib, tw_n, nullptr, epi, ChainEpi{}, s);
+  return band_image_g<1>(n, G, nimg, Ib, tw_n, nullptr, map, epi, ChainEpi{}, s);
 }
 
 hipError_t launch_band_image_chain(int n, int G, int nimg, const float2* Ib, const float2* tw_n,
                                    const ChainEpi& ch, hipStream_t s) {
   if (!ch.m || !ch.grad) return hipErrorInvalidValue;
-  return band_image_g<2>(n, G, nimg, Ib, tw_n, nullptr, FidelityEpi{}, ch, s);
+  return band_image_g<2>(n, G, nimg, Ib, tw_n, nullptr, PlaneMap{}, FidelityEpi{}, ch, s);
 }
 
 }  // namespace huvk

@@ -46,16 +46,24 @@ hipError_t launch_rows_band_c(int n, int n1, int B, int nclips, const float2* ma
 hipError_t launch_cols_band_c(int n, int n1, int B, int BB, int nclips, const float2* tmp,
                               const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                               hipStream_t s);
-// kern: [Q][nplanes][Kmax] boxes (W = 2 coarse_band(m) + 1, Q = m / 32; copy q
-// multiplied by e^{2 pi i kx q / m}), lam: [nplanes][Kmax]; Mq: one box per
-// clip; coarse: [nclips][nplanes][m][Q][32], row y, column x = Q j + q at
+// One plane's kernels in a stack: `count` boxes from `first`, the `negative`
+// ones first with negative eigenvalues; box k is scaled by
+// sqrt(|eigenvalue_k| / scale) (eigenvalues over n^4).
+struct PlaneStack {
+  int first, count, negative;
+  float scale;
+};
+// kern: [Q][total] boxes (W = 2 coarse_band(m) + 1, Q = m / 32; copy q
+// multiplied by e^{2 pi i kx q / m}), stacks: device array of nplanes; Mq: one
+// box per clip; coarse: [nclips][nplanes][m][Q][32], row y, column x = Q j + q at
 // [y][q][j] (class-major).  Boxes are W x W ([kx + BB][ky + BB])
 // for xlanes = 1 and column-paired (W + 1) x W (launch_cols_band's Mp) for 2.
 // S kernel splits (fields_splits): coarse then holds S partial image sets,
 // [S][nclips][nplanes][m][m], summed by launch_coarse_rows.
-int fields_splits(int m, int nclips, int Kmax);
-hipError_t launch_socs_fields(int m, int xnb, int xlanes, int nclips, int nplanes, int Kmax, int S,
-                              const float2* kern, const float* lam, const float2* Mq,
+int fields_splits(int m, int images, int Kmax);
+hipError_t launch_socs_fields(int m, int xnb, int xlanes, int nclips, int nplanes,
+                              const PlaneStack* stacks, int total, int S, const float2* kern,
+                              const float2* Mq,
                               const float2* tw_m, float* coarse, hipStream_t s);
 hipError_t launch_coarse_rows(int m, int B, int nimg, int S, const float* coarse,
                               const float2* tw_m, float2* tmp1, hipStream_t s);
@@ -66,9 +74,20 @@ hipError_t launch_coarse_cols(int m, int B, int nimg, float flare, const float2*
 bool coarse_fused_supported(int m);
 hipError_t launch_coarse_fused(int m, int B, int nimg, int S, const float* coarse, float flare,
                                const float2* tw_m, float2* Ib, hipStream_t s);
-// Ib: [nimg][2G+1][G+1] Hermitian half band (gy + G, gx).
+// Planes that share images: `nplanes` planes of a clip have `nd` distinct
+// images; plane p shows image src[p], and image u belongs to the planes
+// list[off[u]] .. list[off[u + 1] - 1] (device arrays; src null: each plane
+// has its own).
+struct PlaneMap {
+  int nplanes = 1, nd = 1;
+  const int* src = nullptr;
+  const int* off = nullptr;
+  const int* list = nullptr;
+};
+// Ib: [nimg][2G+1][G+1] Hermitian half band (gy + G, gx).  With a map, nimg
+// counts distinct images ([clip][nd]) and out holds [clip][nplanes].
 hipError_t launch_band_image(int n, int G, int nimg, const float2* Ib, const float2* tw_n,
-                             float* out, hipStream_t s);
+                             float* out, const PlaneMap& map, hipStream_t s);
 
 // The ILT fidelity term evaluated where band_image would store the image
 // (images img = target * ncond + condition): r = sigma(steepness (dose I -
@@ -86,8 +105,11 @@ struct FidelityEpi {
   float* G = nullptr;
   double* partial = nullptr;
 };
+// With a map (over the conditions), nimg still counts (target, condition)
+// images and Ib holds [target][nd].
 hipError_t launch_band_image_fidelity(int n, int G, int nimg, const float2* Ib,
-                                      const float2* tw_n, const FidelityEpi& epi, hipStream_t s);
+                                      const float2* tw_n, const PlaneMap& map,
+                                      const FidelityEpi& epi, hipStream_t s);
 
 // The ILT chain rule evaluated where band_image would store the image: image
 // j is dC/dm of ILT row j, and row (orows ? orows[j] : j) of grad receives

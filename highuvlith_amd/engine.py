@@ -276,6 +276,24 @@ def build_kernel_set(optics, points, grid, defocus_nm, wavelength_nm, max_kernel
     return _take_kernel_set(lib, h, grid, defocus_nm, wavelength_nm)
 
 
+def real_fields(ks):
+    """The real fields of a SparseKernelSet on masks with a real transmittance:
+    Hermitian functions (R, 2B+1, 2B+1) [kx + B][ky + B] with sum_k lambda_k |E_k|^2 =
+    sum_j v_j^2 (eigenvalues normalised); R = 0 where the set has no such form."""
+    lib = _lib.load()
+    eig = np.ascontiguousarray(ks.eigenvalues / ks.normalization_divisor)
+    vals = np.ascontiguousarray(np.stack([ks.values.real, ks.values.imag], -1))
+    sup = np.ascontiguousarray(ks.support, dtype=np.int64)
+    band, count = C.c_int(), C.c_int()
+    args = (ks.n, ks.num_kernels, len(sup), i64ptr(sup), dptr(eig), dptr(vals))
+    check(lib.huv_real_fields(*args, 0, None, C.byref(band), C.byref(count)))
+    w = 2 * band.value + 1
+    out = np.zeros((count.value, w, w, 2))
+    if count.value:
+        check(lib.huv_real_fields(*args, count.value, dptr(out), C.byref(band), C.byref(count)))
+    return out[..., 0] + 1j * out[..., 1]
+
+
 def build_kernel_sets_device(ctx, optics, points, grid, defocus_nm, wavelength_nm, max_kernels,
                              kernel_energy_fraction=1.0, method=None):
     """Kernel sets of several focus planes with the TCC factor, its Gram product

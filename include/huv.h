@@ -124,6 +124,18 @@ huv_status huv_kernels_copy(const huv_host_kernels* ks, int64_t* support, int64_
                             double* eigenvalues, double* values);
 void huv_kernels_free(huv_host_kernels* ks);
 
+/* The real fields of a kernel set on masks with a real transmittance (no
+ * counterpart in the reference): sum_k lambda_k |E_k|^2 = sum_j v_j^2, each v_j
+ * the field of a Hermitian function on the box |kx|, |ky| <= band; what the
+ * device images real masks with where two fields to a transform are fewer than
+ * num_kernels.  Arguments as huv_kset_upload.  *count = number of fields (0
+ * where the set has no such form), *band = box half-width; `fields` receives
+ * up to `capacity` boxes [j][kx + band][ky + band] of interleaved complex
+ * (NULL with capacity 0 to size the buffer). */
+huv_status huv_real_fields(int n, int num_kernels, int64_t num_support, const int64_t* support,
+                           const double* eigenvalues, const double* values, int64_t capacity,
+                           double* fields, int* band, int* count);
+
 /* Rasterise painted rectangles (later ones win) over a background with exact
  * area coverage (mask.rs:590, 1365-1571).  rects: nrects x (x, y, w, h, re, im);
  * out: n x n interleaved complex. */
