@@ -541,26 +541,55 @@ struct CoarseFft {
 };
 
 // ---------------------------------------------------------------------------
-// coarse_rows: coarse row pairs -> FFT_M forward, keep gx in [0, G] and
-// [M - G, M) (G = 2B).  tmp1 layout [img][kk][pair] with kk in [0, 2G].
-// ---------------------------------------------------------------------------
 // coarse[i] = sum_j coarse[j * count + i], j = 0 .. S-1 in order (float4 lanes).
-__global__ void k_sum_splits(float* __restrict__ coarse, int S, int64_t count4) {
+// Latency-bound for the few images that are split at all: the partials of U
+// splits are requested before the first is added, and a work-group is one wave,
+// so a single 64^2 image uses 16 CUs (18 splits: 8.0 -> 3.6 us; four work-groups
+// of 256 threads added one load at a time).
+// ---------------------------------------------------------------------------
+template <int U>
+__global__ __launch_bounds__(64) void k_sum_splits(float* __restrict__ coarse, int S,
+                                                   int64_t count4) {
   float4* c4 = reinterpret_cast<float4*>(coarse);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count4;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    float4 v = c4[i];
-    for (int j = 1; j < S; ++j) {
-      const float4 w = c4[j * count4 + i];
-      v.x += w.x;
-      v.y += w.y;
-      v.z += w.z;
-      v.w += w.w;
+  for (int64_t i = blockIdx.x * (int64_t)64 + threadIdx.x; i < count4;
+       i += (int64_t)gridDim.x * 64) {
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j0 = 0; j0 < S; j0 += U) {
+      float4 w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = c4[min(j0 + u, S - 1) * count4 + i];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // a select, not a branch that the load would sink into
+        const bool on = j0 + u < S;
+        v.x += on ? w[u].x : 0.f;
+        v.y += on ? w[u].y : 0.f;
+        v.z += on ? w[u].z : 0.f;
+        v.w += on ? w[u].w : 0.f;
+      }
     }
     c4[i] = v;
   }
 }
 
+static hipError_t sum_splits(float* coarse, int S, int64_t count, hipStream_t s) {
+  if (S <= 1) return hipSuccess;
+  const int64_t count4 = count / 4;  // M^2 is a multiple of 4
+  const int blocks = (int)std::min<int64_t>((count4 + 63) / 64, 16384);
+  // all of a row's partials in one round of requests where they fit
+  if (S <= 8)
+    hipLaunchKernelGGL(k_sum_splits<8>, dim3(blocks), dim3(64), 0, s, coarse, S, count4);
+  else if (S <= 16)
+    hipLaunchKernelGGL(k_sum_splits<16>, dim3(blocks), dim3(64), 0, s, coarse, S, count4);
+  else
+    hipLaunchKernelGGL(k_sum_splits<32>, dim3(blocks), dim3(64), 0, s, coarse, S, count4);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// coarse_rows: coarse row pairs -> FFT_M forward, keep gx in [0, G] and
+// [M - G, M) (G = 2B).  tmp1 layout [img][kk][pair] with kk in [0, 2G].
+// ---------------------------------------------------------------------------
 template <int M, int TEAMS>
 __global__ __launch_bounds__(TEAMS * CoarseFft<M>::N2) void k_coarse_rows(
     const float* __restrict__ coarse, int B, const float2* __restrict__ tw_m,
@@ -1314,15 +1343,9 @@ static hipError_t coarse_rows_m(int B, int nimg, int S, const float* coarse, con
                                 float2* tmp1, hipStream_t s) {
   constexpr int TEAMS = 256 / CoarseFft<M>::N2;
   dim3 grid((M / 2 + TEAMS - 1) / TEAMS, nimg);
-  if (S > 1) {
-    // fold the kernel-split partials into the first set (M^2 is a multiple of 4)
-    const int64_t count4 = (int64_t)nimg * M * M / 4;
-    const int blocks = (int)std::min<int64_t>((count4 + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_sum_splits, dim3(blocks), dim3(256), 0, s, const_cast<float*>(coarse), S,
-                       count4);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
+  // fold the kernel-split partials into the first set
+  const hipError_t e = sum_splits(const_cast<float*>(coarse), S, (int64_t)nimg * M * M, s);
+  if (e != hipSuccess) return e;
   HUV_LAUNCH((k_coarse_rows<M, TEAMS>), grid, dim3(256), 0, s, coarse, B, tw_m, tmp1);
 }
 
@@ -1342,14 +1365,8 @@ hipError_t launch_coarse_rows(int m, int B, int nimg, int S, const float* coarse
 template <int M, int THREADS>
 static hipError_t coarse_fused_m(int B, int nimg, int S, const float* coarse, float flare,
                                  const float2* tw_m, float2* Ib, hipStream_t s) {
-  if (S > 1) {
-    const int64_t count4 = (int64_t)nimg * M * M / 4;
-    const int blocks = (int)std::min<int64_t>((count4 + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_sum_splits, dim3(blocks), dim3(256), 0, s, const_cast<float*>(coarse), S,
-                       count4);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
+  const hipError_t e = sum_splits(const_cast<float*>(coarse), S, (int64_t)nimg * M * M, s);
+  if (e != hipSuccess) return e;
   constexpr size_t shmem = (size_t)(M / 2) * (M + 1) * sizeof(c32);
   auto kern = k_coarse_fused<M, THREADS>;
   static const hipError_t attr = hipFuncSetAttribute(
