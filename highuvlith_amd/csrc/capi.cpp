@@ -229,6 +229,12 @@ Ctx::~Ctx() {
   if (pin_h) hipHostFree(pin_h);
   if (pin_d) hipFree(pin_d);
   if (dl_h) hipHostFree(dl_h);
+  for (FeatureSlot& f : feature_slots) {
+    if (f.busy) hipEventSynchronize(f.done);
+    if (f.done) hipEventDestroy(f.done);
+    if (f.h) hipHostFree(f.h);
+    if (f.d) hipFree(f.d);
+  }
   if (own_stream) hipStreamDestroy(own_stream);
 }
 
@@ -251,6 +257,30 @@ bool Ctx::staging(size_t bytes, hipError_t& e) {
   }
   pin_cap = bytes;
   return true;
+}
+
+Ctx::FeatureSlot* Ctx::feature_slot(size_t bytes, hipError_t& e) {
+  FeatureSlot& f = feature_slots[feature_next];
+  feature_next ^= 1;
+  e = hipSuccess;
+  if (!f.done) e = hipEventCreateWithFlags(&f.done, hipEventDisableTiming);
+  if (e == hipSuccess && f.busy) e = hipEventSynchronize(f.done);
+  if (e != hipSuccess) return nullptr;
+  f.busy = false;
+  if (bytes <= f.cap) return &f;
+  if (f.h) hipHostFree(f.h);
+  if (f.d) hipFree(f.d);
+  f.h = f.d = nullptr;
+  f.cap = 0;
+  e = hipHostMalloc((void**)&f.h, bytes, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipMalloc((void**)&f.d, bytes);
+  if (e != hipSuccess) {
+    if (f.h) hipHostFree(f.h);
+    f.h = f.d = nullptr;
+    return nullptr;
+  }
+  f.cap = bytes;
+  return &f;
 }
 
 bool Ctx::download_area(size_t bytes, hipError_t& e) {
@@ -520,6 +550,16 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   std::vector<int64_t> coff((size_t)nclips + 1, 0), eoff((size_t)nclips + 1, 0);
   std::vector<huv::RectFeature> fs;
   std::vector<huv::RectCell> cl;
+  // The call's cell limit counts the cells of one grid per clip: where these
+  // could reach it, the clips are resolved that way.
+  double bound = 0.0;
+  for (int i = 0; i < nclips; ++i) {
+    const double r = 2.0 * (double)(rb.offsets[i + 1] - rb.offsets[i]) + 1.0;
+    bound += r * r;
+  }
+  const bool whole = bound > (double)kRectMaxCells;
+  std::vector<std::array<double, 4>> boxes;
+  std::vector<Pt> v;
   const double half = n * rb.pixel_nm / 2.0;
   // overlaps of at most 1e-9 of the field length count as none (mask.rs:838-841,1099-1108)
   const double eps = 1e-9 * (2.0 * half);
@@ -533,7 +573,7 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
       fs.push_back({q[0], q[1], q[2], q[3], huv::cd(q[4], q[5])});
     }
     const huv::cd bg(rb.background[2 * i], rb.background[2 * i + 1]);
-    if (!huv::resolve_rect_cells(fs, bg, n, rb.pixel_nm, kRectMaxGrid, cl))
+    if (!huv::resolve_rect_cells(fs, bg, n, rb.pixel_nm, kRectMaxGrid, cl, whole))
       return fail(HUV_INVALID_PARAMETER,
                   "clip " + std::to_string(i) + ": more than 2^20 edge-grid cells; rasterise it instead");
     for (const auto& e : cl) cells.insert(cells.end(), {e.x0, e.x1, e.y0, e.y1, e.w.real(), e.w.imag()});
@@ -541,7 +581,7 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
     if (coff[i + 1] > kRectMaxCells) return fail(HUV_INVALID_PARAMETER, "too many rectangle cells in one call");
     if (rb.polys) {
       // bounding boxes of the clip's features, for the overlap rule
-      std::vector<std::array<double, 4>> boxes;
+      boxes.clear();
       for (const auto& f : fs) {
         if (!(f.w > 0 && f.h > 0)) continue;
         const double x0 = std::max(f.x - f.w / 2, -half), x1 = std::min(f.x + f.w / 2, half);
@@ -550,15 +590,18 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
       }
       const huv_polygons& P = *rb.polys;
       for (int64_t j = P.poly_offsets[i]; j < P.poly_offsets[i + 1]; ++j) {
-        std::vector<Pt> v;
-        for (int64_t k = P.vertex_offsets[j]; k < P.vertex_offsets[j + 1]; ++k)
+        v.clear();
+        bool inside = true;  // the clip then keeps the polygon as it is
+        for (int64_t k = P.vertex_offsets[j]; k < P.vertex_offsets[j + 1]; ++k) {
           v.push_back({P.vertices[2 * k], P.vertices[2 * k + 1]});
+          inside = inside && std::fabs(v.back().first) <= half && std::fabs(v.back().second) <= half;
+        }
         if (v.size() < 3) continue;
         if (!polygon_simple(v))
           return fail(HUV_INVALID_PARAMETER, "clip " + std::to_string(i) + ", polygon " +
                                                  std::to_string(j - P.poly_offsets[i]) +
                                                  ": edges cross; rasterise it instead");
-        v = clip_polygon(v, half);
+        if (!inside) v = clip_polygon(v, half);
         if (v.empty()) continue;
         double twice = 0.0;
         std::array<double, 4> bb{v[0].first, v[0].first, v[0].second, v[0].second};
@@ -602,24 +645,33 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   const size_t pdc_b = nedges > 0 ? pdc.size() * sizeof(double) : 0;
   const size_t bytes = cell_b + off_b + bg_b + edge_b + eoff_b + pdc_b;
   hipError_t e;
-  // the staging area may still feed an earlier copy on the stream
-  e = hipStreamSynchronize(c->stream());
-  if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-  if (!c->staging(bytes, e)) return hip_fail(e, "staging buffer");
-  if (cell_b) std::memcpy(c->pin_h, cells.data(), cell_b);
-  std::memcpy(c->pin_h + cell_b, coff.data(), off_b);
-  std::memcpy(c->pin_h + cell_b + off_b, rb.background, bg_b);
-  char* ph = c->pin_h + cell_b + off_b + bg_b;
+  // per-call geometry is not recorded into a caller's graph
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  e = hipStreamIsCapturing(c->stream(), &cap);
+  if (e == hipSuccess && cap != hipStreamCaptureStatusNone) e = hipErrorStreamCaptureUnsupported;
+  if (e != hipSuccess) return hip_fail(e, "feature upload");
+  Ctx::FeatureSlot* slot = c->feature_slot(bytes, e);
+  if (!slot) return hip_fail(e, "staging buffer");
+  if (cell_b) std::memcpy(slot->h, cells.data(), cell_b);
+  std::memcpy(slot->h + cell_b, coff.data(), off_b);
+  std::memcpy(slot->h + cell_b + off_b, rb.background, bg_b);
+  char* ph = slot->h + cell_b + off_b + bg_b;
   if (nedges > 0) {
     std::memcpy(ph, edges.data(), edge_b);
     std::memcpy(ph + edge_b, eoff.data(), eoff_b);
     std::memcpy(ph + edge_b + eoff_b, pdc.data(), pdc_b);
   }
-  e = hipMemcpyAsync(c->pin_d, c->pin_h, bytes, hipMemcpyHostToDevice, c->stream());
+  e = hipMemcpyAsync(slot->d, slot->h, bytes, hipMemcpyHostToDevice, c->stream());
   if (e != hipSuccess) return hip_fail(e, "rectangle upload");
-  const double* d_cells = (const double*)c->pin_d;
-  const int64_t* d_coff = (const int64_t*)(c->pin_d + cell_b);
-  const double* d_bg = (const double*)(c->pin_d + cell_b + off_b);
+  // whatever returns from here on has queued the copy at least
+  struct Mark {
+    Ctx::FeatureSlot* s;
+    hipStream_t st;
+    ~Mark() { s->busy = hipEventRecord(s->done, st) == hipSuccess; }
+  } mark{slot, c->stream()};
+  const double* d_cells = (const double*)slot->d;
+  const int64_t* d_coff = (const int64_t*)(slot->d + cell_b);
+  const double* d_bg = (const double*)(slot->d + cell_b + off_b);
   const int nk = 2 * B + 1;
   double2* X = nullptr;
   double2* Y = nullptr;
@@ -639,7 +691,7 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   if (e != hipSuccess) return hip_fail(e, "rect_band launch");
   c->stage_end(ST_RECT_BAND, ev);
   if (nedges > 0) {
-    const char* pd = c->pin_d + cell_b + off_b + bg_b;
+    const char* pd = slot->d + cell_b + off_b + bg_b;
     c->stage_begin(ST_POLY_BAND, &ev);
     e = huvk::launch_poly_band((const double*)pd, (const int64_t*)(pd + edge_b),
                                (const double*)(pd + edge_b + eoff_b), nclips, n, L, B, BB, Mq, Mp,

@@ -81,6 +81,20 @@ struct Ctx {
   char* pin_d = nullptr;
   size_t pin_cap = 0;
   bool staging(size_t bytes, hipError_t& e);
+  // Staged feature geometry: two such pairs used in turn, each with an event
+  // after the last kernel that reads it, so a call plans and uploads while the
+  // previous call's images are still computed.
+  struct FeatureSlot {
+    char* h = nullptr;
+    char* d = nullptr;
+    size_t cap = 0;
+    hipEvent_t done = nullptr;
+    bool busy = false;
+  };
+  FeatureSlot feature_slots[2];
+  int feature_next = 0;
+  // The next slot with room for `bytes`, its earlier use finished.
+  FeatureSlot* feature_slot(size_t bytes, hipError_t& e);
   // Pinned, device-mapped host buffer for small per-step downloads (the ILT
   // driver's reduction and cost partials, which its kernels write there
   // directly through dl_d), grown on demand.

@@ -51,24 +51,33 @@ __global__ __launch_bounds__(256) void k_rect_tables(const double* __restrict__ 
   Y[idx] = ya;
 }
 
-// One thread per tile of kRectT consecutive rows (ky + BB) x kRectT consecutive
+// A lane takes a tile of kRectT consecutive rows (ky + BB) x kRectT consecutive
 // columns (kx + BB), row tiles fastest: per cell it loads kRectT row and
-// kRectT column coefficients for kRectT^2 products.  Work-groups
-// [clip * bpc, (clip + 1) * bpc) cover one clip's box.
+// kRectT column coefficients for kRectT^2 products.  The SL waves of a
+// work-group share its 64 tiles and take every SL-th cell each, the next cell's
+// coefficients requested before the current one's products; their sums are
+// added in a fixed tree.  Work-groups [clip * gpc, (clip + 1) * gpc) cover one
+// clip's box.  A chain of loads over the cells bounds a small batch (one clip,
+// 100 cells, B = 13: 50 us with one wave a tile group and no request ahead,
+// 7.5 us so), so it takes eight waves; a full chip takes two (96 clips of 43
+// cells, B = 47: 25.6 us).
 constexpr int kRectT = 4;
 
-__global__ __launch_bounds__(256) void k_rect_band(const double2* __restrict__ X,
-                                                   const double2* __restrict__ Y,
-                                                   const int64_t* __restrict__ coff,
-                                                   const double* __restrict__ bg, int n, int B,
-                                                   int BB, int bpc, float2* __restrict__ Mq,
-                                                   float2* __restrict__ Mp) {
+template <int SL>
+__global__ __launch_bounds__(64 * SL) void k_rect_band(const double2* __restrict__ X,
+                                                       const double2* __restrict__ Y,
+                                                       const int64_t* __restrict__ coff,
+                                                       const double* __restrict__ bg, int n, int B,
+                                                       int BB, int gpc, float2* __restrict__ Mq,
+                                                       float2* __restrict__ Mp) {
+  __shared__ double red[SL / 2][2 * kRectT * kRectT][64];
   const int W = 2 * BB + 1, nk = 2 * B + 1;
   const int G = (W + kRectT - 1) / kRectT;
-  const int clip = blockIdx.x / bpc;
-  const int t = (blockIdx.x - clip * bpc) * blockDim.x + threadIdx.x;
-  if (t >= G * G) return;
-  const int gc = t / G, gr = t - gc * G;
+  const int clip = blockIdx.x / gpc;
+  const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
+  const int t = (blockIdx.x - clip * gpc) * 64 + lane;
+  const bool tile = t < G * G;
+  const int gc = tile ? t / G : 0, gr = tile ? t - gc * G : 0;
   int xi[kRectT], yi[kRectT];
   bool xl[kRectT], yl[kRectT];
 #pragma unroll
@@ -85,26 +94,60 @@ __global__ __launch_bounds__(256) void k_rect_band(const double2* __restrict__ X
   for (int i = 0; i < kRectT; ++i)
 #pragma unroll
     for (int j = 0; j < kRectT; ++j) re[i][j] = im[i][j] = 0.0;
-  const int64_t c0 = coff[clip], c1 = coff[clip + 1];
-  const double2* xr = X + c0 * nk;
-  const double2* yr = Y + c0 * nk;
-  for (int64_t c = c0; c < c1; ++c, xr += nk, yr += nk) {
+  const int64_t c0 = coff[clip] + slice, c1 = coff[clip + 1];
+  if (c0 < c1) {
     double2 x[kRectT], y[kRectT];
-#pragma unroll
-    for (int j = 0; j < kRectT; ++j) {
-      x[j] = xr[xi[j]];
-      y[j] = yr[yi[j]];
-    }
-#pragma unroll
-    for (int i = 0; i < kRectT; ++i)
+    auto load = [&](int64_t c, double2* a, double2* b) {
 #pragma unroll
       for (int j = 0; j < kRectT; ++j) {
-        re[i][j] = fma(x[j].x, y[i].x, re[i][j]);
-        re[i][j] = fma(-x[j].y, y[i].y, re[i][j]);
-        im[i][j] = fma(x[j].x, y[i].y, im[i][j]);
-        im[i][j] = fma(x[j].y, y[i].x, im[i][j]);
+        a[j] = X[c * nk + xi[j]];
+        b[j] = Y[c * nk + yi[j]];
       }
+    };
+    load(c0, x, y);
+    for (int64_t c = c0; c < c1; c += SL) {
+      double2 xn[kRectT], yn[kRectT];
+      load(c + SL < c1 ? c + SL : c, xn, yn);
+#pragma unroll
+      for (int i = 0; i < kRectT; ++i)
+#pragma unroll
+        for (int j = 0; j < kRectT; ++j) {
+          re[i][j] = fma(x[j].x, y[i].x, re[i][j]);
+          re[i][j] = fma(-x[j].y, y[i].y, re[i][j]);
+          im[i][j] = fma(x[j].x, y[i].y, im[i][j]);
+          im[i][j] = fma(x[j].y, y[i].x, im[i][j]);
+        }
+#pragma unroll
+      for (int j = 0; j < kRectT; ++j) {
+        x[j] = xn[j];
+        y[j] = yn[j];
+      }
+    }
   }
+#pragma unroll
+  for (int h = SL / 2; h >= 1; h /= 2) {
+    if (slice >= h && slice < 2 * h) {
+#pragma unroll
+      for (int i = 0; i < kRectT; ++i)
+#pragma unroll
+        for (int j = 0; j < kRectT; ++j) {
+          red[slice - h][2 * (i * kRectT + j)][lane] = re[i][j];
+          red[slice - h][2 * (i * kRectT + j) + 1][lane] = im[i][j];
+        }
+    }
+    __syncthreads();
+    if (slice < h) {
+#pragma unroll
+      for (int i = 0; i < kRectT; ++i)
+#pragma unroll
+        for (int j = 0; j < kRectT; ++j) {
+          re[i][j] += red[slice][2 * (i * kRectT + j)][lane];
+          im[i][j] += red[slice][2 * (i * kRectT + j) + 1][lane];
+        }
+    }
+    __syncthreads();
+  }
+  if (slice != 0 || !tile) return;
   const double nn = (double)n * (double)n;
   float2* mq = Mq + (size_t)clip * W * W;
   float2* mp = Mp ? Mp + (size_t)clip * (W + 1) * W : nullptr;
@@ -303,10 +346,17 @@ hipError_t launch_rect_band(const double2* X, const double2* Y, const int64_t* c
   if (B < 0 || BB < B || BB > 1024) return hipErrorInvalidValue;
   const int W = 2 * BB + 1;
   const int G = (W + kRectT - 1) / kRectT;
-  const int bpc = (G * G + 255) / 256;
-  if ((int64_t)bpc * nclips >= (1ll << 31)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_rect_band, dim3((unsigned)(bpc * nclips)), dim3(256), 0, s, X, Y, coff,
-                     bg, n, B, BB, bpc, Mq, Mp);
+  const int gpc = (G * G + 63) / 64;
+  if ((int64_t)gpc * nclips >= (1ll << 31)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(gpc * nclips));
+  // Up to two work-groups per CU: eight waves each, else two (512 clips of 64
+  // cells, B = 47: 4608 work-groups fill the chip without more).
+  if (gpc * nclips <= 512)
+    hipLaunchKernelGGL(k_rect_band<8>, grid, dim3(512), 0, s, X, Y, coff, bg, n, B, BB, gpc, Mq,
+                       Mp);
+  else
+    hipLaunchKernelGGL(k_rect_band<2>, grid, dim3(128), 0, s, X, Y, coff, bg, n, B, BB, gpc, Mq,
+                       Mp);
   return hipGetLastError();
 }
 

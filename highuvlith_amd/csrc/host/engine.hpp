@@ -209,8 +209,10 @@ struct RectCell {
   cd w;
 };
 // Painter's-rule resolution of rectangles into disjoint cells (see the
-// definition); false when the edge grid would exceed max_cells cells.
+// definition); false when the edge grid would exceed max_cells cells.  whole:
+// on one grid over all edges, whose cells are the ones a call's limit counts.
 bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd background, int n,
-                        double pixel_nm, int64_t max_cells, std::vector<RectCell>& out);
+                        double pixel_nm, int64_t max_cells, std::vector<RectCell>& out,
+                        bool whole = false);
 
 }  // namespace huv

@@ -381,41 +381,49 @@ void rasterize_rects(const std::vector<RectFeature>& rects, cd bg, int n, double
 }
 
 // Disjoint cells of painted rectangles (mask.rs:1365-1424, compress): the
-// rectangles are clipped to the field, the field and rectangle edges are
-// merged within 1e-12 L, each rectangle paints its cells in order (the later
-// one wins), runs of equal value along x become one cell and consecutive
-// rows with identical content one row.  Cells equal to the background are
-// dropped; each cell keeps value - background.
-bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, double pixel,
-                        int64_t max_cells, std::vector<RectCell>& out) {
-  out.clear();
-  const double half = n * pixel / 2.0;
-  const double eps = 1e-12 * (2.0 * half);
-  struct R { double x0, x1, y0, y1; cd v; };
-  std::vector<R> rs;
-  for (const auto& f : rects) {
-    if (!(f.w > 0 && f.h > 0)) continue;
-    const double x0 = std::max(f.x - f.w / 2, -half), x1 = std::min(f.x + f.w / 2, half);
-    const double y0 = std::max(f.y - f.h / 2, -half), y1 = std::min(f.y + f.h / 2, half);
-    if (x1 - x0 <= 0 || y1 - y0 <= 0) continue;
-    rs.push_back({x0, x1, y0, y1, f.value});
+// rectangles are clipped to the field, their edges are merged within 1e-12 L,
+// each rectangle paints its cells in order (the later one wins), runs of equal
+// value along x become one cell and consecutive rows with identical content
+// one row.  Cells equal to the background are dropped; each cell keeps
+// value - background.
+//
+// The picture is resolved per group of overlapping rectangles, on that group's
+// own edges: a rectangle that meets no other is one cell whatever else the clip
+// holds, where a grid over all edges cuts it at every other rectangle's edges
+// (43 contacts of a jittered array: 43 cells instead of about 400, and a tenth of
+// the host time).  The limit on the whole clip's edge grid stays as it is.
+namespace {
+
+struct PaintRect {
+  double x0, x1, y0, y1;
+  int cls;  // index of its value; 0 is the background
+};
+
+// Cells of the rectangles g (painter order) on their own merged edges.
+void resolve_group(const std::vector<PaintRect>& g, const std::vector<cd>& values, double eps,
+                   std::vector<RectCell>& out) {
+  const cd bg = values[0];
+  if (g.size() == 1) {
+    if (g[0].cls) out.push_back({g[0].x0, g[0].x1, g[0].y0, g[0].y1, values[g[0].cls] - bg});
+    return;
   }
-  if (rs.empty()) return true;
-  std::vector<double> xe{-half, half}, ye{-half, half};
-  for (auto& r : rs) {
+  std::vector<double> xe, ye;
+  xe.reserve(2 * g.size());
+  ye.reserve(2 * g.size());
+  for (const auto& r : g) {
     xe.push_back(r.x0); xe.push_back(r.x1);
     ye.push_back(r.y0); ye.push_back(r.y1);
   }
   dedup(xe, eps);
   dedup(ye, eps);
   const int64_t nx = (int64_t)xe.size() - 1, ny = (int64_t)ye.size() - 1;
-  if (nx < 1 || ny < 1 || nx > max_cells / ny) return false;
-  std::vector<cd> cells((size_t)(nx * ny), bg);
-  for (auto& r : rs) {
-    const int64_t i0 = edge_index(ye, r.y0, eps), i1 = edge_index(ye, r.y1, eps);
-    const int64_t j0 = edge_index(xe, r.x0, eps), j1 = edge_index(xe, r.x1, eps);
-    for (int64_t i = i0; i < std::min(i1, ny); ++i)
-      for (int64_t j = j0; j < std::min(j1, nx); ++j) cells[i * nx + j] = r.v;
+  if (nx < 1 || ny < 1) return;
+  std::vector<int> cells((size_t)(nx * ny), 0);
+  for (const auto& r : g) {
+    const int64_t i0 = edge_index(ye, r.y0, eps), i1 = std::min(edge_index(ye, r.y1, eps), ny);
+    const int64_t j0 = edge_index(xe, r.x0, eps), j1 = std::min(edge_index(xe, r.x1, eps), nx);
+    for (int64_t i = i0; i < i1; ++i)
+      for (int64_t j = j0; j < j1; ++j) cells[i * nx + j] = r.cls;
   }
   int64_t i = 0;
   while (i < ny) {
@@ -425,13 +433,84 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
       ++k;
     int64_t j = 0;
     while (j < nx) {
-      const cd v = cells[i * nx + j];
+      const int v = cells[i * nx + j];
       int64_t e = j + 1;
       while (e < nx && cells[i * nx + e] == v) ++e;
-      if (v != bg) out.push_back({xe[j], xe[e], ye[i], ye[k], v - bg});
+      if (v) out.push_back({xe[j], xe[e], ye[i], ye[k], values[v] - bg});
       j = e;
     }
     i = k;
+  }
+}
+
+// Overlap groups are found pair by pair; clips of more rectangles are one group
+// (as is every clip with `whole`).
+constexpr size_t kGroupMaxRects = 2048;
+
+}  // namespace
+
+bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, double pixel,
+                        int64_t max_cells, std::vector<RectCell>& out, bool whole) {
+  out.clear();
+  const double half = n * pixel / 2.0;
+  const double eps = 1e-12 * (2.0 * half);
+  std::vector<PaintRect> rs;
+  std::vector<cd> values{bg};
+  rs.reserve(rects.size());
+  for (const auto& f : rects) {
+    if (!(f.w > 0 && f.h > 0)) continue;
+    const double x0 = std::max(f.x - f.w / 2, -half), x1 = std::min(f.x + f.w / 2, half);
+    const double y0 = std::max(f.y - f.h / 2, -half), y1 = std::min(f.y + f.h / 2, half);
+    if (x1 - x0 <= 0 || y1 - y0 <= 0) continue;
+    // equal values beyond the first 64 distinct ones keep classes of their own,
+    // which only splits cells
+    int cls = -1;
+    for (size_t v = 0; v < values.size() && cls < 0 && v < 64; ++v)
+      if (values[v] == f.value) cls = (int)v;
+    if (cls < 0) {
+      cls = (int)values.size();
+      values.push_back(f.value);
+    }
+    rs.push_back({x0, x1, y0, y1, cls});
+  }
+  if (rs.empty()) return true;
+  const size_t R = rs.size();
+  if ((double)(2 * R + 1) * (double)(2 * R + 1) > (double)max_cells) {
+    // the clip's whole edge grid, field edges included, against the limit
+    std::vector<double> xe{-half, half}, ye{-half, half};
+    for (const auto& r : rs) {
+      xe.push_back(r.x0); xe.push_back(r.x1);
+      ye.push_back(r.y0); ye.push_back(r.y1);
+    }
+    dedup(xe, eps);
+    dedup(ye, eps);
+    const int64_t nx = (int64_t)xe.size() - 1, ny = (int64_t)ye.size() - 1;
+    if (nx < 1 || ny < 1 || nx > max_cells / ny) return false;
+  }
+  whole = whole || R > kGroupMaxRects;
+  std::vector<int> root(R);
+  for (size_t i = 0; i < R; ++i) root[i] = whole ? 0 : (int)i;
+  auto find = [&](int i) {
+    while (root[i] != i) i = root[i] = root[root[i]];
+    return i;
+  };
+  if (!whole)
+    for (size_t i = 0; i < R; ++i)
+      for (size_t j = 0; j < i; ++j)
+        if (rs[i].x0 < rs[j].x1 && rs[j].x0 < rs[i].x1 && rs[i].y0 < rs[j].y1 &&
+            rs[j].y0 < rs[i].y1) {
+          const int a = find((int)i), b = find((int)j);
+          root[std::max(a, b)] = std::min(a, b);
+        }
+  // groups in the order of their first rectangle, painter order within each
+  std::vector<std::vector<int>> members(R);
+  for (size_t i = 0; i < R; ++i) members[find((int)i)].push_back((int)i);
+  std::vector<PaintRect> g;
+  for (size_t i = 0; i < R; ++i) {
+    if (members[i].empty()) continue;
+    g.clear();
+    for (int k : members[i]) g.push_back(rs[k]);
+    resolve_group(g, values, eps, out);
   }
   return true;
 }

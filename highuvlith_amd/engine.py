@@ -694,7 +694,7 @@ def band_spectrum_rects_device(ctx, clips, grid, band, backgrounds=0.0):
 
 def socs_images_rects_device(ctx, grid, arrays, planes, out):
     """Images of rectangle masks (arrays = rect_arrays(...)) into out (N, P, n, n) f32 CUDA,
-    on torch's current stream; the call synchronises that stream before staging."""
+    on torch's current stream; the geometry is copied before the call returns."""
     import torch
     offsets, rects, bg = arrays
     nclips, n = len(offsets) - 1, grid.size
@@ -712,7 +712,7 @@ def socs_images_rects_device(ctx, grid, arrays, planes, out):
 def socs_images_features_device(ctx, grid, arrays, polygons, planes, out):
     """Images of masks of rectangles (arrays = rect_arrays(...)) and simple polygons
     (polygons = PolygonArrays(...)) into out (N, P, n, n) f32 CUDA, on torch's
-    current stream; the call synchronises that stream before staging."""
+    current stream; the geometry is copied before the call returns."""
     import torch
     offsets, rects, bg = arrays
     nclips, n = len(offsets) - 1, grid.size

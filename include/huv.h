@@ -319,8 +319,9 @@ huv_status huv_band_spectrum(huv_ctx* ctx, int nclips, int n, int band, const fl
  * path for rectangles, mask.rs:616-657 with compress / axis_coefficients /
  * add_term_spectrum at mask.rs:1365-1502): S[k] = n^2 c(m) e^{-i pi (mx+my)(n-1)/n}
  * for |kx|, |ky| <= band, FP64 evaluation; out: DEVICE, nclips x (2B+1) x (2B+1)
- * interleaved complex FP32 in huv_band_spectrum's layout [kx+B][ky+B].
- * Synchronises the context stream before staging the geometry. */
+ * interleaved complex FP32 in huv_band_spectrum's layout [kx+B][ky+B].  The
+ * geometry is copied before the call returns, which may wait for the feature
+ * call before the previous one; not for use while the stream is captured. */
 huv_status huv_band_spectrum_rects(huv_ctx* ctx, int nclips, int n, double pixel_nm, int band,
                                    const int64_t* offsets, const double* rects,
                                    const double* background, float* out);
