@@ -100,7 +100,8 @@ huv_status ilt_buffers(Ctx* c, const huv_ilt* p, int T, IltBuffers& b) {
   b.reg_part = b.fid_part + TC * kBpi;
   b.cost_d = b.reg_part + (size_t)T * kBpi;
   if (p->m > 64) {
-    const size_t ng0 = TC * W2 * p->m, nab = TC * b.KS * W * p->m;
+    // fields between the adjoint's passes: none on m = 128, which keeps them in LDS
+    const size_t ng0 = TC * W2 * p->m, nab = p->m > 128 ? TC * b.KS * W * p->m : 0;
     a = (char*)c->ws.get(Workspace::ILT9, (ng0 + nab) * sizeof(float2), e);
     if (!a) return hip_fail(e, "ILT workspace");
     b.g0tmp = (float2*)a;
@@ -264,15 +265,15 @@ huv_status ilt_eval(huv_ilt* p, int T, const float* targets, const int* trows,
     const double n2 = (double)n * n;
     const float g0_scale = 1.0f / ((float)m * (float)m);
     const float lam_scale = (float)n2;  // device lambda carries 1/n^4
+    const float2* tw_m = c->twiddles(m, e);
+    if (!tw_m) return hip_fail(e, "twiddle table");
     if (m <= 64) {
       e = huvk::launch_ilt_adjoint(m, T * C, b.KS, Mq, b.Gb, B, C, dK, dkern, dlam, lam_scale,
-                                   g0_scale, (float)p->flare, b.G0g, b.Rout, s);
+                                   g0_scale, (float)p->flare, tw_m, b.G0g, b.Rout, s);
     } else {
       if ((int64_t)T * C * b.KS > 65535)
         return fail(HUV_INVALID_PARAMETER, "targets x conditions x kernels exceeds 65535 per "
                                            "evaluation on coarse grids above 64: pass fewer targets");
-      const float2* tw_m = c->twiddles(m, e);
-      if (!tw_m) return hip_fail(e, "twiddle table");
       e = huvk::launch_ilt_adjoint_big(m, T * C, b.KS, Mq, b.Gb, B, C, dK, dkern, dlam,
                                        lam_scale, g0_scale, (float)p->flare, tw_m, b.g0tmp,
                                        b.G0g, b.abuf, b.Rout, s);

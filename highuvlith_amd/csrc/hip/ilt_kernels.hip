@@ -106,66 +106,91 @@ constexpr int PW_THREADS = 256;
 // (The fidelity term of each image and G = dC/dI are evaluated by the
 // band-image stage itself, launch_band_image_fidelity.)
 
-// Regularisers on m (ilt.rs:606-645): cost partials per block and gradient.
-__global__ __launch_bounds__(PW_THREADS) void k_ilt_reg(
+// Regularisers on m (ilt.rs:606-645): cost partials per block and gradient.  A
+// thread takes four neighbouring pixels: nine gradient magnitudes (four pixels,
+// their left neighbour and the four above) from seven loads, where one pixel at a
+// time takes three magnitudes and nine loads each.  Latency-bound: 1024 threads a
+// work-group and 32-bit indexes (5 targets of 1024^2: 91 -> 27 us).  n is a
+// power of two, n >= 256; chunks are whole groups of four.
+constexpr int kRegThreads = 1024;
+__global__ __launch_bounds__(kRegThreads) void k_ilt_reg(
     const float* __restrict__ m, int n, int blocks_per_img, float tv_w, float tv_eps, float bin_w,
     float* __restrict__ reg_grad, double* __restrict__ partial) {
-  __shared__ double sh[PW_THREADS];
+  __shared__ double sh[kRegThreads];
   const int tgt = blockIdx.y;
-  const int64_t npix = (int64_t)n * n;
+  const int npix = n * n, sh_n = 31 - __clz(n), mask = n - 1;
   const float* mm = m + (size_t)tgt * npix;
   float* rg = reg_grad + (size_t)tgt * npix;
   const float inv_n = 1.0f / (float)npix;
   double acc = 0.0;
-  const int64_t chunk = (npix + blocks_per_img - 1) / blocks_per_img;
-  const int64_t lo = blockIdx.x * chunk, hi = min(npix, lo + chunk);
-  auto sval = [&](int i, int j, float& gx, float& gy) {
-    const float v = mm[(size_t)i * n + j];
-    gx = mm[(size_t)i * n + (j + 1) % n] - v;
-    gy = mm[(size_t)((i + 1) % n) * n + j] - v;
-    return sqrtf(gx * gx + gy * gy + tv_eps * tv_eps);
-  };
-  for (int64_t p = lo + threadIdx.x; p < hi; p += PW_THREADS) {
-    const int i = (int)(p / n), j = (int)(p % n);
-    float g = 0.0f;
+  const int quads = npix / 4, chunk = (quads + blocks_per_img - 1) / blocks_per_img;
+  const int lo = blockIdx.x * chunk, hi = min(quads, lo + chunk);
+  auto mag = [&](float gx, float gy) { return sqrtf(gx * gx + gy * gy + tv_eps * tv_eps); };
+  for (int q = lo + threadIdx.x; q < hi; q += kRegThreads) {
+    const int p = 4 * q, i = p >> sh_n, j = p & mask;
+    const float* row = mm + ((size_t)i << sh_n);
+    const float4 c4 = *reinterpret_cast<const float4*>(row + j);
+    const float c[4] = {c4.x, c4.y, c4.z, c4.w};
+    float g[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (tv_w > 0.0f) {
-      float gx, gy, lx, ly, ux, uy;
-      const float s0 = sval(i, j, gx, gy);
-      const float sl = sval(i, (j + n - 1) % n, lx, ly);
-      const float su = sval((i + n - 1) % n, j, ux, uy);
-      acc += (double)(tv_w * (s0 - tv_eps) * inv_n);
-      g += tv_w * (-(gx + gy) / s0 + lx / sl + uy / su) * inv_n;
+      const float* dn = mm + ((size_t)((i + 1) & mask) << sh_n);
+      const float* up = mm + ((size_t)((i - 1) & mask) << sh_n);
+      const float4 d4 = *reinterpret_cast<const float4*>(dn + j);
+      const float4 u4 = *reinterpret_cast<const float4*>(up + j);
+      const float cr = row[(j + 4) & mask], ur = up[(j + 4) & mask];
+      const float cl = row[(j - 1) & mask], dl = dn[(j - 1) & mask];
+      const float d[4] = {d4.x, d4.y, d4.z, d4.w}, u[5] = {u4.x, u4.y, u4.z, u4.w, ur};
+      float lx = c[0] - cl, sl = mag(lx, dl - cl);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float gx = (k < 3 ? c[k + 1] : cr) - c[k], gy = d[k] - c[k];
+        const float ux = u[k + 1] - u[k], uy = c[k] - u[k];
+        const float s0 = mag(gx, gy), su = mag(ux, uy);
+        acc += (double)(tv_w * (s0 - tv_eps) * inv_n);
+        g[k] += tv_w * (-(gx + gy) / s0 + lx / sl + uy / su) * inv_n;
+        lx = gx;
+        sl = s0;
+      }
     }
     if (bin_w > 0.0f) {
-      const float v = mm[p];
-      acc += (double)(bin_w * 4.0f * v * (1.0f - v) * inv_n);
-      g += bin_w * 4.0f * (1.0f - 2.0f * v) * inv_n;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        acc += (double)(bin_w * 4.0f * c[k] * (1.0f - c[k]) * inv_n);
+        g[k] += bin_w * 4.0f * (1.0f - 2.0f * c[k]) * inv_n;
+      }
     }
-    rg[p] = g;
+    *reinterpret_cast<float4*>(rg + p) = make_float4(g[0], g[1], g[2], g[3]);
   }
-  const double s = block_sum<PW_THREADS>(acc, sh);
+  const double s = block_sum<kRegThreads>(acc, sh);
   if (threadIdx.x == 0) partial[(size_t)tgt * blocks_per_img + blockIdx.x] = s;
 }
 
-// cost[t] = sum_c w_c (1/N) sum_blocks fid[t, c] + sum_blocks reg[t]  (fixed order).
-__global__ void k_ilt_cost_reduce(const double* __restrict__ fid, const double* __restrict__ reg,
-                                  int ntargets, int ncond, int bpi, int reg_bpi,
-                                  const float* __restrict__ weight, double inv_n,
-                                  double* __restrict__ cost) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ntargets) return;
+// cost[t] = sum_c w_c (1/N) sum_blocks fid[t, c] + sum_blocks reg[t]  (fixed
+// order).  One wave per target fetches 64 partials at a time into LDS and every
+// lane adds them in order; a lone thread waiting for each load took 13.3 us for
+// 160 partials, this takes 6.8.
+__global__ __launch_bounds__(64) void k_ilt_cost_reduce(
+    const double* __restrict__ fid, const double* __restrict__ reg, int ncond, int bpi,
+    int reg_bpi, const float* __restrict__ weight, double inv_n, double* __restrict__ cost) {
+  __shared__ double sh[64];
+  const int t = blockIdx.x, lane = threadIdx.x;
+  auto add_in_order = [&](const double* p, int count, double s) {
+    for (int b0 = 0; b0 < count; b0 += 64) {
+      const int nb = min(64, count - b0);
+      __syncthreads();
+      if (lane < nb) sh[lane] = p[b0 + lane];
+      __syncthreads();
+      for (int b = 0; b < nb; ++b) s += sh[b];
+    }
+    return s;
+  };
   double total = 0.0;
   for (int c = 0; c < ncond; ++c) {
-    double s = 0.0;
-    const double* p = fid + ((size_t)t * ncond + c) * bpi;
-    for (int b = 0; b < bpi; ++b) s += p[b];
+    const double s = add_in_order(fid + ((size_t)t * ncond + c) * bpi, bpi, 0.0);
     total += (double)weight[c] * s * inv_n;
   }
-  if (reg) {
-    const double* p = reg + (size_t)t * reg_bpi;
-    for (int b = 0; b < reg_bpi; ++b) total += p[b];
-  }
-  cost[t] = total;
+  if (reg) total = add_in_order(reg + (size_t)t * reg_bpi, reg_bpi, total);
+  if (lane == 0) cost[t] = total;
 }
 
 // ---------------------------------------------------------------------------
@@ -173,167 +198,216 @@ __global__ void k_ilt_cost_reduce(const double* __restrict__ fid, const double* 
 //   k_ilt_g0:      one work-group per image (target, condition): G0_b on the
 //                  coarse grid, G0[img][y][x] (real), from the |g| <= 2B band
 //                  Gb of F(G), layout [gx + 2B][gy + 2B], flare adjoint applied.
-//   k_ilt_adjoint: work-group (image, split s) takes the kernels k = s, s + KS,
-//                  ...: field A_k, product with G0_b, back to the |f| <= B band,
-//                  accumulating lambda_k conj(K_k) F(G0_b . A_k) / n^2 into its
-//                  own partial band Rpart[img][s][fx + B][fy + B]; k_ilt_hband
-//                  sums the KS partials in a fixed order.
+//   k_ilt_adjoint: work-group (image, kernel k < KS): field A_k, product with
+//                  G0_b, back to the |f| <= B band; lambda_k conj(K_k)
+//                  F(G0_b . A_k) / n^2 into Rpart[img][k][fx + B][fy + B] (zero
+//                  beyond the condition's own count); k_ilt_hband sums the KS
+//                  bands in a fixed order.
 // ---------------------------------------------------------------------------
+// Transforms of length M = N1 x N2 run in teams of N1 threads of one wave (8 x 16
+// for M = 128, 8 x 8 for 64, 4 x 8 for 32), N2 values a thread: thread t holds
+// x[t + N1 i] and gets X[t + N1 i], so a forward transform follows an inverse
+// one without an exchange.  One transform a thread (64 values in registers, one
+// wave a work-group, half its lanes idle in the row passes) took 23 us for the
+// G0 of 64 images and 45 us for their 768 (image, kernel) adjoints at M = 64;
+// this takes 10.4 and 17.9.  At M = 128 one launch with the field in LDS takes
+// 67 us for 480 jobs, row, column and output passes through memory 82.
 template <int M>
-__global__ __launch_bounds__(M) void k_ilt_g0(const float2* __restrict__ Gb, int B, float g0_scale,
-                                              float flare, float* __restrict__ G0g) {
-  constexpr int TP = M + 1;
+struct AdjTeam {
+  static constexpr int N2 = M == 128 ? 16 : 8, N1 = M / N2;
+  static constexpr int THREADS = M == 128 ? 512 : 256, TEAMS = THREADS / N1;
+  static constexpr int EX = (N1 + 1) * N2;  // exchange area of a team
+  static constexpr int TP = M + 1;          // tile row stride
+  static_assert(N2 % N1 == 0 && 64 % N1 == 0, "teams lie in one wave");
+};
+
+// w[k] = e^{-2 pi i t k / M}; ex: the team's exchange area.
+template <int SIGN, int M>
+__device__ __forceinline__ void team_fft(c32* v, int t, const c32* w, c32* ex) {
+  constexpr int N1 = AdjTeam<M>::N1, N2 = AdjTeam<M>::N2, R = N2 / N1;
+  fft_reg<SIGN, N2>(v);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int k = 0; k < N2; ++k)
+    ex[t + (N1 + 1) * k] =
+        k == 0 ? v[0] : cmul(v[k], SIGN < 0 ? w[k] : c32{w[k].re, -w[k].im});
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    c32 u[N1];
+#pragma unroll
+    for (int i = 0; i < N1; ++i) u[i] = ex[i + (N1 + 1) * (t + N1 * r)];
+    fft_reg<SIGN, N1>(u);
+#pragma unroll
+    for (int k = 0; k < N1; ++k) v[r + R * k] = u[k];
+  }
+}
+
+// signed frequency of FFT bin h if |f| <= band, else a value outside the band
+__device__ __forceinline__ int band_freq(int h, int M, int band) {
+  if (h <= band) return h;
+  if (h - M >= -band) return h - M;
+  return 1 << 20;
+}
+
+template <int M>
+__global__ __launch_bounds__(AdjTeam<M>::THREADS) void k_ilt_g0(const float2* __restrict__ Gb, int B,
+                                                float g0_scale, float flare,
+                                                const float2* __restrict__ tw_m,
+                                                float* __restrict__ G0g) {
+  using A = AdjTeam<M>;
+  constexpr int N1 = A::N1, N2 = A::N2, TP = A::TP;
   extern __shared__ unsigned char smem_raw[];
   c32* T = reinterpret_cast<c32*>(smem_raw);  // (4B+1) x TP
   const int G = 2 * B, W2 = 4 * B + 1;
   const int img = blockIdx.x;
-  const int tid = threadIdx.x;
+  const int lane = threadIdx.x & 63, per = 64 / N1;  // teams of a wave
+  const int t = lane / per, team = (threadIdx.x >> 6) * per + lane % per;
+  c32* ex = T + (size_t)W2 * TP + team * A::EX;
   const float2* gb = Gb + (size_t)img * W2 * W2;
-  // x pass over the 4B+1 band rows gy
-  for (int iy = tid; iy < W2; iy += M) {
-    c32 v[M];
+  c32 w[N2];
 #pragma unroll
-    for (int h = 0; h < M; ++h) {
-      v[h] = c32{0.f, 0.f};
-      // gx = h (h <= 2B) or h - M (>= -2B)
-      if (h <= G) {
-        const float2 a = gb[(size_t)(h + G) * W2 + iy];
-        v[h] = c32{a.x, a.y};
-      }
-      if (h - M >= -G) {
-        const float2 a = gb[(size_t)(h - M + G) * W2 + iy];
-        v[h] = cadd(v[h], c32{a.x, a.y});
+  for (int k = 0; k < N2; ++k) w[k] = tw_lookup<-1>(tw_m, t * k);
+  // x pass over the 4B+1 band rows gy; every lane takes part in the exchanges
+  for (int r0 = 0; r0 < W2; r0 += A::TEAMS) {
+    const int iy = r0 + team;
+    const bool act = iy < W2;
+    c32 v[N2];
+#pragma unroll
+    for (int i = 0; i < N2; ++i) {
+      const int gx = band_freq(t + N1 * i, M, G);
+      v[i] = c32{0.f, 0.f};
+      if (act && gx <= G) {
+        const float2 a = gb[(size_t)(gx + G) * W2 + iy];
+        // flare adjoint: non-DC terms scale by (1 - phi)
+        const float f = (gx == 0 && iy == G) ? 1.0f : 1.0f - flare;
+        v[i] = c32{a.x * f, a.y * f};
       }
     }
-    // flare adjoint: non-DC terms scale by (1 - phi)
-    const int gy = iy - G;
+    team_fft<+1, M>(v, t, w, ex);
+    if (act) {
 #pragma unroll
-    for (int h = 0; h < M; ++h)
-      if (!(h == 0 && gy == 0)) v[h] = cscale(v[h], 1.0f - flare);
-    fft_reg<+1, M>(v);
-#pragma unroll
-    for (int j = 0; j < M; ++j) T[iy * TP + j] = v[j];
+      for (int i = 0; i < N2; ++i) T[iy * TP + t + N1 * i] = v[i];
+    }
   }
   __syncthreads();
-  const int j = tid;
-  c32 d[M];
-#pragma unroll
-  for (int h = 0; h < M; ++h) {
-    d[h] = c32{0.f, 0.f};
-    if (h <= G) d[h] = T[(h + G) * TP + j];
-    if (h - M >= -G) d[h] = cadd(d[h], T[(h - M + G) * TP + j]);
-  }
-  fft_reg<+1, M>(d);
   float* g0 = G0g + (size_t)img * M * M;
+  for (int x0 = 0; x0 < M; x0 += A::TEAMS) {
+    const int x = x0 + team;
+    const bool act = x < M;
+    c32 v[N2];
 #pragma unroll
-  for (int y = 0; y < M; ++y) g0[y * M + j] = d[y].re * g0_scale;
+    for (int i = 0; i < N2; ++i) {
+      const int gy = band_freq(t + N1 * i, M, G);
+      v[i] = act && gy <= G ? T[(gy + G) * TP + x] : c32{0.f, 0.f};
+    }
+    team_fft<+1, M>(v, t, w, ex);
+    if (act) {
+#pragma unroll
+      for (int i = 0; i < N2; ++i) g0[(t + N1 * i) * M + x] = v[i].re * g0_scale;
+    }
+  }
 }
 
+// One (image, kernel) per work-group: rows ky of E = IFFT(K . M), columns back
+// and forth through the product with G0_b, rows fy out; the field stays in LDS.
 template <int M>
-__global__ __launch_bounds__(M) void k_ilt_adjoint(
+__global__ __launch_bounds__(AdjTeam<M>::THREADS) void k_ilt_adjoint(
     const float2* __restrict__ Mq, const float* __restrict__ G0g, int B, int ncond,
     const int* __restrict__ cond_K, const float2* const* __restrict__ cond_kern,
-    const float* const* __restrict__ cond_lam, float lam_scale, float2* __restrict__ Rpart) {
-  constexpr int TP = M + 1;
+    const float* const* __restrict__ cond_lam, float lam_scale, const float2* __restrict__ tw_m,
+    float2* __restrict__ Rpart) {
+  using A = AdjTeam<M>;
+  constexpr int N1 = A::N1, N2 = A::N2, TP = A::TP;
   extern __shared__ unsigned char smem_raw[];
   const int W = 2 * B + 1;
-  c32* T = reinterpret_cast<c32*>(smem_raw);                  // W x TP
-  c32* P1 = T + (size_t)W * TP;                               // W x TP
-  float* G0 = reinterpret_cast<float*>(P1 + (size_t)W * TP);  // M x TP
-  const int img = blockIdx.x, split = blockIdx.y, KS = gridDim.y;
+  c32* T = reinterpret_cast<c32*>(smem_raw);  // W x TP
+  const int img = blockIdx.x, k = blockIdx.y;
   const int tgt = img / ncond, c = img % ncond;
-  const int tid = threadIdx.x;
+  float2* ro = Rpart + ((size_t)img * gridDim.y + k) * W * W;
+  if (k >= cond_K[c]) {  // whole work-group
+    for (int i = threadIdx.x; i < W * W; i += A::THREADS) ro[i] = make_float2(0.f, 0.f);
+    return;
+  }
+  const int lane = threadIdx.x & 63, per = 64 / N1;
+  const int t = lane / per, team = (threadIdx.x >> 6) * per + lane % per;
+  c32* ex = T + (size_t)W * TP + team * A::EX;
   const float2* mq = Mq + (size_t)tgt * W * W;
-  {
-    const float* g0 = G0g + (size_t)img * M * M;
-    for (int y = 0; y < M; ++y) G0[y * TP + tid] = g0[y * M + tid];
+  const float2* kern = cond_kern[c] + (size_t)k * W * W;
+  const float* g0 = G0g + (size_t)img * M * M;
+  c32 w[N2];
+#pragma unroll
+  for (int i = 0; i < N2; ++i) w[i] = tw_lookup<-1>(tw_m, t * i);
+  for (int r0 = 0; r0 < W; r0 += A::TEAMS) {
+    const int iy = r0 + team;
+    const bool act = iy < W;
+    c32 v[N2];
+#pragma unroll
+    for (int i = 0; i < N2; ++i) {
+      const int kx = band_freq(t + N1 * i, M, B);
+      v[i] = c32{0.f, 0.f};
+      if (act && kx <= B) {
+        const float2 a = kern[(size_t)(kx + B) * W + iy], b = mq[(size_t)(kx + B) * W + iy];
+        v[i] = cmul(c32{a.x, a.y}, c32{b.x, b.y});
+      }
+    }
+    team_fft<+1, M>(v, t, w, ex);
+    if (act) {
+#pragma unroll
+      for (int i = 0; i < N2; ++i) T[iy * TP + t + N1 * i] = v[i];
+    }
   }
   __syncthreads();
-
-  // ---- per kernel: field, product, back to the |f| <= B band ----
-  const int K = cond_K[c];
-  const float2* kern = cond_kern[c];
-  const float* lam = cond_lam[c];
-  c32 R[2 * 15 + 1];  // accumulator row fy = tid - B (B <= 15)
+  for (int x0 = 0; x0 < M; x0 += A::TEAMS) {
+    const int x = x0 + team;
+    const bool act = x < M;
+    c32 v[N2];
+    float g[N2];
 #pragma unroll
-  for (int i = 0; i < 31; ++i) R[i] = c32{0.f, 0.f};
-  for (int k = split; k < K; k += KS) {
-    // x pass (rows iy in [0, 2B]): E row = IFFT_M(K . M)
-    for (int iy = tid; iy < W; iy += M) {
-      const float2* kk = kern + (size_t)k * W * W + iy;
-      const float2* mm = mq + iy;
-      c32 v[M];
-#pragma unroll
-      for (int h = 0; h < M; ++h) {
-        v[h] = c32{0.f, 0.f};
-        if (h <= B) {
-          const float2 a = kk[(size_t)(h + B) * W], b = mm[(size_t)(h + B) * W];
-          v[h] = cmul(c32{a.x, a.y}, c32{b.x, b.y});
-        }
-        if (h - M >= -B) {
-          const float2 a = kk[(size_t)(h - M + B) * W], b = mm[(size_t)(h - M + B) * W];
-          v[h] = cmac(v[h], c32{a.x, a.y}, c32{b.x, b.y});
-        }
-      }
-      fft_reg<+1, M>(v);
-#pragma unroll
-      for (int j = 0; j < M; ++j) T[iy * TP + j] = v[j];
+    for (int i = 0; i < N2; ++i) {
+      g[i] = act ? g0[(t + N1 * i) * M + x] : 0.f;
+      const int ky = band_freq(t + N1 * i, M, B);
+      v[i] = act && ky <= B ? T[(ky + B) * TP + x] : c32{0.f, 0.f};
     }
-    __syncthreads();
-    // y pass (column j): E column, times G0_b, forward FFT_M, keep |fy| <= B
-    {
-      const int j = tid;
-      c32 d[M];
+    team_fft<+1, M>(v, t, w, ex);
 #pragma unroll
-      for (int h = 0; h < M; ++h) {
-        d[h] = c32{0.f, 0.f};
-        if (h <= B) d[h] = T[(h + B) * TP + j];
-        if (h - M >= -B) d[h] = cadd(d[h], T[(h - M + B) * TP + j]);
-      }
-      fft_reg<+1, M>(d);
+    for (int i = 0; i < N2; ++i) v[i] = cscale(v[i], g[i]);
+    team_fft<-1, M>(v, t, w, ex);
+    // the column's band rows replace it (read above by this team alone)
+    if (act) {
 #pragma unroll
-      for (int y = 0; y < M; ++y) d[y] = cscale(d[y], G0[y * TP + j]);
-      fft_reg<-1, M>(d);
-#pragma unroll
-      for (int h = 0; h < M; ++h) {
-        if (h <= B) P1[(h + B) * TP + j] = d[h];
-        if (h - M >= -B) P1[(h - M + B) * TP + j] = d[h];
+      for (int i = 0; i < N2; ++i) {
+        const int fy = band_freq(t + N1 * i, M, B);
+        if (fy <= B) T[(fy + B) * TP + x] = v[i];
       }
     }
-    __syncthreads();
-    // x stage (row fy): forward FFT_M over x, keep |fx| <= B, accumulate
-    if (tid < W) {
-      c32 v[M];
-#pragma unroll
-      for (int j = 0; j < M; ++j) v[j] = P1[tid * TP + j];
-      fft_reg<-1, M>(v);
-      const float l = lam[k] * lam_scale;
-      const float2* kk = kern + (size_t)k * W * W + tid;  // K[k][fx + B][fy + B], fy = tid - B
-#pragma unroll
-      for (int i = 0; i < 31; ++i) {
-        const int fx = i - 15;
-        if (fx >= -B && fx <= B) {
-          const c32 val = v[(fx + M) % M];
-          const float2 kv = kk[(size_t)(fx + B) * W];
-          R[i] = cadd(R[i], cscale(cconjmul(c32{kv.x, kv.y}, val), l));
-        }
-      }
-    }
-    __syncthreads();
   }
-  if (tid < W) {
-    float2* ro = Rpart + ((size_t)img * KS + split) * W * W + tid;
+  __syncthreads();
+  const float l = cond_lam[c][k] * lam_scale;
+  for (int r0 = 0; r0 < W; r0 += A::TEAMS) {
+    const int iy = r0 + team;
+    const bool act = iy < W;
+    c32 v[N2];
 #pragma unroll
-    for (int i = 0; i < 31; ++i) {
-      const int fx = i - 15;
-      if (fx >= -B && fx <= B) ro[(size_t)(fx + B) * W] = make_float2(R[i].re, R[i].im);
+    for (int i = 0; i < N2; ++i) v[i] = act ? T[iy * TP + t + N1 * i] : c32{0.f, 0.f};
+    team_fft<-1, M>(v, t, w, ex);
+    if (act) {
+#pragma unroll
+      for (int i = 0; i < N2; ++i) {
+        const int fx = band_freq(t + N1 * i, M, B);
+        if (fx > B) continue;
+        const float2 kv = kern[(size_t)(fx + B) * W + iy];
+        const c32 r = cscale(cconjmul(c32{kv.x, kv.y}, v[i]), l);
+        ro[(size_t)(fx + B) * W + iy] = make_float2(r.re, r.im);
+      }
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Adjoint on coarse grids M = 128, 192, 256 (band half-width B up to 63): the
-// same algebra as k_ilt_g0 / k_ilt_adjoint, with the length-M transforms done
+// Adjoint on coarse grids M = 192, 256 (band half-width B up to 63), and G0_b on
+// M = 128 (whose 2B-band rows do not fit LDS beside the exchange areas; its
+// adjoint is k_ilt_adjoint): the same algebra as k_ilt_g0 / k_ilt_adjoint, with the length-M transforms done
 // by teams of threads (four-step, LDS) and the per-(image, kernel) field held
 // in HBM between passes.  A job is (image, kernel) with image = target x
 // ncond + condition and kernel k < KS (KS = the largest kernel count; jobs
@@ -353,13 +427,6 @@ struct AdjFft {
   static constexpr int TEAMS = 256 / N2;
 };
 constexpr int kAdjColTeams = 8;
-
-// signed frequency of FFT bin h if |f| <= band, else a value outside the band
-__device__ __forceinline__ int band_freq(int h, int M, int band) {
-  if (h <= band) return h;
-  if (h - M >= -band) return h - M;
-  return 1 << 20;
-}
 
 template <int M>
 __global__ __launch_bounds__(256) void k_ilt_g0_rows(const float2* __restrict__ Gb, int B,
@@ -518,21 +585,29 @@ __global__ __launch_bounds__(256) void k_ilt_adj_out(
 // R_c = sum over the KS partial bands of image (tgt, c), in split order.
 // With a complex absorber a and c = 1 - a (ilt.rs:672,715), 2 Re[conj(c) Q]
 // has the spectrum conj(c) R(f) + c conj(R(-f)); inv_n2 = 1 / n^2.
-__global__ void k_ilt_hband(const float2* __restrict__ Rin, int B, int ncond, int KS,
-                            const float* __restrict__ weight, float cr, float ci, float inv_n2,
-                            float2* __restrict__ H) {
+// A work-group takes 32 bins (fy fastest, as the bands are stored); its eight
+// groups of 32 lanes take every eighth of the KS bands each, added up in group
+// order.  One thread a bin in the order of H read a line per lane and waited for
+// each band in turn (5 targets, 3 conditions, KS = 32: 35 -> 6.1 us).
+constexpr int kHbSlices = 8;
+__global__ __launch_bounds__(32 * kHbSlices) void k_ilt_hband(
+    const float2* __restrict__ Rin, int B, int ncond, int KS, const float* __restrict__ weight,
+    float cr, float ci, float inv_n2, float2* __restrict__ H) {
+  __shared__ c32 part[kHbSlices][32];
   const int tgt = blockIdx.y;
   const int W = 2 * B + 1;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (B + 1) * W) return;
-  const int fx = idx % (B + 1), fy = idx / (B + 1) - B;
+  const int o = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int idx = blockIdx.x * 32 + o, count = (B + 1) * W;
+  const int at = min(idx, count - 1);
+  const int fx = at / W, fy = at % W - B;
+  const size_t ia = (size_t)(fx + B) * W + (fy + B), ib = (size_t)(B - fx) * W + (B - fy);
   c32 acc{0.f, 0.f};
   for (int c = 0; c < ncond; ++c) {
     c32 p{0.f, 0.f}, q{0.f, 0.f};
-    for (int sp = 0; sp < KS; ++sp) {
-      const float2* r = Rin + (((size_t)tgt * ncond + c) * KS + sp) * W * W;
-      const float2 a = r[(size_t)(fx + B) * W + (fy + B)];
-      const float2 b = r[(size_t)(B - fx) * W + (B - fy)];
+    const float2* r = Rin + ((size_t)tgt * ncond + c) * KS * W * W;
+#pragma unroll 4
+    for (int sp = g; sp < KS; sp += kHbSlices) {
+      const float2 a = r[(size_t)sp * W * W + ia], b = r[(size_t)sp * W * W + ib];
       p = cadd(p, c32{a.x, a.y});
       q = cadd(q, c32{b.x, b.y});
     }
@@ -541,7 +616,13 @@ __global__ void k_ilt_hband(const float2* __restrict__ Rin, int B, int ncond, in
     const c32 v = cmul(c32{cr, ci}, c32{q.re, -q.im});
     acc = cadd(acc, cscale(cadd(u, v), weight[c]));
   }
-  H[(size_t)tgt * (B + 1) * W + idx] = make_float2(acc.re * inv_n2, acc.im * inv_n2);
+  part[g][o] = acc;
+  __syncthreads();
+  if (g != 0 || idx >= count) return;
+#pragma unroll
+  for (int k = 1; k < kHbSlices; ++k) acc = cadd(acc, part[k][o]);
+  H[(size_t)tgt * count + (fy + B) * (B + 1) + fx] =
+      make_float2(acc.re * inv_n2, acc.im * inv_n2);
 }
 
 // Local proxy gradient (ilt.rs:719-721): dcdm[t] = sum_c w_c G0_c with
@@ -820,7 +901,7 @@ hipError_t launch_ilt_mask_rows(const float* theta, const int* rows, const float
 
 hipError_t launch_ilt_reg(const float* m, int n, int ntargets, int bpi, float tv_w, float tv_eps,
                           float bin_w, float* reg_grad, double* partial, hipStream_t s) {
-  hipLaunchKernelGGL(k_ilt_reg, dim3(bpi, ntargets), dim3(PW_THREADS), 0, s, m, n, bpi, tv_w,
+  hipLaunchKernelGGL(k_ilt_reg, dim3(bpi, ntargets), dim3(kRegThreads), 0, s, m, n, bpi, tv_w,
                      tv_eps, bin_w, reg_grad, partial);
   return hipGetLastError();
 }
@@ -828,8 +909,28 @@ hipError_t launch_ilt_reg(const float* m, int n, int ntargets, int bpi, float tv
 hipError_t launch_ilt_cost_reduce(const double* fid, const double* reg, int ntargets, int ncond,
                                   int bpi, int reg_bpi, const float* weight, double inv_n,
                                   double* cost, hipStream_t s) {
-  hipLaunchKernelGGL(k_ilt_cost_reduce, dim3((ntargets + 63) / 64), dim3(64), 0, s, fid, reg,
-                     ntargets, ncond, bpi, reg_bpi, weight, inv_n, cost);
+  hipLaunchKernelGGL(k_ilt_cost_reduce, dim3(ntargets), dim3(64), 0, s, fid, reg, ncond, bpi,
+                     reg_bpi, weight, inv_n, cost);
+  return hipGetLastError();
+}
+
+// the (image, kernel) adjoints of a coarse grid up to 128
+template <int M>
+static hipError_t adjoint_jobs(int nimg, int KS, const float2* Mq, const float* G0g, int B,
+                               int ncond, const int* cond_K, const float2* const* cond_kern,
+                               const float* const* cond_lam, float lam_scale, const float2* tw_m,
+                               float2* Rpart, hipStream_t s) {
+  using A = AdjTeam<M>;
+  if (4 * B + 1 > M) return hipErrorInvalidValue;
+  constexpr size_t ex = (size_t)A::TEAMS * A::EX;
+  auto bytes = [](int b) { return ((size_t)(2 * b + 1) * A::TP + ex) * sizeof(c32); };
+  auto k1 = k_ilt_adjoint<M>;
+  // sized for the largest band, once per instantiation
+  static const hipError_t a1 = hipFuncSetAttribute(
+      (const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes((M - 1) / 4));
+  if (a1 != hipSuccess) return a1;
+  hipLaunchKernelGGL(k1, dim3(nimg, KS), dim3(A::THREADS), bytes(B), s, Mq, G0g, B, ncond, cond_K,
+                     cond_kern, cond_lam, lam_scale, tw_m, Rpart);
   return hipGetLastError();
 }
 
@@ -837,34 +938,33 @@ template <int M>
 static hipError_t adjoint_m(int nimg, int KS, const float2* Mq, const float2* Gb, int B, int ncond,
                             const int* cond_K, const float2* const* cond_kern,
                             const float* const* cond_lam, float lam_scale, float g0_scale,
-                            float flare, float* G0g, float2* Rpart, hipStream_t s) {
-  const int W = 2 * B + 1, W2 = 4 * B + 1;
-  const size_t sh0 = (size_t)W2 * (M + 1) * sizeof(c32);
-  const size_t sh1 = (size_t)2 * W * (M + 1) * sizeof(c32) + (size_t)M * (M + 1) * sizeof(float);
+                            float flare, const float2* tw_m, float* G0g, float2* Rpart,
+                            hipStream_t s) {
+  using A = AdjTeam<M>;
+  if (4 * B + 1 > M) return hipErrorInvalidValue;
+  constexpr size_t ex = (size_t)A::TEAMS * A::EX;
+  auto bytes = [](int b) { return ((size_t)(4 * b + 1) * A::TP + ex) * sizeof(c32); };
   auto k0 = k_ilt_g0<M>;
-  auto k1 = k_ilt_adjoint<M>;
-  // sized for the largest band (B = 15), once per instantiation
   static const hipError_t a0 = hipFuncSetAttribute(
-      (const void*)k0, hipFuncAttributeMaxDynamicSharedMemorySize, (int)((61 * (M + 1)) * sizeof(c32)));
-  static const hipError_t a1 = hipFuncSetAttribute(
-      (const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize,
-      (int)(2 * 31 * (M + 1) * sizeof(c32) + M * (M + 1) * sizeof(float)));
+      (const void*)k0, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes((M - 1) / 4));
   if (a0 != hipSuccess) return a0;
-  if (a1 != hipSuccess) return a1;
-  hipLaunchKernelGGL(k0, dim3(nimg), dim3(M), sh0, s, Gb, B, g0_scale, flare, G0g);
-  hipLaunchKernelGGL(k1, dim3(nimg, KS), dim3(M), sh1, s, Mq, G0g, B, ncond, cond_K, cond_kern,
-                     cond_lam, lam_scale, Rpart);
-  return hipGetLastError();
+  hipLaunchKernelGGL(k0, dim3(nimg), dim3(A::THREADS), bytes(B), s, Gb, B, g0_scale, flare, tw_m,
+                     G0g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return adjoint_jobs<M>(nimg, KS, Mq, G0g, B, ncond, cond_K, cond_kern, cond_lam, lam_scale, tw_m,
+                         Rpart, s);
 }
 
 hipError_t launch_ilt_adjoint(int m, int nimg, int KS, const float2* Mq, const float2* Gb, int B,
                               int ncond, const int* cond_K, const float2* const* cond_kern,
                               const float* const* cond_lam, float lam_scale, float g0_scale,
-                              float flare, float* G0g, float2* Rpart, hipStream_t s) {
+                              float flare, const float2* tw_m, float* G0g, float2* Rpart,
+                              hipStream_t s) {
   if (B > 15 || KS < 1) return hipErrorInvalidValue;
   switch (m) {
-    case 32: return adjoint_m<32>(nimg, KS, Mq, Gb, B, ncond, cond_K, cond_kern, cond_lam, lam_scale, g0_scale, flare, G0g, Rpart, s);
-    case 64: return adjoint_m<64>(nimg, KS, Mq, Gb, B, ncond, cond_K, cond_kern, cond_lam, lam_scale, g0_scale, flare, G0g, Rpart, s);
+    case 32: return adjoint_m<32>(nimg, KS, Mq, Gb, B, ncond, cond_K, cond_kern, cond_lam, lam_scale, g0_scale, flare, tw_m, G0g, Rpart, s);
+    case 64: return adjoint_m<64>(nimg, KS, Mq, Gb, B, ncond, cond_K, cond_kern, cond_lam, lam_scale, g0_scale, flare, tw_m, G0g, Rpart, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -882,6 +982,12 @@ static hipError_t adjoint_big_m(int nimg, int KS, const float2* Mq, const float2
                      flare, tw_m, g0tmp);
   hipLaunchKernelGGL(k_ilt_g0_cols<M>, dim3(blocks(M, F::TEAMS), nimg), dim3(256), 0, s, g0tmp, B,
                      g0_scale, tw_m, G0g);
+  if constexpr (M == 128) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return adjoint_jobs<M>(nimg, KS, Mq, G0g, B, ncond, cond_K, cond_kern, cond_lam, lam_scale,
+                           tw_m, Rpart, s);
+  } else {
   hipLaunchKernelGGL(k_ilt_adj_rows<M>, dim3(blocks(W, F::TEAMS), jobs), dim3(256), 0, s, Mq, B,
                      ncond, KS, cond_K, cond_kern, tw_m, buf);
   hipLaunchKernelGGL(k_ilt_adj_cols<M>, dim3(blocks(M, kAdjColTeams), jobs),
@@ -889,6 +995,7 @@ static hipError_t adjoint_big_m(int nimg, int KS, const float2* Mq, const float2
   hipLaunchKernelGGL(k_ilt_adj_out<M>, dim3(blocks(W, F::TEAMS), jobs), dim3(256), 0, s, buf, B,
                      ncond, KS, cond_K, cond_kern, cond_lam, lam_scale, tw_m, Rpart);
   return hipGetLastError();
+  }
 }
 
 hipError_t launch_ilt_adjoint_big(int m, int nimg, int KS, const float2* Mq, const float2* Gb,
@@ -910,8 +1017,8 @@ hipError_t launch_ilt_hband(const float2* Rin, int B, int ntargets, int ncond, i
                             const float* weight, float cr, float ci, float inv_n2, float2* H,
                             hipStream_t s) {
   const int cnt = (B + 1) * (2 * B + 1);
-  hipLaunchKernelGGL(k_ilt_hband, dim3((cnt + 127) / 128, ntargets), dim3(128), 0, s, Rin, B,
-                     ncond, KS, weight, cr, ci, inv_n2, H);
+  hipLaunchKernelGGL(k_ilt_hband, dim3((cnt + 31) / 32, ntargets), dim3(32 * kHbSlices), 0, s, Rin,
+                     B, ncond, KS, weight, cr, ci, inv_n2, H);
   return hipGetLastError();
 }
 

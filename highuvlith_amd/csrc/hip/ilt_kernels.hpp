@@ -19,12 +19,14 @@ hipError_t launch_ilt_cost_reduce(const double* fid, const double* reg, int ntar
                                   int bpi, int reg_bpi, const float* weight, double inv_n,
                                   double* cost, hipStream_t s);
 // Adjoint band of nimg = ntargets x ncond images on coarse grid m (32 or 64):
-// G0g scratch [nimg][m][m] floats, Rpart [nimg][KS][2B+1][2B+1] partial bands
-// (the kernels of each condition dealt over KS work-groups per image).
+// G0g scratch [nimg][m][m] floats, Rpart [nimg][KS][2B+1][2B+1] one band per
+// kernel (KS = the largest kernel count, zero bands past a condition's own
+// count); tw_m: the W_m table.
 hipError_t launch_ilt_adjoint(int m, int nimg, int KS, const float2* Mq, const float2* Gb, int B,
                               int ncond, const int* cond_K, const float2* const* cond_kern,
                               const float* const* cond_lam, float lam_scale, float g0_scale,
-                              float flare, float* G0g, float2* Rpart, hipStream_t s);
+                              float flare, const float2* tw_m, float* G0g, float2* Rpart,
+                              hipStream_t s);
 // The same adjoint for coarse grids m = 128, 192, 256: team FFTs through HBM
 // (g0tmp: nimg x (4B+1) x m complex; buf: nimg x KS x (2B+1) x m complex;
 // tw_m: the W_m table); Rpart holds one band per kernel (KS = the largest
