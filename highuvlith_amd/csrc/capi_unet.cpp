@@ -33,10 +33,10 @@ struct Acts {
   int N = 0, H = 0, W = 0;
   std::vector<void*> owned;
   bf16_t* x8 = nullptr;
-  std::vector<bf16_t*> e1, e2, pool, cat, d1, d2;        // forward
+  std::vector<bf16_t*> e1, e2, pool, d1, d2;             // forward
   std::vector<bf16_t*> ge1, ge2, gpool, gcat, gd1, gd2;  // gradients
   bf16_t *xt = nullptr, *dyt = nullptr, *tmp = nullptr;
-  float *out = nullptr, *dout = nullptr, *part = nullptr, *hpart = nullptr, *bpart = nullptr;
+  float *out = nullptr, *dout = nullptr, *part = nullptr, *hpart = nullptr;
   double* lpart = nullptr;
   size_t part_floats = 0;
   void release() {
@@ -131,16 +131,15 @@ huv_status ensure_acts(huv_unet* u, int N, int H, int W) {
 #define A(ptr, count) if ((st = alloc_t(a, &(ptr), (size_t)(count))) != HUV_OK) return st
   A(a.x8, P * 8);
   a.e1.resize(L); a.e2.resize(L); a.ge1.resize(L); a.ge2.resize(L);
-  a.pool.resize(L); a.gpool.resize(L); a.cat.resize(L); a.gcat.resize(L);
+  a.pool.resize(L); a.gpool.resize(L); a.gcat.resize(L);
   a.d1.resize(L); a.d2.resize(L); a.gd1.resize(L); a.gd2.resize(L);
   size_t maxt = (size_t)P * 8;
-  size_t part = 0, bpart = 0;
+  size_t part = 0;
   auto note_conv = [&](const Conv& c, int l) {
     const int Hl = H >> l, Wl = W >> l;
     const size_t ws = (size_t)wgrad_splits(c, N, Hl, Wl);
-    part = std::max(part, ws * c.cout * 9 * c.cin);
+    part = std::max(part, ws * ((size_t)c.cout * 9 * c.cin + c.cout));
     part = std::max(part, (size_t)bias_splits(c, N, Hl, Wl) * c.cout);
-    bpart = std::max(bpart, ws * c.cout);
   };
   for (int l = 0; l < L; ++l) {
     const int64_t Pl = P >> (2 * l);
@@ -152,7 +151,7 @@ huv_status ensure_acts(huv_unet* u, int N, int H, int W) {
     if (l < L - 1) {
       A(a.pool[l], (Pl / 4) * c); A(a.gpool[l], (Pl / 4) * c);
       const int ct = u->ch(l + 1) + c;
-      A(a.cat[l], Pl * ct); A(a.gcat[l], Pl * ct);
+      A(a.gcat[l], Pl * ct);
       A(a.d1[l], Pl * c); A(a.d2[l], Pl * c); A(a.gd1[l], Pl * c); A(a.gd2[l], Pl * c);
       maxt = std::max(maxt, (size_t)(Pl * ct));
       note_conv(u->dec1[l], l);
@@ -163,7 +162,6 @@ huv_status ensure_acts(huv_unet* u, int N, int H, int W) {
   A(a.out, P); A(a.dout, P);
   a.part_floats = std::max(part, (size_t)1);
   A(a.part, a.part_floats);
-  A(a.bpart, std::max(bpart, (size_t)1));
   A(a.hpart, (size_t)kHeadBlocks * (u->base + 1));
   A(a.lpart, kLossBlocks);
 #undef A
@@ -183,77 +181,82 @@ huv_status refresh_bf16(huv_unet* u) {
   return HUV_OK;
 }
 
-huv_status conv_fwd(huv_unet* u, const Conv& c, const bf16_t* x, int l, bf16_t* y) {
+huvk::ConvIn input(const bf16_t* x, int c) { return huvk::ConvIn{x, c}; }
+// The decoder's input at level l: the level below upsampled, then the skip.
+huvk::ConvIn decoder_input(huv_unet* u, int l) {
   const Acts& a = u->a;
-  HCHK(huvk::launch_conv3x3_fwd(x, a.N, a.H >> l, a.W >> l, c.cin, wbf(u, c), u->p + c.b_off,
-                                c.cout, 1, y, S(u)),
+  const bf16_t* up = l == u->levels - 2 ? a.e2[u->levels - 1] : a.d2[l + 1];
+  return huvk::ConvIn{a.e2[l], u->ch(l), up, u->ch(l + 1)};
+}
+
+huv_status conv_fwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, int l, bf16_t* y,
+                    bf16_t* pool = nullptr) {
+  const Acts& a = u->a;
+  HCHK(huvk::launch_conv3x3_fwd(x, a.N, a.H >> l, a.W >> l, wbf(u, c), u->p + c.b_off, c.cout, 1,
+                                nullptr, y, pool, S(u)),
        "U-Net conv forward");
   return HUV_OK;
 }
 
-huv_status forward(huv_unet* u, const float* in) {
+huv_status forward(huv_unet* u, const float* in, float* out) {
   Acts& a = u->a;
   const int L = u->levels;
   const int64_t P = (int64_t)a.N * a.H * a.W;
+  // 32-bit indices of 8-channel groups of the widest tensor (the decoder's input at level 0)
+  HCHK(P * (u->ch(1) + u->ch(0)) / 8 < (1ll << 30) ? hipSuccess : hipErrorInvalidValue,
+       "U-Net size");
   HCHK(huvk::launch_pack_input(in, P, a.x8, S(u)), "U-Net input");
   huv_status st;
   for (int l = 0; l < L; ++l) {
-    const bf16_t* src = l == 0 ? a.x8 : a.pool[l - 1];
+    const huvk::ConvIn src = l == 0 ? input(a.x8, 8) : input(a.pool[l - 1], u->ch(l - 1));
     if ((st = conv_fwd(u, u->enc1[l], src, l, a.e1[l])) != HUV_OK) return st;
-    if ((st = conv_fwd(u, u->enc2[l], a.e1[l], l, a.e2[l])) != HUV_OK) return st;
-    if (l < L - 1)
-      HCHK(huvk::launch_maxpool_fwd(a.e2[l], a.N, a.H >> l, a.W >> l, u->ch(l), a.pool[l], S(u)),
-           "U-Net pool");
+    if ((st = conv_fwd(u, u->enc2[l], input(a.e1[l], u->ch(l)), l, a.e2[l],
+                       l < L - 1 ? a.pool[l] : nullptr)) != HUV_OK)
+      return st;
   }
   for (int l = L - 2; l >= 0; --l) {
-    const bf16_t* up = l == L - 2 ? a.e2[L - 1] : a.d2[l + 1];
-    HCHK(huvk::launch_upcat_fwd(up, u->ch(l + 1), a.e2[l], u->ch(l), a.N, a.H >> l, a.W >> l,
-                                a.cat[l], S(u)),
-         "U-Net upsample");
-    if ((st = conv_fwd(u, u->dec1[l], a.cat[l], l, a.d1[l])) != HUV_OK) return st;
-    if ((st = conv_fwd(u, u->dec2[l], a.d1[l], l, a.d2[l])) != HUV_OK) return st;
+    if ((st = conv_fwd(u, u->dec1[l], decoder_input(u, l), l, a.d1[l])) != HUV_OK) return st;
+    if ((st = conv_fwd(u, u->dec2[l], input(a.d1[l], u->ch(l)), l, a.d2[l])) != HUV_OK) return st;
   }
-  HCHK(huvk::launch_head_fwd(a.d2[0], P, u->base, u->p + u->head_w, u->p + u->head_b, a.out,
-                             S(u)),
+  HCHK(huvk::launch_head_fwd(a.d2[0], P, u->base, u->p + u->head_w, u->p + u->head_b, out, S(u)),
        "U-Net head");
   return HUV_OK;
 }
 
-// Gradients of one conv (+ReLU) layer: masks dy in place, writes dW, db into
-// u->g and (if dx) the input gradient.
-huv_status conv_bwd(huv_unet* u, const Conv& c, const bf16_t* x, const bf16_t* y, bf16_t* dy,
-                    int l, bf16_t* dx) {
+// Gradients of one conv layer from dy (zero where the layer's ReLU was): dW and
+// db into u->g and (if dx) the input gradient, zeroed where dx_mask, the output
+// of the layer that made the input, is not positive.
+huv_status conv_bwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, const bf16_t* dy, int l,
+                    bf16_t* dx, const bf16_t* dx_mask) {
   Acts& a = u->a;
   const int H = a.H >> l, W = a.W >> l;
   const int splits = wgrad_splits(c, a.N, H, W);
+  const int64_t weights = (int64_t)c.cout * 9 * c.cin;
   if (wgrad_nhwc(c, W)) {
-    if (y) HCHK(huvk::launch_relu_mask(dy, y, a.N, H, W, c.cout, S(u)), "U-Net relu mask");
-    HCHK(huvk::launch_conv3x3_wgrad_nhwc(dy, x, a.N, H, W, c.cin, c.cout, splits, a.part, a.bpart,
-                                         S(u)),
+    HCHK(huvk::launch_conv3x3_wgrad_nhwc(dy, x, a.N, H, W, c.cout, splits, a.part, S(u)),
          "U-Net weight gradient");
-    HCHK(huvk::launch_sum_splits(a.part, splits, (int64_t)c.cout * 9 * c.cin, u->g + c.w_off,
-                                 S(u)),
+    // the biases follow the weights in the partials and in the parameters
+    HCHK(huvk::launch_sum_splits(a.part, splits, weights + c.cout, u->g + c.w_off, S(u)),
          "U-Net split sum");
-    HCHK(huvk::launch_sum_splits(a.bpart, splits, c.cout, u->g + c.b_off, S(u)),
-         "U-Net bias split sum");
-    if (dx)
-      HCHK(huvk::launch_conv3x3_fwd(dy, a.N, H, W, c.cout, wrot(u, c), nullptr, c.cin, 0, dx,
-                                    S(u)),
-           "U-Net data gradient");
-    return HUV_OK;
+  } else {
+    const bf16_t* xin = x.X;
+    if (x.Cu > 0) {
+      HCHK(huvk::launch_upcat_fwd(x.U, x.Cu, x.X, x.C, a.N, H, W, a.tmp, S(u)), "U-Net upsample");
+      xin = a.tmp;
+    }
+    HCHK(huvk::launch_nhwc_to_nchw(dy, a.N, H, W, c.cout, a.dyt, S(u)), "U-Net transpose");
+    HCHK(huvk::launch_nhwc_to_nchw(xin, a.N, H, W, c.cin, a.xt, S(u)), "U-Net transpose");
+    HCHK(huvk::launch_conv3x3_wgrad(a.dyt, a.xt, a.N, H, W, c.cin, c.cout, splits, a.part, S(u)),
+         "U-Net weight gradient");
+    HCHK(huvk::launch_sum_splits(a.part, splits, weights, u->g + c.w_off, S(u)), "U-Net split sum");
+    // bias partials reuse the (already consumed) weight-gradient split buffer
+    const int bsplits = bias_splits(c, a.N, H, W);
+    HCHK(huvk::launch_channel_sum(a.dyt, a.N, H * W, c.cout, a.part, bsplits, u->g + c.b_off, S(u)),
+         "U-Net bias gradient");
   }
-  HCHK(huvk::launch_relu_mask_t(dy, y, a.N, H, W, c.cout, a.dyt, S(u)), "U-Net relu mask");
-  HCHK(huvk::launch_nhwc_to_nchw(x, a.N, H, W, c.cin, a.xt, S(u)), "U-Net transpose");
-  HCHK(huvk::launch_conv3x3_wgrad(a.dyt, a.xt, a.N, H, W, c.cin, c.cout, splits, a.part, S(u)),
-       "U-Net weight gradient");
-  HCHK(huvk::launch_sum_splits(a.part, splits, (int64_t)c.cout * 9 * c.cin, u->g + c.w_off, S(u)),
-       "U-Net split sum");
-  // bias partials reuse the (already consumed) weight-gradient split buffer
-  const int bsplits = bias_splits(c, a.N, H, W);
-  HCHK(huvk::launch_channel_sum(a.dyt, a.N, H * W, c.cout, a.part, bsplits, u->g + c.b_off, S(u)),
-       "U-Net bias gradient");
   if (dx)
-    HCHK(huvk::launch_conv3x3_fwd(dy, a.N, H, W, c.cout, wrot(u, c), nullptr, c.cin, 0, dx, S(u)),
+    HCHK(huvk::launch_conv3x3_fwd(input(dy, c.cout), a.N, H, W, wrot(u, c), nullptr, c.cin, 0,
+                                  dx_mask, dx, nullptr, S(u)),
          "U-Net data gradient");
   return HUV_OK;
 }
@@ -270,24 +273,24 @@ huv_status backward(huv_unet* u) {
        "U-Net head sum");
   huv_status st;
   for (int l = 0; l <= L - 2; ++l) {
-    if ((st = conv_bwd(u, u->dec2[l], a.d1[l], a.d2[l], a.gd2[l], l, a.gd1[l])) != HUV_OK) return st;
-    if ((st = conv_bwd(u, u->dec1[l], a.cat[l], a.d1[l], a.gd1[l], l, a.gcat[l])) != HUV_OK) return st;
+    const huvk::ConvIn cat = decoder_input(u, l);
+    if ((st = conv_bwd(u, u->dec2[l], input(a.d1[l], u->ch(l)), a.gd2[l], l, a.gd1[l], a.d1[l])) != HUV_OK)
+      return st;
+    if ((st = conv_bwd(u, u->dec1[l], cat, a.gd1[l], l, a.gcat[l], nullptr)) != HUV_OK) return st;
     bf16_t* gup = l == L - 2 ? a.ge2[L - 1] : a.gd2[l + 1];
-    HCHK(huvk::launch_upcat_bwd(a.gcat[l], u->ch(l + 1), u->ch(l), a.N, a.H >> l, a.W >> l, gup,
-                                a.ge2[l], 0, S(u)),
+    HCHK(huvk::launch_upcat_bwd_u(a.gcat[l], cat.Cu, cat.C, a.N, a.H >> l, a.W >> l, cat.U, gup,
+                                  S(u)),
          "U-Net upsample gradient");
   }
   for (int l = L - 1; l >= 0; --l) {
-    const int H = a.H >> l, W = a.W >> l;
-    if (l < L - 1) {
-      HCHK(huvk::launch_maxpool_bwd(a.e2[l], a.gpool[l], a.N, H, W, u->ch(l), a.tmp, S(u)),
-           "U-Net pool gradient");
-      HCHK(huvk::launch_add_bf16(a.ge2[l], a.tmp, (int64_t)a.N * H * W * u->ch(l), S(u)),
+    if (l < L - 1)
+      HCHK(huvk::launch_skip_pool_bwd(a.e2[l], a.gpool[l], a.gcat[l], u->ch(l + 1), a.N, a.H >> l,
+                                      a.W >> l, u->ch(l), a.ge2[l], S(u)),
            "U-Net skip gradient");
-    }
-    if ((st = conv_bwd(u, u->enc2[l], a.e1[l], a.e2[l], a.ge2[l], l, a.ge1[l])) != HUV_OK) return st;
-    const bf16_t* src = l == 0 ? a.x8 : a.pool[l - 1];
-    if ((st = conv_bwd(u, u->enc1[l], src, a.e1[l], a.ge1[l], l, l == 0 ? nullptr : a.gpool[l - 1])) != HUV_OK)
+    if ((st = conv_bwd(u, u->enc2[l], input(a.e1[l], u->ch(l)), a.ge2[l], l, a.ge1[l], a.e1[l])) != HUV_OK)
+      return st;
+    const huvk::ConvIn src = l == 0 ? input(a.x8, 8) : input(a.pool[l - 1], u->ch(l - 1));
+    if ((st = conv_bwd(u, u->enc1[l], src, a.ge1[l], l, l == 0 ? nullptr : a.gpool[l - 1], nullptr)) != HUV_OK)
       return st;
   }
   return HUV_OK;
@@ -437,11 +440,7 @@ huv_status huv_unet_forward(huv_unet* u, int N, int H, int W, const float* in, f
   std::lock_guard<std::mutex> lk(u->ctx->mu);
   hipSetDevice(u->ctx->device);
   if ((st = ensure_acts(u, N, H, W)) != HUV_OK) return st;
-  if ((st = forward(u, in)) != HUV_OK) return st;
-  HCHK(hipMemcpyAsync(out, u->a.out, (size_t)N * H * W * sizeof(float), hipMemcpyDeviceToDevice,
-                      S(u)),
-       "U-Net output copy");
-  return HUV_OK;
+  return forward(u, in, out);
 }
 
 huv_status huv_unet_loss_grad(huv_unet* u, int N, int H, int W, const float* in,
@@ -452,7 +451,7 @@ huv_status huv_unet_loss_grad(huv_unet* u, int N, int H, int W, const float* in,
   std::lock_guard<std::mutex> lk(u->ctx->mu);
   hipSetDevice(u->ctx->device);
   if ((st = ensure_acts(u, N, H, W)) != HUV_OK) return st;
-  if ((st = forward(u, in)) != HUV_OK) return st;
+  if ((st = forward(u, in, u->a.out)) != HUV_OK) return st;
   const int64_t P = (int64_t)N * H * W;
   HCHK(huvk::launch_mse(u->a.out, target, P, u->a.dout, u->a.lpart, kLossBlocks, S(u)), "U-Net loss");
   if ((st = backward(u)) != HUV_OK) return st;

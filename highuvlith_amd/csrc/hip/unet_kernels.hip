@@ -18,6 +18,8 @@
 //             words.  Split-K partials are summed in a fixed order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "unet_kernels.hpp"
 
 namespace huvk {
@@ -38,17 +40,38 @@ __device__ __forceinline__ bf16x8 ld8(const bf16_t* p) {
 }
 __device__ __forceinline__ bf16x8 zero8() { return __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0)); }
 
+// Eight BF16 values as one 16-byte word.
+union B8 {
+  uint4 u;
+  bf16_t h[8];
+};
+
+// The maximum of four, channel by channel, keeping the winner's bits.
+__device__ __forceinline__ B8 max4(const B8& v0, const B8& v1, const B8& v2, const B8& v3) {
+  B8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    bf16_t m = v0.h[e];
+    if (bf2f(v1.h[e]) > bf2f(m)) m = v1.h[e];
+    if (bf2f(v2.h[e]) > bf2f(m)) m = v2.h[e];
+    if (bf2f(v3.h[e]) > bf2f(m)) m = v3.h[e];
+    o.h[e] = m;
+  }
+  return o;
+}
+
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution.  Work-group = 4 waves along pixels; each wave
 // computes BM x BN blocks of 32 pixels x 32 output channels.  The operands
 // of step s + 1 are loaded before the products of step s are issued.
 // ---------------------------------------------------------------------------
 template <int BM, int BN>
-__global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ X, int N, int H,
-                                                     int W, int Cin,
+__global__ __launch_bounds__(256) void k_conv3x3_fwd(ConvIn in, int N, int H, int W,
                                                      const bf16_t* __restrict__ Wt,
                                                      const float* __restrict__ bias, int Cout,
-                                                     int relu, bf16_t* __restrict__ Y) {
+                                                     int relu, const bf16_t* __restrict__ mask,
+                                                     bf16_t* __restrict__ Y) {
+  const int Cin = in.Cu + in.C;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int half = lane >> 5, li = lane & 31;
   const int64_t NP = (int64_t)N * H * W;
@@ -82,7 +105,7 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ 
     for (int bm = 0; bm < BM; ++bm) {
       const int yy = py[bm] + dy, xx = px[bm] + dx;
       const bool v = kv && pv[bm] && yy >= 0 && yy < H && xx >= 0 && xx < W;
-      a[bm] = v ? ld8(X + (((int64_t)pn[bm] * H + yy) * W + xx) * Cin + cb * 8) : zero8();
+      a[bm] = v ? ld8(in.at(pn[bm], yy, xx, H, W, cb * 8)) : zero8();
     }
 #pragma unroll
     for (int bn = 0; bn < BN; ++bn) {
@@ -125,7 +148,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ 
         if (p < NP) {
           float v = acc[bm][bn][r] + bv;
           if (relu) v = fmaxf(v, 0.f);
-          Y[p * Cout + co[bn]] = f2bf(v);
+          const bool off = mask && bf2f(mask[p * Cout + co[bn]]) <= 0.f;
+          Y[p * Cout + co[bn]] = off ? (bf16_t)0 : f2bf(v);
         }
       }
   }
@@ -134,41 +158,51 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ 
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution with the input and the weights staged in LDS.
 // Work-group = 4 waves over an output tile of TH = 2 BM rows x 64 columns of
-// one image; wave w takes columns x0 + 32 (w % 2) .. + 31 of rows
-// y0 + w / 2 + 2 b (b < BM), and BN blocks of 32 output channels, so one
-// weight fragment feeds BM products.  Input channels run in chunks of CC:
-// the (TH + 2) x (64 + 2) x CC halo and the chunk's 9 x CC weights of the
-// 32 BN output channels are loaded once per chunk (zero outside the image
-// and beyond Cout) and read by all four waves from LDS; A = 32 pixels x 16 k
-// per MFMA step (two 8-channel blocks of (tap, channel) index 2s and
-// 2s + 1), B = 16 k x 32 output channels.  Needs W % 64 == 0 and
-// H % TH == 0.
+// one image; wave w takes columns x0 + 32 (w % 2) .. + 31 of the BM rows from
+// y0 + BM (w / 2), and BN blocks of 32 output channels, so one weight fragment
+// feeds BM products.  Input channels run in chunks of CC: the (TH + 2) x (64 + 2)
+// x CC halo and the chunk's 9 x CC weights of the 32 BN output channels are
+// loaded once per chunk (zero outside the image and beyond Cout) and read by all
+// four waves from LDS; A = 32 pixels x 16 k per MFMA step (two 8-channel blocks of
+// (tap, channel) index 2s and 2s + 1), B = 16 k x 32 output channels.  Needs
+// W % 64 == 0 and H % TH == 0.
+//
+// The output leaves through LDS in 16-byte runs of channels, where the ReLU mask
+// of the layer below (mask: dX zeroed where that layer's output is not positive)
+// and the 2 x 2 maximum (pool) cost no pass of their own; the decoder's input is
+// read from its two sources (the half-resolution map and the skip), so the
+// concatenation is never written.  A forward pass of 32 fields of 512^2 (4 levels,
+// base 32): 5222 -> 3790 us with the three passes gone; the loss gradient of 8 of
+// them 6273 -> 5194 us, with the masks, the sum and the pooling of the backward
+// pass fused likewise.  What bounds it: the LDS (two 16-byte reads per 1 1/3 products
+// of a wave) and the waits between the chunks' loads and their products.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int CC>
-__global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(const bf16_t* __restrict__ X, int N,
-                                                         int H, int W, int Cin,
+__global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H, int W,
                                                          const bf16_t* __restrict__ Wt,
                                                          const float* __restrict__ bias, int Cout,
-                                                         int relu, bf16_t* __restrict__ Y) {
+                                                         int relu, const bf16_t* __restrict__ mask,
+                                                         bf16_t* __restrict__ Y,
+                                                         bf16_t* __restrict__ pool) {
   constexpr int TH = 2 * BM, TW = 64, HR = TH + 2, HC = TW + 2;
   constexpr int PS = CC + 8;  // pixel stride in the tile (bf16), spreads the LDS banks
   constexpr int CB = CC / 8, KBC = 9 * CB, STEPS = (KBC + 1) / 2;
-  constexpr int WS = 9 * CC + 8;  // output-channel stride of the staged weights (bf16)
-  __shared__ __attribute__((aligned(16))) bf16_t tile[HR * HC * PS];
+  constexpr int WS = 9 * CC + 8;   // output-channel stride of the staged weights (bf16)
+  constexpr int OS = 32 * BN + 8;  // pixel stride of the staged output (bf16)
+  constexpr int IN_LDS = HR * HC * PS, OUT_LDS = TH * TW * OS;
+  __shared__ __attribute__((aligned(16))) bf16_t tile[IN_LDS > OUT_LDS ? IN_LDS : OUT_LDS];
   __shared__ __attribute__((aligned(16))) bf16_t wts[32 * BN * WS];
+  const int Cin = in.Cu + in.C;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int half = lane >> 5, li = lane & 31;
   const int tilesX = W / TW, tilesY = H / TH;
-  int blk = blockIdx.x;
-  const int tx = blk % tilesX;
-  blk /= tilesX;
-  const int ty = blk % tilesY, n = blk / tilesY;
-  const int x0 = tx * TW, y0 = ty * TH;
+  const int x0 = (int)blockIdx.x % tilesX * TW, y0 = (int)blockIdx.x / tilesX % tilesY * TH;
+  const int n = (int)blockIdx.x / (tilesX * tilesY);
   const int cobase = blockIdx.y * 32 * BN;
   const int px = 32 * (wave & 1) + li;  // this lane's A row (pixel column) in the tile
-  int co[BN];
-#pragma unroll
-  for (int bn = 0; bn < BN; ++bn) co[bn] = cobase + 32 * bn + li;
+  const int py0 = BM * (wave >> 1);     // first output row of the wave in the tile
+  constexpr int HALO = HR * HC * CB, HIT = (HALO + 255) / 256;
+  constexpr int WGT = 32 * BN * KBC, WIT = (WGT + 255) / 256;
   f32x16 acc[BM][BN];
 #pragma unroll
   for (int bm = 0; bm < BM; ++bm)
@@ -176,31 +210,41 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(const bf16_t* __restric
     for (int bn = 0; bn < BN; ++bn)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bm][bn][r] = 0.f;
-
   for (int c0 = 0; c0 < Cin; c0 += CC) {
     // Every load of the chunk is issued before the first LDS store, so their
     // latencies overlap.
-    constexpr int HALO = HR * HC * CB, HIT = (HALO + 255) / 256;
-    constexpr int WGT = 32 * BN * KBC, WIT = (WGT + 255) / 256;
+    // Buffer loads with 32-bit offsets into the image (or its half-resolution
+    // part): a pixel outside it, and an output channel beyond Cout, gets an
+    // offset past the end, which reads zero.
     uint4 hv[HIT], wv[WIT];
+    const bool up = c0 < in.Cu;
+    const int sh = up ? 1 : 0, cs = up ? in.Cu : in.C, ws = W >> sh;
+    const int image = (H >> sh) * ws * cs;
+    const bf16_t* src = (up ? in.U : in.X) + (size_t)n * image;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(src), (short)0, image * (int)sizeof(bf16_t), 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(Wt), (short)0, Cout * 9 * Cin * (int)sizeof(bf16_t), 0x00020000);
+    const int soff = (up ? c0 : c0 - in.Cu) * (int)sizeof(bf16_t);
 #pragma unroll
     for (int k = 0; k < HIT; ++k) {
       const int i = threadIdx.x + 256 * k;
       const int cb = i % CB, pix = i / CB;
       const int yy = y0 - 1 + pix / HC, xx = x0 - 1 + pix % HC;
-      hv[k] = make_uint4(0, 0, 0, 0);
-      if (i < HALO && yy >= 0 && yy < H && xx >= 0 && xx < W)
-        hv[k] = *reinterpret_cast<const uint4*>(X + (((size_t)n * H + yy) * W + xx) * Cin + c0 +
-                                                8 * cb);
+      const bool v = i < HALO && yy >= 0 && yy < H && xx >= 0 && xx < W;
+      const int off = (((yy >> sh) * ws + (xx >> sh)) * cs + 8 * cb) * (int)sizeof(bf16_t);
+      hv[k] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(xr, v ? off + soff : -1, 0, 0));
     }
 #pragma unroll
     for (int k = 0; k < WIT; ++k) {
       const int i = threadIdx.x + 256 * k;
       const int kb = i % KBC, col = i / KBC;  // kb = tap * CB + cb
       const int tap = kb / CB, cb = kb % CB, c = cobase + col;
-      wv[k] = make_uint4(0, 0, 0, 0);
-      if (i < WGT && c < Cout)
-        wv[k] = *reinterpret_cast<const uint4*>(Wt + ((size_t)c * 9 + tap) * Cin + c0 + 8 * cb);
+      const bool v = i < WGT && c < Cout;
+      const int off = ((c * 9 + tap) * Cin + c0 + 8 * cb) * (int)sizeof(bf16_t);
+      wv[k] = __builtin_bit_cast(uint4,
+                                 __builtin_amdgcn_raw_buffer_load_b128(wr, v ? off : -1, 0, 0));
     }
     __syncthreads();  // the previous chunk has been consumed
 #pragma unroll
@@ -228,8 +272,7 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(const bf16_t* __restric
       }
 #pragma unroll
       for (int bm = 0; bm < BM; ++bm) {
-        const int py = (wave >> 1) + 2 * bm;
-        const bf16x8 a0 = ld8(tile + ((py + dy) * HC + px + dx) * PS + 8 * cb);
+        const bf16x8 a0 = ld8(tile + ((py0 + bm + dy) * HC + px + dx) * PS + 8 * cb);
         const bf16x8 a = kv ? a0 : zero8();
 #pragma unroll
         for (int bn = 0; bn < BN; ++bn)
@@ -237,21 +280,52 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(const bf16_t* __restric
       }
     }
   }
+  __syncthreads();  // the tile has been read by every wave
 #pragma unroll
-  for (int bm = 0; bm < BM; ++bm) {
-    const size_t prow = ((size_t)n * H + y0 + (wave >> 1) + 2 * bm) * W + x0 + 32 * (wave & 1);
+  for (int bn = 0; bn < BN; ++bn) {
+    const int co = cobase + 32 * bn + li;
+    const float bv = bias && co < Cout ? bias[co] : 0.f;
 #pragma unroll
-    for (int bn = 0; bn < BN; ++bn) {
-      if (co[bn] >= Cout) continue;
-      const float bv = bias ? bias[co[bn]] : 0.f;
+    for (int bm = 0; bm < BM; ++bm)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int i = 8 * (r / 4) + 4 * half + (r % 4);
         float v = acc[bm][bn][r] + bv;
         if (relu) v = fmaxf(v, 0.f);
-        Y[(prow + i) * Cout + co[bn]] = f2bf(v);
+        tile[((py0 + bm) * TW + 32 * (wave & 1) + i) * OS + 32 * bn + li] = f2bf(v);
       }
+  }
+  __syncthreads();
+  constexpr int G8 = 4 * BN;  // 8-channel groups of the block
+  for (int i = threadIdx.x; i < TH * TW * G8; i += 256) {
+    const int g = i % G8, q = i / G8, c = cobase + 8 * g;
+    if (c >= Cout) continue;
+    const size_t at = (((size_t)n * H + y0 + q / TW) * W + x0 + q % TW) * Cout + c;
+    B8 v;
+    v.u = *reinterpret_cast<const uint4*>(tile + q * OS + 8 * g);
+    if (mask) {
+      B8 y;
+      y.u = *reinterpret_cast<const uint4*>(mask + at);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (bf2f(y.h[e]) <= 0.f) v.h[e] = 0;
     }
+    *reinterpret_cast<uint4*>(Y + at) = v.u;
+  }
+  if (!pool) return;
+  for (int i = threadIdx.x; i < TH * TW / 4 * G8; i += 256) {
+    const int g = i % G8, q = i / G8, c = cobase + 8 * g;
+    if (c >= Cout) continue;
+    const int yo = q / (TW / 2), xo = q % (TW / 2);
+    const bf16_t* b = tile + (2 * yo * TW + 2 * xo) * OS + 8 * g;
+    B8 v0, v1, v2, v3;
+    v0.u = *reinterpret_cast<const uint4*>(b);
+    v1.u = *reinterpret_cast<const uint4*>(b + OS);
+    v2.u = *reinterpret_cast<const uint4*>(b + TW * OS);
+    v3.u = *reinterpret_cast<const uint4*>(b + (TW + 1) * OS);
+    *reinterpret_cast<uint4*>(
+        pool + (((size_t)n * (H / 2) + y0 / 2 + yo) * (W / 2) + x0 / 2 + xo) * Cout + c) =
+        max4(v0, v1, v2, v3).u;
   }
 }
 
@@ -268,21 +342,12 @@ __global__ void k_conv_weight_rot(const bf16_t* __restrict__ Wt, int Cout, int C
   }
 }
 
-// Eight BF16 values as one 16-byte word.
-union B8 {
-  uint4 u;
-  bf16_t h[8];
-};
-
 // ---------------------------------------------------------------------------
 // NHWC -> NCHW through a 64-pixel x 32-channel LDS tile (HW % 64 == 0, C % 8
 // == 0): each thread reads one 16-byte run of 8 channels of a pixel and
-// writes one 16-byte run of 8 pixels of a channel.  MASK: the ReLU mask of
-// the backward pass, dY zeroed (in place, and in the copy) where Y <= 0.
+// writes one 16-byte run of 8 pixels of a channel.
 // ---------------------------------------------------------------------------
-template <bool MASK>
-__global__ __launch_bounds__(256) void k_transpose_t(bf16_t* __restrict__ dY,
-                                                     const bf16_t* __restrict__ Y, int N, int HW,
+__global__ __launch_bounds__(256) void k_transpose_t(const bf16_t* __restrict__ X, int N, int HW,
                                                      int C, bf16_t* __restrict__ out) {
   constexpr int TP = 64, TC = 32, LP = TP + 8;  // padded pixel stride (16-byte aligned rows)
   __shared__ __align__(16) bf16_t tile[TC][LP];
@@ -291,21 +356,8 @@ __global__ __launch_bounds__(256) void k_transpose_t(bf16_t* __restrict__ dY,
   {
     const int px = threadIdx.x >> 2, ch = 8 * (threadIdx.x & 3);
     if (c0 + ch < C) {
-      const int64_t idx = (p0 + px) * C + c0 + ch;
       B8 v;
-      v.u = *reinterpret_cast<const uint4*>(dY + idx);
-      if (MASK && Y) {
-        B8 y;
-        y.u = *reinterpret_cast<const uint4*>(Y + idx);
-        bool any = false;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (bf2f(y.h[k]) <= 0.f) {
-            v.h[k] = 0;
-            any = true;
-          }
-        if (any) *reinterpret_cast<uint4*>(dY + idx) = v.u;
-      }
+      v.u = *reinterpret_cast<const uint4*>(X + (p0 + px) * C + c0 + ch);
 #pragma unroll
       for (int k = 0; k < 8; ++k) tile[ch + k][px] = v.h[k];
     }
@@ -461,12 +513,14 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad(const bf16_t* __restrict_
 // kx - 1 pixels (the one- and two-pixel shifts are funnel shifts of the
 // aligned word and the next), acc[kx] += A B, so each wave owns its three
 // taps outright.  Wave 0 of the work-groups of input block 0 also sums dY
-// over the pixels (the bias gradient).  part[split][co][tap][ci],
-// bpart[split][co].  Needs W % 64 == 0, Cin % 8 == 0, Cout % 8 == 0.
+// over the pixels (the bias gradient).  part[split]: [co][tap][ci], then [co]
+// biases (the order of the parameters).  Needs W % 64 == 0, Cin % 8 == 0, Cout % 8 == 0.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(192) void k_conv3x3_wgrad_nhwc(
-    const bf16_t* __restrict__ dY, const bf16_t* __restrict__ X, int N, int H, int W, int Cin,
-    int Cout, int rows_per_split, float* __restrict__ part, float* __restrict__ bpart) {
+    const bf16_t* __restrict__ dY, ConvIn in, int N, int H, int W, int Cout, int rows_per_split,
+    float* __restrict__ part) {
+  const int Cin = in.Cu + in.C;
+  const size_t stride = (size_t)Cout * 9 * Cin + Cout;  // a split's weights, then biases
   constexpr int SEG = 64, LP = SEG + 8;  // staged rows: 72 pixels (66 used), 16-byte aligned
   constexpr int NT = 192;
   constexpr int DT = SEG * 4, DI = (DT + NT - 1) / NT;            // dY: 64 px x 4 groups
@@ -483,7 +537,7 @@ __global__ __launch_bounds__(192) void k_conv3x3_wgrad_nhwc(
   const int split = blockIdx.y;
   const int rows = N * H;
   const int r0 = split * rows_per_split, r1 = min(rows, r0 + rows_per_split);
-  const bool bias = bpart != nullptr && cib == 0 && ky == 0;
+  const bool bias = cib == 0 && ky == 0;
   f32x16 acc[3];
 #pragma unroll
   for (int b = 0; b < 3; ++b)
@@ -503,8 +557,7 @@ __global__ __launch_bounds__(192) void k_conv3x3_wgrad_nhwc(
         const int jj = rem >> 2, cg = rem & 3;
         const int yy = yfirst + r, xx = x0 + jj - 1;
         if (r < nrow && yy >= 0 && yy < H && xx >= 0 && xx < W && ci0 + 8 * cg < Cin)
-          return *reinterpret_cast<const uint4*>(X + (((size_t)n * H + yy) * W + xx) * Cin + ci0 +
-                                                 8 * cg);
+          return *reinterpret_cast<const uint4*>(in.at(n, yy, xx, H, W, ci0 + 8 * cg));
         return make_uint4(0, 0, 0, 0);
       };
       auto x_store = [&](int t, const B8& v) {
@@ -590,30 +643,12 @@ __global__ __launch_bounds__(192) void k_conv3x3_wgrad_nhwc(
     for (int r = 0; r < 16; ++r) {
       const int co = co0 + 8 * (r / 4) + 4 * half + (r % 4);
       if (co < Cout && ci < Cin)
-        part[(((size_t)split * Cout + co) * 9 + 3 * ky + kx) * Cin + ci] = acc[kx][r];
+        part[(size_t)split * stride + ((size_t)co * 9 + 3 * ky + kx) * Cin + ci] = acc[kx][r];
     }
   if (bias) {
     bsum += __shfl_xor(bsum, 32);  // the two pixel halves of channel li
-    if (half == 0 && co0 + li < Cout) bpart[(size_t)split * Cout + co0 + li] = bsum;
-  }
-}
-
-// dY *= (Y > 0), in place (NHWC, 8 channels per thread).
-__global__ void k_relu_mask(bf16_t* __restrict__ dY, const bf16_t* __restrict__ Y,
-                            int64_t count8) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count8;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    B8 v, yv;
-    v.u = reinterpret_cast<const uint4*>(dY)[i];
-    yv.u = reinterpret_cast<const uint4*>(Y)[i];
-    bool any = false;
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (bf2f(yv.h[k]) <= 0.f) {
-        v.h[k] = 0;
-        any = true;
-      }
-    if (any) reinterpret_cast<uint4*>(dY)[i] = v.u;
+    if (half == 0 && co0 + li < Cout)
+      part[(size_t)split * stride + (size_t)Cout * 9 * Cin + co0 + li] = bsum;
   }
 }
 
@@ -686,34 +721,32 @@ __global__ void k_maxpool_fwd(const bf16_t* __restrict__ X, int N, int H, int W,
     const bf16_t* b = X + (((size_t)n * H + 2 * yo) * W + 2 * xo) * C + 8 * g;
     const B8 v0 = ld_b8(b), v1 = ld_b8(b + C), v2 = ld_b8(b + (size_t)W * C),
              v3 = ld_b8(b + (size_t)W * C + C);
-    B8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      // the maximum is one of the inputs: keep its bits (no rounding)
-      bf16_t m = v0.h[e];
-      if (bf2f(v1.h[e]) > bf2f(m)) m = v1.h[e];
-      if (bf2f(v2.h[e]) > bf2f(m)) m = v2.h[e];
-      if (bf2f(v3.h[e]) > bf2f(m)) m = v3.h[e];
-      o.h[e] = m;
-    }
+    const B8 o = max4(v0, v1, v2, v3);
     st_b8(Y + (size_t)q * C + 8 * g, o);
   }
 }
 
-// dX: dY routed to the first maximum of each 2 x 2 window, zero elsewhere.
-__global__ void k_maxpool_bwd(const bf16_t* __restrict__ X, const bf16_t* __restrict__ dY, int N,
-                              int H, int W, int C, bf16_t* __restrict__ dX) {
-  const int Ho = H / 2, Wo = W / 2, G = C / 8;
+// The gradient of an encoder level's output X (N, H, W, C): dP (of the pooled
+// map) routed to the first maximum of each 2 x 2 window, added to the skip's part
+// of dcat (channels Cu .. Cu + C - 1 of Cu + C), zero where X is not positive (the
+// ReLU that made X): one pass over the four tensors.
+__global__ void k_skip_pool_bwd(const bf16_t* __restrict__ X, const bf16_t* __restrict__ dP,
+                                const bf16_t* __restrict__ dcat, int Cu, int N, int H, int W,
+                                int C, bf16_t* __restrict__ dX) {
+  const int Ho = H / 2, Wo = W / 2, G = C / 8, Ct = Cu + C;
   const int total = N * Ho * Wo * G;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
     const int g = i % G, q = i / G;
     const int xo = q % Wo, t = q / Wo, yo = t % Ho, n = t / Ho;
-    const size_t base = (((size_t)n * H + 2 * yo) * W + 2 * xo) * C + 8 * g;
-    const size_t o[4] = {0, (size_t)C, (size_t)W * C, (size_t)W * C + C};
+    const size_t p = ((size_t)n * H + 2 * yo) * W + 2 * xo;
+    const size_t o[4] = {p, p + 1, p + W, p + W + 1};
     B8 v[4], d[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = ld_b8(X + base + o[k]);
-    const B8 dy = ld_b8(dY + (size_t)q * C + 8 * g);
+    for (int k = 0; k < 4; ++k) {
+      v[k] = ld_b8(X + o[k] * C + 8 * g);
+      d[k] = ld_b8(dcat + o[k] * Ct + Cu + 8 * g);
+    }
+    const B8 dy = ld_b8(dP + (size_t)q * C + 8 * g);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       int arg = 0;
@@ -724,10 +757,14 @@ __global__ void k_maxpool_bwd(const bf16_t* __restrict__ X, const bf16_t* __rest
         if (x > m) { m = x; arg = k; }
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) d[k].h[e] = k == arg ? dy.h[e] : (bf16_t)0;
+      for (int k = 0; k < 4; ++k) {
+        const bf16_t r = k == arg ? dy.h[e] : (bf16_t)0;
+        const bf16_t sum = f2bf(bf2f(d[k].h[e]) + bf2f(r));
+        d[k].h[e] = bf2f(v[k].h[e]) <= 0.f ? (bf16_t)0 : sum;
+      }
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) st_b8(dX + base + o[k], d[k]);
+    for (int k = 0; k < 4; ++k) st_b8(dX + o[k] * C + 8 * g, d[k]);
   }
 }
 
@@ -749,9 +786,10 @@ __global__ void k_upcat_fwd(const bf16_t* __restrict__ U, int Cu, const bf16_t* 
   }
 }
 
-// dU = sum of dcat's first Cu channels over each 2 x 2 block
+// dU = sum of dcat's first Cu channels over each 2 x 2 block, zero where U (a
+// ReLU's output) is not positive
 __global__ void k_upcat_bwd_u(const bf16_t* __restrict__ dcat, int Cu, int Cs, int N, int H,
-                              int W, bf16_t* __restrict__ dU) {
+                              int W, const bf16_t* __restrict__ U, bf16_t* __restrict__ dU) {
   const int Ct = Cu + Cs, Hh = H / 2, Wh = W / 2, G = Cu / 8;
   const int total = N * Hh * Wh * G;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
@@ -760,34 +798,14 @@ __global__ void k_upcat_bwd_u(const bf16_t* __restrict__ dcat, int Cu, int Cs, i
     const size_t b = (((size_t)n * H + 2 * y) * W + 2 * x) * Ct + 8 * g;
     const B8 a0 = ld_b8(dcat + b), a1 = ld_b8(dcat + b + Ct), a2 = ld_b8(dcat + b + (size_t)W * Ct),
              a3 = ld_b8(dcat + b + (size_t)W * Ct + Ct);
+    const B8 u = ld_b8(U + (size_t)q * Cu + 8 * g);
     B8 o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      o.h[e] = f2bf((bf2f(a0.h[e]) + bf2f(a1.h[e])) + (bf2f(a2.h[e]) + bf2f(a3.h[e])));
-    st_b8(dU + (size_t)q * Cu + 8 * g, o);
-  }
-}
-
-// dS (+)= dcat's last Cs channels
-__global__ void k_upcat_bwd_s(const bf16_t* __restrict__ dcat, int Cu, int Cs, int64_t P,
-                              bf16_t* __restrict__ dS, int accumulate) {
-  const int Ct = Cu + Cs, G = Cs / 8;
-  const int64_t total = P * G;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int g = (int)(i % G);
-    const int64_t p = i / G;
-    const B8 v = ld_b8(dcat + (size_t)p * Ct + Cu + 8 * g);
-    bf16_t* d = dS + (size_t)p * Cs + 8 * g;
-    if (accumulate) {
-      const B8 w = ld_b8(d);
-      B8 o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o.h[e] = f2bf(bf2f(w.h[e]) + bf2f(v.h[e]));
-      st_b8(d, o);
-    } else {
-      st_b8(d, v);
+    for (int e = 0; e < 8; ++e) {
+      const bf16_t sum = f2bf((bf2f(a0.h[e]) + bf2f(a1.h[e])) + (bf2f(a2.h[e]) + bf2f(a3.h[e])));
+      o.h[e] = bf2f(u.h[e]) <= 0.f ? (bf16_t)0 : sum;
     }
+    st_b8(dU + (size_t)q * Cu + 8 * g, o);
   }
 }
 
@@ -810,16 +828,25 @@ __global__ __launch_bounds__(kHeadThreads) void k_head_bwd(
     const bf16_t* __restrict__ Y, const float* __restrict__ dout, int64_t P,
     const float* __restrict__ w, bf16_t* __restrict__ dY, float* __restrict__ part) {
   __shared__ float sh[kHeadThreads];
-  float acc[C + 1];
+  float acc[C + 1], wr[C];
 #pragma unroll
   for (int c = 0; c <= C; ++c) acc[c] = 0.f;
+#pragma unroll
+  for (int c = 0; c < C; ++c) wr[c] = w[c];
   for (int64_t p = blockIdx.x * (int64_t)kHeadThreads + threadIdx.x; p < P;
        p += (int64_t)gridDim.x * kHeadThreads) {
     const float g = dout[p];
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-      dY[p * C + c] = f2bf(g * w[c]);
-      acc[c] += g * bf2f(Y[p * C + c]);
+    for (int c8 = 0; c8 < C; c8 += 8) {
+      const B8 y = ld_b8(Y + p * C + c8);
+      B8 d;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = bf2f(y.h[e]);
+        d.h[e] = v <= 0.f ? (bf16_t)0 : f2bf(g * wr[c8 + e]);  // the ReLU that made Y
+        acc[c8 + e] += g * v;
+      }
+      st_b8(dY + p * C + c8, d);
     }
     acc[C] += g;
   }
@@ -867,12 +894,6 @@ __global__ void k_pack_input(const float* __restrict__ in, int64_t P, bf16_t* __
   }
 }
 
-__global__ void k_add_bf16(bf16_t* __restrict__ dS, const bf16_t* __restrict__ dX, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    dS[i] = f2bf(bf2f(dS[i]) + bf2f(dX[i]));
-}
-
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                        float* __restrict__ v, int64_t n, float lr, float b1, float b2, float eps,
                        float c1, float c2) {
@@ -903,25 +924,32 @@ static dim3 grid1d(int64_t n, int threads = 256) {
   return dim3((unsigned)b);
 }
 
-hipError_t launch_conv3x3_fwd(const bf16_t* X, int N, int H, int W, int Cin, const bf16_t* Wt,
-                              const float* bias, int Cout, int relu, bf16_t* Y, hipStream_t s) {
-  if (Cin % 8 != 0 || Cout < 1 || N < 1 || H < 1 || W < 1) return hipErrorInvalidValue;
+hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_t* Wt,
+                              const float* bias, int Cout, int relu, const bf16_t* mask, bf16_t* Y,
+                              bf16_t* pool, hipStream_t s) {
+  const int Cin = in.Cu + in.C;
+  if (in.C % 8 != 0 || in.Cu % 8 != 0 || Cout % 8 != 0 || Cout < 8 || N < 1 || H < 1 || W < 1 ||
+      (pool && (H % 2 != 0 || W % 2 != 0)))
+    return hipErrorInvalidValue;
   const int64_t NP = (int64_t)N * H * W;
-  if (W % 64 == 0 && H % 4 == 0 && Cin % 8 == 0 && (Cin <= 16 || Cin % 16 == 0) &&
-      (int64_t)N * (H / 4) * (W / 64) < (1ll << 31)) {
+  // a chunk of input channels comes from one source
+  const int chunk = Cin == 8 ? 8 : Cin % 32 != 0 || in.Cu % 32 != 0 ? 16 : 32;
+  if (W % 64 == 0 && H % 4 == 0 && Cin % chunk == 0 && in.Cu % chunk == 0 &&
+      (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) &&
+      (int64_t)H * W * std::max(in.C, in.Cu) < (1ll << 30)) {  // 32-bit byte offsets
     // tiles of 4 rows x 64 columns: BM = 2 pixel blocks per wave
     dim3 grid((unsigned)((int64_t)N * (H / 4) * (W / 64)),
               (unsigned)((Cout + (Cout <= 32 ? 31 : 63)) / (Cout <= 32 ? 32 : 64)));
-#define HUV_CONV_LDS(BN_, CC_)                                                                    \
-  hipLaunchKernelGGL((k_conv3x3_fwd_lds<2, BN_, CC_>), grid, dim3(256), 0, s, X, N, H, W, Cin, Wt, \
-                     bias, Cout, relu, Y)
+#define HUV_CONV_LDS(BN_, CC_)                                                                  \
+  hipLaunchKernelGGL((k_conv3x3_fwd_lds<2, BN_, CC_>), grid, dim3(256), 0, s, in, N, H, W, Wt, \
+                     bias, Cout, relu, mask, Y, pool)
     if (Cout <= 32) {
-      if (Cin == 8) HUV_CONV_LDS(1, 8);
-      else if (Cin % 32 != 0) HUV_CONV_LDS(1, 16);
+      if (chunk == 8) HUV_CONV_LDS(1, 8);
+      else if (chunk == 16) HUV_CONV_LDS(1, 16);
       else HUV_CONV_LDS(1, 32);
     } else {
-      if (Cin == 8) HUV_CONV_LDS(2, 8);
-      else if (Cin % 32 != 0) HUV_CONV_LDS(2, 16);
+      if (chunk == 8) HUV_CONV_LDS(2, 8);
+      else if (chunk == 16) HUV_CONV_LDS(2, 16);
       else HUV_CONV_LDS(2, 32);
     }
 #undef HUV_CONV_LDS
@@ -930,14 +958,16 @@ hipError_t launch_conv3x3_fwd(const bf16_t* X, int N, int H, int W, int Cin, con
   constexpr int BM = 2;
   if (Cout <= 32) {
     dim3 grid((unsigned)((NP + 4 * 32 * BM - 1) / (4 * 32 * BM)), (unsigned)((Cout + 31) / 32));
-    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 1>), grid, dim3(256), 0, s, X, N, H, W, Cin, Wt, bias,
-                       Cout, relu, Y);
+    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 1>), grid, dim3(256), 0, s, in, N, H, W, Wt, bias, Cout,
+                       relu, mask, Y);
   } else {
     dim3 grid((unsigned)((NP + 4 * 32 * BM - 1) / (4 * 32 * BM)), (unsigned)((Cout + 63) / 64));
-    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 2>), grid, dim3(256), 0, s, X, N, H, W, Cin, Wt, bias,
-                       Cout, relu, Y);
+    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 2>), grid, dim3(256), 0, s, in, N, H, W, Wt, bias, Cout,
+                       relu, mask, Y);
   }
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !pool) return e;
+  return launch_maxpool_fwd(Y, N, H, W, Cout, pool, s);
 }
 
 hipError_t launch_conv_weight_rot(const bf16_t* Wt, int Cout, int Cin, bf16_t* Wr,
@@ -951,16 +981,7 @@ hipError_t launch_nhwc_to_nchw(const bf16_t* X, int N, int H, int W, int C, bf16
                                hipStream_t s) {
   if ((H * W) % 64 != 0 || C % 8 != 0) return hipErrorInvalidValue;
   dim3 grid((unsigned)((int64_t)N * H * W / 64), (unsigned)((C + 31) / 32));
-  hipLaunchKernelGGL((k_transpose_t<false>), grid, dim3(256), 0, s, const_cast<bf16_t*>(X),
-                     nullptr, N, H * W, C, XT);
-  return hipGetLastError();
-}
-
-hipError_t launch_relu_mask_t(bf16_t* dY, const bf16_t* Y, int N, int H, int W, int C,
-                              bf16_t* dYT, hipStream_t s) {
-  if ((H * W) % 64 != 0 || C % 8 != 0) return hipErrorInvalidValue;
-  dim3 grid((unsigned)((int64_t)N * H * W / 64), (unsigned)((C + 31) / 32));
-  hipLaunchKernelGGL((k_transpose_t<true>), grid, dim3(256), 0, s, dY, Y, N, H * W, C, dYT);
+  hipLaunchKernelGGL(k_transpose_t, grid, dim3(256), 0, s, X, N, H * W, C, XT);
   return hipGetLastError();
 }
 
@@ -982,23 +1003,15 @@ hipError_t launch_conv3x3_wgrad(const bf16_t* dYT, const bf16_t* XT, int N, int 
   return hipGetLastError();
 }
 
-hipError_t launch_conv3x3_wgrad_nhwc(const bf16_t* dY, const bf16_t* X, int N, int H, int W,
-                                     int Cin, int Cout, int splits, float* part, float* bpart,
-                                     hipStream_t s) {
-  if (W % 64 != 0 || Cin % 8 != 0 || Cout % 8 != 0 || splits < 1 || splits > N * H)
+hipError_t launch_conv3x3_wgrad_nhwc(const bf16_t* dY, const ConvIn& in, int N, int H, int W,
+                                     int Cout, int splits, float* part, hipStream_t s) {
+  if (W % 64 != 0 || in.C % 8 != 0 || in.Cu % 8 != 0 || Cout % 8 != 0 || splits < 1 ||
+      splits > N * H)
     return hipErrorInvalidValue;
   const int rps = (N * H + splits - 1) / splits;
-  const int blocks = ((Cout + 31) / 32) * ((Cin + 31) / 32);
-  hipLaunchKernelGGL(k_conv3x3_wgrad_nhwc, dim3(blocks, splits), dim3(192), 0, s, dY, X, N, H, W,
-                     Cin, Cout, rps, part, bpart);
-  return hipGetLastError();
-}
-
-hipError_t launch_relu_mask(bf16_t* dY, const bf16_t* Y, int N, int H, int W, int C,
-                            hipStream_t s) {
-  if (C % 8 != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_relu_mask, grid1d((int64_t)N * H * W * C / 8), dim3(256), 0, s, dY, Y,
-                     (int64_t)N * H * W * C / 8);
+  const int blocks = ((Cout + 31) / 32) * ((in.Cu + in.C + 31) / 32);
+  hipLaunchKernelGGL(k_conv3x3_wgrad_nhwc, dim3(blocks, splits), dim3(192), 0, s, dY, in, N, H, W,
+                     Cout, rps, part);
   return hipGetLastError();
 }
 
@@ -1029,11 +1042,12 @@ hipError_t launch_maxpool_fwd(const bf16_t* X, int N, int H, int W, int C, bf16_
   return hipGetLastError();
 }
 
-hipError_t launch_maxpool_bwd(const bf16_t* X, const bf16_t* dY, int N, int H, int W, int C,
-                              bf16_t* dX, hipStream_t s) {
-  if (C % 8 != 0 || (int64_t)N * H * W * C / 8 >= (1ll << 30)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_maxpool_bwd, grid1d((int64_t)N * (H / 2) * (W / 2) * C / 8), dim3(256), 0,
-                     s, X, dY, N, H, W, C, dX);
+hipError_t launch_skip_pool_bwd(const bf16_t* X, const bf16_t* dP, const bf16_t* dcat, int Cu,
+                                int N, int H, int W, int C, bf16_t* dX, hipStream_t s) {
+  if (C % 8 != 0 || Cu % 8 != 0 || (int64_t)N * H * W * (Cu + C) / 8 >= (1ll << 30))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_skip_pool_bwd, grid1d((int64_t)N * (H / 2) * (W / 2) * C / 8), dim3(256), 0,
+                     s, X, dP, dcat, Cu, N, H, W, C, dX);
   return hipGetLastError();
 }
 
@@ -1046,16 +1060,12 @@ hipError_t launch_upcat_fwd(const bf16_t* U, int Cu, const bf16_t* S, int Cs, in
   return hipGetLastError();
 }
 
-hipError_t launch_upcat_bwd(const bf16_t* dcat, int Cu, int Cs, int N, int H, int W, bf16_t* dU,
-                            bf16_t* dS, int accumulate, hipStream_t s) {
+hipError_t launch_upcat_bwd_u(const bf16_t* dcat, int Cu, int Cs, int N, int H, int W,
+                              const bf16_t* U, bf16_t* dU, hipStream_t s) {
   if (Cu % 8 != 0 || Cs % 8 != 0 || (int64_t)N * H * W * (Cu + Cs) / 8 >= (1ll << 30))
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_upcat_bwd_u, grid1d((int64_t)N * (H / 2) * (W / 2) * Cu / 8), dim3(256), 0,
-                     s, dcat, Cu, Cs, N, H, W, dU);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_upcat_bwd_s, grid1d((int64_t)N * H * W * Cs / 8), dim3(256), 0, s, dcat, Cu,
-                     Cs, (int64_t)N * H * W, dS, accumulate);
+                     s, dcat, Cu, Cs, N, H, W, U, dU);
   return hipGetLastError();
 }
 
@@ -1089,11 +1099,6 @@ hipError_t launch_mse(const float* out, const float* target, int64_t P, float* d
 
 hipError_t launch_pack_input(const float* in, int64_t P, bf16_t* X8, hipStream_t s) {
   hipLaunchKernelGGL(k_pack_input, grid1d(P), dim3(256), 0, s, in, P, X8);
-  return hipGetLastError();
-}
-
-hipError_t launch_add_bf16(bf16_t* dS, const bf16_t* dX, int64_t count, hipStream_t s) {
-  hipLaunchKernelGGL(k_add_bf16, grid1d(count), dim3(256), 0, s, dS, dX, count);
   return hipGetLastError();
 }
 
