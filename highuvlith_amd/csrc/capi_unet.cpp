@@ -95,11 +95,7 @@ bool wgrad_nhwc(const Conv& c, int W) { return W % 64 == 0 && c.cin % 8 == 0 && 
 
 int wgrad_splits(const Conv& c, int N, int H, int W) {
   const int rows = N * H;
-  if (wgrad_nhwc(c, W)) {
-    // about 1024 work-groups (four 3-wave groups per CU)
-    const int tiles = ((c.cout + 31) / 32) * ((c.cin + 31) / 32);
-    return std::max(1, std::min((1024 + tiles - 1) / tiles, rows));
-  }
+  if (wgrad_nhwc(c, W)) return huvk::wgrad_nhwc_splits(N, H, W, c.cin, c.cout);
   const int cob = (c.cout + 31) / 32;
   const int tiles = (cob >= 2 ? (cob + 1) / 2 : cob) * ((c.cin + 31) / 32) * 3;
   int s = (1024 + tiles - 1) / tiles;

@@ -41,7 +41,9 @@ hipError_t launch_conv3x3_wgrad(const bf16_t* dYT, const bf16_t* XT, int N, int 
                                 int Cin, int Cout, int splits, float* part, hipStream_t s);
 // Weight and bias gradient partials straight from the NHWC tensors dY (ReLU
 // already applied) and `in`: part[split] = [co][t][ci] then [co]; W % 64 == 0, Cout
-// a multiple of 8; rows (n, y) are split into `splits` contiguous ranges.
+// a multiple of 8, Cu of 32; the rows of the 64-pixel column strips are split into
+// `splits` contiguous ranges (wgrad_nhwc_splits: as many as fill the card).
+int wgrad_nhwc_splits(int N, int H, int W, int Cin, int Cout);
 hipError_t launch_conv3x3_wgrad_nhwc(const bf16_t* dY, const ConvIn& in, int N, int H, int W,
                                      int Cout, int splits, float* part, hipStream_t s);
 // out[i] = sum_s part[s][i] (fixed order), i < count.
