@@ -26,6 +26,7 @@ namespace huvk {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void lds_void;
 
 __device__ __forceinline__ float bf2f(bf16_t b) { return __uint_as_float((uint32_t)b << 16); }
 __device__ __forceinline__ bf16_t f2bf(float f) {
@@ -33,6 +34,13 @@ __device__ __forceinline__ bf16_t f2bf(float f) {
   if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)0x7fc0;  // NaN
   u += 0x7fffu + ((u >> 16) & 1u);                              // round to nearest even
   return (bf16_t)(u >> 16);
+}
+
+// Two values rounded to nearest even, the first in the low half (one instruction).
+__device__ __forceinline__ uint32_t f2bf2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
 
 __device__ __forceinline__ bf16x8 ld8(const bf16_t* p) {
@@ -156,26 +164,18 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(ConvIn in, int N, int H, in
 }
 
 // ---------------------------------------------------------------------------
-// Forward 3x3 convolution with the input and the weights staged in LDS.
-// Work-group = 4 waves over an output tile of TH = 2 BM rows x 64 columns of
-// one image; wave w takes columns x0 + 32 (w % 2) .. + 31 of the BM rows from
-// y0 + BM (w / 2), and BN blocks of 32 output channels, so one weight fragment
-// feeds BM products.  Input channels run in chunks of CC: the (TH + 2) x (64 + 2)
-// x CC halo and the chunk's 9 x CC weights of the 32 BN output channels are
-// loaded once per chunk (zero outside the image and beyond Cout) and read by all
-// four waves from LDS; A = 32 pixels x 16 k per MFMA step (two 8-channel blocks of
-// (tap, channel) index 2s and 2s + 1), B = 16 k x 32 output channels.  Needs
-// W % 64 == 0 and H % TH == 0.
-//
-// The output leaves through LDS in 16-byte runs of channels, where the ReLU mask
-// of the layer below (mask: dX zeroed where that layer's output is not positive)
-// and the 2 x 2 maximum (pool) cost no pass of their own; the decoder's input is
-// read from its two sources (the half-resolution map and the skip), so the
-// concatenation is never written.  A forward pass of 32 fields of 512^2 (4 levels,
-// base 32): 5222 -> 3790 us with the three passes gone; the loss gradient of 8 of
-// them 6273 -> 5194 us, with the masks, the sum and the pooling of the backward
-// pass fused likewise.  What bounds it: the LDS (two 16-byte reads per 1 1/3 products
-// of a wave) and the waits between the chunks' loads and their products.
+// Forward 3x3 convolution of few input channels (the first layer's 8), input and
+// weights staged in LDS.  Work-group = 4 waves over an output tile of TH = 2 BM rows
+// x 64 columns of one image; wave w takes columns x0 + 32 (w % 2) .. + 31 of the BM
+// rows from y0 + BM (w / 2), and BN blocks of 32 output channels, so one weight
+// fragment feeds BM products.  Input channels run in chunks of CC: the (TH + 2) x
+// (64 + 2) x CC halo and the chunk's 9 x CC weights of the 32 BN output channels are
+// loaded once per chunk (zero outside the image and beyond Cout) and read by all four
+// waves from LDS; A = 32 pixels x 16 k per MFMA step (two 8-channel blocks of (tap,
+// channel) index 2s and 2s + 1, so at 8 channels a product spans two taps), B = 16 k x
+// 32 output channels.  The output leaves through LDS in 16-byte runs of channels, with
+// the ReLU mask and the 2 x 2 maximum as below.  Bound by the writes: 32 fields of
+// 512^2, 32 channels, 184 us.  Needs W % 64 == 0 and H % TH == 0.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int CC>
 __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H, int W,
@@ -318,6 +318,202 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H
     if (c >= Cout) continue;
     const int yo = q / (TW / 2), xo = q % (TW / 2);
     const bf16_t* b = tile + (2 * yo * TW + 2 * xo) * OS + 8 * g;
+    B8 v0, v1, v2, v3;
+    v0.u = *reinterpret_cast<const uint4*>(b);
+    v1.u = *reinterpret_cast<const uint4*>(b + OS);
+    v2.u = *reinterpret_cast<const uint4*>(b + TW * OS);
+    v3.u = *reinterpret_cast<const uint4*>(b + (TW + 1) * OS);
+    *reinterpret_cast<uint4*>(
+        pool + (((size_t)n * (H / 2) + y0 / 2 + yo) * (W / 2) + x0 / 2 + xo) * Cout + c) =
+        max4(v0, v1, v2, v3).u;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Forward 3x3 convolution with channels in chunks of CC = 16 or 32, staged in LDS.
+// Work-group = 4 waves over a tile of TH rows x 64 columns of one image and 32 COW
+// output channels: wave w takes one block of 32 output channels, 32 columns and BM
+// rows.  A chunk's weights of the block (9 taps x CC channels) stay in the wave's
+// registers; each input row of the tile is read from LDS once per column shift and
+// feeds the output rows above, at and below it, so a chunk costs (BM + 2) + 3 operand
+// reads of 16 bytes per 3 BM products.  The sums run over (chunk, tap, channel) for
+// every output, whatever BM.
+//
+// The products are weights x pixels: a lane ends up with four consecutive channels
+// of one pixel at a time, which leave through LDS in 16-byte runs, where the ReLU
+// mask of the layer below (mask: dX zeroed where that layer's output is not positive)
+// and the 2 x 2 maximum (pool) cost no pass of their own; the decoder's input is
+// read from its two sources (the half-resolution map and the skip), so the
+// concatenation is never written.
+//
+// What bounds it: at 64 and more output channels the matrix cores, 1030 TFLOP/s over
+// the layers of a forward pass (a large library product: 1190); at 32 the copies of
+// halo and weights, 0.7 of the card's copy rate.  Blocks of 2 rows x 32 columns x 64
+// channels per wave, with both operands read anew for every tap and copied through
+// registers, took 2557 and 1262 us of a forward pass of 32 fields of 512^2 (4 levels,
+// base 32), now 1874 and 1246: 3790 -> 3110 us altogether, and 4245 -> 3670 for the
+// loss gradient of 8 of them.  Needs W % 64 == 0 and H % TH == 0.
+// ---------------------------------------------------------------------------
+template <int BM, int COW, int CC>
+__global__ __launch_bounds__(256, 2) void k_conv3x3_rows(ConvIn in, int N, int H, int W,
+                                                         const bf16_t* __restrict__ Wt,
+                                                         const float* __restrict__ bias, int Cout,
+                                                         int relu, const bf16_t* __restrict__ mask,
+                                                         bf16_t* __restrict__ Y,
+                                                         bf16_t* __restrict__ pool) {
+  constexpr int TH = 2 * BM / COW, TW = 64, HR = TH + 2, HC = TW + 2;
+  constexpr int CB = CC / 8, S = CC / 16;  // 16-byte pieces of a pixel; products per tap
+  constexpr int OS = 32 * COW + 8;         // pixel stride of the staged output
+  constexpr int IN_RUNS = (HR * HC * CB + 63) / 64;  // 64 pieces a wave copies at once
+  constexpr int W_RUNS = 32 * COW * 9 * CB / 64;
+  constexpr int IN_LDS = IN_RUNS * 512, W_LDS = W_RUNS * 512, OUT_LDS = TH * TW * OS;
+  __shared__ __attribute__((aligned(16)))
+  bf16_t lds[IN_LDS + W_LDS > OUT_LDS ? IN_LDS + W_LDS : OUT_LDS];
+  const int Cin = in.Cu + in.C;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int half = lane >> 5, li = lane & 31;
+  const int cw = wave % COW, col = wave / COW % 2, rg = wave / (2 * COW);
+  const int tilesX = W / TW, tilesY = H / TH;
+  const int tiles = N * tilesY * tilesX, cogroups = (Cout + 32 * COW - 1) / (32 * COW);
+  // The channel groups of a tile, and tiles with a common edge, run on one XCD
+  // (work-groups are dealt to the 8 XCDs in turn) where the tiles can be dealt out.
+  int t = blockIdx.x / cogroups, cg = blockIdx.x % cogroups;
+  if (tiles % 8 == 0) {
+    const int j = blockIdx.x / 8;
+    cg = j % cogroups;
+    t = (int)blockIdx.x % 8 * (tiles / 8) + j / cogroups;
+  }
+  const int x0 = t % tilesX * TW, y0 = t / tilesX % tilesY * TH, n = t / (tilesX * tilesY);
+  const int cobase = cg * 32 * COW;
+  // The 16-byte pieces of a pixel (or of one tap of an output channel) are permuted by
+  // its column (channel), so that the reads of consecutive lanes do not meet in a bank.
+  auto swz = [](int c) { return CB == 4 ? (c >> 1) & 3 : (c >> 2) & 1; };
+  int abase[3][S], wbase[S];  // this lane's operand pieces at the wave's first row, and tap 0
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) {
+      const int c = 32 * col + li + dx;
+      abase[dx][q] = (rg * BM * HC + c) * CC + 8 * ((2 * q + half) ^ swz(c));
+    }
+    wbase[q] = IN_LDS + (32 * cw + li) * CC + 8 * ((2 * q + half) ^ swz(li));
+  }
+  f32x16 acc[BM];
+#pragma unroll
+  for (int bm = 0; bm < BM; ++bm)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[bm][r] = 0.f;
+  for (int c0 = 0; c0 < Cin; c0 += CC) {
+    // The chunk goes from memory to LDS without registers, 64 pieces per wave and copy,
+    // by buffer loads with 32-bit offsets into the image (or its half-resolution part):
+    // a pixel outside it, and an output channel beyond Cout, gets an offset past the
+    // end, which reads zero.
+    const bool up = c0 < in.Cu;
+    const int sh = up ? 1 : 0, cs = up ? in.Cu : in.C, ws = W >> sh;
+    const int image = (H >> sh) * ws * cs;
+    const bf16_t* src = (up ? in.U : in.X) + (size_t)n * image;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(src), (short)0, image * (int)sizeof(bf16_t), 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(Wt), (short)0, Cout * 9 * Cin * (int)sizeof(bf16_t), 0x00020000);
+    const int soff = (up ? c0 : c0 - in.Cu) * (int)sizeof(bf16_t);
+    __syncthreads();  // the previous chunk has been consumed
+#pragma unroll 1
+    for (int k = wv; k < W_RUNS; k += 4) {
+      const int i = 64 * k + lane, c = i / CB % (32 * COW), tap = i / (CB * 32 * COW);
+      const int cb = i % CB ^ swz(c);
+      const int off = (((cobase + c) * 9 + tap) * Cin + c0 + 8 * cb) * (int)sizeof(bf16_t);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(lds + IN_LDS + 512 * k), 16,
+                                               cobase + c < Cout ? off : -1, 0, 0, 0);
+    }
+#pragma unroll 1
+    for (int k = wv; k < IN_RUNS; k += 4) {
+      const int i = 64 * k + lane, pix = i / CB, row = pix / HC, c = pix - row * HC;
+      const int cb = i % CB ^ swz(c);
+      const int yy = y0 - 1 + row, xx = x0 - 1 + c;
+      const bool v = row < HR && yy >= 0 && yy < H && xx >= 0 && xx < W;
+      const int off = (((yy >> sh) * ws + (xx >> sh)) * cs + 8 * cb) * (int)sizeof(bf16_t);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(lds + 512 * k), 16,
+                                               v ? off + soff : -1, 0, 0, 0);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's copies have landed (vmcnt 0)
+    __syncthreads();
+    bf16x8 wf[9 * S];
+#pragma unroll
+    for (int k = 0; k < 9 * S; ++k) wf[k] = ld8(lds + wbase[k % S] + k / S * (32 * COW * CC));
+    // units of one input row and column shift, the next one's operands being read
+    // during this one's products (and no earlier: registers)
+    bf16x8 a[S], an[S];
+#pragma unroll
+    for (int q = 0; q < S; ++q) a[q] = ld8(lds + abase[0][q]);
+#pragma unroll
+    for (int u = 0; u < 3 * (BM + 2); ++u) {
+      const int rho = u / 3, dx = u % 3, rn = (u + 1) / 3, dn = (u + 1) % 3;
+      if (rn < BM + 2) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) an[q] = ld8(lds + abase[dn][q] + rn * (HC * CC));
+      }
+#pragma unroll
+      for (int q = 0; q < S; ++q)
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy) {
+          const int bm = rho - dy;
+          if (bm >= 0 && bm < BM)
+            acc[bm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[(dy * 3 + dx) * S + q], a[q],
+                                                              acc[bm], 0, 0, 0);
+        }
+#pragma unroll
+      for (int q = 0; q < S; ++q) a[q] = an[q];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();  // the tile has been read by every wave
+  int hb = half;
+  asm volatile("" : "+v"(hb));  // the biases are not loaded before the products
+  float bv[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int co = cobase + 32 * cw + 8 * (r / 4) + 4 * hb + (r % 4);
+    bv[r] = bias && co < Cout ? bias[co] : 0.f;
+  }
+#pragma unroll
+  for (int bm = 0; bm < BM; ++bm) {
+    bf16_t* o = lds + ((rg * BM + bm) * TW + 32 * col + li) * OS + 32 * cw + 4 * half;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = acc[bm][4 * q + e] + bv[4 * q + e];
+        if (relu) v[e] = fmaxf(v[e], 0.f);
+      }
+      *reinterpret_cast<uint2*>(o + 8 * q) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+    }
+  }
+  __syncthreads();
+  constexpr int G8 = 4 * COW;  // 8-channel groups of the block
+  for (int i = tid; i < TH * TW * G8; i += 256) {
+    const int g = i % G8, q = i / G8, c = cobase + 8 * g;
+    if (c >= Cout) continue;
+    const size_t at = (((size_t)n * H + y0 + q / TW) * W + x0 + q % TW) * Cout + c;
+    B8 v;
+    v.u = *reinterpret_cast<const uint4*>(lds + q * OS + 8 * g);
+    if (mask) {
+      B8 m;
+      m.u = *reinterpret_cast<const uint4*>(mask + at);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (bf2f(m.h[e]) <= 0.f) v.h[e] = 0;
+    }
+    *reinterpret_cast<uint4*>(Y + at) = v.u;
+  }
+  if (!pool) return;
+  for (int i = tid; i < TH * TW / 4 * G8; i += 256) {
+    const int g = i % G8, q = i / G8, c = cobase + 8 * g;
+    const int yo = q / (TW / 2), xo = q % (TW / 2);
+    if (c >= Cout) continue;
+    const bf16_t* b = lds + (2 * yo * TW + 2 * xo) * OS + 8 * g;
     B8 v0, v1, v2, v3;
     v0.u = *reinterpret_cast<const uint4*>(b);
     v1.u = *reinterpret_cast<const uint4*>(b + OS);
@@ -1052,24 +1248,38 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
   const int64_t NP = (int64_t)N * H * W;
   // a chunk of input channels comes from one source
   const int chunk = Cin == 8 ? 8 : Cin % 32 != 0 || in.Cu % 32 != 0 ? 16 : 32;
-  if (W % 64 == 0 && H % 4 == 0 && Cin % chunk == 0 && in.Cu % chunk == 0 &&
-      (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) &&
+  if (chunk > 8 && W % 64 == 0 && H % 8 == 0 && Cin % chunk == 0 && in.Cu % chunk == 0 &&
       (int64_t)H * W * std::max(in.C, in.Cu) < (1ll << 30)) {  // 32-bit byte offsets
+    const int cow = Cout <= 32 ? 1 : 2, groups = (Cout + 32 * cow - 1) / (32 * cow);
+    auto blocks = [&](int th) { return (int64_t)N * (H / th) * (W / 64) * groups; };
+    // Tiles of 8 rows where two work-groups per CU come of it, else of 4 (more reads per
+    // product): with the limit at 256, 3790 -> 3810 us for the gradient of 8 of 512^2.
+    const int th = blocks(8) >= 512 ? 8 : 4;
+    if (blocks(th) < (1ll << 31)) {
+#define HUV_CONV_ROWS(BM_, COW_, CC_)                                                          \
+  hipLaunchKernelGGL((k_conv3x3_rows<BM_, COW_, CC_>), dim3((unsigned)blocks(th)), dim3(256), \
+                     0, s, in, N, H, W, Wt, bias, Cout, relu, mask, Y, pool)
+      if (cow == 1) {
+        if (chunk == 16) { if (th == 8) HUV_CONV_ROWS(4, 1, 16); else HUV_CONV_ROWS(2, 1, 16); }
+        else { if (th == 8) HUV_CONV_ROWS(4, 1, 32); else HUV_CONV_ROWS(2, 1, 32); }
+      } else {
+        if (chunk == 16) { if (th == 8) HUV_CONV_ROWS(8, 2, 16); else HUV_CONV_ROWS(4, 2, 16); }
+        else { if (th == 8) HUV_CONV_ROWS(8, 2, 32); else HUV_CONV_ROWS(4, 2, 32); }
+      }
+#undef HUV_CONV_ROWS
+      return hipGetLastError();
+    }
+  }
+  if (chunk == 8 && W % 64 == 0 && H % 4 == 0 && (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) &&
+      (int64_t)H * W * in.C < (1ll << 30)) {
     // tiles of 4 rows x 64 columns: BM = 2 pixel blocks per wave
     dim3 grid((unsigned)((int64_t)N * (H / 4) * (W / 64)),
               (unsigned)((Cout + (Cout <= 32 ? 31 : 63)) / (Cout <= 32 ? 32 : 64)));
-#define HUV_CONV_LDS(BN_, CC_)                                                                  \
-  hipLaunchKernelGGL((k_conv3x3_fwd_lds<2, BN_, CC_>), grid, dim3(256), 0, s, in, N, H, W, Wt, \
-                     bias, Cout, relu, mask, Y, pool)
-    if (Cout <= 32) {
-      if (chunk == 8) HUV_CONV_LDS(1, 8);
-      else if (chunk == 16) HUV_CONV_LDS(1, 16);
-      else HUV_CONV_LDS(1, 32);
-    } else {
-      if (chunk == 8) HUV_CONV_LDS(2, 8);
-      else if (chunk == 16) HUV_CONV_LDS(2, 16);
-      else HUV_CONV_LDS(2, 32);
-    }
+#define HUV_CONV_LDS(BN_)                                                                          \
+  hipLaunchKernelGGL((k_conv3x3_fwd_lds<2, BN_, 8>), grid, dim3(256), 0, s, in, N, H, W, Wt, bias, \
+                     Cout, relu, mask, Y, pool)
+    if (Cout <= 32) HUV_CONV_LDS(1);
+    else HUV_CONV_LDS(2);
 #undef HUV_CONV_LDS
     return hipGetLastError();
   }

@@ -54,3 +54,15 @@ def test_output_and_gradient(ctx, levels, base, n, h, w):
     loss2, g2 = net.loss_and_grad(torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda(),
                                   want_grad=True)
     assert loss2 == loss and np.array_equal(g, g2)
+
+
+@pytest.mark.parametrize("levels,base", [(3, 64), (3, 32), (2, 16)])
+def test_batch_equals_its_fields(ctx, levels, base):
+    """A batch is convolved in taller tiles than a single field: the same bits."""
+    import torch
+    net = UN.UNet(ctx, levels=levels, base=base, seed=2)
+    x = torch.rand((16, 256, 256), generator=torch.Generator().manual_seed(base)).cuda()
+    out = net.forward(x).cpu().numpy()
+    for k in (0, 7, 15):
+        one = net.forward(x[k:k + 1].contiguous()).cpu().numpy()
+        assert np.array_equal(one[0], out[k])
