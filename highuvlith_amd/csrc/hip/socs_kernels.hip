@@ -12,13 +12,15 @@
 // once per image and evaluated on the n x n output grid.
 //
 // Stages (one launch each, all batched over clips / images):
-//   rows_band    mask rows (real, FP32) -> row spectra, band |kx| <= B kept
-//   cols_band    row spectra -> M[ky][kx] band, twisted per x class q
+//   rows_pruned  mask rows (real, FP32) -> row spectra, band |kx| <= B kept
+//   cols_pruned  row spectra -> M[ky][kx] band (rows_band and cols_band: B > 63)
 //   socs_fields  K kernels x band -> coarse intensity (fields in registers)
 //   coarse_rows  coarse rows -> |gx| <= 2B
 //   coarse_cols  -> intensity band I^[gy][gx], 1/m^2, flare on non-DC terms
 //   band_image   band -> n x n image rows (C2R), written once to HBM
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "fft_lds.hpp"
 #include "socs_kernels.hpp"
@@ -204,6 +206,283 @@ __global__ __launch_bounds__(TEAMS * N2) void k_cols_band_c(
           if (col == 0) put_p(-1, ky + BB, make_float2(0.f, 0.f));  // the zero column
         }
       });
+}
+
+// ---------------------------------------------------------------------------
+// Pruned forward transforms: of a length N = 32 L only the bins |k| < 16 T (T = 2 or
+// 4) are wanted.  L lanes share a transform; lane n1 holds x[n1 + L n2], n2 < 32, and
+// transforms over n2 in registers:
+//   Y[n1][k2] = FFT_32(x[n1 + L .])[k2] W_N^{n1 k2}
+//   X[k2 + 32 k1] = sum_{n1} Y[n1][k2] W_L^{n1 k1},  -T/2 <= k1 < T/2
+// so after one exchange through LDS the second half is T sums of L terms per k2 (a
+// decimation in time that stops at length T) instead of transforms of length L of
+// which most bins would be dropped, and every lane has work in both halves.
+//
+// What bounds them: the rows the reads of the rasters (24 of 2048^2: 151 -> 98 us, 4.1
+// TB/s; 49 of 1024^2 60.7 -> 51; 74 of 512^2 28 -> 18; 2048 of 1024^2, band 47, 591 ->
+// 539; 19 complex ones of 1024^2 47 -> 31.7), before the instructions of the full
+// transforms and the gathers of their twiddles; the columns the latency of one load,
+// one exchange and one store (band 15 of 21 of 512^2 11.6 -> 5.4; band 63 of 24 of
+// 2048^2 33 -> 21.5; band 47 of 512 of 1024^2 152 -> 93).  tmp is row-contiguous: a row's
+// bins are one run to write, and the lanes of one n1 read neighbouring columns.
+// ---------------------------------------------------------------------------
+// o[i] = sum_n v[n] W_L^{n (i - T / 2)}
+template <int L, int T>
+__device__ __forceinline__ void dft_pruned(const c32* v, c32* o);
+
+template <int L, int T, int I>
+__device__ __forceinline__ void dft_pruned_join(const c32* e, const c32* d, c32* o) {
+  if constexpr (I < T) {
+    o[I] = cadd(e[I], twiddle<-1, I - T / 2, L>(d[I]));
+    dft_pruned_join<L, T, I + 1>(e, d, o);
+  }
+}
+
+template <int L, int T>
+__device__ __forceinline__ void dft_pruned(const c32* v, c32* o) {
+  if constexpr (L == T) {
+    c32 u[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) u[i] = v[i];
+    fft_reg<-1, T>(u);
+#pragma unroll
+    for (int i = 0; i < T; ++i) o[i] = u[(i + T / 2) % T];
+  } else {
+    c32 a[L / 2], b[L / 2], e[T], d[T];
+#pragma unroll
+    for (int i = 0; i < L / 2; ++i) {
+      a[i] = v[2 * i];
+      b[i] = v[2 * i + 1];
+    }
+    dft_pruned<L / 2, T>(a, e);
+    dft_pruned<L / 2, T>(b, d);
+    dft_pruned_join<L, T, 0>(e, d, o);
+  }
+}
+
+template <int T, int I = 0>
+__device__ __forceinline__ void tw64_if(c32* o, bool on) {
+  if constexpr (I < T) {
+    const c32 y = twiddle<-1, I - T / 2, 64>(o[I]);
+    o[I] = on ? y : o[I];
+    tw64_if<T, I + 1>(o, on);
+  }
+}
+
+// The second half: lane t of a transform's L lanes; the transforms of a wave are
+// interleaved CN at a time (lane = transform + CN t within a wave for L = 64).
+// emit(k, X[k]) once per bin over the L lanes; Y[n1][k2] at y[k2 (L + 1) + n1].
+template <int L, int T, int CN, typename Emit>
+__device__ __forceinline__ void pruned_sums(int t, const c32* y, Emit emit) {
+  c32 o[T];
+  if constexpr (L == 64) {
+    // two lanes per k2: the even and the odd n1
+    const int k2 = t >> 1, odd = t & 1;
+    c32 v[32];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) v[j] = y[k2 * (L + 1) + 2 * j + odd];
+    dft_pruned<32, T>(v, o);
+    tw64_if<T>(o, odd != 0);
+#pragma unroll
+    for (int i = 0; i < T / 2; ++i) {
+      // the even lane finishes the bins below zero, the odd lane the others
+      const c32 give = odd ? o[i] : o[i + T / 2], keep = odd ? o[i + T / 2] : o[i];
+      const c32 got = {__shfl_xor(give.re, CN), __shfl_xor(give.im, CN)};
+      emit(k2 + 32 * (i + (odd ? 0 : -T / 2)), odd ? cadd(got, keep) : cadd(keep, got));
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 32 / L; ++q) {
+      const int k2 = t + L * q;
+      c32 v[L];
+#pragma unroll
+      for (int j = 0; j < L; ++j) v[j] = y[k2 * (L + 1) + j];
+      dft_pruned<L, T>(v, o);
+#pragma unroll
+      for (int i = 0; i < T; ++i) emit(k2 + 32 * (i - T / 2), o[i]);
+    }
+  }
+}
+
+// rows_pruned: row spectra |k| <= B < 16 T of real row pairs z = a + i b (CX = false)
+// or of complex rows (CX), to tmp[item][k + B], item = pair or row over all clips.
+// One wave per work-group, 64 / L items at a time, `per` times; a lane keeps the 31
+// factors W_N^{n1 k2} of its n1 in registers.
+template <int L, int T, bool CX>
+__global__ __launch_bounds__(64) void k_rows_pruned(const float* __restrict__ masks, int64_t items,
+                                                    int per, int B,
+                                                    const float2* __restrict__ tw_n,
+                                                    float2* __restrict__ tmp) {
+  constexpr int N = 32 * L, TEAMS = 64 / L, TS = 32 * (L + 1) + (L == 8 ? 4 : 0);
+  __shared__ c32 sh[TEAMS * TS];
+  const int team = threadIdx.x / L, t = threadIdx.x % L;
+  const int nk = 2 * B + 1;
+  c32 tw[32];
+#pragma unroll
+  for (int k = 1; k < 32; ++k) tw[k] = tw_lookup<-1>(tw_n, t * k);
+  for (int g = 0; g < per; ++g) {
+    const int64_t item = ((int64_t)blockIdx.x * per + g) * TEAMS + team;
+    if (item - team >= items) break;  // the whole wave
+    const bool active = item < items;
+    const float* a = masks + (active ? item : 0) * (2 * N);
+    c32 v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const int x = t + L * i;
+      if constexpr (CX) {
+        const float2 z = reinterpret_cast<const float2*>(a)[x];
+        v[i] = c32{z.x, z.y};
+      } else if constexpr (L >= 32) {
+        v[i] = c32{__builtin_nontemporal_load(a + x), __builtin_nontemporal_load(a + N + x)};
+      } else {
+        v[i] = c32{a[x], a[N + x]};
+      }
+    }
+    fft_reg<-1, 32>(v);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      sh[team * TS + k * (L + 1) + t] = k == 0 ? v[0] : cmul(v[k], tw[k]);
+    __syncthreads();
+    float2* out = tmp + (active ? item : 0) * nk + B;
+    pruned_sums<L, T, 1>(t, sh + team * TS, [&](int k, c32 x) {
+      if (active && k >= -B && k <= B) out[k] = make_float2(x.re, x.im);
+    });
+  }
+}
+
+// The value of the band box at (kx, ky): the column's bin times the pixel transfer,
+// zero beyond B (and to the box's mirror image and the column-paired copy).
+struct BandBox {
+  float2 *mq, *mp;
+  int BB, W;
+  __device__ __forceinline__ void put_p(int col, int row, float2 v) const {
+    mp[((size_t)((col + 1) >> 1) * W + row) * 2 + ((col + 1) & 1)] = v;
+  }
+  __device__ __forceinline__ void put(int kx, int ky, float2 v) const {
+    mq[(size_t)(kx + BB) * W + (ky + BB)] = v;
+    if (mp) put_p(kx + BB, ky + BB, v);
+  }
+};
+
+// cols_pruned: the band box of real rasters from tmp[clip][pair][k + B] (layout and
+// outputs as cols_band's).  Work-group = the columns kx and -kx of KX values of kx, L
+// lanes each: with z_p the pair spectra, P[ky] = FFT_{n/2}(z_.[kx]) and Q[ky] =
+// FFT_{n/2}(z_.[-kx]) give the even and odd rows' transforms (P[ky] + conj Q[-ky]) / 2
+// and (P[ky] - conj Q[-ky]) / (2 i), and M[ky][kx] is the first plus W_n^{ky} times
+// the second.  Lanes of one n1 read neighbouring columns.
+template <int L, int T, int KX>
+__global__ __launch_bounds__(2 * KX * L) void k_cols_pruned(
+    const float2* __restrict__ tmp, int B, int BB, const float2* __restrict__ tw_n,
+    const float* __restrict__ sinc_t, float2* __restrict__ Mq, float2* __restrict__ Mp) {
+  constexpr int NP = 32 * L, N = 2 * NP, CN = 2 * KX, NT = CN * L;
+  constexpr int CS = 32 * (L + 1) + (CN < 16 ? 16 / CN : 1);  // a column's stride
+  constexpr int OS = 32 * T + 1;
+  __shared__ c32 sh[CN * (CS > OS ? CS : OS)];
+  const int tid = threadIdx.x, c = tid % CN, t = tid / CN;
+  const int clip = blockIdx.y, kx0 = blockIdx.x * KX;
+  const int nk = 2 * B + 1, W = 2 * BB + 1;
+  const int kx = kx0 + c % KX;
+  const bool live = kx <= B;
+  const float2* src = tmp + (size_t)clip * NP * nk + (live ? B + (c < KX ? kx : -kx) : 0);
+  {
+    c32 v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const float2 z = src[(t + L * i) * nk];
+      v[i] = c32{z.x, z.y};
+    }
+    c32 tw[32];
+#pragma unroll
+    for (int k = 1; k < 32; ++k) tw[k] = tw_lookup<-1>(tw_n, 2 * t * k);
+    fft_reg<-1, 32>(v);
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      sh[c * CS + k * (L + 1) + t] = k == 0 ? v[0] : cmul(v[k], tw[k]);
+  }
+  __syncthreads();
+  c32 o[T * 32 / L];
+  int n = 0;
+  pruned_sums<L, T, CN>(t, sh + c * CS, [&](int, c32 x) { o[n++] = x; });
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 32 / L; ++q)
+#pragma unroll
+    for (int i = 0; i < T; ++i) sh[c * OS + t + L * q + 32 * i] = o[q * T + i];
+  __syncthreads();
+  const BandBox box{Mq + (size_t)clip * W * W, Mp ? Mp + (size_t)clip * (W + 1) * W : nullptr, BB, W};
+  for (int i = tid; i < KX * W; i += NT) {
+    const int j = i / W, x = kx0 + j, y = i % W - BB;
+    if (x > BB) break;
+    float2 m = make_float2(0.f, 0.f);
+    if (x <= B && y >= -B && y <= B) {
+      const c32 p = sh[j * OS + y + 16 * T], q = sh[(j + KX) * OS - y + 16 * T];
+      const c32 e = {0.5f * (p.re + q.re), 0.5f * (p.im - q.im)};
+      const c32 d = {0.5f * (p.im + q.im), -0.5f * (p.re - q.re)};
+      const c32 r = cscale(cadd(e, cmul(d, tw_lookup<-1>(tw_n, y < 0 ? y + N : y))),
+                           sinc_t[x + B] * sinc_t[y + B]);
+      m = make_float2(r.re, r.im);
+    }
+    box.put(x, y, m);
+    if (x > 0) box.put(-x, -y, make_float2(m.x, -m.y));
+    else if (box.mp) box.put_p(-1, y + BB, make_float2(0.f, 0.f));  // the zero column
+  }
+}
+
+// cols_pruned_c: the band box of complex rasters from tmp[clip][row][k + B]; KX columns
+// per work-group, L lanes each.
+template <int L, int T, int KX>
+__global__ __launch_bounds__(KX * L) void k_cols_pruned_c(
+    const float2* __restrict__ tmp, int B, int BB, const float2* __restrict__ tw_n,
+    const float* __restrict__ sinc_t, float2* __restrict__ Mq, float2* __restrict__ Mp) {
+  constexpr int N = 32 * L;
+  constexpr int CS = 32 * (L + 1) + (KX < 16 ? 16 / KX : 1);
+  constexpr int OS = 32 * T + 1;
+  __shared__ c32 sh[KX * (CS > OS ? CS : OS)];
+  const int tid = threadIdx.x, c = tid % KX, t = tid / KX;
+  const int clip = blockIdx.y, kx = (int)blockIdx.x * KX + c - BB;
+  const int nk = 2 * B + 1, W = 2 * BB + 1;
+  const bool live = kx >= -B && kx <= B;
+  const float2* src = tmp + (size_t)clip * N * nk + (live ? B + kx : 0);
+  {
+    c32 v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const float2 z = src[(t + L * i) * nk];
+      v[i] = c32{z.x, z.y};
+    }
+    c32 tw[32];
+#pragma unroll
+    for (int k = 1; k < 32; ++k) tw[k] = tw_lookup<-1>(tw_n, t * k);
+    fft_reg<-1, 32>(v);
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      sh[c * CS + k * (L + 1) + t] = k == 0 ? v[0] : cmul(v[k], tw[k]);
+  }
+  __syncthreads();
+  float2 o[T * 32 / (L < 64 ? L : 64)];
+  int ks[T * 32 / (L < 64 ? L : 64)], n = 0;
+  pruned_sums<L, T, KX>(t, sh + c * CS, [&](int k, c32 x) {
+    ks[n] = k;
+    o[n++] = make_float2(x.re, x.im);
+  });
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < T * 32 / (L < 64 ? L : 64); ++i)
+    sh[c * OS + ks[i] + 16 * T] = c32{o[i].x, o[i].y};
+  __syncthreads();
+  const BandBox box{Mq + (size_t)clip * W * W, Mp ? Mp + (size_t)clip * (W + 1) * W : nullptr, BB, W};
+  for (int i = tid; i < KX * W; i += KX * L) {
+    const int j = i / W, x = (int)blockIdx.x * KX + j - BB, y = i % W - BB;
+    if (x > BB) break;
+    float2 m = make_float2(0.f, 0.f);
+    if (x >= -B && x <= B && y >= -B && y <= B) {
+      const c32 r = cscale(sh[j * OS + y + 16 * T], sinc_t[x + B] * sinc_t[y + B]);
+      m = make_float2(r.re, r.im);
+    }
+    box.put(x, y, m);
+    if (x == -BB && box.mp) box.put_p(-1, y + BB, make_float2(0.f, 0.f));  // the zero column
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1188,6 +1467,7 @@ static hipError_t rows_band_n(int B, int nclips, const float* masks, const float
              tmp);
 }
 
+// The factorisations of the four-step kernels; the pruned ones have one form.
 int band_fft_default(int n) {
   switch (n) {
     case 256: return 16;
@@ -1221,8 +1501,87 @@ int band_fft_options(int n, int* n1s) {
     default: return hipErrorInvalidValue;                              \
   }
 
+// The pruned transforms take every band up to 63, which is every band of an image (a
+// coarse grid of at most 256); wider ones (the density filter's) would need more outer
+// bins than T = 4 and keep the four-step kernels, whose layout of tmp is their own.
+static bool band_pruned(int B) { return B <= 63; }
+static bool band_n1_ok(int n, int n1) {
+  int o[4];
+  const int k = band_fft_options(n, o);
+  return n1 == 0 ? k > 0 : std::find(o, o + k, n1) != o + k;
+}
+
+template <int L, int T, bool CX>
+static hipError_t rows_pruned(int64_t items, int B, const float* masks, const float2* tw_n,
+                              float2* tmp, hipStream_t s) {
+  constexpr int TEAMS = 64 / L;
+  const int64_t groups = (items + TEAMS - 1) / TEAMS, resident = 256 * 9;  // nine per CU (LDS)
+  const int64_t per = (groups + resident - 1) / resident;
+  if (per >= (1ll << 31)) return hipErrorInvalidValue;
+  HUV_LAUNCH((k_rows_pruned<L, T, CX>), dim3((unsigned)((groups + per - 1) / per)), dim3(64), 0, s,
+             masks, items, (int)per, B, tw_n, tmp);
+}
+
+template <bool CX>
+static hipError_t rows_pruned_n(int n, int B, int nclips, const float* masks, const float2* tw_n,
+                                float2* tmp, hipStream_t s) {
+  const int64_t items = (int64_t)nclips * (CX ? n : n / 2);
+#define HUV_ROWS_PRUNED(L_)                                                    \
+  return B <= 31 ? rows_pruned<L_, 2, CX>(items, B, masks, tw_n, tmp, s)       \
+                 : rows_pruned<L_, 4, CX>(items, B, masks, tw_n, tmp, s)
+  switch (n) {
+    case 256: HUV_ROWS_PRUNED(8);
+    case 512: HUV_ROWS_PRUNED(16);
+    case 1024: HUV_ROWS_PRUNED(32);
+    case 2048: HUV_ROWS_PRUNED(64);
+    default: return hipErrorInvalidValue;
+  }
+#undef HUV_ROWS_PRUNED
+}
+
+template <int L, int T, int KX, bool CX>
+static hipError_t cols_pruned(int B, int BB, int nclips, const float2* tmp, const float2* tw_n,
+                              const float* sinc_t, float2* Mq, float2* Mp, hipStream_t s) {
+  if constexpr (CX) {
+    HUV_LAUNCH((k_cols_pruned_c<L, T, KX>), dim3((2 * BB + KX) / KX, nclips), dim3(KX * L), 0, s,
+               tmp, B, BB, tw_n, sinc_t, Mq, Mp);
+  } else {
+    HUV_LAUNCH((k_cols_pruned<L, T, KX>), dim3((BB + KX) / KX, nclips), dim3(2 * KX * L), 0, s, tmp,
+               B, BB, tw_n, sinc_t, Mq, Mp);
+  }
+}
+
+template <bool CX>
+static hipError_t cols_pruned_n(int n, int B, int BB, int nclips, const float2* tmp,
+                                const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
+                                hipStream_t s) {
+#define HUV_COLS_PRUNED(L_, KX_)                                                                  \
+  return B <= 31 ? cols_pruned<L_, 2, KX_, CX>(B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s)       \
+                 : cols_pruned<L_, 4, KX_, CX>(B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s)
+  if constexpr (CX) {
+    switch (n) {
+      case 256: HUV_COLS_PRUNED(8, 16);
+      case 512: HUV_COLS_PRUNED(16, 8);
+      case 1024: HUV_COLS_PRUNED(32, 8);
+      case 2048: HUV_COLS_PRUNED(64, 4);
+      default: return hipErrorInvalidValue;
+    }
+  } else {
+    switch (n) {
+      case 256: HUV_COLS_PRUNED(4, 16);
+      case 512: HUV_COLS_PRUNED(8, 8);
+      case 1024: HUV_COLS_PRUNED(16, 8);
+      case 2048: HUV_COLS_PRUNED(32, 4);
+      default: return hipErrorInvalidValue;
+    }
+  }
+#undef HUV_COLS_PRUNED
+}
+
 hipError_t launch_rows_band(int n, int n1, int B, int nclips, const float* masks,
                             const float2* tw_n, float2* tmp, hipStream_t s) {
+  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
+  if (band_pruned(B)) return rows_pruned_n<false>(n, B, nclips, masks, tw_n, tmp, s);
   HUV_BAND_FFT_SWITCH(rows_band_n, B, nclips, masks, tw_n, tmp, s)
 }
 
@@ -1239,6 +1598,9 @@ hipError_t launch_cols_band(int n, int n1, int B, int BB, int nclips, const floa
                             const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                             hipStream_t s) {
   if (BB < B || 2 * BB + 1 > n) return hipErrorInvalidValue;
+  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
+  if (band_pruned(B))
+    return cols_pruned_n<false>(n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s);
   HUV_BAND_FFT_SWITCH(cols_band_n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s)
 }
 
@@ -1252,6 +1614,9 @@ static hipError_t rows_band_c_n(int B, int nclips, const float2* masks, const fl
 
 hipError_t launch_rows_band_c(int n, int n1, int B, int nclips, const float2* masks,
                               const float2* tw_n, float2* tmp, hipStream_t s) {
+  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
+  if (band_pruned(B))
+    return rows_pruned_n<true>(n, B, nclips, reinterpret_cast<const float*>(masks), tw_n, tmp, s);
   HUV_BAND_FFT_SWITCH(rows_band_c_n, B, nclips, masks, tw_n, tmp, s)
 }
 
@@ -1268,6 +1633,8 @@ hipError_t launch_cols_band_c(int n, int n1, int B, int BB, int nclips, const fl
                               const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                               hipStream_t s) {
   if (BB < B || 2 * BB + 1 > n) return hipErrorInvalidValue;
+  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
+  if (band_pruned(B)) return cols_pruned_n<true>(n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s);
   HUV_BAND_FFT_SWITCH(cols_band_c_n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s)
 }
 

@@ -39,7 +39,7 @@ hipError_t launch_cols_band(int n, int n1, int B, int BB, int nclips, const floa
                             const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                             hipStream_t s);
 // Complex rasters (masks: [nclips][n][n] interleaved complex): every row is
-// transformed (tmp: [nclips][2B+1][n]) and both signs of kx are column
+// transformed (tmp: nclips n (2B+1) values) and both signs of kx are column
 // passes; Mq / Mp as for launch_cols_band.
 hipError_t launch_rows_band_c(int n, int n1, int B, int nclips, const float2* masks,
                               const float2* tw_n, float2* tmp, hipStream_t s);
