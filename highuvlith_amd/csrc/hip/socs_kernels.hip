@@ -944,9 +944,10 @@ __global__ __launch_bounds__(TEAMS * CoarseFft<M>::N2) void k_coarse_cols(
 // coarse_fused: coarse_rows and coarse_cols of one image in one work-group,
 // the row spectra kept in LDS ((M/2) x (M + 1) complex; M = 64, 128, 192).
 // Transforms M = N1 x N2 run in place in the LDS rows, teams of N2 threads:
-//  row pass, pair y2 (z = row 2 y2 + i row 2 y2 + 1, x = Q j + q read from
-//    the class-major image): thread n1 < N1 takes x = n1 + N1 n2, FFT_N2,
-//    twiddle W_M^{n1 k2}, to slot n1 + N1 k2; after a barrier thread k2
+//  copy: row pairs z = row 2 y2 + i row 2 y2 + 1 from the class-major image, in
+//    its order (whole lines), to x = Q j + q of pair y2; the twiddles beside them.
+//  row pass, pair y2: thread n1 < N1 takes x = n1 + N1 n2, FFT_N2, twiddle
+//    W_M^{n1 k2}, to the same slots n1 + N1 k2; after a barrier thread k2
 //    takes slots n1 + N1 k2 (n1 < N1), FFT_N1, back to the same slots: the
 //    pair's frequency k = k2 + N2 k1 sits at slot k1 + N1 k2.
 //  column pass, column gx in [0, G] (G = 2B): c[2 y2] = A, c[2 y2 + 1] = B
@@ -956,6 +957,11 @@ __global__ __launch_bounds__(TEAMS * CoarseFft<M>::N2) void k_coarse_cols(
 //    kept: Ib[img][gy + G][gx] = v / M^2, times (1 - flare) except at the
 //    origin.  Every read of a column's slots precedes the barrier after
 //    which they are rewritten; columns never share slots.
+// One work-group per CU and image: bound by the latencies of its steps.  With as many
+// waves as the registers allow (M = 128: 16, one step per pass; M = 192: 12, two
+// steps), copied in whole lines and with the twiddles in LDS, 38 images of M = 128
+// take 13.7 us (8 waves that gather rows and twiddles from memory 17.3), 1024 of
+// M = 192 93 us (127).
 // ---------------------------------------------------------------------------
 template <int M, int THREADS>
 __global__ __launch_bounds__(THREADS) void k_coarse_fused(const float* __restrict__ coarse, int B,
@@ -964,30 +970,48 @@ __global__ __launch_bounds__(THREADS) void k_coarse_fused(const float* __restric
                                                           float2* __restrict__ Ib) {
   constexpr int N1 = CoarseFft<M>::N1, N2 = CoarseFft<M>::N2, Q = M / 32;
   constexpr int NP = M / 2, PS = M + 1, TEAMS = THREADS / N2;
-  extern __shared__ c32 zs[];  // [NP][PS]
+  extern __shared__ c32 zs[];  // [NP][PS], then the twiddles W_M^k
+  float2* const twl = reinterpret_cast<float2*>(zs + NP * PS);
   const int img = blockIdx.x;
   const int team = threadIdx.x / N2, t = threadIdx.x % N2;
   const int G = 2 * B;
   auto slot = [](int k) { return k / N2 + N1 * (k % N2); };
   const float* base = coarse + (size_t)img * M * M;
+  // The image as it lies in memory (class-major rows) to x order, a row pair as z; the
+  // row pass below takes and leaves its thread's own slots.
+  constexpr int ELEMS = NP * M, U = 8;
+  for (int i0 = threadIdx.x; i0 < ELEMS; i0 += U * THREADS) {
+    float za[U], zb[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int i = i0 + k * THREADS, y2 = i / M, at = i % M;
+      if (i < ELEMS) {
+        za[k] = base[2 * y2 * M + at];
+        zb[k] = base[(2 * y2 + 1) * M + at];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int i = i0 + k * THREADS, y2 = i / M, at = i % M;
+      if (i < ELEMS) zs[y2 * PS + at % 32 * Q + at / 32] = c32{za[k], zb[k]};
+    }
+  }
+  for (int i = threadIdx.x; i < M; i += THREADS) twl[i] = tw_m[i];
+  __syncthreads();
   for (int r0 = 0; r0 < NP; r0 += TEAMS) {
     const int y2 = r0 + team;
     const bool act = y2 < NP;
     c32* row = zs + (act ? y2 : 0) * PS;
+    int tx = t;  // indices computed anew in every step: they would not fit in registers
+    asm volatile("" : "+v"(tx));
     if (act && t < N1) {
-      const float* ra = base + (size_t)(2 * y2) * M;
-      const float* rb = ra + M;
       c32 v[N2];
 #pragma unroll
-      for (int n2 = 0; n2 < N2; ++n2) {
-        const int x = t + N1 * n2;
-        const int at = (x % Q) * 32 + x / Q;  // class-major position of x
-        v[n2] = c32{ra[at], rb[at]};
-      }
+      for (int n2 = 0; n2 < N2; ++n2) v[n2] = row[t + N1 * n2];
       fft_small<-1, N2>(v);
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2) {
-        if (k2 > 0) v[k2] = cmul(v[k2], tw_lookup<-1>(tw_m, (t * k2) % M));
+        if (k2 > 0) v[k2] = cmul(v[k2], tw_lookup<-1>(twl, (tx * k2) % M));
         row[t + N1 * k2] = v[k2];
       }
     }
@@ -1008,6 +1032,8 @@ __global__ __launch_bounds__(THREADS) void k_coarse_fused(const float* __restric
   for (int c0 = 0; c0 <= G; c0 += TEAMS) {
     const int gx = c0 + team;
     const bool act = gx <= G;
+    int tx = t;
+    asm volatile("" : "+v"(tx));
     const int gxa = act ? gx : 0;
     const int sp = slot(gxa), sm = slot((M - gxa) % M), sw = gxa == 0 ? slot(M / 2) : sm;
     // exchange-area slot of column value y
@@ -1016,7 +1042,7 @@ __global__ __launch_bounds__(THREADS) void k_coarse_fused(const float* __restric
     if (act && t < N1) {
 #pragma unroll
       for (int n2 = 0; n2 < N2; ++n2) {
-        const int y = t + N1 * n2;
+        const int y = tx + N1 * n2;
         const c32 zp = zs[(y >> 1) * PS + sp], zn = zs[(y >> 1) * PS + sm];
         // A = (Z[k] + conj Z[M-k]) / 2 ; B = (Z[k] - conj Z[M-k]) / (2i)
         v[n2] = (y & 1) == 0 ? c32{0.5f * (zp.re + zn.re), 0.5f * (zp.im - zn.im)}
@@ -1024,7 +1050,7 @@ __global__ __launch_bounds__(THREADS) void k_coarse_fused(const float* __restric
       }
       fft_small<-1, N2>(v);
 #pragma unroll
-      for (int k2 = 1; k2 < N2; ++k2) v[k2] = cmul(v[k2], tw_lookup<-1>(tw_m, (t * k2) % M));
+      for (int k2 = 1; k2 < N2; ++k2) v[k2] = cmul(v[k2], tw_lookup<-1>(twl, (tx * k2) % M));
     }
     __syncthreads();
     if (act && t < N1) {
@@ -1750,7 +1776,7 @@ static hipError_t coarse_fused_m(int B, int nimg, int S, const float* coarse, fl
                                  const float2* tw_m, float2* Ib, hipStream_t s) {
   const hipError_t e = sum_splits(const_cast<float*>(coarse), S, (int64_t)nimg * M * M, s);
   if (e != hipSuccess) return e;
-  constexpr size_t shmem = (size_t)(M / 2) * (M + 1) * sizeof(c32);
+  constexpr size_t shmem = ((size_t)(M / 2) * (M + 1) + M) * sizeof(c32);
   auto kern = k_coarse_fused<M, THREADS>;
   static const hipError_t attr = hipFuncSetAttribute(
       (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
@@ -1763,8 +1789,8 @@ hipError_t launch_coarse_fused(int m, int B, int nimg, int S, const float* coars
   if (S < 1 || 4 * B + 1 > m) return hipErrorInvalidValue;
   switch (m) {
     case 64: return coarse_fused_m<64, 512>(B, nimg, S, coarse, flare, tw_m, Ib, s);
-    case 128: return coarse_fused_m<128, 512>(B, nimg, S, coarse, flare, tw_m, Ib, s);
-    case 192: return coarse_fused_m<192, 512>(B, nimg, S, coarse, flare, tw_m, Ib, s);
+    case 128: return coarse_fused_m<128, 1024>(B, nimg, S, coarse, flare, tw_m, Ib, s);
+    case 192: return coarse_fused_m<192, 768>(B, nimg, S, coarse, flare, tw_m, Ib, s);
     default: return hipErrorNotSupported;
   }
 }
