@@ -189,7 +189,7 @@ huv_status conv_fwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, int l, bf
                     bf16_t* pool = nullptr) {
   const Acts& a = u->a;
   HCHK(huvk::launch_conv3x3_fwd(x, a.N, a.H >> l, a.W >> l, wbf(u, c), u->p + c.b_off, c.cout, 1,
-                                nullptr, y, pool, S(u)),
+                                huvk::ConvOut{y, nullptr, pool}, S(u)),
        "U-Net conv forward");
   return HUV_OK;
 }
@@ -219,11 +219,18 @@ huv_status forward(huv_unet* u, const float* in, float* out) {
   return HUV_OK;
 }
 
+// Whether the data gradient of dec1[l] goes to its two sources in one pass.
+bool split_gcat(huv_unet* u, int l) {
+  const Acts& a = u->a;
+  return huvk::conv3x3_by_rows(input(nullptr, u->ch(l)), a.N, a.H >> l, a.W >> l,
+                               u->ch(l + 1) + u->ch(l));
+}
+
 // Gradients of one conv layer from dy (zero where the layer's ReLU was): dW and
 // db into u->g and (if dx) the input gradient, zeroed where dx_mask, the output
-// of the layer that made the input, is not positive.
+// of the layer that made the input, is not positive; see ConvOut for the rest.
 huv_status conv_bwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, const bf16_t* dy, int l,
-                    bf16_t* dx, const bf16_t* dx_mask) {
+                    const huvk::ConvOut& dx) {
   Acts& a = u->a;
   const int H = a.H >> l, W = a.W >> l;
   const int splits = wgrad_splits(c, a.N, H, W);
@@ -250,9 +257,9 @@ huv_status conv_bwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, const bf1
     HCHK(huvk::launch_channel_sum(a.dyt, a.N, H * W, c.cout, a.part, bsplits, u->g + c.b_off, S(u)),
          "U-Net bias gradient");
   }
-  if (dx)
-    HCHK(huvk::launch_conv3x3_fwd(input(dy, c.cout), a.N, H, W, wrot(u, c), nullptr, c.cin, 0,
-                                  dx_mask, dx, nullptr, S(u)),
+  if (dx.Y)
+    HCHK(huvk::launch_conv3x3_fwd(input(dy, c.cout), a.N, H, W, wrot(u, c), nullptr, c.cin, 0, dx,
+                                  S(u)),
          "U-Net data gradient");
   return HUV_OK;
 }
@@ -270,23 +277,32 @@ huv_status backward(huv_unet* u) {
   huv_status st;
   for (int l = 0; l <= L - 2; ++l) {
     const huvk::ConvIn cat = decoder_input(u, l);
-    if ((st = conv_bwd(u, u->dec2[l], input(a.d1[l], u->ch(l)), a.gd2[l], l, a.gd1[l], a.d1[l])) != HUV_OK)
+    if ((st = conv_bwd(u, u->dec2[l], input(a.d1[l], u->ch(l)), a.gd2[l], l,
+                       huvk::ConvOut{a.gd1[l], a.d1[l]})) != HUV_OK)
       return st;
-    if ((st = conv_bwd(u, u->dec1[l], cat, a.gd1[l], l, a.gcat[l], nullptr)) != HUV_OK) return st;
+    // the concatenation's gradient: the skip's part to gcat and the upsampled part
+    // summed by the convolution, or the whole to gcat
     bf16_t* gup = l == L - 2 ? a.ge2[L - 1] : a.gd2[l + 1];
-    HCHK(huvk::launch_upcat_bwd_u(a.gcat[l], cat.Cu, cat.C, a.N, a.H >> l, a.W >> l, cat.U, gup,
-                                  S(u)),
-         "U-Net upsample gradient");
+    huvk::ConvOut gcat{a.gcat[l]};
+    if (split_gcat(u, l)) gcat = huvk::ConvOut{a.gcat[l], nullptr, nullptr, gup, cat.U, cat.Cu};
+    if ((st = conv_bwd(u, u->dec1[l], cat, a.gd1[l], l, gcat)) != HUV_OK) return st;
+    if (gcat.Cu == 0)
+      HCHK(huvk::launch_upcat_bwd_u(a.gcat[l], cat.Cu, cat.C, a.N, a.H >> l, a.W >> l, cat.U, gup,
+                                    S(u)),
+           "U-Net upsample gradient");
   }
   for (int l = L - 1; l >= 0; --l) {
     if (l < L - 1)
-      HCHK(huvk::launch_skip_pool_bwd(a.e2[l], a.gpool[l], a.gcat[l], u->ch(l + 1), a.N, a.H >> l,
+      HCHK(huvk::launch_skip_pool_bwd(a.e2[l], a.gpool[l], a.gcat[l],
+                                      split_gcat(u, l) ? 0 : u->ch(l + 1), a.N, a.H >> l,
                                       a.W >> l, u->ch(l), a.ge2[l], S(u)),
            "U-Net skip gradient");
-    if ((st = conv_bwd(u, u->enc2[l], input(a.e1[l], u->ch(l)), a.ge2[l], l, a.ge1[l], a.e1[l])) != HUV_OK)
+    if ((st = conv_bwd(u, u->enc2[l], input(a.e1[l], u->ch(l)), a.ge2[l], l,
+                       huvk::ConvOut{a.ge1[l], a.e1[l]})) != HUV_OK)
       return st;
     const huvk::ConvIn src = l == 0 ? input(a.x8, 8) : input(a.pool[l - 1], u->ch(l - 1));
-    if ((st = conv_bwd(u, u->enc1[l], src, a.ge1[l], l, l == 0 ? nullptr : a.gpool[l - 1], nullptr)) != HUV_OK)
+    if ((st = conv_bwd(u, u->enc1[l], src, a.ge1[l], l,
+                       huvk::ConvOut{l == 0 ? nullptr : a.gpool[l - 1]})) != HUV_OK)
       return st;
   }
   return HUV_OK;

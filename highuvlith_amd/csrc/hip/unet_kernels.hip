@@ -68,6 +68,18 @@ __device__ __forceinline__ B8 max4(const B8& v0, const B8& v1, const B8& v2, con
   return o;
 }
 
+// The sum of four, channel by channel, zero where u (a ReLU's output) is not positive.
+__device__ __forceinline__ B8 sum4_masked(const B8& a0, const B8& a1, const B8& a2, const B8& a3,
+                                          const B8& u) {
+  B8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bf16_t sum = f2bf((bf2f(a0.h[e]) + bf2f(a1.h[e])) + (bf2f(a2.h[e]) + bf2f(a3.h[e])));
+    o.h[e] = bf2f(u.h[e]) <= 0.f ? (bf16_t)0 : sum;
+  }
+  return o;
+}
+
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution.  Work-group = 4 waves along pixels; each wave
 // computes BM x BN blocks of 32 pixels x 32 output channels.  The operands
@@ -358,9 +370,7 @@ template <int BM, int COW, int CC>
 __global__ __launch_bounds__(256, 2) void k_conv3x3_rows(ConvIn in, int N, int H, int W,
                                                          const bf16_t* __restrict__ Wt,
                                                          const float* __restrict__ bias, int Cout,
-                                                         int relu, const bf16_t* __restrict__ mask,
-                                                         bf16_t* __restrict__ Y,
-                                                         bf16_t* __restrict__ pool) {
+                                                         int relu, ConvOut out) {
   constexpr int TH = 2 * BM / COW, TW = 64, HR = TH + 2, HC = TW + 2;
   constexpr int CB = CC / 8, S = CC / 16;  // 16-byte pieces of a pixel; products per tap
   constexpr int OS = 32 * COW + 8;         // pixel stride of the staged output
@@ -493,35 +503,41 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_rows(ConvIn in, int N, int H
   }
   __syncthreads();
   constexpr int G8 = 4 * COW;  // 8-channel groups of the block
+  const int Cu = out.Cu, Cy = Cout - Cu;
   for (int i = tid; i < TH * TW * G8; i += 256) {
     const int g = i % G8, q = i / G8, c = cobase + 8 * g;
-    if (c >= Cout) continue;
-    const size_t at = (((size_t)n * H + y0 + q / TW) * W + x0 + q % TW) * Cout + c;
+    if (c >= Cout || c < Cu) continue;
+    const size_t at = (((size_t)n * H + y0 + q / TW) * W + x0 + q % TW) * Cy + c - Cu;
     B8 v;
     v.u = *reinterpret_cast<const uint4*>(lds + q * OS + 8 * g);
-    if (mask) {
+    if (out.mask) {
       B8 m;
-      m.u = *reinterpret_cast<const uint4*>(mask + at);
+      m.u = *reinterpret_cast<const uint4*>(out.mask + at);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         if (bf2f(m.h[e]) <= 0.f) v.h[e] = 0;
     }
-    *reinterpret_cast<uint4*>(Y + at) = v.u;
+    *reinterpret_cast<uint4*>(out.Y + at) = v.u;
   }
-  if (!pool) return;
+  if (!out.pool && cobase >= Cu) return;
   for (int i = tid; i < TH * TW / 4 * G8; i += 256) {
     const int g = i % G8, q = i / G8, c = cobase + 8 * g;
+    if (c >= Cout || (!out.pool && c >= Cu)) continue;
     const int yo = q / (TW / 2), xo = q % (TW / 2);
-    if (c >= Cout) continue;
     const bf16_t* b = lds + (2 * yo * TW + 2 * xo) * OS + 8 * g;
     B8 v0, v1, v2, v3;
     v0.u = *reinterpret_cast<const uint4*>(b);
     v1.u = *reinterpret_cast<const uint4*>(b + OS);
     v2.u = *reinterpret_cast<const uint4*>(b + TW * OS);
     v3.u = *reinterpret_cast<const uint4*>(b + (TW + 1) * OS);
-    *reinterpret_cast<uint4*>(
-        pool + (((size_t)n * (H / 2) + y0 / 2 + yo) * (W / 2) + x0 / 2 + xo) * Cout + c) =
-        max4(v0, v1, v2, v3).u;
+    const size_t p = ((size_t)n * (H / 2) + y0 / 2 + yo) * (W / 2) + x0 / 2 + xo;
+    if (out.pool) {
+      *reinterpret_cast<uint4*>(out.pool + p * Cout + c) = max4(v0, v1, v2, v3).u;
+    } else {
+      B8 u;
+      u.u = *reinterpret_cast<const uint4*>(out.U + p * Cu + c);
+      *reinterpret_cast<uint4*>(out.dU + p * Cu + c) = sum4_masked(v0, v1, v2, v3, u).u;
+    }
   }
 }
 
@@ -1113,12 +1129,7 @@ __global__ void k_upcat_bwd_u(const bf16_t* __restrict__ dcat, int Cu, int Cs, i
     const B8 a0 = ld_b8(dcat + b), a1 = ld_b8(dcat + b + Ct), a2 = ld_b8(dcat + b + (size_t)W * Ct),
              a3 = ld_b8(dcat + b + (size_t)W * Ct + Ct);
     const B8 u = ld_b8(U + (size_t)q * Cu + 8 * g);
-    B8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bf16_t sum = f2bf((bf2f(a0.h[e]) + bf2f(a1.h[e])) + (bf2f(a2.h[e]) + bf2f(a3.h[e])));
-      o.h[e] = bf2f(u.h[e]) <= 0.f ? (bf16_t)0 : sum;
-    }
+    const B8 o = sum4_masked(a0, a1, a2, a3, u);
     st_b8(dU + (size_t)q * Cu + 8 * g, o);
   }
 }
@@ -1238,27 +1249,42 @@ static dim3 grid1d(int64_t n, int threads = 256) {
   return dim3((unsigned)b);
 }
 
-hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_t* Wt,
-                              const float* bias, int Cout, int relu, const bf16_t* mask, bf16_t* Y,
-                              bf16_t* pool, hipStream_t s) {
+// A chunk of input channels comes from one source.
+static int conv_chunk(const ConvIn& in) {
   const int Cin = in.Cu + in.C;
+  return Cin == 8 ? 8 : Cin % 32 != 0 || in.Cu % 32 != 0 ? 16 : 32;
+}
+
+bool conv3x3_by_rows(const ConvIn& in, int N, int H, int W, int Cout) {
+  const int chunk = conv_chunk(in);
+  return chunk > 8 && W % 64 == 0 && H % 8 == 0 && (in.Cu + in.C) % chunk == 0 &&
+         in.Cu % chunk == 0 &&
+         (int64_t)H * W * std::max(in.C, in.Cu) < (1ll << 30) &&  // 32-bit byte offsets
+         (int64_t)N * (H / 4) * (W / 64) * ((Cout + 31) / 32) < (1ll << 31);
+}
+
+hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_t* Wt,
+                              const float* bias, int Cout, int relu, const ConvOut& out,
+                              hipStream_t s) {
+  const int Cin = in.Cu + in.C;
+  const bf16_t* mask = out.mask;
+  bf16_t *Y = out.Y, *pool = out.pool;
+  const bool rows = conv3x3_by_rows(in, N, H, W, Cout);
   if (in.C % 8 != 0 || in.Cu % 8 != 0 || Cout % 8 != 0 || Cout < 8 || N < 1 || H < 1 || W < 1 ||
-      (pool && (H % 2 != 0 || W % 2 != 0)))
+      (pool && (H % 2 != 0 || W % 2 != 0)) ||
+      (out.Cu > 0 && (!rows || pool || mask || out.Cu % 8 != 0 || out.Cu > Cout)))
     return hipErrorInvalidValue;
   const int64_t NP = (int64_t)N * H * W;
-  // a chunk of input channels comes from one source
-  const int chunk = Cin == 8 ? 8 : Cin % 32 != 0 || in.Cu % 32 != 0 ? 16 : 32;
-  if (chunk > 8 && W % 64 == 0 && H % 8 == 0 && Cin % chunk == 0 && in.Cu % chunk == 0 &&
-      (int64_t)H * W * std::max(in.C, in.Cu) < (1ll << 30)) {  // 32-bit byte offsets
+  const int chunk = conv_chunk(in);
+  if (rows) {
     const int cow = Cout <= 32 ? 1 : 2, groups = (Cout + 32 * cow - 1) / (32 * cow);
     auto blocks = [&](int th) { return (int64_t)N * (H / th) * (W / 64) * groups; };
     // Tiles of 8 rows where two work-groups per CU come of it, else of 4 (more reads per
     // product): with the limit at 256, 3790 -> 3810 us for the gradient of 8 of 512^2.
     const int th = blocks(8) >= 512 ? 8 : 4;
-    if (blocks(th) < (1ll << 31)) {
 #define HUV_CONV_ROWS(BM_, COW_, CC_)                                                          \
   hipLaunchKernelGGL((k_conv3x3_rows<BM_, COW_, CC_>), dim3((unsigned)blocks(th)), dim3(256), \
-                     0, s, in, N, H, W, Wt, bias, Cout, relu, mask, Y, pool)
+                     0, s, in, N, H, W, Wt, bias, Cout, relu, out)
       if (cow == 1) {
         if (chunk == 16) { if (th == 8) HUV_CONV_ROWS(4, 1, 16); else HUV_CONV_ROWS(2, 1, 16); }
         else { if (th == 8) HUV_CONV_ROWS(4, 1, 32); else HUV_CONV_ROWS(2, 1, 32); }
@@ -1267,8 +1293,7 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
         else { if (th == 8) HUV_CONV_ROWS(8, 2, 32); else HUV_CONV_ROWS(4, 2, 32); }
       }
 #undef HUV_CONV_ROWS
-      return hipGetLastError();
-    }
+    return hipGetLastError();
   }
   if (chunk == 8 && W % 64 == 0 && H % 4 == 0 && (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) &&
       (int64_t)H * W * in.C < (1ll << 30)) {

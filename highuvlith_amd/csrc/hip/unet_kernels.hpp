@@ -24,12 +24,25 @@ struct ConvIn {
     return X + (((size_t)n * H + y) * W + x) * C + (c - Cu);
   }
 };
-// Y = act(conv3x3(in) + bias), pad 1, stride 1.  relu: 0/1.  bias may be NULL.  Y
-// has Cout channels (a multiple of 8).  mask (optional, Y's shape): Y zeroed
-// where mask <= 0.  pool (optional): the 2 x 2 maximum of Y, (N, H/2, W/2, Cout).
+// A convolution's output: Y, with Cout - Cu channels.  mask (optional, Y's shape): Y
+// zeroed where mask <= 0.  pool (optional): the 2 x 2 maximum of Y, (N, H/2, W/2, Cout).
+// Cu > 0 (neither mask nor pool; only where conv3x3_by_rows): the first Cu channels go
+// to dU (N, H/2, W/2, Cu) instead, summed over 2 x 2 and zero where U, of that shape, is
+// not positive: the gradient of the upsampled half of a concatenation.
+struct ConvOut {
+  bf16_t* Y = nullptr;
+  const bf16_t* mask = nullptr;
+  bf16_t* pool = nullptr;
+  bf16_t* dU = nullptr;
+  const bf16_t* U = nullptr;
+  int Cu = 0;
+};
+// out = act(conv3x3(in) + bias), pad 1, stride 1, Cout channels (a multiple of 8).
+// relu: 0/1.  bias may be NULL.
 hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_t* Wt,
-                              const float* bias, int Cout, int relu, const bf16_t* mask, bf16_t* Y,
-                              bf16_t* pool, hipStream_t s);
+                              const float* bias, int Cout, int relu, const ConvOut& out,
+                              hipStream_t s);
+bool conv3x3_by_rows(const ConvIn& in, int N, int H, int W, int Cout);
 // Wr[ci][t][co] = W[co][8 - t][ci] (the kernel of the data gradient).
 hipError_t launch_conv_weight_rot(const bf16_t* Wt, int Cout, int Cin, bf16_t* Wr, hipStream_t s);
 // XT[n][c][y][x] = X[n][y][x][c] (H W a multiple of 64, C of 8; likewise below).
