@@ -185,16 +185,17 @@ huvk::ConvIn decoder_input(huv_unet* u, int l) {
   return huvk::ConvIn{a.e2[l], u->ch(l), up, u->ch(l + 1)};
 }
 
-huv_status conv_fwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, int l, bf16_t* y,
-                    bf16_t* pool = nullptr) {
+huv_status conv_fwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, int l,
+                    const huvk::ConvOut& y) {
   const Acts& a = u->a;
-  HCHK(huvk::launch_conv3x3_fwd(x, a.N, a.H >> l, a.W >> l, wbf(u, c), u->p + c.b_off, c.cout, 1,
-                                huvk::ConvOut{y, nullptr, pool}, S(u)),
+  HCHK(huvk::launch_conv3x3_fwd(x, a.N, a.H >> l, a.W >> l, wbf(u, c), u->p + c.b_off, c.cout, 1, y,
+                                S(u)),
        "U-Net conv forward");
   return HUV_OK;
 }
 
-huv_status forward(huv_unet* u, const float* in, float* out) {
+// keep: the backward pass follows and reads every activation.
+huv_status forward(huv_unet* u, const float* in, float* out, bool keep) {
   Acts& a = u->a;
   const int L = u->levels;
   const int64_t P = (int64_t)a.N * a.H * a.W;
@@ -205,14 +206,25 @@ huv_status forward(huv_unet* u, const float* in, float* out) {
   huv_status st;
   for (int l = 0; l < L; ++l) {
     const huvk::ConvIn src = l == 0 ? input(a.x8, 8) : input(a.pool[l - 1], u->ch(l - 1));
-    if ((st = conv_fwd(u, u->enc1[l], src, l, a.e1[l])) != HUV_OK) return st;
-    if ((st = conv_fwd(u, u->enc2[l], input(a.e1[l], u->ch(l)), l, a.e2[l],
-                       l < L - 1 ? a.pool[l] : nullptr)) != HUV_OK)
+    if ((st = conv_fwd(u, u->enc1[l], src, l, huvk::ConvOut{a.e1[l]})) != HUV_OK) return st;
+    if ((st = conv_fwd(u, u->enc2[l], input(a.e1[l], u->ch(l)), l,
+                       huvk::ConvOut{a.e2[l], nullptr, l < L - 1 ? a.pool[l] : nullptr})) != HUV_OK)
       return st;
   }
   for (int l = L - 2; l >= 0; --l) {
-    if ((st = conv_fwd(u, u->dec1[l], decoder_input(u, l), l, a.d1[l])) != HUV_OK) return st;
-    if ((st = conv_fwd(u, u->dec2[l], input(a.d1[l], u->ch(l)), l, a.d2[l])) != HUV_OK) return st;
+    if ((st = conv_fwd(u, u->dec1[l], decoder_input(u, l), l, huvk::ConvOut{a.d1[l]})) != HUV_OK)
+      return st;
+    const huvk::ConvIn x = input(a.d1[l], u->ch(l));
+    huvk::ConvOut y{a.d2[l]};
+    if (l == 0 && huvk::conv3x3_by_rows(x, a.N, a.H, a.W, u->base)) {
+      // the head with the last layer, which a pass without gradient need not write
+      y.head = out;
+      y.head_w = u->p + u->head_w;
+      y.head_b = u->p + u->head_b;
+      if (!keep) y.Y = nullptr;
+    }
+    if ((st = conv_fwd(u, u->dec2[l], x, l, y)) != HUV_OK) return st;
+    if (y.head) return HUV_OK;
   }
   HCHK(huvk::launch_head_fwd(a.d2[0], P, u->base, u->p + u->head_w, u->p + u->head_b, out, S(u)),
        "U-Net head");
@@ -452,7 +464,7 @@ huv_status huv_unet_forward(huv_unet* u, int N, int H, int W, const float* in, f
   std::lock_guard<std::mutex> lk(u->ctx->mu);
   hipSetDevice(u->ctx->device);
   if ((st = ensure_acts(u, N, H, W)) != HUV_OK) return st;
-  return forward(u, in, out);
+  return forward(u, in, out, false);
 }
 
 huv_status huv_unet_loss_grad(huv_unet* u, int N, int H, int W, const float* in,
@@ -463,7 +475,7 @@ huv_status huv_unet_loss_grad(huv_unet* u, int N, int H, int W, const float* in,
   std::lock_guard<std::mutex> lk(u->ctx->mu);
   hipSetDevice(u->ctx->device);
   if ((st = ensure_acts(u, N, H, W)) != HUV_OK) return st;
-  if ((st = forward(u, in, u->a.out)) != HUV_OK) return st;
+  if ((st = forward(u, in, u->a.out, true)) != HUV_OK) return st;
   const int64_t P = (int64_t)N * H * W;
   HCHK(huvk::launch_mse(u->a.out, target, P, u->a.dout, u->a.lpart, kLossBlocks, S(u)), "U-Net loss");
   if ((st = backward(u)) != HUV_OK) return st;

@@ -503,6 +503,20 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_rows(ConvIn in, int N, int H
   }
   __syncthreads();
   constexpr int G8 = 4 * COW;  // 8-channel groups of the block
+  if (out.head) {
+    // the 1 x 1 head on this block's channels, which are all there are
+    for (int i = tid; i < TH * TW; i += 256) {
+      float h = out.head_b[0];
+      for (int c = 0; c < Cout; c += 8) {
+        B8 v;
+        v.u = *reinterpret_cast<const uint4*>(lds + i * OS + c);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h += bf2f(v.h[e]) * out.head_w[c + e];
+      }
+      out.head[((size_t)n * H + y0 + i / TW) * W + x0 + i % TW] = h;
+    }
+    if (!out.Y) return;
+  }
   const int Cu = out.Cu, Cy = Cout - Cu;
   for (int i = tid; i < TH * TW * G8; i += 256) {
     const int g = i % G8, q = i / G8, c = cobase + 8 * g;
@@ -1272,6 +1286,7 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
   const bool rows = conv3x3_by_rows(in, N, H, W, Cout);
   if (in.C % 8 != 0 || in.Cu % 8 != 0 || Cout % 8 != 0 || Cout < 8 || N < 1 || H < 1 || W < 1 ||
       (pool && (H % 2 != 0 || W % 2 != 0)) ||
+      (out.head && (!rows || Cout > 64 || !out.head_w || !out.head_b)) || (!Y && !out.head) ||
       (out.Cu > 0 && (!rows || pool || mask || out.Cu % 8 != 0 || out.Cu > Cout)))
     return hipErrorInvalidValue;
   const int64_t NP = (int64_t)N * H * W;

@@ -28,7 +28,9 @@ struct ConvIn {
 // zeroed where mask <= 0.  pool (optional): the 2 x 2 maximum of Y, (N, H/2, W/2, Cout).
 // Cu > 0 (neither mask nor pool; only where conv3x3_by_rows): the first Cu channels go
 // to dU (N, H/2, W/2, Cu) instead, summed over 2 x 2 and zero where U, of that shape, is
-// not positive: the gradient of the upsampled half of a concatenation.
+// not positive: the gradient of the upsampled half of a concatenation.  head (only where
+// conv3x3_by_rows, Cout <= 64): head_b[0] + sum over the channels of Y head_w, FP32 per
+// pixel; Y may then be null.
 struct ConvOut {
   bf16_t* Y = nullptr;
   const bf16_t* mask = nullptr;
@@ -36,6 +38,8 @@ struct ConvOut {
   bf16_t* dU = nullptr;
   const bf16_t* U = nullptr;
   int Cu = 0;
+  float* head = nullptr;
+  const float *head_w = nullptr, *head_b = nullptr;
 };
 // out = act(conv3x3(in) + bias), pad 1, stride 1, Cout channels (a multiple of 8).
 // relu: 0/1.  bias may be NULL.
