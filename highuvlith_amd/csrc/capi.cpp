@@ -547,6 +547,7 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   // Host plan: disjoint cells per clip (painter's rule), staged with the cell
   // offsets and backgrounds in one pinned upload.
   std::vector<double> cells, edges, pdc((size_t)nclips * 2, 0.0);
+  bool edges_real = true;  // no polygon edge has an imaginary weight
   std::vector<int64_t> coff((size_t)nclips + 1, 0), eoff((size_t)nclips + 1, 0);
   std::vector<huv::RectFeature> fs;
   std::vector<huv::RectCell> cl;
@@ -621,6 +622,7 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
         boxes.push_back(bb);
         const huv::cd w = huv::cd(P.values[2 * j], P.values[2 * j + 1]) - bg;
         const double sg = twice > 0 ? 1.0 : -1.0;
+        edges_real = edges_real && w.imag() == 0.0;
         pdc[2 * i] += w.real() * 0.5 * std::fabs(twice);
         pdc[2 * i + 1] += w.imag() * 0.5 * std::fabs(twice);
         for (size_t k = 0; k < v.size(); ++k) {
@@ -694,8 +696,8 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
     const char* pd = slot->d + cell_b + off_b + bg_b;
     c->stage_begin(ST_POLY_BAND, &ev);
     e = huvk::launch_poly_band((const double*)pd, (const int64_t*)(pd + edge_b),
-                               (const double*)(pd + edge_b + eoff_b), nclips, n, L, B, BB, Mq, Mp,
-                               c->stream());
+                               (const double*)(pd + edge_b + eoff_b), edges_real, nclips, n, L, B,
+                               BB, Mq, Mp, c->stream());
     if (e != hipSuccess) return hip_fail(e, "poly_band launch");
     c->stage_end(ST_POLY_BAND, ev);
   }

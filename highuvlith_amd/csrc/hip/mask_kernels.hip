@@ -62,6 +62,7 @@ __global__ __launch_bounds__(256) void k_rect_tables(const double* __restrict__ 
 // 7.5 us so), so it takes eight waves; a full chip takes two (96 clips of 43
 // cells, B = 47: 25.6 us).
 constexpr int kRectT = 4;
+constexpr int kPolySlices = 8;
 
 template <int SL>
 __global__ __launch_bounds__(64 * SL) void k_rect_band(const double2* __restrict__ X,
@@ -176,6 +177,66 @@ __global__ __launch_bounds__(64 * SL) void k_rect_band(const double2* __restrict
   }
 }
 
+// One edge's term of a tile's bins: x the edge's column table, yv its row entries.
+__device__ __forceinline__ void poly_edge(const double4* x, const int* xi, const double4* yv,
+                                          double dx, double dy, double dk, int mx0, int my0,
+                                          double (&ar)[kRectT][kRectT],
+                                          double (&ai)[kRectT][kRectT]) {
+#pragma unroll
+  for (int j = 0; j < kRectT; ++j) {
+    const double4 xv = x[xi[j]];  // one column at a time (register budget)
+    const double kx = dk * (mx0 + j);
+#pragma unroll
+    for (int i = 0; i < kRectT; ++i) {
+      const double ky = dk * (my0 + i);
+      const double kn = kx * dy - ky * dx;
+      const double u = 0.5 * (kx * dx + ky * dy);
+      const double su = xv.w * yv[i].z + xv.z * yv[i].w;
+      double r = __builtin_amdgcn_rcp(u);
+      r = fma(r, fma(-u, r, 1.0), r);
+      r = fma(r, fma(-u, r, 1.0), r);
+      const double sc = fabs(u) < 1e-4 ? 1.0 - u * u * (1.0 / 6.0) : su * r;
+      const double a = kn * sc;
+      const double hr = xv.x * yv[i].x - xv.y * yv[i].y;
+      const double hi = xv.x * yv[i].y + xv.y * yv[i].x;
+      ar[i][j] = fma(a, hr, ar[i][j]);
+      ai[i][j] = fma(a, hi, ai[i][j]);
+    }
+  }
+}
+
+// The bin of orders (mx, my) from its edge sum (re, im): i / |k|^2 of it, or the area at
+// the origin, in the box's scale and phase.
+__device__ __forceinline__ double2 poly_bin(int mx, int my, double re, double im,
+                                            const double* pdc, double dk, double L, double nf) {
+  double fr, fi;
+  if (mx == 0 && my == 0) {
+    fr = pdc[0];
+    fi = pdc[1];
+  } else {
+    const double kx = dk * mx, ky = dk * my;
+    const double inv = 1.0 / (kx * kx + ky * ky);
+    fr = -im * inv;
+    fi = re * inv;
+  }
+  double tt = (double)(mx + my) * (nf - 1.0) / nf;
+  tt -= 2.0 * rint(0.5 * tt);
+  double sv, cv;
+  sincospi(-tt, &sv, &cv);
+  const double scale = nf * nf / (L * L);
+  return make_double2(scale * (fr * cv - fi * sv), scale * (fr * sv + fi * cv));
+}
+
+// Adds v to what the rectangle pass stored at (col, row).
+__device__ __forceinline__ void poly_add(float2* mq, float2* mp, int W, int col, int row,
+                                         double vr, double vi) {
+  float2* q = mq + (size_t)col * W + row;
+  const float2 old = *q;
+  const float2 v = make_float2((float)((double)old.x + vr), (float)((double)old.y + vi));
+  *q = v;
+  if (mp) mp[((size_t)((col + 1) >> 1) * W + row) * 2 + ((col + 1) & 1)] = v;
+}
+
 // Simple polygons (mask.rs:1286-1352): for k = 2 pi m / L != 0
 //   \iint_P e^{-ik.r} = (i/|k|^2) sum_e s (kx dy - ky dx) sinc(k.d/2) e^{-ik.r_mid}
 // with s the polygon's orientation sign, and the area at k = 0.  edges:
@@ -183,8 +244,8 @@ __global__ __launch_bounds__(64 * SL) void k_rect_band(const double2* __restrict
 // clip = sum of (value - background) area.  The box bins |kx|, |ky| <= B get
 //   (N^2/L^2) e^{-i pi (mx + my)(N - 1)/N} x integral
 // added to what the rectangle pass stored (plain and column-paired).
-// wpc work-groups per clip (of up to 512 threads), one thread per tile of
-// kRectT rows x kRectT columns.  The clip's edges
+// The form for bands above 63: wpc work-groups per clip (of up to 512 threads), one
+// thread per tile of kRectT rows x kRectT columns.  The clip's edges
 // are taken in chunks; for each chunk the work-group first tabulates, per edge
 // and order m in [-B, B], w e^{-i kx cx} with (cos, sin)(kx dx / 2) and
 // e^{-i ky cy} with (cos, sin)(ky dy / 2) in LDS, then every tile reads its
@@ -248,33 +309,12 @@ __global__ __launch_bounds__(512) void k_poly_band(const double* __restrict__ ed
         double4 yv[kRectT];
 #pragma unroll
         for (int i = 0; i < kRectT; ++i) yv[i] = tab[(chunk + el) * nk + yi[i]];
-#pragma unroll
-        for (int j = 0; j < kRectT; ++j) {
-          const double4 xv = tab[el * nk + xi[j]];  // one column at a time (register budget)
-          const double kx = dk * (mx0 + j);
-#pragma unroll
-          for (int i = 0; i < kRectT; ++i) {
-            const double ky = dk * (my0 + i);
-            const double kn = kx * dy - ky * dx;
-            const double u = 0.5 * (kx * dx + ky * dy);
-            const double su = xv.w * yv[i].z + xv.z * yv[i].w;
-            double r = __builtin_amdgcn_rcp(u);
-            r = fma(r, fma(-u, r, 1.0), r);
-            r = fma(r, fma(-u, r, 1.0), r);
-            const double sc = fabs(u) < 1e-4 ? 1.0 - u * u * (1.0 / 6.0) : su * r;
-            const double a = kn * sc;
-            const double hr = xv.x * yv[i].x - xv.y * yv[i].y;
-            const double hi = xv.x * yv[i].y + xv.y * yv[i].x;
-            ar[i][j] = fma(a, hr, ar[i][j]);
-            ai[i][j] = fma(a, hi, ai[i][j]);
-          }
-        }
+        poly_edge(tab + el * nk, xi, yv, dx, dy, dk, mx0, my0, ar, ai);
       }
     }
   }
   if (!active) return;
   const double nf = (double)n;
-  const double scale = nf * nf / (L * L);
   float2* mq = Mq + (size_t)clip * W * W;
   float2* mp = Mp ? Mp + (size_t)clip * (W + 1) * W : nullptr;
 #pragma unroll
@@ -286,37 +326,165 @@ __global__ __launch_bounds__(512) void k_poly_band(const double* __restrict__ ed
       const int row = kRectT * gr + i, my = my0 + i;
       if (row >= W) break;
       if (mx < -B || mx > B || my < -B || my > B) continue;
-      double fr, fi;
-      if (mx == 0 && my == 0) {
-        fr = pdc[2 * clip];
-        fi = pdc[2 * clip + 1];
-      } else {
-        const double kx = dk * mx, ky = dk * my;
-        const double inv = 1.0 / (kx * kx + ky * ky);  // i / |k|^2
-        fr = -ai[i][j] * inv;
-        fi = ar[i][j] * inv;
+      const double2 v = poly_bin(mx, my, ar[i][j], ai[i][j], pdc + 2 * clip, dk, L, nf);
+      poly_add(mq, mp, W, col, row, v.x, v.y);
+    }
+  }
+}
+
+// The same for bands up to 63.  Work-group = 64 tiles x 8 waves, each wave taking every
+// eighth edge (one of a chunk of eight), so that few clips fill the chip: wpc
+// work-groups per clip.  The tables of a chunk are products of two short ones, orders
+// 16 a and b < 16 (m = 16 a + b), so an edge and axis take at most 24 pairs of sincos
+// instead of 2 B + 1.  HERM, where no edge has an imaginary weight: only the columns
+// kx <= 0 are summed, each bin's conjugate going to its mirror image.
+// What bounds it: the FP64 products and one work-group's registers per CU.  96 clips of
+// real polygons, B = 47: 430 us with one thread per tile, every bin and long tables
+// (192 work-groups of five waves), 413 with half the bins and half the work-groups, 238
+// so; at 128 registers, for two work-groups per CU, it spills (416).
+template <bool HERM>
+__global__ __launch_bounds__(512) void k_poly_band_sliced(
+    const double* __restrict__ edges, const int64_t* __restrict__ eoff,
+    const double* __restrict__ pdc, int n, double L, int B, int BB, int wpc,
+    float2* __restrict__ Mq, float2* __restrict__ Mp) {
+  constexpr int E = kPolySlices;
+  extern __shared__ double4 tab[];  // [axis][edge in chunk][m + B], then the short tables
+  const int W = 2 * BB + 1, nk = 2 * B + 1;
+  const int G = (W + kRectT - 1) / kRectT;
+  const int clip = blockIdx.x / wpc;
+  const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
+  const int t = (blockIdx.x - clip * wpc) * 64 + lane;  // tile index
+  const int64_t e0 = eoff[clip], e1 = eoff[clip + 1];
+  if (e0 == e1) return;  // uniform over the work-group
+  const bool active = t < (HERM ? BB / kRectT + 1 : G) * G;
+  const int gc = active ? t / G : 0, gr = active ? t - (t / G) * G : 0;
+  const int mx0 = kRectT * gc - BB, my0 = kRectT * gr - BB;
+  const double dk = 2.0 * M_PI / L;
+  const int A = (B + 15) / 16, NS = 2 * A + 1 + 16;  // orders 16 (-A .. A), then 0 .. 15
+  double4* const sht = tab + 2 * E * nk;             // [axis][edge][NS]
+  int xi[kRectT], yi[kRectT];
+#pragma unroll
+  for (int j = 0; j < kRectT; ++j) {
+    xi[j] = min(max(mx0 + j + B, 0), nk - 1);
+    yi[j] = min(max(my0 + j + B, 0), nk - 1);
+  }
+  double ar[kRectT][kRectT], ai[kRectT][kRectT];
+#pragma unroll
+  for (int i = 0; i < kRectT; ++i)
+#pragma unroll
+    for (int j = 0; j < kRectT; ++j) ar[i][j] = ai[i][j] = 0.0;
+  for (int64_t cb = e0; cb < e1; cb += E) {
+    const int ne = (int)min((int64_t)E, e1 - cb);
+    for (int q = threadIdx.x; q < 2 * ne * NS; q += 512) {
+      const int axis = q / (ne * NS), r = q - axis * ne * NS;
+      const int el = r / NS, i = r - el * NS;
+      const double* p = edges + 6 * (cb + el);
+      const double k = dk * (i <= 2 * A ? 16 * (i - A) : i - 2 * A - 1);
+      double sv, cv, sh, ch;
+      sincos(k * (axis == 0 ? p[2] : p[3]), &sv, &cv);
+      sincos(0.5 * k * (axis == 0 ? p[0] : p[1]), &sh, &ch);
+      double pr = cv, pi = -sv;  // e^{-i k c}, times the edge weight on the x axis, once
+      if (axis == 0 && i <= 2 * A) {
+        const double wr = p[4], wi = p[5];
+        const double tr = wr * pr - wi * pi;
+        pi = wr * pi + wi * pr;
+        pr = tr;
       }
-      double tt = (double)(mx + my) * (nf - 1.0) / nf;
-      tt -= 2.0 * rint(0.5 * tt);
-      double sv, cv;
-      sincospi(-tt, &sv, &cv);
-      const double vr = scale * (fr * cv - fi * sv), vi = scale * (fr * sv + fi * cv);
-      float2* q = mq + (size_t)col * W + row;
-      const float2 old = *q;
-      const float2 v = make_float2((float)((double)old.x + vr), (float)((double)old.y + vi));
-      *q = v;
-      if (mp) mp[((size_t)((col + 1) >> 1) * W + row) * 2 + ((col + 1) & 1)] = v;
+      sht[(axis * E + el) * NS + i] = make_double4(pr, pi, ch, sh);
+    }
+    __syncthreads();  // the short tables; and the previous chunk has been consumed
+    for (int q = threadIdx.x; q < 2 * ne * nk; q += 512) {
+      const int axis = q / (ne * nk), r = q - axis * ne * nk;
+      const int el = r / nk, mi = r - el * nk, m = mi - B + 16 * A;
+      const double4* s = sht + (axis * E + el) * NS;
+      const double4 u = s[m >> 4], v = s[2 * A + 1 + (m & 15)];
+      tab[(axis * E + el) * nk + mi] =
+          make_double4(u.x * v.x - u.y * v.y, u.x * v.y + u.y * v.x, u.z * v.z - u.w * v.w,
+                       u.w * v.z + u.z * v.w);
+    }
+    __syncthreads();
+    if (active && slice < ne) {
+      const double dx = edges[6 * (cb + slice)], dy = edges[6 * (cb + slice) + 1];
+      double4 yv[kRectT];
+#pragma unroll
+      for (int i = 0; i < kRectT; ++i) yv[i] = tab[(E + slice) * nk + yi[i]];
+      poly_edge(tab + slice * nk, xi, yv, dx, dy, dk, mx0, my0, ar, ai);
+    }
+  }
+  // the waves' sums, by halves
+  double* const red = reinterpret_cast<double*>(tab);
+#pragma unroll
+  for (int h = E / 2; h >= 1; h /= 2) {
+    __syncthreads();
+    if (slice >= h && slice < 2 * h) {
+#pragma unroll
+      for (int i = 0; i < kRectT; ++i)
+#pragma unroll
+        for (int j = 0; j < kRectT; ++j) {
+          double* r = red + ((slice - h) * 2 * kRectT * kRectT + 2 * (i * kRectT + j)) * 64 + lane;
+          r[0] = ar[i][j];
+          r[64] = ai[i][j];
+        }
+    }
+    __syncthreads();
+    if (slice < h) {
+#pragma unroll
+      for (int i = 0; i < kRectT; ++i)
+#pragma unroll
+        for (int j = 0; j < kRectT; ++j) {
+          const double* r = red + (slice * 2 * kRectT * kRectT + 2 * (i * kRectT + j)) * 64 + lane;
+          ar[i][j] += r[0];
+          ai[i][j] += r[64];
+        }
+    }
+  }
+  if (!active || slice != 0) return;
+  float2* mq = Mq + (size_t)clip * W * W;
+  float2* mp = Mp ? Mp + (size_t)clip * (W + 1) * W : nullptr;
+#pragma unroll
+  for (int j = 0; j < kRectT; ++j) {
+    const int col = kRectT * gc + j, mx = mx0 + j;
+    if (col >= W || (HERM && mx > 0)) break;
+#pragma unroll
+    for (int i = 0; i < kRectT; ++i) {
+      const int row = kRectT * gr + i, my = my0 + i;
+      if (row >= W) break;
+      if (mx < -B || mx > B || my < -B || my > B) continue;
+      const double2 v = poly_bin(mx, my, ar[i][j], ai[i][j], pdc + 2 * clip, dk, L, (double)n);
+      poly_add(mq, mp, W, col, row, v.x, v.y);
+      if (HERM && mx < 0) poly_add(mq, mp, W, 2 * BB - col, 2 * BB - row, v.x, -v.y);
     }
   }
 }
 
 hipError_t launch_poly_band(const double* edges, const int64_t* eoff, const double* pdc,
-                            int nclips, int n, double L, int B, int BB, float2* Mq, float2* Mp,
-                            hipStream_t s) {
+                            bool real, int nclips, int n, double L, int B, int BB, float2* Mq,
+                            float2* Mp, hipStream_t s) {
   if (nclips <= 0) return hipSuccess;
   if (B < 0 || BB < B || B > kPolyMaxBand || BB > 1024) return hipErrorInvalidValue;
   const int W = 2 * BB + 1, nk = 2 * B + 1;
   const int G = (W + kRectT - 1) / kRectT;
+  // Eight edges' tables take up to 78 KiB of LDS at 63, the widest band of an image; a
+  // wider one would leave most waves without an edge.
+  if (B <= 63) {
+    const int tiles = (real ? BB / kRectT + 1 : G) * G, wpc = (tiles + 63) / 64;
+    if ((int64_t)wpc * nclips >= (1ll << 31)) return hipErrorInvalidValue;
+    const int ns = 2 * ((B + 15) / 16) + 17;
+    const size_t lds = std::max((size_t)2 * kPolySlices * (nk + ns) * sizeof(double4),
+                                (size_t)kPolySlices * kRectT * kRectT * 64 * sizeof(double));
+    auto kern = real ? k_poly_band_sliced<true> : k_poly_band_sliced<false>;
+    // sized for B = 63, once each
+    constexpr int most = 2 * kPolySlices * (127 + 25) * (int)sizeof(double4);
+    static const hipError_t attr[2] = {
+        hipFuncSetAttribute((const void*)k_poly_band_sliced<false>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, most),
+        hipFuncSetAttribute((const void*)k_poly_band_sliced<true>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, most)};
+    if (attr[real] != hipSuccess) return attr[real];
+    hipLaunchKernelGGL(kern, dim3((unsigned)(wpc * nclips)), dim3(512), lds, s, edges, eoff, pdc, n,
+                       L, B, BB, wpc, Mq, Mp);
+    return hipGetLastError();
+  }
   const int wpc = (G * G + 511) / 512;
   const int threads = ((((G * G + wpc - 1) / wpc) + 63) / 64) * 64;
   if ((int64_t)wpc * nclips >= (1ll << 31)) return hipErrorInvalidValue;

@@ -26,8 +26,9 @@ constexpr int kPolyMaxBand = 511;
 // (dx, dy, cx, cy, re, im) per edge, (re, im) = orientation sign x (value -
 // background); eoff: nclips + 1 edge offsets; pdc: per clip sum of
 // (value - background) x area (nm^2).
+// real: no edge has an imaginary weight (half of the bins are then computed).
 hipError_t launch_poly_band(const double* edges, const int64_t* eoff, const double* pdc,
-                            int nclips, int n, double L, int B, int BB, float2* Mq, float2* Mp,
+                            bool real, int nclips, int n, double L, int B, int BB, float2* Mq, float2* Mp,
                             hipStream_t s);
 
 }  // namespace huvk
