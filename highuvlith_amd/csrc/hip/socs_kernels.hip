@@ -330,7 +330,9 @@ __global__ __launch_bounds__(64) void k_rows_pruned(const float* __restrict__ ma
     for (int i = 0; i < 32; ++i) {
       const int x = t + L * i;
       if constexpr (CX) {
-        const float2 z = reinterpret_cast<const float2*>(a)[x];
+        // 8 bytes at the 4-byte alignment that a caller's pairs of floats have
+        typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+        const f2 z = reinterpret_cast<const f2*>(a)[x];
         v[i] = c32{z.x, z.y};
       } else if constexpr (L >= 32) {
         v[i] = c32{__builtin_nontemporal_load(a + x), __builtin_nontemporal_load(a + N + x)};
@@ -1229,8 +1231,13 @@ __device__ __forceinline__ void chain_task(float beta, const c32* d, int C, int 
 // img / ncond, condition img % ncond).  MODE 2 (chain): the image is dC/dm of
 // ILT row img, and dC/dtheta goes to row (ch.orows ? ch.orows[img] : img) of
 // ch.grad (chain_task).
+//
+// Five waves per SIMD where the image form of four folds fits 96 registers without
+// spilling: 38 images of 1024^2 are then one generation of work-groups instead of 1.2
+// (complex call 144.2 -> 139.6 us).  The other forms would spill 3 to 15 registers
+// (three planes of 512^2 59.3 -> 61.8 us, the gradient of 512^2 254 -> 258).
 template <int TMIN, int TMAX, int MODE>
-__global__ __launch_bounds__(256) void k_band_image(const float2* __restrict__ Ib, int n, int G,
+__global__ __launch_bounds__(256, TMIN == -2 && MODE == 0 ? 5 : 1) void k_band_image(const float2* __restrict__ Ib, int n, int G,
                                                     int nimg, const float2* __restrict__ tw_n,
                                                     float* __restrict__ out, PlaneMap map,
                                                     FidelityEpi epi, ChainEpi ch) {
