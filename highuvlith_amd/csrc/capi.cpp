@@ -314,39 +314,26 @@ void Ctx::drop_graph(GraphEntry& g) {
 }
 
 void Ctx::forget_kset(uint64_t id) {
-  bool busy = false;
-  for (auto it = graphs.begin(); it != graphs.end();) {
-    if (std::find(it->second.ksets.begin(), it->second.ksets.end(), id) != it->second.ksets.end()) {
-      if (!busy) hipStreamSynchronize(stream());
-      if (!busy && own_stream) hipStreamSynchronize(own_stream);
-      busy = true;
-      drop_graph(it->second);
-      it = graphs.erase(it);
-    } else {
-      ++it;
-    }
-  }
-  for (auto it = plane_tables.begin(); it != plane_tables.end();) {
-    if (std::find(it->first.begin(), it->first.end(), id) != it->first.end()) {
-      if (!busy) hipStreamSynchronize(stream());
-      busy = true;
-      hipFree(it->second);
-      it = plane_tables.erase(it);
-    } else {
-      ++it;
-    }
-  }
-  for (auto it = plane_packs.begin(); it != plane_packs.end();) {
-    if (std::find(it->first.begin(), it->first.end(), id) != it->first.end()) {
-      if (!busy) hipStreamSynchronize(stream());
-      busy = true;
-      hipFree(it->second.kern);
-      hipFree(it->second.tab);
-      it = plane_packs.erase(it);
-    } else {
-      ++it;
-    }
-  }
+  bool idle = false;
+  auto wait = [&] {  // before the first entry goes
+    if (idle) return;
+    hipStreamSynchronize(stream());
+    if (own_stream) hipStreamSynchronize(own_stream);
+    idle = true;
+  };
+  forget_entries(graphs, id, [&](GraphEntry& g) {
+    wait();
+    drop_graph(g);
+  });
+  forget_entries(plane_tables, id, [&](void* t) {
+    wait();
+    hipFree(t);
+  });
+  forget_entries(plane_packs, id, [&](PlanePack& p) {
+    wait();
+    hipFree(p.kern);
+    hipFree(p.tab);
+  });
 }
 
 huv_status band_stage(Ctx* c, int nclips, int n, int B, int BB, const float* masks, float2* Mq,
@@ -1135,9 +1122,8 @@ huv_status kset_real(huv_kset* ks, bool boxes) {
 // tables, uploaded once per distinct plane list.
 huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, bool real_masks,
                        const int** dK, const float2* const** dkern, const float* const** dlam) {
-  std::vector<uint64_t> key;
-  for (int p = 0; p < nplanes; ++p) key.push_back(planes[p]->id);
-  key.push_back((uint64_t)real_masks);
+  PlaneKey key{{}, {(uint64_t)real_masks}};
+  for (int p = 0; p < nplanes; ++p) key.ksets.push_back(planes[p]->id);
   const size_t offk = 0, offp = ((size_t)nplanes * sizeof(int) + 63) / 64 * 64;
   const size_t offl = offp + (size_t)nplanes * sizeof(void*);
   const size_t tbl = offl + (size_t)nplanes * sizeof(void*);
@@ -1184,15 +1170,12 @@ huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, bool real_m
 huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool paired,
                       bool real_masks, const Ctx::PlanePack** pack) {
   const int BB = huvk::coarse_band(m), Q = huvk::coarse_classes(m);
-  std::vector<uint64_t> key;
-  for (int p = 0; p < nplanes; ++p) key.push_back(planes[p]->id);
-  key.push_back((uint64_t)m);
-  key.push_back((uint64_t)paired);
-  key.push_back((uint64_t)real_masks);
+  PlaneKey key{{}, {(uint64_t)m, (uint64_t)paired, (uint64_t)real_masks}};
+  for (int p = 0; p < nplanes; ++p) key.ksets.push_back(planes[p]->id);
   auto it = c->plane_packs.find(key);
   if (it == c->plane_packs.end() && c->fixed_mode) {
     // a stack built by an earlier call for complex masks serves real ones too
-    key.back() = 0;
+    key.form.back() = 0;
     it = c->plane_packs.find(key);
     if (it == c->plane_packs.end())
       return fail(HUV_INVALID_PARAMETER,
@@ -1581,8 +1564,7 @@ huv_status socs_shape(Ctx* c, int nclips, int n, const MaskSource& src, int npla
 
 // Runs body() eagerly, or replays / records a graph of it keyed by `key`.
 template <class Body>
-huv_status graph_run(Ctx* c, const std::vector<uint64_t>& key, const std::vector<uint64_t>& ksets,
-                     Body body) {
+huv_status graph_run(Ctx* c, const PlaneKey& key, Body body) {
   auto it = c->graphs.find(key);
   if (it != c->graphs.end() && it->second.generation == c->ws.generation) {
     hipStream_t own = c->own_stream, act = c->active;
@@ -1636,7 +1618,6 @@ huv_status graph_run(Ctx* c, const std::vector<uint64_t>& key, const std::vector
   Ctx::GraphEntry ge;
   ge.graph = g;
   ge.generation = gen;
-  ge.ksets = ksets;
   e = hipGraphInstantiate(&ge.exec, g, nullptr, nullptr, 0);
   if (e != hipSuccess) {
     hipGraphDestroy(g);
@@ -1660,8 +1641,7 @@ huv_status socs_groups(Ctx* c, int ngroups, const huv_clip_group* groups, const 
   };
   const bool pt = opts && opts->pixel_transfer;
   std::vector<GroupPlan> plan;
-  std::vector<uint64_t> key{(uint64_t)tag, (uint64_t)pt, (uint64_t)ngroups};
-  std::vector<uint64_t> ksets;
+  PlaneKey key{{}, {(uint64_t)tag, (uint64_t)pt, (uint64_t)ngroups}};
   for (int i = 0; i < ngroups; ++i) {
     const huv_clip_group& g = groups[i];
     if (g.nclips == 0) continue;
@@ -1671,14 +1651,11 @@ huv_status socs_groups(Ctx* c, int ngroups, const huv_clip_group* groups, const 
                                &gp.t, &computed);
     if (st != HUV_OK) return st;
     plan.push_back(gp);
-    key.insert(key.end(), {(uint64_t)g.n, (uint64_t)g.nclips, (uint64_t)(uintptr_t)g.masks,
+    key.form.insert(key.form.end(), {(uint64_t)g.n, (uint64_t)g.nclips, (uint64_t)(uintptr_t)g.masks,
                            (uint64_t)(uintptr_t)g.out, (uint64_t)g.nplanes, (uint64_t)gp.t.m,
                            (uint64_t)gp.t.n1, (uint64_t)gp.t.xnb, (uint64_t)gp.t.xlanes,
                            (uint64_t)gp.t.chunks});
-    for (int p = 0; p < g.nplanes; ++p) {
-      key.push_back(g.planes[p]->id);
-      ksets.push_back(g.planes[p]->id);
-    }
+    for (int p = 0; p < g.nplanes; ++p) key.ksets.push_back(g.planes[p]->id);
   }
   auto body = [&]() -> huv_status {
     for (const auto& gp : plan) {
@@ -1688,7 +1665,7 @@ huv_status socs_groups(Ctx* c, int ngroups, const huv_clip_group* groups, const 
     }
     return HUV_OK;
   };
-  if (opts && opts->graph) return graph_run(c, key, ksets, body);
+  if (opts && opts->graph) return graph_run(c, key, body);
   return body();
 }
 

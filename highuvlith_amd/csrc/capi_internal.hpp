@@ -12,6 +12,7 @@
 #include "../../include/huv.h"
 #include "hip/socs_kernels.hpp"
 #include "host/engine.hpp"
+#include "host/plane_key.hpp"
 
 // A kernel set built on the host (huv_kernels_build) or with the device's
 // help (huv_kernels_build_device).
@@ -49,8 +50,9 @@ struct Ctx {
   std::map<int, float2*> tw;
   std::map<long, float*> sinc;
   // Device copies of per-plane pointer tables and packed kernel stacks, keyed
-  // by the ids of the kernel sets in a plane list (dropped when a set dies).
-  std::map<std::vector<uint64_t>, void*> plane_tables;
+  // by the kernel sets of a plane list (dropped when a set dies).  A table's
+  // form: whether it is the one for real masks.
+  std::map<PlaneKey, void*> plane_tables;
   struct PlanePack {
     float2* kern = nullptr;  // [Q][total] boxes (W x W or column-paired)
     int* tab = nullptr;      // nd PlaneStacks, then map.src, map.off, map.list
@@ -60,21 +62,20 @@ struct Ctx {
     const huvk::PlaneStack* stacks() const { return (const huvk::PlaneStack*)tab; }
     huvk::PlaneMap map;      // src null where every plane has its own image
   };
-  // keyed by the kernel-set ids followed by the coarse size, the box layout
-  // and whether the stack is the one for real masks
-  std::map<std::vector<uint64_t>, PlanePack> plane_packs;
+  // form: the coarse size, the box layout and whether the stack is the one for
+  // real masks
+  std::map<PlaneKey, PlanePack> plane_packs;
   // Launch shapes chosen by the autotuner, keyed by (n, band, nplanes, Kmax).
   std::map<std::vector<int>, huv_socs_tuning> tuned;
   bool autotune = false;
-  // Captured launch sequences, keyed by the call's pointers, sizes and
-  // kernel-set ids; valid while the workspace generation is unchanged.
+  // Captured launch sequences, keyed by the call's kernel sets, pointers and
+  // sizes; valid while the workspace generation is unchanged.
   struct GraphEntry {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint64_t generation = 0;
-    std::vector<uint64_t> ksets;
   };
-  std::map<std::vector<uint64_t>, GraphEntry> graphs;
+  std::map<PlaneKey, GraphEntry> graphs;
   // Pinned host staging area and its device mirror for small per-step
   // uploads (the ILT driver's coefficients and row lists), grown on demand.
   char* pin_h = nullptr;
