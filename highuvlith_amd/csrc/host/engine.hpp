@@ -144,13 +144,15 @@ struct KernelSet {
 // The real fields v_j (j < R) of a kernel set on masks with a real
 // transmittance: sum_k lambda_k |E_k|^2 = sum_j v_j^2 with each v_j the field
 // of a Hermitian function on the |kx|, |ky| <= B box (real_form.cpp); mu[j] is
-// v_j's squared norm (decreasing), the ones dropped sum to at most 2^-28 of the
-// trace.  False (no form) for more than kRealFieldsMaxKernels kernels, negative
-// or non-finite input.  support / eig / values as huv_kset_upload.
+// v_j's squared norm (decreasing).  The ones dropped move an image by at most
+// 2^-25 of peak times the mean of the mask's squared transmittance, peak being the
+// largest intensity one unit order gives (the clear field, as a rule).  False (no
+// form) for more than kRealFieldsMaxKernels kernels, negative or non-finite
+// input.  support / eig / values as huv_kset_upload.
 constexpr int kRealFieldsMaxKernels = 128;
 struct RealFields {
   int B = 0, R = 0;
-  double trace = 0.0;
+  double trace = 0.0, peak = 0.0;
   std::vector<double> mu;
   std::vector<double> v;  // R vectors of (2B+1)^2
 };
@@ -158,7 +160,8 @@ bool real_fields(int n, int B, int K, int64_t S, const int64_t* support, const d
                  const double* values, RealFields& out);
 // The Hermitian function of v_j at (kx, ky), |kx|, |ky| <= B.
 cd real_field_value(const RealFields& f, int j, int kx, int ky);
-// Whether two sets give every real mask the same image (to 2^-26 of it).
+// Whether two sets give every real mask the same image (their forms are within 2^-26
+// of peak).
 bool same_real_form(const RealFields& a, const RealFields& b);
 
 struct BuildSettings {

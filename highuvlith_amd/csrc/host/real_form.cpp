@@ -32,11 +32,15 @@ double dotr(const double* a, const double* b, size_t n) {
   return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
-// The dropped eigenvalues' sum relative to the trace: a sixteenth of an FP32
-// ulp of the image.
-constexpr double kDrop = 1.0 / (double)(1 << 28);
-// How far two planes' forms may differ (Frobenius norm over the trace) to
-// count as one: a quarter of an FP32 ulp.
+// Both limits are parts of the largest intensity that one unit order gives (peak),
+// the clear field where the optics pass the zero order: a form of norm q moves no
+// image of a mask by more than q times the mean of its squared transmittance.
+// (The trace would be no such scale: it grows with the band's area, to 153 .. 2469
+// clear fields for the annular source at 2 nm, 512^2 .. 2048^2.)
+// The dropped eigenvalues' sum: what one FP32 rounding of the clear field is.
+constexpr double kDrop = 1.0 / (double)(1 << 25);
+// How far two planes' forms may differ (Frobenius norm) to count as one: half of
+// that.  Opposite focus planes of a point-symmetric source are 1e-12 apart.
 constexpr double kSame = 1.0 / (double)(1 << 26);
 
 }  // namespace
@@ -91,10 +95,19 @@ bool real_fields(int n, int B, int K, int64_t S, const int64_t* support, const d
   if (!hermitian_eigen_desc(gram, F, F, mu, U)) return false;
   double trace = 0.0;
   for (double m : mu) trace += std::max(m, 0.0);
-  if (!(trace > 0.0)) return false;
+  std::vector<double> power(half + 1, 0.0);  // sum of |v(f)|^2 over the half box
+  for (int i = 0; i < F; ++i) {
+    const double* p = v.data() + (size_t)i * N;
+    for (size_t x = 0; x < half; ++x)
+      power[x] += 0.5 * (p[2 * x] * p[2 * x] + p[2 * x + 1] * p[2 * x + 1]);
+    power[half] += p[N - 1] * p[N - 1];
+  }
+  double peak = 0.0;
+  for (double p : power) peak = std::max(peak, p);
+  if (!(peak > 0.0) || !std::isfinite(trace)) return false;
   int R = F;
   double tail = 0.0;
-  while (R > 1 && tail + std::max(mu[R - 1], 0.0) <= kDrop * trace) tail += std::max(mu[--R], 0.0);
+  while (R > 1 && tail + std::max(mu[R - 1], 0.0) <= kDrop * peak) tail += std::max(mu[--R], 0.0);
   for (int j = 0; j < R; ++j) {
     double im = 0.0;
     for (int i = 0; i < F; ++i) im = std::max(im, std::fabs(U[(size_t)j * F + i].imag()));
@@ -103,6 +116,7 @@ bool real_fields(int n, int B, int K, int64_t S, const int64_t* support, const d
   out.B = B;
   out.R = R;
   out.trace = trace;
+  out.peak = peak;
   out.mu.assign(mu.begin(), mu.begin() + R);
   out.v.assign((size_t)R * N, 0.0);
   for (int j = 0; j < R; ++j) {
@@ -131,9 +145,8 @@ cd real_field_value(const RealFields& f, int j, int kx, int ky) {
 // with orthonormal coordinates; both defects are formed without cancellation.
 bool same_real_form(const RealFields& a, const RealFields& b) {
   if (a.R < 1 || a.R != b.R || a.B != b.B) return false;
-  if (std::fabs(a.trace - b.trace) > kSame * a.trace) return false;
   for (int j = 0; j < a.R; ++j)
-    if (std::fabs(a.mu[j] - b.mu[j]) > kSame * a.trace) return false;
+    if (std::fabs(a.mu[j] - b.mu[j]) > kSame * a.peak) return false;
   const int R = a.R;
   const size_t N = (size_t)(2 * a.B + 1) * (2 * a.B + 1);
   std::vector<double> c((size_t)R * R);  // c[i][l]: b_l = sum_i c[i][l] a_i / mu_i
@@ -159,7 +172,7 @@ bool same_real_form(const RealFields& a, const RealFields& b) {
     }
     res += dotr(r.data(), r.data(), N);
   }
-  return std::sqrt(in) + 2.0 * std::sqrt(res * a.trace) <= kSame * a.trace;
+  return std::sqrt(in) + 2.0 * std::sqrt(res * a.trace) <= kSame * a.peak;
 }
 
 }  // namespace huv
