@@ -1083,13 +1083,35 @@ static huv::cd packed_value(const huv::RealFields& f, int j, int kx, int ky) {
   return (a + huv::cd(0, 1) * b) / std::sqrt(pow2_scale(f.mu[0]));
 }
 
+// The set's form into ks->rf, with the fields where they are fewer than the kernels
+// or always (`all`); without a form, or the memory for one, ks->rf stays empty.
+static bool kset_form(huv_kset* ks, bool all) {
+  try {
+    if (huv::real_form(ks->n, ks->B, ks->K, ks->S, ks->support.data(), ks->lam_host.data(),
+                       ks->values.data(), !all, ks->rf))
+      return true;
+  } catch (const std::exception&) {
+  }
+  ks->rf = huv::RealFields();
+  return false;
+}
+
+// Whether two sets give every real mask the same image.
+static bool same_images(huv_kset* a, huv_kset* b) {
+  if (a == b) return true;
+  try {
+    return huv::same_eigenvalues(a->rf, b->rf) && (!a->rf.v.empty() || kset_form(a, true)) &&
+           (!b->rf.v.empty() || kset_form(b, true)) && huv::same_real_form(a->rf, b->rf);
+  } catch (const std::exception&) {
+    return false;
+  }
+}
+
 huv_status kset_real(huv_kset* ks, bool boxes) {
   if (!ks->real_done) {
-    if (huv::real_fields(ks->n, ks->B, ks->K, ks->S, ks->support.data(), ks->lam_host.data(),
-                         ks->values.data(), ks->rf)) {
-      const int kr = (ks->rf.R + 1) / 2;
-      ks->Kr = kr < ks->K ? kr : 0;
-    }
+    // Nothing to gain, as a rule out of focus: the eigenvalues tell, before any field
+    // is computed.
+    if (kset_form(ks, false) && !ks->rf.v.empty()) ks->Kr = (ks->rf.R + 1) / 2;
     ks->real_done = true;
   }
   if (!boxes || !ks->Kr || ks->kern_r) return HUV_OK;
@@ -1192,13 +1214,15 @@ huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool 
         const huv_status st = kset_real(planes[p], false);
         if (st != HUV_OK) return st;
         for (int t = 0; t < (int)rep.size() && u == (int)rep.size(); ++t)
-          if (planes[rep[t]] == planes[p] || huv::same_real_form(planes[rep[t]]->rf, planes[p]->rf))
-            u = t;
+          if (same_images(planes[rep[t]], planes[p])) u = t;
       }
       src[p] = u;
       if (u == (int)rep.size()) rep.push_back(p);
     }
     pk.nd = (int)rep.size();
+    // fields computed for the comparison alone
+    for (int p = 0; p < nplanes; ++p)
+      if (!planes[p]->Kr) std::vector<double>().swap(planes[p]->rf.v);
     // longest stacks first: the field work-groups of the last plane end a launch
     auto count = [&](int t) { return real_masks && planes[t]->Kr ? planes[t]->Kr : planes[t]->K; };
     std::vector<int> order(pk.nd), where(pk.nd);

@@ -104,6 +104,9 @@ struct ColMatrix {
 // tridiagonalisation + phase normalisation + implicit QL (linalg.rs:324-551).
 bool hermitian_eigen_desc(const std::vector<cd>& h, int64_t n, int64_t count,
                           std::vector<double>& values, std::vector<cd>& vectors);
+// The same for a real symmetric matrix, whose vectors are real; count 0: values alone.
+bool symmetric_eigen_desc(std::vector<double> a, int64_t n, int64_t count,
+                          std::vector<double>& values, std::vector<double>& vectors);
 
 // Leading eigenpairs of X X^H by randomized subspace iteration
 // (linalg.rs:657-679).  Gaussian stream: splitmix64 + Box-Muller (the
@@ -154,14 +157,21 @@ struct RealFields {
   int B = 0, R = 0;
   double trace = 0.0, peak = 0.0;
   std::vector<double> mu;
-  std::vector<double> v;  // R vectors of (2B+1)^2
+  std::vector<double> v;  // R vectors of (2B+1)^2, padded to an even length
 };
-bool real_fields(int n, int B, int K, int64_t S, const int64_t* support, const double* eig,
-                 const double* values, RealFields& out);
+// fewer_only: v only where two fields to a transform are fewer than K (the rest costs
+// a fifth to a third of v).
+bool real_form(int n, int B, int K, int64_t S, const int64_t* support, const double* eig,
+               const double* values, bool fewer_only, RealFields& out);
+inline bool real_fields(int n, int B, int K, int64_t S, const int64_t* support, const double* eig,
+                        const double* values, RealFields& out) {
+  return real_form(n, B, K, S, support, eig, values, false, out);
+}
 // The Hermitian function of v_j at (kx, ky), |kx|, |ky| <= B.
 cd real_field_value(const RealFields& f, int j, int kx, int ky);
 // Whether two sets give every real mask the same image (their forms are within 2^-26
-// of peak).
+// of peak); same_eigenvalues, which needs no v, is a necessary condition.
+bool same_eigenvalues(const RealFields& a, const RealFields& b);
 bool same_real_form(const RealFields& a, const RealFields& b);
 
 struct BuildSettings {

@@ -115,7 +115,8 @@ void orthonormalize(ColMatrix& m, Rng& rng) {
   }
 }
 
-// Implicit QL for a real symmetric tridiagonal (linalg.rs:343-415).
+// Implicit QL for a real symmetric tridiagonal (linalg.rs:343-415); z may be empty
+// (eigenvalues alone).
 bool tql2(std::vector<double>& d, std::vector<double>& e, std::vector<double>& z) {
   const int64_t n = (int64_t)d.size();
   double dmax = 0, emax = 0;
@@ -159,6 +160,7 @@ bool tql2(std::vector<double>& d, std::vector<double>& e, std::vector<double>& z
         p = s * r;
         d[i + 1] = g + p;
         g = c * r - b;
+        if (z.empty()) continue;
         double* zi = z.data() + i * n;
         double* zi1 = z.data() + (i + 1) * n;
         for (int64_t k = 0; k < n; ++k) {
@@ -299,6 +301,71 @@ bool hermitian_eigen_desc(const std::vector<cd>& hin, int64_t n, int64_t count,
       cd* tail = vectors.data() + c * n + k + 1;
       const cd t = dotc(u.data(), tail, m) * 2.0;
       for (int64_t i = 0; i < m; ++i) tail[i] -= u[i] * t;
+    }
+  }
+  return true;
+}
+
+bool symmetric_eigen_desc(std::vector<double> a, int64_t n, int64_t count,
+                          std::vector<double>& values, std::vector<double>& vectors) {
+  values.clear();
+  vectors.clear();
+  if (n == 0) return true;
+  count = std::min(count, n);
+  double scale = 0.0;
+  for (double v : a) scale = std::max(scale, std::fabs(v));
+  const double inv = scale > 0.0 ? 1.0 / scale : 1.0;
+  for (double& v : a) v *= inv;
+  std::vector<double> d((size_t)n), e((size_t)n, 0.0), p((size_t)n);
+  // Reflector k zeroes column k below its first subdiagonal element and is kept in
+  // the column's place (unit norm; all zero for none).
+  for (int64_t k = 0; k + 2 < n; ++k) {
+    const int64_t m = n - k - 1;
+    double* u = a.data() + k * n + k + 1;
+    double alpha2 = 0.0;
+    for (int64_t i = 0; i < m; ++i) alpha2 += u[i] * u[i];
+    if (alpha2 == 0.0) continue;
+    const double beta = -std::copysign(std::sqrt(alpha2), u[0]);
+    e[k] = beta;
+    const double un = std::sqrt(2.0 * beta * (beta - u[0]));
+    u[0] -= beta;
+    for (int64_t i = 0; i < m; ++i) u[i] /= un;
+    std::fill(p.begin(), p.begin() + m, 0.0);
+    for (int64_t j = 0; j < m; ++j) {
+      const double* c = a.data() + (k + 1 + j) * n + k + 1;
+      const double uj = 2.0 * u[j];
+      for (int64_t i = 0; i < m; ++i) p[i] += c[i] * uj;
+    }
+    double kk = 0.0;
+    for (int64_t i = 0; i < m; ++i) kk += u[i] * p[i];
+    for (int64_t i = 0; i < m; ++i) p[i] -= u[i] * kk;
+    for (int64_t j = 0; j < m; ++j) {
+      double* c = a.data() + (k + 1 + j) * n + k + 1;
+      const double pj = p[j], uj = u[j];
+      for (int64_t i = 0; i < m; ++i) c[i] -= u[i] * pj + p[i] * uj;
+    }
+  }
+  if (n >= 2) e[n - 2] = a[(n - 2) * n + n - 1];
+  for (int64_t i = 0; i < n; ++i) d[i] = a[i * n + i];
+  std::vector<double> z(count > 0 ? (size_t)(n * n) : 0, 0.0);
+  for (int64_t i = 0; i < n && count > 0; ++i) z[i * n + i] = 1.0;
+  if (!tql2(d, e, z)) return false;
+  std::vector<int64_t> order((size_t)n);
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int64_t x, int64_t y) { return d[y] < d[x]; });
+  values.resize((size_t)n);
+  for (int64_t i = 0; i < n; ++i) values[i] = d[order[i]] * scale;
+  vectors.resize((size_t)(n * count));
+  for (int64_t c = 0; c < count; ++c) {
+    double* w = vectors.data() + c * n;
+    std::copy(z.begin() + order[c] * n, z.begin() + (order[c] + 1) * n, w);
+    for (int64_t k = n - 3; k >= 0; --k) {
+      const double* u = a.data() + k * n + k + 1;
+      const int64_t m = n - k - 1;
+      double t = 0.0;
+      for (int64_t i = 0; i < m; ++i) t += u[i] * w[k + 1 + i];
+      t *= 2.0;
+      for (int64_t i = 0; i < m; ++i) w[k + 1 + i] -= u[i] * t;
     }
   }
   return true;
