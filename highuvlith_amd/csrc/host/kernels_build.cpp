@@ -391,7 +391,11 @@ void rasterize_rects(const std::vector<RectFeature>& rects, cd bg, int n, double
 // own edges: a rectangle that meets no other is one cell whatever else the clip
 // holds, where a grid over all edges cuts it at every other rectangle's edges
 // (43 contacts of a jittered array: 43 cells instead of about 400, and a tenth of
-// the host time).  The limit on the whole clip's edge grid stays as it is.
+// the host time).  Groups that touch are also resolved together, where shapes made
+// of slabs or a tiling run on (1024 squares of one value in 32 rows: one cell), and
+// the fewer cells taken: a grid over a brickwork of many values may cut more than it
+// joins.  So a clip never has more cells than one grid over all edges gives it.  The
+// limit on the whole clip's edge grid stays as it is.
 namespace {
 
 struct PaintRect {
@@ -443,6 +447,22 @@ void resolve_group(const std::vector<PaintRect>& g, const std::vector<cd>& value
   }
 }
 
+// Disjoint sets of rectangles; a set's name is its first rectangle.
+struct Groups {
+  std::vector<int> root;
+  explicit Groups(size_t n) : root(n) {
+    for (size_t i = 0; i < n; ++i) root[i] = (int)i;
+  }
+  int find(int i) {
+    while (root[i] != i) i = root[i] = root[root[i]];
+    return i;
+  }
+  void join(int i, int j) {
+    const int a = find(i), b = find(j);
+    root[std::max(a, b)] = std::min(a, b);
+  }
+};
+
 // Overlap groups are found pair by pair; clips of more rectangles are one group
 // (as is every clip with `whole`).
 constexpr size_t kGroupMaxRects = 2048;
@@ -488,29 +508,47 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
     if (nx < 1 || ny < 1 || nx > max_cells / ny) return false;
   }
   whole = whole || R > kGroupMaxRects;
-  std::vector<int> root(R);
-  for (size_t i = 0; i < R; ++i) root[i] = whole ? 0 : (int)i;
-  auto find = [&](int i) {
-    while (root[i] != i) i = root[i] = root[root[i]];
-    return i;
-  };
+  // overlapping rectangles, and those that touch along an edge as well
+  Groups over(R), near(R);
   if (!whole)
     for (size_t i = 0; i < R; ++i)
-      for (size_t j = 0; j < i; ++j)
-        if (rs[i].x0 < rs[j].x1 && rs[j].x0 < rs[i].x1 && rs[i].y0 < rs[j].y1 &&
-            rs[j].y0 < rs[i].y1) {
-          const int a = find((int)i), b = find((int)j);
-          root[std::max(a, b)] = std::min(a, b);
-        }
+      for (size_t j = 0; j < i; ++j) {
+        const double ox = std::min(rs[i].x1, rs[j].x1) - std::max(rs[i].x0, rs[j].x0);
+        const double oy = std::min(rs[i].y1, rs[j].y1) - std::max(rs[i].y0, rs[j].y0);
+        if (ox > 0 && oy > 0) over.join((int)i, (int)j);
+        if ((ox > eps && oy >= -eps) || (oy > eps && ox >= -eps)) near.join((int)i, (int)j);
+      }
+  else
+    for (size_t i = 1; i < R; ++i) {
+      over.join((int)i, 0);
+      near.join((int)i, 0);
+    }
   // groups in the order of their first rectangle, painter order within each
-  std::vector<std::vector<int>> members(R);
-  for (size_t i = 0; i < R; ++i) members[find((int)i)].push_back((int)i);
+  std::vector<std::vector<int>> members(R), parts(R);
+  for (size_t i = 0; i < R; ++i) members[near.find((int)i)].push_back((int)i);
   std::vector<PaintRect> g;
-  for (size_t i = 0; i < R; ++i) {
-    if (members[i].empty()) continue;
+  std::vector<RectCell> joined;
+  for (const std::vector<int>& near_group : members) {
+    if (near_group.empty()) continue;
+    const size_t before = out.size();
+    for (int k : near_group) parts[over.find(k)].push_back(k);
+    size_t count = 0;
+    for (int k : near_group) {
+      if (parts[k].empty()) continue;
+      g.clear();
+      for (int t : parts[k]) g.push_back(rs[t]);
+      parts[k].clear();
+      resolve_group(g, values, eps, out);
+      ++count;
+    }
+    if (count < 2) continue;
     g.clear();
-    for (int k : members[i]) g.push_back(rs[k]);
-    resolve_group(g, values, eps, out);
+    for (int k : near_group) g.push_back(rs[k]);
+    joined.clear();
+    resolve_group(g, values, eps, joined);
+    if (joined.size() >= out.size() - before) continue;
+    out.resize(before);
+    out.insert(out.end(), joined.begin(), joined.end());
   }
   return true;
 }

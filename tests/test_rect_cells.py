@@ -1,0 +1,149 @@
+"""Cells of rectangle lists (resolve_rect_cells): the picture is the painter's one, and
+no list is cut into more cells than one grid over all its edges gives, with equal
+neighbours along x and equal neighbouring rows joined.
+"""
+import os
+import subprocess
+
+import pytest
+
+import highuvlith_amd as H
+
+HOST = os.path.join(os.path.dirname(os.path.abspath(H.__file__)), "csrc", "host")
+
+HEAD = r"""
+#include <chrono>
+#include <cmath>
+#include <cstdio>
+#include <functional>
+#include <random>
+#include <set>
+#include "engine.hpp"
+using namespace huv;
+typedef std::vector<RectFeature> List;
+static const int N = 1024;
+static const double PX = 1.0, HALF = 512.0;
+static std::mt19937_64 gen(11);
+static double uni(double a, double b) { return std::uniform_real_distribution<double>(a, b)(gen); }
+
+// Cells of one grid over all edges, and the value at (x, y).
+static long one_grid(const List& l, cd bg) {
+  std::set<double> xs, ys;
+  for (auto& r : l) {
+    for (double s : {-0.5, 0.5}) {
+      xs.insert(std::min(HALF, std::max(-HALF, r.x + s * r.w)));
+      ys.insert(std::min(HALF, std::max(-HALF, r.y + s * r.h)));
+    }
+  }
+  auto near = [](const std::set<double>& s) {
+    std::vector<double> o;
+    for (double v : s) if (o.empty() || v - o.back() > 1e-12 * 2 * HALF) o.push_back(v);
+    return o;
+  };
+  const std::vector<double> x = near(xs), y = near(ys);
+  auto at = [](const std::vector<double>& e, double v) {
+    return std::lower_bound(e.begin(), e.end(), std::min(HALF, std::max(-HALF, v)) - 1e-9) - e.begin();
+  };
+  const long nx = (long)x.size() - 1, ny = (long)y.size() - 1;
+  if (nx < 1 || ny < 1) return 0;
+  std::vector<std::vector<cd>> c(ny, std::vector<cd>(nx, bg));
+  for (auto& r : l)
+    for (long i = at(y, r.y - r.h / 2); i < std::min<long>(ny, at(y, r.y + r.h / 2)); ++i)
+      for (long j = at(x, r.x - r.w / 2); j < std::min<long>(nx, at(x, r.x + r.w / 2)); ++j)
+        c[i][j] = r.value;
+  long cells = 0;
+  for (long i = 0; i < ny; ++i) {
+    if (i && c[i] == c[i - 1]) continue;
+    for (long j = 0; j < nx; ++j) cells += c[i][j] != bg && (j == 0 || c[i][j] != c[i][j - 1]);
+  }
+  return cells;
+}
+
+static List tiles(int nx, int ny, double sx, double sy, double fill, double shift, cd v) {
+  List l;
+  for (int i = 0; i < ny; ++i)
+    for (int j = 0; j < nx; ++j)
+      l.push_back({sx * (j - 0.5 * nx + 0.5) + shift * (i % 2), sy * (i - 0.5 * ny + 0.5), sx * fill,
+                   sy * fill, v});
+  return l;
+}
+
+static List scatter(int n, double most, int values) {
+  List l;
+  for (int i = 0; i < n; ++i)
+    l.push_back({std::round(uni(-520, 520)), std::round(uni(-520, 520)), std::round(uni(1, most)),
+                 std::round(uni(1, most)), cd(1.0 + i % values, 0.25 * (i % 3))});
+  return l;
+}
+
+// 0, or what is wrong with the cells of l
+static int check(const List& l, cd bg) {
+  std::vector<RectCell> cells;
+  if (!resolve_rect_cells(l, bg, N, PX, 1 << 20, cells)) return 1;
+  if ((long)cells.size() > one_grid(l, bg)) {
+    std::printf("%zu rectangles: %zu cells, one grid %ld\n", l.size(), cells.size(), one_grid(l, bg));
+    return 2;
+  }
+  for (int t = 0; t < 400; ++t) {
+    double x = uni(-HALF, HALF), y = uni(-HALF, HALF);
+    if (t % 2 && !l.empty()) {  // near a rectangle
+      const RectFeature& r = l[(size_t)uni(0, l.size()) % l.size()];
+      x = r.x + uni(-0.6, 0.6) * r.w;
+      y = r.y + uni(-0.6, 0.6) * r.h;
+    }
+    if (std::fabs(x) >= HALF || std::fabs(y) >= HALF) continue;
+    cd want = bg, got = bg;
+    for (auto& r : l)
+      if (std::fabs(x - r.x) < r.w / 2 && std::fabs(y - r.y) < r.h / 2) want = r.value;
+    int in = 0;
+    for (auto& c : cells)
+      if (x > c.x0 && x < c.x1 && y > c.y0 && y < c.y1) {
+        got = bg + c.w;
+        ++in;
+      }
+    if (in > 1 || std::abs(got - want) > 1e-12) return 3;
+  }
+  return 0;
+}
+"""
+
+BODIES = {
+    # shapes made of slabs, tilings, steps and bricks: joined across touching edges
+    "touching": r"""
+int main() {
+  for (cd bg : {cd(0, 0), cd(0.3, -0.1)}) {
+    std::vector<RectCell> cells;
+    if (!resolve_rect_cells(tiles(32, 32, 16, 16, 1, 0, 1.0), bg, N, PX, 1 << 20, cells)) return 9;
+    if (cells.size() != 1) return 8;
+    List steps, ls;
+    for (int i = 0; i < 60; ++i) steps.push_back({-300.0 + 10 * i, 4.0 * i, 10, 20, 1.0});
+    for (int i = 0; i < 5; ++i)
+      for (int j = 0; j < 5; ++j) {
+        ls.push_back({-440.0 + 180 * j, -440.0 + 180 * i, 20, 80, 1.0});
+        ls.push_back({-405.0 + 180 * j, -470.0 + 180 * i, 50, 20, 1.0});
+      }
+    for (const List& l : {tiles(32, 32, 16, 16, 1, 0, 1.0), tiles(20, 40, 40, 20, 1, 20, 1.0),
+                          tiles(9, 9, 30, 30, 1, 3.7, 0.5), tiles(7, 7, 40, 40, 0.5, 0, 1.0),
+                          steps, ls, List{}, scatter(1, 90, 1)})
+      if (int e = check(l, bg)) return e;
+    for (int n : {2, 3, 8, 30, 90})
+      for (double most : {40.0, 200.0})
+        for (int r = 0; r < 6; ++r)
+          if (int e = check(scatter(n, most, 1 + r), bg)) return e;
+  }
+  return 0;
+}
+""",
+}
+
+
+@pytest.mark.parametrize("case", sorted(BODIES))
+def test_cells(tmp_path, case):
+    src, exe = tmp_path / "cells.cpp", tmp_path / "cells"
+    src.write_text(HEAD + BODIES[case])
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", HOST, str(src)]
+                   + [os.path.join(HOST, f) for f in ("kernels_build.cpp", "linalg.cpp",
+                                                      "optics_source.cpp")]
+                   + ["-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
