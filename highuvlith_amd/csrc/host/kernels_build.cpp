@@ -476,20 +476,28 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
   const double eps = 1e-12 * (2.0 * half);
   std::vector<PaintRect> rs;
   std::vector<cd> values{bg};
+  std::map<std::pair<double, double>, int> more;  // classes from the 16th on
   rs.reserve(rects.size());
   for (const auto& f : rects) {
     if (!(f.w > 0 && f.h > 0)) continue;
     const double x0 = std::max(f.x - f.w / 2, -half), x1 = std::min(f.x + f.w / 2, half);
     const double y0 = std::max(f.y - f.h / 2, -half), y1 = std::min(f.y + f.h / 2, half);
     if (x1 - x0 <= 0 || y1 - y0 <= 0) continue;
-    // equal values beyond the first 64 distinct ones keep classes of their own,
-    // which only splits cells
+    // few values, as a rule: the first 16 by comparison, the others by a search
     int cls = -1;
-    for (size_t v = 0; v < values.size() && cls < 0 && v < 64; ++v)
+    for (size_t v = 0; v < std::min<size_t>(values.size(), 16) && cls < 0; ++v)
       if (values[v] == f.value) cls = (int)v;
     if (cls < 0) {
-      cls = (int)values.size();
-      values.push_back(f.value);
+      // + 0.0: the two zeros are one value
+      const std::pair<double, double> key(f.value.real() + 0.0, f.value.imag() + 0.0);
+      const auto it = more.find(key);
+      if (it != more.end()) {
+        cls = it->second;
+      } else {
+        cls = (int)values.size();
+        values.push_back(f.value);
+        if (cls >= 16) more[key] = cls;
+      }
     }
     rs.push_back({x0, x1, y0, y1, cls});
   }

@@ -108,6 +108,24 @@ static int check(const List& l, cd bg) {
 """
 
 BODIES = {
+    # equal neighbours are joined however many values the clip has
+    "values": r"""
+int main() {
+  for (int values : {3, 15, 16, 17, 63, 64, 65, 66, 150}) {
+    List l;
+    for (int i = 0; i < 300; ++i)  // a strip of pairs of equal slabs, then one over them
+      l.push_back({-500.0 + 3 * i, 100, 3, 50, cd(1.0 + i / 2 % values, 0)});
+    for (int i = 0; i < 60; ++i) l.push_back({-300.0 + 8 * i, 90, 8, 9, cd(1.0 + values - i / 4 % 3, 0)});
+    l.push_back({0, 0, 30, 30, cd(-0.0, 0.0)});
+    l.push_back({0, 40, 30, 30, cd(0.0, -0.0)});
+    for (cd bg : {cd(0, 0), cd(5, 0)})
+      if (int e = check(l, bg)) return e;
+    for (int r = 0; r < 4; ++r)
+      if (int e = check(scatter(120, 200, values), cd(0, 0))) return e;
+  }
+  return 0;
+}
+""",
     # shapes made of slabs, tilings, steps and bricks: joined across touching edges
     "touching": r"""
 int main() {
