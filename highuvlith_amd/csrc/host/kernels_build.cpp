@@ -463,8 +463,47 @@ struct Groups {
   }
 };
 
-// Overlap groups are found pair by pair; clips of more rectangles are one group
-// (as is every clip with `whole`).
+// Joins overlapping rectangles in `over`, and those and the ones that touch along an
+// edge in `near`.  A sweep along the axis across which the rectangles are shorter: each
+// is compared with those that have not ended before it begins (an array of 45 x 45: 0.5
+// ms where all pairs take 8).
+void find_groups(const std::vector<PaintRect>& rs, double eps, Groups& over, Groups& near) {
+  const size_t R = rs.size();
+  double w = 0.0, h = 0.0;
+  for (const auto& r : rs) {
+    w += r.x1 - r.x0;
+    h += r.y1 - r.y0;
+  }
+  // (along, across) extents of a rectangle
+  struct Box { double a0, a1, b0, b1; int i; };
+  std::vector<Box> boxes(R);
+  for (size_t i = 0; i < R; ++i) {
+    const PaintRect& r = rs[i];
+    boxes[i] = w <= h ? Box{r.x0, r.x1, r.y0, r.y1, (int)i} : Box{r.y0, r.y1, r.x0, r.x1, (int)i};
+  }
+  std::sort(boxes.begin(), boxes.end(), [](const Box& p, const Box& q) {
+    return p.a0 != q.a0 ? p.a0 < q.a0 : p.i < q.i;
+  });
+  std::vector<Box> open;
+  for (const Box& p : boxes) {
+    size_t kept = 0;
+    for (const Box& q : open) {
+      if (q.a1 < p.a0 - eps) continue;
+      open[kept++] = q;
+      const double ob = std::min(p.b1, q.b1) - std::max(p.b0, q.b0);
+      if (ob < -eps) continue;
+      const double oa = std::min(p.a1, q.a1) - std::max(p.a0, q.a0);
+      const bool meet = oa > 0 && ob > 0;
+      if (meet) over.join(p.i, q.i);
+      if (meet || oa > eps || ob > eps) near.join(p.i, q.i);
+    }
+    open.resize(kept);
+    open.push_back(p);
+  }
+}
+
+// A clip of more rectangles is one group (as is every clip with `whole`): it is within
+// the limit on the edge grid only if most edges are common ones.
 constexpr size_t kGroupMaxRects = 2048;
 
 }  // namespace
@@ -518,40 +557,38 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
   whole = whole || R > kGroupMaxRects;
   // overlapping rectangles, and those that touch along an edge as well
   Groups over(R), near(R);
-  if (!whole)
-    for (size_t i = 0; i < R; ++i)
-      for (size_t j = 0; j < i; ++j) {
-        const double ox = std::min(rs[i].x1, rs[j].x1) - std::max(rs[i].x0, rs[j].x0);
-        const double oy = std::min(rs[i].y1, rs[j].y1) - std::max(rs[i].y0, rs[j].y0);
-        if (ox > 0 && oy > 0) over.join((int)i, (int)j);
-        if ((ox > eps && oy >= -eps) || (oy > eps && ox >= -eps)) near.join((int)i, (int)j);
-      }
-  else
+  if (whole) {
     for (size_t i = 1; i < R; ++i) {
       over.join((int)i, 0);
       near.join((int)i, 0);
     }
+  } else {
+    find_groups(rs, eps, over, near);
+  }
   // groups in the order of their first rectangle, painter order within each
-  std::vector<std::vector<int>> members(R), parts(R);
-  for (size_t i = 0; i < R; ++i) members[near.find((int)i)].push_back((int)i);
+  struct Member { int near, over, i; };
+  std::vector<Member> order(R);
+  for (size_t i = 0; i < R; ++i) order[i] = {near.find((int)i), over.find((int)i), (int)i};
+  std::sort(order.begin(), order.end(), [](const Member& p, const Member& q) {
+    return p.near != q.near ? p.near < q.near : p.over != q.over ? p.over < q.over : p.i < q.i;
+  });
   std::vector<PaintRect> g;
   std::vector<RectCell> joined;
-  for (const std::vector<int>& near_group : members) {
-    if (near_group.empty()) continue;
-    const size_t before = out.size();
-    for (int k : near_group) parts[over.find(k)].push_back(k);
-    size_t count = 0;
-    for (int k : near_group) {
-      if (parts[k].empty()) continue;
+  for (size_t i = 0; i < R;) {
+    const size_t first = i, before = out.size();
+    int count = 0;
+    while (i < R && order[i].near == order[first].near) {
       g.clear();
-      for (int t : parts[k]) g.push_back(rs[t]);
-      parts[k].clear();
+      const int part = order[i].over;
+      for (; i < R && order[i].over == part; ++i) g.push_back(rs[order[i].i]);
       resolve_group(g, values, eps, out);
       ++count;
     }
     if (count < 2) continue;
+    std::sort(order.begin() + first, order.begin() + i,
+              [](const Member& p, const Member& q) { return p.i < q.i; });
     g.clear();
-    for (int k : near_group) g.push_back(rs[k]);
+    for (size_t k = first; k < i; ++k) g.push_back(rs[order[k].i]);
     joined.clear();
     resolve_group(g, values, eps, joined);
     if (joined.size() >= out.size() - before) continue;

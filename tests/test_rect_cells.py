@@ -108,6 +108,41 @@ static int check(const List& l, cd bg) {
 """
 
 BODIES = {
+    # an aligned array of 2025 rectangles takes less than one look at every pair does
+    "array": r"""
+static volatile long sink;
+int main() {
+  for (double shift : {0.0, 3.0})
+    for (bool turned : {false, true}) {
+      List l = tiles(45, 45, 16, 20, 0.5, shift, 1.0);
+      if (turned)
+        for (auto& r : l) {
+          std::swap(r.x, r.y);
+          std::swap(r.w, r.h);
+        }
+      if (int e = check(l, cd(0, 0))) return e;
+      std::vector<RectCell> cells;
+      double cost[2] = {1e9, 1e9};
+      for (int k = 0; k < 20; ++k) {
+        const auto t0 = std::chrono::steady_clock::now();
+        resolve_rect_cells(l, cd(0, 0), N, PX, 1 << 20, cells);
+        const auto t1 = std::chrono::steady_clock::now();
+        long n = 0;
+        for (size_t i = 0; i < l.size(); ++i)
+          for (size_t j = 0; j < i; ++j)
+            n += l[i].x - l[i].w / 2 < l[j].x + l[j].w / 2 && l[j].x - l[j].w / 2 < l[i].x + l[i].w / 2 &&
+                 l[i].y - l[i].h / 2 < l[j].y + l[j].h / 2 && l[j].y - l[j].h / 2 < l[i].y + l[i].h / 2;
+        sink = n;
+        const auto t2 = std::chrono::steady_clock::now();
+        cost[0] = std::min(cost[0], std::chrono::duration<double>(t1 - t0).count());
+        cost[1] = std::min(cost[1], std::chrono::duration<double>(t2 - t1).count());
+      }
+      std::printf("%.3f ms, every pair %.3f ms\n", 1e3 * cost[0], 1e3 * cost[1]);
+      if (cost[0] > cost[1]) return 7;
+    }
+  return 0;
+}
+""",
     # equal neighbours are joined however many values the clip has
     "values": r"""
 int main() {
