@@ -538,14 +538,30 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   std::vector<int64_t> coff((size_t)nclips + 1, 0), eoff((size_t)nclips + 1, 0);
   std::vector<huv::RectFeature> fs;
   std::vector<huv::RectCell> cl;
-  // The call's cell limit counts the cells of one grid per clip: where these
-  // could reach it, the clips are resolved that way.
+  auto load = [&](int i) {
+    fs.clear();
+    for (int64_t r = rb.offsets[i]; r < rb.offsets[i + 1]; ++r) {
+      const double* q = rb.rects + 6 * r;
+      fs.push_back({q[0], q[1], q[2], q[3], huv::cd(q[4], q[5])});
+    }
+  };
+  // The call's cell limit counts the cells of one grid per clip, of which there are
+  // fewer here: they are counted only where two bounds, one of the rectangles' numbers
+  // and one of their edges, do not exclude that they reach it.
   double bound = 0.0;
   for (int i = 0; i < nclips; ++i) {
     const double r = 2.0 * (double)(rb.offsets[i + 1] - rb.offsets[i]) + 1.0;
     bound += r * r;
   }
-  const bool whole = bound > (double)kRectMaxCells;
+  if (bound > (double)kRectMaxCells) {
+    bound = 0.0;
+    for (int i = 0; i < nclips; ++i) {
+      load(i);
+      bound += (double)huv::rect_grid_cells_bound(fs, n, rb.pixel_nm);
+    }
+  }
+  const bool count = bound > (double)kRectMaxCells;
+  int64_t grid = 0, clip_grid = 0;  // cells of one grid per clip
   std::vector<std::array<double, 4>> boxes;
   std::vector<Pt> v;
   const double half = n * rb.pixel_nm / 2.0;
@@ -555,18 +571,15 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
     return fail(HUV_UNSUPPORTED, "polygon masks support band half-widths up to " +
                                      std::to_string(huvk::kPolyMaxBand));
   for (int i = 0; i < nclips; ++i) {
-    fs.clear();
-    for (int64_t r = rb.offsets[i]; r < rb.offsets[i + 1]; ++r) {
-      const double* q = rb.rects + 6 * r;
-      fs.push_back({q[0], q[1], q[2], q[3], huv::cd(q[4], q[5])});
-    }
+    load(i);
     const huv::cd bg(rb.background[2 * i], rb.background[2 * i + 1]);
-    if (!huv::resolve_rect_cells(fs, bg, n, rb.pixel_nm, kRectMaxGrid, cl, whole))
+    if (!huv::resolve_rect_cells(fs, bg, n, rb.pixel_nm, kRectMaxGrid, cl, count ? &clip_grid : nullptr))
       return fail(HUV_INVALID_PARAMETER,
                   "clip " + std::to_string(i) + ": more than 2^20 edge-grid cells; rasterise it instead");
     for (const auto& e : cl) cells.insert(cells.end(), {e.x0, e.x1, e.y0, e.y1, e.w.real(), e.w.imag()});
     coff[i + 1] = (int64_t)(cells.size() / 6);
-    if (coff[i + 1] > kRectMaxCells) return fail(HUV_INVALID_PARAMETER, "too many rectangle cells in one call");
+    grid += clip_grid;
+    if (grid > kRectMaxCells) return fail(HUV_INVALID_PARAMETER, "too many rectangle cells in one call");
     if (rb.polys) {
       // bounding boxes of the clip's features, for the overlap rule
       boxes.clear();

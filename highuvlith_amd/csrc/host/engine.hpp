@@ -222,10 +222,12 @@ struct RectCell {
   cd w;
 };
 // Painter's-rule resolution of rectangles into disjoint cells (see the
-// definition); false when the edge grid would exceed max_cells cells.  whole:
-// on one grid over all edges, whose cells are the ones a call's limit counts.
+// definition); false when the edge grid would exceed max_cells cells.  grid_cells,
+// if given: the cells of one grid over all edges, which a call's limit counts.
 bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd background, int n,
                         double pixel_nm, int64_t max_cells, std::vector<RectCell>& out,
-                        bool whole = false);
+                        int64_t* grid_cells = nullptr);
+// At least that count, without painting.
+int64_t rect_grid_cells_bound(const std::vector<RectFeature>& rects, int n, double pixel_nm);
 
 }  // namespace huv

@@ -502,26 +502,52 @@ void find_groups(const std::vector<PaintRect>& rs, double eps, Groups& over, Gro
   }
 }
 
-// A clip of more rectangles is one group (as is every clip with `whole`): it is within
-// the limit on the edge grid only if most edges are common ones.
+// A clip of more rectangles is one group: it is within the limit on the edge grid only if
+// most edges are common ones.
 constexpr size_t kGroupMaxRects = 2048;
 
 }  // namespace
 
+// The rectangle as the field clips it; false for an empty one.
+static bool clip_rect(const RectFeature& f, double half, PaintRect& r) {
+  if (!(f.w > 0 && f.h > 0)) return false;
+  r.x0 = std::max(f.x - f.w / 2, -half), r.x1 = std::min(f.x + f.w / 2, half);
+  r.y0 = std::max(f.y - f.h / 2, -half), r.y1 = std::min(f.y + f.h / 2, half);
+  return r.x1 - r.x0 > 0 && r.y1 - r.y0 > 0;
+}
+
+// A row of the grid that A rectangles reach into holds at most 2 A - 1 runs.
+int64_t rect_grid_cells_bound(const std::vector<RectFeature>& rects, int n, double pixel) {
+  const double half = n * pixel / 2.0;
+  const double eps = 1e-12 * (2.0 * half);
+  std::vector<double> ye;
+  std::vector<PaintRect> rs;
+  PaintRect r{};
+  for (const auto& f : rects) {
+    if (!clip_rect(f, half, r)) continue;
+    rs.push_back(r);
+    ye.push_back(r.y0);
+    ye.push_back(r.y1);
+  }
+  dedup(ye, eps);
+  int64_t cells = 0;
+  for (const auto& q : rs) cells += 2 * (edge_index(ye, q.y1, eps) - edge_index(ye, q.y0, eps));
+  return cells;
+}
+
 bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, double pixel,
-                        int64_t max_cells, std::vector<RectCell>& out, bool whole) {
+                        int64_t max_cells, std::vector<RectCell>& out, int64_t* grid_cells) {
   out.clear();
+  if (grid_cells) *grid_cells = 0;
   const double half = n * pixel / 2.0;
   const double eps = 1e-12 * (2.0 * half);
   std::vector<PaintRect> rs;
   std::vector<cd> values{bg};
   std::map<std::pair<double, double>, int> more;  // classes from the 16th on
   rs.reserve(rects.size());
+  PaintRect box{};
   for (const auto& f : rects) {
-    if (!(f.w > 0 && f.h > 0)) continue;
-    const double x0 = std::max(f.x - f.w / 2, -half), x1 = std::min(f.x + f.w / 2, half);
-    const double y0 = std::max(f.y - f.h / 2, -half), y1 = std::min(f.y + f.h / 2, half);
-    if (x1 - x0 <= 0 || y1 - y0 <= 0) continue;
+    if (!clip_rect(f, half, box)) continue;
     // few values, as a rule: the first 16 by comparison, the others by a search
     int cls = -1;
     for (size_t v = 0; v < std::min<size_t>(values.size(), 16) && cls < 0; ++v)
@@ -538,7 +564,8 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
         if (cls >= 16) more[key] = cls;
       }
     }
-    rs.push_back({x0, x1, y0, y1, cls});
+    box.cls = cls;
+    rs.push_back(box);
   }
   if (rs.empty()) return true;
   const size_t R = rs.size();
@@ -554,10 +581,15 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
     const int64_t nx = (int64_t)xe.size() - 1, ny = (int64_t)ye.size() - 1;
     if (nx < 1 || ny < 1 || nx > max_cells / ny) return false;
   }
-  whole = whole || R > kGroupMaxRects;
+  std::vector<PaintRect> g;
+  std::vector<RectCell> joined;
+  if (grid_cells) {
+    resolve_group(rs, values, eps, joined);
+    *grid_cells = (int64_t)joined.size();
+  }
   // overlapping rectangles, and those that touch along an edge as well
   Groups over(R), near(R);
-  if (whole) {
+  if (R > kGroupMaxRects) {
     for (size_t i = 1; i < R; ++i) {
       over.join((int)i, 0);
       near.join((int)i, 0);
@@ -572,8 +604,6 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
   std::sort(order.begin(), order.end(), [](const Member& p, const Member& q) {
     return p.near != q.near ? p.near < q.near : p.over != q.over ? p.over < q.over : p.i < q.i;
   });
-  std::vector<PaintRect> g;
-  std::vector<RectCell> joined;
   for (size_t i = 0; i < R;) {
     const size_t first = i, before = out.size();
     int count = 0;

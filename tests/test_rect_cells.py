@@ -108,6 +108,39 @@ static int check(const List& l, cd bg) {
 """
 
 BODIES = {
+    # a call's limit counts one grid's cells, whatever the clip is cut into; the bound
+    # that spares the count holds, and lets 512 clips of 200 scattered contacts pass
+    "limit": r"""
+int main() {
+  std::vector<RectCell> with, without;
+  for (int values : {1, 5, 100})
+    for (int n : {0, 1, 2, 9, 60, 200})
+      for (double most : {20.0, 300.0}) {
+        const List l = scatter(n, most, values);
+        int64_t grid = -1;
+        if (!resolve_rect_cells(l, cd(0, 0), N, PX, 1 << 20, with, &grid)) return 1;
+        if (grid != one_grid(l, cd(0, 0))) return 2;
+        if (rect_grid_cells_bound(l, N, PX) < grid) return 3;
+        resolve_rect_cells(l, cd(0, 0), N, PX, 1 << 20, without);
+        if (with.size() != without.size()) return 4;
+      }
+  for (const List& l : {tiles(32, 32, 16, 16, 1, 0, 1.0), tiles(20, 40, 40, 20, 1, 20, 1.0),
+                        tiles(50, 45, 16, 16, 0.5, 0, 1.0)}) {
+    int64_t grid = -1;
+    if (!resolve_rect_cells(l, cd(0, 0), N, PX, 1 << 20, with, &grid)) return 5;
+    if (grid != one_grid(l, cd(0, 0)) || rect_grid_cells_bound(l, N, PX) < grid) return 6;
+  }
+  int64_t calls = 0;
+  for (int c = 0; c < 512; ++c) {
+    List l;
+    for (int i = 0; i < 200; ++i)
+      l.push_back({-480 + 64.0 * (i % 15) + uni(0, 8), -480 + 64.0 * (i / 15) + uni(0, 8), uni(12, 24),
+                   uni(12, 24), 1.0});
+    calls += rect_grid_cells_bound(l, N, PX);
+  }
+  return calls <= 1 << 26 ? 0 : 7;
+}
+""",
     # an aligned array of 2025 rectangles takes less than one look at every pair does
     "array": r"""
 static volatile long sink;
@@ -200,3 +233,21 @@ def test_cells(tmp_path, case):
                    + ["-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.gpu
+def test_a_call_of_many_rectangles(gpu_ctx):
+    """520 clips of 190 contacts: above the limit by their number, far below by their
+    cells.  Tolerance as for the groups: one rounding to FP32 of FP64 sums."""
+    import numpy as np
+    from test_gpu_rect_groups import _reference
+    rng = np.random.default_rng(1)
+    n, px, band = 256, 2.0, 7
+    site = np.arange(190)
+    lists = [[(*map(float, p), 1.0) for p in np.stack(
+        [-240 + 34 * (site % 14) + rng.uniform(0, 8, 190), -240 + 34 * (site // 14)
+         + rng.uniform(0, 8, 190), rng.uniform(8, 30, 190), rng.uniform(8, 30, 190)], 1)]
+             for _ in range(520)]
+    got = H.engine.band_spectrum_rects_device(gpu_ctx, lists, H.GridConfig(n, px), band).cpu().numpy()
+    for c in range(0, 520, 40):
+        assert np.abs(got[c] - _reference(lists[c], 0.0, n, px, band)).max() <= 1.2e-7 * n * n, c
