@@ -666,11 +666,10 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   e = hipMemcpyAsync(slot->d, slot->h, bytes, hipMemcpyHostToDevice, c->stream());
   if (e != hipSuccess) return hip_fail(e, "rectangle upload");
   // whatever returns from here on has queued the copy at least
-  struct Mark {
-    Ctx::FeatureSlot* s;
-    hipStream_t st;
-    ~Mark() { s->busy = hipEventRecord(s->done, st) == hipSuccess; }
-  } mark{slot, c->stream()};
+  const hipStream_t st = c->stream();
+  const SlotMark mark(
+      slot, [=] { return hipEventRecord(slot->done, st) == hipSuccess; },
+      [=] { hipStreamSynchronize(st); });
   const double* d_cells = (const double*)slot->d;
   const int64_t* d_coff = (const int64_t*)(slot->d + cell_b);
   const double* d_bg = (const double*)(slot->d + cell_b + off_b);

@@ -13,6 +13,7 @@
 #include "hip/socs_kernels.hpp"
 #include "host/engine.hpp"
 #include "host/plane_key.hpp"
+#include "host/slot_mark.hpp"
 
 // A kernel set built on the host (huv_kernels_build) or with the device's
 // help (huv_kernels_build_device).
