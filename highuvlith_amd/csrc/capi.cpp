@@ -1192,6 +1192,30 @@ huv_status plane_table(Ctx* c, int nplanes, huv_kset* const* planes, bool real_m
   return HUV_OK;
 }
 
+// Allocation and upload by a thread that is capturing a stream (on): in relaxed
+// capture mode and on a stream of its own, so that nothing of it is recorded.
+struct RelaxedCapture {
+  bool on;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  explicit RelaxedCapture(bool o) : on(o) {
+    if (on) hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  RelaxedCapture(const RelaxedCapture&) = delete;
+  ~RelaxedCapture() {
+    if (on) hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  hipError_t upload(void* d, const void* h, size_t bytes) const {
+    if (!on) return hipMemcpy(d, h, bytes, hipMemcpyHostToDevice);
+    hipStream_t s = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (e != hipSuccess) return e;
+    e = hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    hipStreamDestroy(s);
+    return e;
+  }
+};
+
 // Kernel stacks of a plane list packed into one buffer [Q][total][W][W] for
 // coarse grid m (W = 2 BB + 1, BB = (m - 1) / 4 >= every set's band, Q = m / 32;
 // copy q multiplied by e^{2 pi i kx q / m} in FP64) and each box scaled by the root of
@@ -1207,16 +1231,29 @@ huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool 
   PlaneKey key{{}, {(uint64_t)m, (uint64_t)paired, (uint64_t)real_masks}};
   for (int p = 0; p < nplanes; ++p) key.ksets.push_back(planes[p]->id);
   auto it = c->plane_packs.find(key);
-  if (it == c->plane_packs.end() && c->fixed_mode) {
+  bool capturing = false;
+  if (it == c->plane_packs.end()) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hipStreamIsCapturing(c->stream(), &cap);
+    capturing = cap == hipStreamCaptureStatusActive;
+  }
+  if (it == c->plane_packs.end() && (c->fixed_mode || (capturing && real_masks))) {
     // a stack built by an earlier call for complex masks serves real ones too
     key.form.back() = 0;
     it = c->plane_packs.find(key);
-    if (it == c->plane_packs.end())
+    key.form.back() = (uint64_t)real_masks;
+    if (it == c->plane_packs.end() && c->fixed_mode)
       return fail(HUV_INVALID_PARAMETER,
                   "kernel stacks of this plane list are not built yet: call huv_socs_images once "
                   "with the same kernel sets before the no-allocation entry point");
   }
   if (it == c->plane_packs.end()) {
+    // While the caller's stream is captured, a list known only by its stack for real
+    // masks gets the general one too (a single stack used to serve both); allocation
+    // for any other list is left to fail there.
+    PlaneKey other = key;
+    other.form.back() ^= 1;
+    const RelaxedCapture relaxed(capturing && c->plane_packs.count(other) != 0);
     Ctx::PlanePack pk;
     std::vector<int> src(nplanes), rep;  // distinct image of each plane; its plane
     for (int p = 0; p < nplanes; ++p) {
@@ -1329,8 +1366,8 @@ huv_status plane_pack(Ctx* c, int nplanes, huv_kset* const* planes, int m, bool 
     }
     hipError_t e = hipMalloc(&pk.kern, hk.size() * sizeof(float2));
     if (e == hipSuccess) e = hipMalloc(&pk.tab, tab.size() * sizeof(int));
-    if (e == hipSuccess) e = hipMemcpy(pk.kern, hk.data(), hk.size() * sizeof(float2), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(pk.tab, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = relaxed.upload(pk.kern, hk.data(), hk.size() * sizeof(float2));
+    if (e == hipSuccess) e = relaxed.upload(pk.tab, tab.data(), tab.size() * sizeof(int));
     if (e != hipSuccess) {
       hipFree(pk.kern);
       hipFree(pk.tab);
