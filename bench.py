@@ -101,21 +101,6 @@ def fields_algorithmic_flops(Ks, band, m, nclips):
     return nclips * sum(Ks) * per_kernel
 
 
-def executed_kernel_steps(sets, H, np):
-    """Kernel steps per clip that real masks cost: planes with one real form share an
-    image, and a step transforms two real fields."""
-    steps, seen = 0, []
-    for ks in sets:
-        v = H.engine.real_fields(ks)
-        form = (np.abs(v) ** 2).sum(0)
-        if len(v) and any(f.shape == form.shape and np.abs(f - form).max() <= 1e-6 * form.max()
-                          for f in seen):
-            continue
-        seen.append(form)
-        steps += (len(v) + 1) // 2 if len(v) else ks.num_kernels
-    return steps
-
-
 def measured_traffic(kernel):
     """HBM bytes per launch of `kernel` from the committed PMC summary (None if absent)."""
     try:
@@ -192,7 +177,7 @@ def bench_fixed(args, H, W, np, torch):
     launches = {k: v[1] // args.steps for k, v in stages.items() if v[1] > 0}
     nl = launches["socs_fields"]
     f_ms = step_ms["socs_fields"]
-    clip_steps = executed_kernel_steps(sets, H, np)
+    clip_steps = H.engine.socs_plan(planes)[1]  # what a clip's real mask costs
     exec_flops = fields_flops(nclips, clip_steps, m)
     algo_flops = fields_algorithmic_flops(Ks, B, m, nclips)
     achieved_tf = algo_flops / (f_ms * 1e-3) / 1e12

@@ -150,6 +150,8 @@ SIGNATURES = {
                                   C.POINTER(P)]),
     "huv_kset_destroy": (None, [P]),
     "huv_kset_shape": (C.c_int, [P, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
+    "huv_socs_plan": (C.c_int, [P, C.c_int, C.c_int, C.POINTER(P), C.c_int, C.POINTER(C.c_int),
+                                C.POINTER(C.c_int)]),
     "huv_socs_images": (C.c_int, [P, C.c_int, C.c_int, PF, C.c_int, C.POINTER(P), PF,
                                   C.POINTER(huv_socs_opts)]),
     "huv_socs_images_host": (C.c_int, [P, C.c_int, C.c_int, PF, C.c_int, C.POINTER(P), PF,

@@ -1790,6 +1790,26 @@ huv_status huv_socs_images_spectrum(huv_ctx* c, int nclips, int n, const double*
                       it != c->tuned.end() ? &it->second : nullptr);
 }
 
+huv_status huv_socs_plan(huv_ctx* c, int n, int nplanes, huv_kset* const* planes, int real_masks,
+                         int* images, int* steps) {
+  if (!c || !planes || !images || !steps) return fail(HUV_INVALID_PARAMETER, "null argument");
+  if (nplanes < 1) return fail(HUV_INVALID_PARAMETER, "need nplanes >= 1");
+  huv_status st = validate_planes(c, n, nplanes, planes);
+  if (st != HUV_OK) return st;
+  std::lock_guard<std::mutex> lk(c->mu);
+  hipSetDevice(c->device);
+  auto it = c->tuned.find(tuning_key(n, planes, nplanes));
+  const huv_socs_tuning t = it != c->tuned.end() ? it->second : huv_socs_tuning{0, 0, 0, 0, 0};
+  const int m = t.m ? t.m : planes[0]->m;
+  const int xlanes = t.xlanes ? t.xlanes : huvk::fields_lanes_default(m);
+  const Ctx::PlanePack* pack = nullptr;
+  st = plane_pack(c, nplanes, planes, m, xlanes == 2, real_masks != 0, &pack);
+  if (st != HUV_OK) return st;
+  *images = pack->nd;
+  *steps = pack->total;
+  return HUV_OK;
+}
+
 huv_status huv_socs_images_noalloc(huv_ctx* c, int nclips, int n, const float* masks,
                                    int nplanes, huv_kset* const* planes, float* out,
                                    int pixel_transfer) {

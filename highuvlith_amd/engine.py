@@ -423,6 +423,17 @@ class DeviceKernelSet:
         self.handle = None
 
 
+def socs_plan(planes, real_masks=True):
+    """(images, steps) per clip of a call with these DeviceKernelSets: distinct images,
+    and complex fields transformed for all of them."""
+    ctx = planes[0].ctx
+    arr = (C.c_void_p * len(planes))(*[p.handle.value for p in planes])
+    images, steps = C.c_int(), C.c_int()
+    check(ctx.lib.huv_socs_plan(ctx.handle, planes[0].host.n, len(planes), arr,
+                                int(bool(real_masks)), C.byref(images), C.byref(steps)))
+    return images.value, steps.value
+
+
 def socs_images_device(ctx, masks, planes, out, pixel_transfer=False, graph=False):
     """Launch batched images on torch CUDA tensors (masks (N, n, n) f32, out (N, P, n, n) f32).
 

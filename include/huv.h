@@ -182,6 +182,14 @@ void huv_kset_destroy(huv_kset* ks);
 /* Band half-width B and coarse grid m chosen for this set. */
 huv_status huv_kset_shape(const huv_kset* ks, int* band, int* coarse);
 
+/* What a call with these planes images per clip: *images distinct images (planes whose
+ * real masks give one image share it) and *steps kernel steps in all, a step being one
+ * complex field (two real ones of huv_real_fields).  real_masks: for masks with a real
+ * transmittance, else every plane counts with its own kernels.  Builds what the call
+ * would build. */
+huv_status huv_socs_plan(huv_ctx* ctx, int n, int nplanes, huv_kset* const* planes,
+                         int real_masks, int* images, int* steps);
+
 /* Kernel sets of nplanes focus planes (defocus_nm[p]) built with the device's
  * help (replaces KernelBuilder::build, aerial.rs:1041-1317, for the dense TCC
  * and dense Gram paths): the TCC factor A[f, s] = sqrt(w_s) P(f/f_c + s; z,
