@@ -1537,8 +1537,7 @@ std::vector<int> tuning_key(int n, const huv_kset* const* planes, int nplanes) {
 }
 
 // Times every launch shape on this call's inputs (coordinate descent: coarse
-// grid, then band-FFT factor, then x-pass block, then clip ranges) and
-// records the fastest.
+// grid, then x-pass form and block, then clip ranges) and records the fastest.
 // The last run leaves a valid result in `out`.
 huv_status autotune_socs(Ctx* c, int nclips, int n, const MaskSource& src, int nplanes,
                          huv_kset* const* planes, float* out, bool pt, huv_socs_tuning* best) {
@@ -1576,15 +1575,6 @@ huv_status autotune_socs(Ctx* c, int nclips, int n, const MaskSource& src, int n
     st = time_one(t, ms);
     if (st != HUV_OK) break;
     if (ms < cur_ms) { cur_ms = ms; cur = t; }
-  }
-  int n1s[4];
-  const int nn1 = huvk::band_fft_options(n, n1s);
-  for (int i = 0; i < nn1 && st == HUV_OK; ++i) {
-    huv_socs_tuning t = cur;
-    t.n1 = n1s[i];
-    double ms;
-    st = time_one(t, ms);
-    if (st == HUV_OK && ms < cur_ms) { cur_ms = ms; cur = t; }
   }
   for (int xlanes : {1, 2}) {
     if (!huvk::fields_lanes_supported(cur.m, xlanes)) continue;

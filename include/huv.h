@@ -219,9 +219,10 @@ typedef struct {
 
 /* Launch shape of the SOCS path for one (n, band, planes) combination:
  * coarse grid m (32 Q; sets the number of 32-point transform classes Q),
- * band-FFT factor n1 (four-step n = n1 x n / n1), and the field kernel's
- * x pass: xlanes = 1 or 2 lanes per band row (2 needs m >= 64), xnb = 4, 6
- * or 8 band columns per load block; chunks = 1..16 clip ranges issued one
+ * and the field kernel's x pass: xlanes = 1 or 2 lanes per band row (2 needs
+ * m >= 64), xnb = 4, 6 or 8 band columns per load block; n1, a factor of the
+ * band transforms (n = n1 x n / n1), is checked but has no effect, since the
+ * transforms of an image's band have one form; chunks = 1..16 clip ranges issued one
  * after the other (each range's intermediates are then small enough to stay
  * in the device's last-level cache between stages; the default is sized for
  * that; results do not depend on it).  Zero fields select the built-in
