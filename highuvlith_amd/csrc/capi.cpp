@@ -337,7 +337,7 @@ void Ctx::forget_kset(uint64_t id) {
 }
 
 huv_status band_stage(Ctx* c, int nclips, int n, int B, int BB, const float* masks, float2* Mq,
-                      bool pixel_transfer, int n1, float2* Mp) {
+                      bool pixel_transfer, float2* Mp) {
   hipError_t e;
   const float2* tw_n = c->twiddles(n, e);
   if (!tw_n) return hip_fail(e, "twiddle table");
@@ -348,18 +348,18 @@ huv_status band_stage(Ctx* c, int nclips, int n, int B, int BB, const float* mas
   if (!tmp) return hip_fail(e, "workspace");
   hipEvent_t ev;
   c->stage_begin(ST_ROWS_BAND, &ev);
-  e = huvk::launch_rows_band(n, n1, B, nclips, masks, tw_n, tmp, c->stream());
+  e = huvk::launch_rows_band(n, B, nclips, masks, tw_n, tmp, c->stream());
   if (e != hipSuccess) return hip_fail(e, "rows_band launch");
   c->stage_end(ST_ROWS_BAND, ev);
   c->stage_begin(ST_COLS_BAND, &ev);
-  e = huvk::launch_cols_band(n, n1, B, BB, nclips, tmp, tw_n, st, Mq, Mp, c->stream());
+  e = huvk::launch_cols_band(n, B, BB, nclips, tmp, tw_n, st, Mq, Mp, c->stream());
   if (e != hipSuccess) return hip_fail(e, "cols_band launch");
   c->stage_end(ST_COLS_BAND, ev);
   return HUV_OK;
 }
 
 huv_status band_stage_complex(Ctx* c, int nclips, int n, int B, int BB, const float2* masks,
-                              float2* Mq, bool pixel_transfer, int n1, float2* Mp) {
+                              float2* Mq, bool pixel_transfer, float2* Mp) {
   hipError_t e;
   const float2* tw_n = c->twiddles(n, e);
   if (!tw_n) return hip_fail(e, "twiddle table");
@@ -370,11 +370,11 @@ huv_status band_stage_complex(Ctx* c, int nclips, int n, int B, int BB, const fl
   if (!tmp) return hip_fail(e, "workspace");
   hipEvent_t ev;
   c->stage_begin(ST_ROWS_BAND, &ev);
-  e = huvk::launch_rows_band_c(n, n1, B, nclips, masks, tw_n, tmp, c->stream());
+  e = huvk::launch_rows_band_c(n, B, nclips, masks, tw_n, tmp, c->stream());
   if (e != hipSuccess) return hip_fail(e, "rows_band_c launch");
   c->stage_end(ST_ROWS_BAND, ev);
   c->stage_begin(ST_COLS_BAND, &ev);
-  e = huvk::launch_cols_band_c(n, n1, B, BB, nclips, tmp, tw_n, st, Mq, Mp, c->stream());
+  e = huvk::launch_cols_band_c(n, B, BB, nclips, tmp, tw_n, st, Mq, Mp, c->stream());
   if (e != hipSuccess) return hip_fail(e, "cols_band_c launch");
   c->stage_end(ST_COLS_BAND, ev);
   return HUV_OK;
@@ -1417,7 +1417,7 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
   const int B = planes[0]->B;
   const int m = tune && tune->m ? tune->m : planes[0]->m;
   const int BB = huvk::coarse_band(m);
-  const int n1 = tune ? tune->n1 : 0, xnb = tune ? tune->xnb : 0;
+  const int xnb = tune ? tune->xnb : 0;
   const int xlanes = tune && tune->xlanes ? tune->xlanes : huvk::fields_lanes_default(m);
   if (B > BB || m > n) return fail(HUV_INVALID_PARAMETER, "coarse grid too small for the kernel band");
   if (!huvk::fields_lanes_supported(m, xlanes))
@@ -1484,10 +1484,10 @@ huv_status socs_forward(Ctx* c, int nclips, int n, const MaskSource& src, int np
     const int c0 = i * cc, cn = std::min(cc, nclips - c0), ni = cn * nd;
     if (src.kind == MaskSource::REAL) {
       st = band_stage(c, cn, n, B, BB, src.raster + (size_t)c0 * n * n, Mq + (size_t)c0 * W * W,
-                      pt, n1, Mp ? Mp + (size_t)c0 * (W + 1) * W : nullptr);
+                      pt, Mp ? Mp + (size_t)c0 * (W + 1) * W : nullptr);
     } else if (src.kind == MaskSource::COMPLEX) {
       st = band_stage_complex(c, cn, n, B, BB, (const float2*)src.raster + (size_t)c0 * n * n,
-                              Mq + (size_t)c0 * W * W, pt, n1,
+                              Mq + (size_t)c0 * W * W, pt,
                               Mp ? Mp + (size_t)c0 * (W + 1) * W : nullptr);
     }
     if (st != HUV_OK) return st;
@@ -1716,7 +1716,7 @@ huv_status socs_groups(Ctx* c, int ngroups, const huv_clip_group* groups, const 
     plan.push_back(gp);
     key.form.insert(key.form.end(), {(uint64_t)g.n, (uint64_t)g.nclips, (uint64_t)(uintptr_t)g.masks,
                            (uint64_t)(uintptr_t)g.out, (uint64_t)g.nplanes, (uint64_t)gp.t.m,
-                           (uint64_t)gp.t.n1, (uint64_t)gp.t.xnb, (uint64_t)gp.t.xlanes,
+                           (uint64_t)gp.t.xnb, (uint64_t)gp.t.xlanes,
                            (uint64_t)gp.t.chunks});
     for (int p = 0; p < g.nplanes; ++p) key.ksets.push_back(g.planes[p]->id);
   }
@@ -1871,7 +1871,7 @@ huv_status huv_socs_images_features(huv_ctx* c, int nclips, int n, double pixel_
   if (nclips == 0) return HUV_OK;
   std::lock_guard<std::mutex> lk(c->mu);
   hipSetDevice(c->device);
-  // a launch shape tuned for these planes applies (its band-FFT factor is unused)
+  // a launch shape tuned for these planes applies
   auto it = c->tuned.find(tuning_key(n, planes, nplanes));
   MaskSource src;
   src.kind = MaskSource::FEATURES;

@@ -148,7 +148,7 @@ enum Stage { ST_ROWS_BAND = 0, ST_COLS_BAND, ST_FIELDS, ST_COARSE_ROWS, ST_COARS
 // in boxes of half-width BB >= B (zero beyond B).  Layout Mq[clip][kx + BB][ky + BB];
 // Mp (optional) receives the column-paired copy (huvk::launch_cols_band).
 huv_status band_stage(Ctx* c, int nclips, int n, int B, int BB, const float* masks, float2* Mq,
-                      bool pixel_transfer, int n1 = 0, float2* Mp = nullptr);
+                      bool pixel_transfer, float2* Mp = nullptr);
 
 // Rectangle masks of a batch (host arrays): clip i holds rectangles
 // [offsets[i], offsets[i + 1]) of rects (x, y, w, h, re, im; centre and size
@@ -168,7 +168,7 @@ huv_status validate_rects(int nclips, int n, const RectBatch& rb);
 // Band spectrum of nclips complex n x n rasters (device, interleaved FP32):
 // same output as band_stage, every row and both signs of kx transformed.
 huv_status band_stage_complex(Ctx* c, int nclips, int n, int B, int BB, const float2* masks,
-                              float2* Mq, bool pixel_transfer, int n1 = 0, float2* Mp = nullptr);
+                              float2* Mq, bool pixel_transfer, float2* Mp = nullptr);
 // Band of nclips host spectra (n x n interleaved complex FP64, the FFT layout
 // of Fft2D::forward) into Mq (and Mp): the |k| <= B bins, rounded to FP32 and
 // uploaded through the pinned staging area (synchronises the stream first).

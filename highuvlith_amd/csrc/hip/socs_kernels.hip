@@ -13,7 +13,8 @@
 //
 // Stages (one launch each, all batched over clips / images):
 //   rows_pruned  mask rows (real, FP32) -> row spectra, band |kx| <= B kept
-//   cols_pruned  row spectra -> M[ky][kx] band (rows_band and cols_band: B > 63)
+//   cols_pruned  row spectra -> M[ky][kx] band
+//   (rows_band and cols_band: wider bands than an image's, see band_pruned)
 //   socs_fields  K kernels x band -> coarse intensity (fields in registers)
 //   coarse_rows  coarse rows -> |gx| <= 2B
 //   coarse_cols  -> intensity band I^[gy][gx], 1/m^2, flare on non-DC terms
@@ -124,91 +125,6 @@ __global__ __launch_bounds__(TEAMS * N2) void k_cols_band(
 }
 
 // ---------------------------------------------------------------------------
-// Complex transmittance rasters (compute_from_transmittance with an
-// Array2<Complex64> map, aerial.rs:1789-1799): no Hermitian symmetry, so every
-// row is its own complex transform and both signs of kx are column passes.
-// rows_band_c: row r of clip c (interleaved complex FP32), FFT_n forward,
-// keep k in [0, B] and [n - B, n); tmp layout [clip][kk][row], kk as in
-// rows_band (kk <= B -> k = kk, kk > B -> k = n - (kk - B)).
-// ---------------------------------------------------------------------------
-template <int N1, int N2, int TEAMS>
-__global__ __launch_bounds__(TEAMS * N2) void k_rows_band_c(const float2* __restrict__ masks,
-                                                            int B, const float2* __restrict__ tw_n,
-                                                            float2* __restrict__ tmp) {
-  constexpr int N = N1 * N2;
-  __shared__ c32 scratch[TEAMS][(N1 + 1) * N2];
-  const int team = threadIdx.x / N2, t = threadIdx.x % N2;
-  const int clip = blockIdx.y;
-  const int row = blockIdx.x * TEAMS + team;
-  const bool active = row < N;
-  const float* r = reinterpret_cast<const float*>(masks + ((size_t)clip * N + (active ? row : 0)) * N);
-  const int nk = 2 * B + 1;
-  float2* out = tmp + (size_t)clip * nk * N;
-  fft_four_step<-1, N1, N2>(
-      t, scratch[team], tw_n,
-      [&](int i) {
-        return active ? c32{__builtin_nontemporal_load(r + 2 * i),
-                            __builtin_nontemporal_load(r + 2 * i + 1)}
-                      : c32{0.f, 0.f};
-      },
-      [&](int k, c32 v) {
-        if (!active) return;
-        int kk = -1;
-        if (k <= B) kk = k;
-        else if (k >= N - B) kk = B + (N - k);
-        if (kk >= 0) out[(size_t)kk * N + row] = make_float2(v.re, v.im);
-      });
-}
-
-// cols_band_c: box column col = kx + BB for kx in [-BB, BB]: FFT_n forward of
-// the row-spectrum column kx along y, keep ky in [-BB, BB]; the box holds
-// M[ky][kx] * pt for |kx|, |ky| <= B and zero elsewhere (plain and, when Mp
-// is set, column-paired with its zero column in front, as cols_band writes).
-template <int N1, int N2, int TEAMS>
-__global__ __launch_bounds__(TEAMS * N2) void k_cols_band_c(
-    const float2* __restrict__ tmp, int B, int BB, const float2* __restrict__ tw_n,
-    const float* __restrict__ sinc_t, float2* __restrict__ Mq, float2* __restrict__ Mp) {
-  constexpr int N = N1 * N2;
-  __shared__ c32 scratch[TEAMS][(N1 + 1) * N2];
-  const int team = threadIdx.x / N2, t = threadIdx.x % N2;
-  const int clip = blockIdx.y;
-  const int W = 2 * BB + 1;
-  const int col = blockIdx.x * TEAMS + team;
-  const bool active = col < W;
-  const int kx = col - BB;
-  const bool live = active && kx >= -B && kx <= B;
-  const int kk = !live ? 0 : (kx >= 0 ? kx : B - kx);
-  const int nk = 2 * B + 1;
-  const float2* src = tmp + ((size_t)clip * nk + kk) * N;
-  float2* mq = Mq + (size_t)clip * W * W;
-  float2* mp = Mp ? Mp + (size_t)clip * (W + 1) * W : nullptr;
-  auto put_p = [&](int c, int r, float2 v) {
-    mp[((size_t)((c + 1) >> 1) * W + r) * 2 + ((c + 1) & 1)] = v;
-  };
-  fft_four_step<-1, N1, N2>(
-      t, scratch[team], tw_n,
-      [&](int i) {
-        if (!live) return c32{0.f, 0.f};
-        const float2 z = src[i];
-        return c32{z.x, z.y};
-      },
-      [&](int k, c32 v) {
-        if (!active) return;
-        int ky;
-        if (k <= BB) ky = k;
-        else if (k >= N - BB) ky = k - N;
-        else return;
-        if (live && ky >= -B && ky <= B) v = cscale(v, sinc_t[kx + B] * sinc_t[ky + B]);
-        else v = c32{0.f, 0.f};
-        mq[(size_t)col * W + (ky + BB)] = make_float2(v.re, v.im);
-        if (mp) {
-          put_p(col, ky + BB, make_float2(v.re, v.im));
-          if (col == 0) put_p(-1, ky + BB, make_float2(0.f, 0.f));  // the zero column
-        }
-      });
-}
-
-// ---------------------------------------------------------------------------
 // Pruned forward transforms: of a length N = 32 L only the bins |k| < 16 T (T = 2 or
 // 4) are wanted.  L lanes share a transform; lane n1 holds x[n1 + L n2], n2 < 32, and
 // transforms over n2 in registers:
@@ -305,7 +221,9 @@ __device__ __forceinline__ void pruned_sums(int t, const c32* y, Emit emit) {
 }
 
 // rows_pruned: row spectra |k| <= B < 16 T of real row pairs z = a + i b (CX = false)
-// or of complex rows (CX), to tmp[item][k + B], item = pair or row over all clips.
+// or of the rows of complex transmittance rasters (CX: compute_from_transmittance with an
+// Array2<Complex64> map, aerial.rs:1789-1799; no Hermitian symmetry, so every row is its
+// own transform), to tmp[item][k + B], item = pair or row over all clips.
 // One wave per work-group, 64 / L items at a time, `per` times; a lane keeps the 31
 // factors W_N^{n1 k2} of its n1 in registers.
 template <int L, int T, bool CX>
@@ -1516,7 +1434,6 @@ static hipError_t rows_band_n(int B, int nclips, const float* masks, const float
              tmp);
 }
 
-// The factorisations of the four-step kernels; the pruned ones have one form.
 int band_fft_default(int n) {
   switch (n) {
     case 256: return 16;
@@ -1537,28 +1454,22 @@ int band_fft_options(int n, int* n1s) {
   }
 }
 
-// Dispatch over the supported four-step factorisations n = N1 x N2.
-#define HUV_BAND_FFT_SWITCH(FN, ...)                                  \
-  switch (n * 100 + (n1 ? n1 : band_fft_default(n))) {                \
-    case 256 * 100 + 8: return FN<8, 32>(__VA_ARGS__);                 \
-    case 256 * 100 + 16: return FN<16, 16>(__VA_ARGS__);               \
-    case 512 * 100 + 8: return FN<8, 64>(__VA_ARGS__);                 \
-    case 512 * 100 + 16: return FN<16, 32>(__VA_ARGS__);               \
-    case 1024 * 100 + 16: return FN<16, 64>(__VA_ARGS__);              \
-    case 1024 * 100 + 32: return FN<32, 32>(__VA_ARGS__);              \
-    case 2048 * 100 + 32: return FN<32, 64>(__VA_ARGS__);              \
-    default: return hipErrorInvalidValue;                              \
+// The four-step factorisation n = N1 x N2 of the wide bands.
+#define HUV_BAND_FFT_SWITCH(FN, ...)              \
+  switch (n) {                                    \
+    case 256: return FN<16, 16>(__VA_ARGS__);     \
+    case 512: return FN<16, 32>(__VA_ARGS__);     \
+    case 1024: return FN<32, 32>(__VA_ARGS__);    \
+    case 2048: return FN<32, 64>(__VA_ARGS__);    \
+    default: return hipErrorInvalidValue;         \
   }
 
 // The pruned transforms take every band up to 63, which is every band of an image (a
-// coarse grid of at most 256); wider ones (the density filter's) would need more outer
-// bins than T = 4 and keep the four-step kernels, whose layout of tmp is their own.
+// coarse grid of at most 256).  Wider ones would need more outer bins than T = 4 and keep
+// the four-step kernels, whose layout of tmp is their own: the density filter's, the ILT
+// gradient's band 2 B on coarse grids of 192 and 256, and whatever width a caller of
+// huv_band_spectrum asks for.
 static bool band_pruned(int B) { return B <= 63; }
-static bool band_n1_ok(int n, int n1) {
-  int o[4];
-  const int k = band_fft_options(n, o);
-  return n1 == 0 ? k > 0 : std::find(o, o + k, n1) != o + k;
-}
 
 template <int L, int T, bool CX>
 static hipError_t rows_pruned(int64_t items, int B, const float* masks, const float2* tw_n,
@@ -1627,9 +1538,8 @@ static hipError_t cols_pruned_n(int n, int B, int BB, int nclips, const float2* 
 #undef HUV_COLS_PRUNED
 }
 
-hipError_t launch_rows_band(int n, int n1, int B, int nclips, const float* masks,
-                            const float2* tw_n, float2* tmp, hipStream_t s) {
-  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
+hipError_t launch_rows_band(int n, int B, int nclips, const float* masks, const float2* tw_n,
+                            float2* tmp, hipStream_t s) {
   if (band_pruned(B)) return rows_pruned_n<false>(n, B, nclips, masks, tw_n, tmp, s);
   HUV_BAND_FFT_SWITCH(rows_band_n, B, nclips, masks, tw_n, tmp, s)
 }
@@ -1643,48 +1553,27 @@ static hipError_t cols_band_n(int B, int BB, int nclips, const float2* tmp, cons
              Mq, Mp);
 }
 
-hipError_t launch_cols_band(int n, int n1, int B, int BB, int nclips, const float2* tmp,
+hipError_t launch_cols_band(int n, int B, int BB, int nclips, const float2* tmp,
                             const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                             hipStream_t s) {
   if (BB < B || 2 * BB + 1 > n) return hipErrorInvalidValue;
-  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
   if (band_pruned(B))
     return cols_pruned_n<false>(n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s);
   HUV_BAND_FFT_SWITCH(cols_band_n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s)
 }
 
-template <int N1, int N2>
-static hipError_t rows_band_c_n(int B, int nclips, const float2* masks, const float2* tw,
-                                float2* tmp, hipStream_t s) {
-  constexpr int TEAMS = 128 / N2 > 0 ? 128 / N2 : 1;
-  dim3 grid((N1 * N2 + TEAMS - 1) / TEAMS, nclips);
-  HUV_LAUNCH((k_rows_band_c<N1, N2, TEAMS>), grid, dim3(TEAMS * N2), 0, s, masks, B, tw, tmp);
+// Complex rasters are imaged only, so their band is at most 63.
+hipError_t launch_rows_band_c(int n, int B, int nclips, const float2* masks, const float2* tw_n,
+                              float2* tmp, hipStream_t s) {
+  if (!band_pruned(B)) return hipErrorInvalidValue;
+  return rows_pruned_n<true>(n, B, nclips, reinterpret_cast<const float*>(masks), tw_n, tmp, s);
 }
 
-hipError_t launch_rows_band_c(int n, int n1, int B, int nclips, const float2* masks,
-                              const float2* tw_n, float2* tmp, hipStream_t s) {
-  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
-  if (band_pruned(B))
-    return rows_pruned_n<true>(n, B, nclips, reinterpret_cast<const float*>(masks), tw_n, tmp, s);
-  HUV_BAND_FFT_SWITCH(rows_band_c_n, B, nclips, masks, tw_n, tmp, s)
-}
-
-template <int N1, int N2>
-static hipError_t cols_band_c_n(int B, int BB, int nclips, const float2* tmp, const float2* tw_n,
-                                const float* sinc_t, float2* Mq, float2* Mp, hipStream_t s) {
-  constexpr int TEAMS = 128 / N2 > 0 ? 128 / N2 : 1;
-  dim3 grid((2 * BB + 1 + TEAMS - 1) / TEAMS, nclips);
-  HUV_LAUNCH((k_cols_band_c<N1, N2, TEAMS>), grid, dim3(TEAMS * N2), 0, s, tmp, B, BB, tw_n,
-             sinc_t, Mq, Mp);
-}
-
-hipError_t launch_cols_band_c(int n, int n1, int B, int BB, int nclips, const float2* tmp,
+hipError_t launch_cols_band_c(int n, int B, int BB, int nclips, const float2* tmp,
                               const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                               hipStream_t s) {
-  if (BB < B || 2 * BB + 1 > n) return hipErrorInvalidValue;
-  if (!band_n1_ok(n, n1)) return hipErrorInvalidValue;
-  if (band_pruned(B)) return cols_pruned_n<true>(n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s);
-  HUV_BAND_FFT_SWITCH(cols_band_c_n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s)
+  if (BB < B || 2 * BB + 1 > n || !band_pruned(B)) return hipErrorInvalidValue;
+  return cols_pruned_n<true>(n, B, BB, nclips, tmp, tw_n, sinc_t, Mq, Mp, s);
 }
 
 template <int M, int XNB, int XS = 1>

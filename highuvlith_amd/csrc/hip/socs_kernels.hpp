@@ -15,9 +15,8 @@ int coarse_classes(int m);
 // Kernel boxes and band spectra are stored at this width.
 int coarse_band(int m);
 
-// Band FFTs of length n run as four-step N1 x (n / N1): band_fft_default(n)
-// is the built-in N1, band_fft_options lists the supported ones (returns the
-// count).  n1 = 0 selects the default.
+// The factors N1 of four-step band transforms n = N1 x (n / N1) that a tuning may name
+// (band_fft_options, returns the count), and the one that is used, for bands above 63.
 int band_fft_default(int n);
 int band_fft_options(int n, int* n1s);
 // x pass of the field kernel: xlanes = 1 (one lane per band row, every
@@ -29,21 +28,21 @@ constexpr int kFieldsXnbDefault2 = 6;
 int fields_lanes_default(int m);
 bool fields_lanes_supported(int m, int xlanes);
 
-hipError_t launch_rows_band(int n, int n1, int B, int nclips, const float* masks,
-                            const float2* tw_n, float2* tmp, hipStream_t s);
+hipError_t launch_rows_band(int n, int B, int nclips, const float* masks, const float2* tw_n,
+                            float2* tmp, hipStream_t s);
 // Mq: [nclips][W][W] band spectrum (W = 2BB+1, [kx + BB][ky + BB]), zero
 // beyond |k| <= B.  Mp (optional, may be null): the same values column-paired,
 // [nclips][(W + 1) / 2][W][2] with column kx + BB at [(kx + BB + 1) / 2][.][(kx + BB + 1) % 2]
 // and a zero column in front (the layout of the two-lane field kernel).
-hipError_t launch_cols_band(int n, int n1, int B, int BB, int nclips, const float2* tmp,
+hipError_t launch_cols_band(int n, int B, int BB, int nclips, const float2* tmp,
                             const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                             hipStream_t s);
 // Complex rasters (masks: [nclips][n][n] interleaved complex): every row is
 // transformed (tmp: nclips n (2B+1) values) and both signs of kx are column
-// passes; Mq / Mp as for launch_cols_band.
-hipError_t launch_rows_band_c(int n, int n1, int B, int nclips, const float2* masks,
-                              const float2* tw_n, float2* tmp, hipStream_t s);
-hipError_t launch_cols_band_c(int n, int n1, int B, int BB, int nclips, const float2* tmp,
+// passes; Mq / Mp as for launch_cols_band.  B <= 63.
+hipError_t launch_rows_band_c(int n, int B, int nclips, const float2* masks, const float2* tw_n,
+                              float2* tmp, hipStream_t s);
+hipError_t launch_cols_band_c(int n, int B, int BB, int nclips, const float2* tmp,
                               const float2* tw_n, const float* sinc_t, float2* Mq, float2* Mp,
                               hipStream_t s);
 // One plane's kernels in a stack: `count` boxes from `first`, the `negative`
