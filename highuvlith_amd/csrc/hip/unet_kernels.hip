@@ -176,35 +176,29 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(ConvIn in, int N, int H, in
 }
 
 // ---------------------------------------------------------------------------
-// Forward 3x3 convolution of few input channels (the first layer's 8), input and
-// weights staged in LDS.  Work-group = 4 waves over an output tile of TH = 2 BM rows
-// x 64 columns of one image; wave w takes columns x0 + 32 (w % 2) .. + 31 of the BM
-// rows from y0 + BM (w / 2), and BN blocks of 32 output channels, so one weight
-// fragment feeds BM products.  Input channels run in chunks of CC: the (TH + 2) x
-// (64 + 2) x CC halo and the chunk's 9 x CC weights of the 32 BN output channels are
-// loaded once per chunk (zero outside the image and beyond Cout) and read by all four
-// waves from LDS; A = 32 pixels x 16 k per MFMA step (two 8-channel blocks of (tap,
-// channel) index 2s and 2s + 1, so at 8 channels a product spans two taps), B = 16 k x
-// 32 output channels.  The output leaves through LDS in 16-byte runs of channels, with
-// the ReLU mask and the 2 x 2 maximum as below.  Bound by the writes: 32 fields of
-// 512^2, 32 channels, 184 us.  Needs W % 64 == 0 and H % TH == 0.
+// Forward 3x3 convolution of the first layer's 8 input channels, input and weights staged
+// in LDS.  Work-group = 4 waves over an output tile of TH = 2 BM rows x 64 columns of one
+// image; wave w takes columns x0 + 32 (w % 2) .. + 31 of the BM rows from y0 + BM (w / 2),
+// and BN blocks of 32 output channels, so one weight fragment feeds BM products.  The
+// (TH + 2) x (64 + 2) x 8 halo and the 9 x 8 weights of the 32 BN output channels are
+// loaded once (zero outside the image and beyond Cout) and read by all four waves from
+// LDS; A = 32 pixels x 16 k per MFMA step, two taps of 8 channels.  The output leaves
+// through LDS in 16-byte runs of channels.  Bound by the writes: 32 fields of 512^2, 32
+// channels, 184 us.  Needs W % 64 == 0 and H % TH == 0.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int CC>
-__global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H, int W,
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(const bf16_t* __restrict__ X, int H, int W,
                                                          const bf16_t* __restrict__ Wt,
                                                          const float* __restrict__ bias, int Cout,
-                                                         int relu, const bf16_t* __restrict__ mask,
-                                                         bf16_t* __restrict__ Y,
-                                                         bf16_t* __restrict__ pool) {
+                                                         int relu, bf16_t* __restrict__ Y) {
+  constexpr int CC = 8, KB = 9, STEPS = (KB + 1) / 2;  // channels, taps, products
   constexpr int TH = 2 * BM, TW = 64, HR = TH + 2, HC = TW + 2;
   constexpr int PS = CC + 8;  // pixel stride in the tile (bf16), spreads the LDS banks
-  constexpr int CB = CC / 8, KBC = 9 * CB, STEPS = (KBC + 1) / 2;
-  constexpr int WS = 9 * CC + 8;   // output-channel stride of the staged weights (bf16)
+  constexpr int WS = KB * CC + 8;  // output-channel stride of the staged weights (bf16)
   constexpr int OS = 32 * BN + 8;  // pixel stride of the staged output (bf16)
   constexpr int IN_LDS = HR * HC * PS, OUT_LDS = TH * TW * OS;
   __shared__ __attribute__((aligned(16))) bf16_t tile[IN_LDS > OUT_LDS ? IN_LDS : OUT_LDS];
   __shared__ __attribute__((aligned(16))) bf16_t wts[32 * BN * WS];
-  const int Cin = in.Cu + in.C;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int half = lane >> 5, li = lane & 31;
   const int tilesX = W / TW, tilesY = H / TH;
@@ -213,8 +207,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H
   const int cobase = blockIdx.y * 32 * BN;
   const int px = 32 * (wave & 1) + li;  // this lane's A row (pixel column) in the tile
   const int py0 = BM * (wave >> 1);     // first output row of the wave in the tile
-  constexpr int HALO = HR * HC * CB, HIT = (HALO + 255) / 256;
-  constexpr int WGT = 32 * BN * KBC, WIT = (WGT + 255) / 256;
+  constexpr int HALO = HR * HC, HIT = (HALO + 255) / 256;
+  constexpr int WGT = 32 * BN * KB, WIT = (WGT + 255) / 256;
   f32x16 acc[BM][BN];
 #pragma unroll
   for (int bm = 0; bm < BM; ++bm)
@@ -222,74 +216,63 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H
     for (int bn = 0; bn < BN; ++bn)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bm][bn][r] = 0.f;
-  for (int c0 = 0; c0 < Cin; c0 += CC) {
-    // Every load of the chunk is issued before the first LDS store, so their
-    // latencies overlap.
-    // Buffer loads with 32-bit offsets into the image (or its half-resolution
-    // part): a pixel outside it, and an output channel beyond Cout, gets an
-    // offset past the end, which reads zero.
-    uint4 hv[HIT], wv[WIT];
-    const bool up = c0 < in.Cu;
-    const int sh = up ? 1 : 0, cs = up ? in.Cu : in.C, ws = W >> sh;
-    const int image = (H >> sh) * ws * cs;
-    const bf16_t* src = (up ? in.U : in.X) + (size_t)n * image;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16_t*>(src), (short)0, image * (int)sizeof(bf16_t), 0x00020000);
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16_t*>(Wt), (short)0, Cout * 9 * Cin * (int)sizeof(bf16_t), 0x00020000);
-    const int soff = (up ? c0 : c0 - in.Cu) * (int)sizeof(bf16_t);
+  // Every load is issued before the first LDS store, so their latencies overlap: buffer
+  // loads with 32-bit offsets into the image, where a pixel outside it, and an output
+  // channel beyond Cout, gets an offset past the end, which reads zero.
+  uint4 hv[HIT], wv[WIT];
+  const int image = H * W * CC;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(X + (size_t)n * image), (short)0, image * (int)sizeof(bf16_t), 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(Wt), (short)0, Cout * KB * CC * (int)sizeof(bf16_t), 0x00020000);
 #pragma unroll
-    for (int k = 0; k < HIT; ++k) {
-      const int i = threadIdx.x + 256 * k;
-      const int cb = i % CB, pix = i / CB;
-      const int yy = y0 - 1 + pix / HC, xx = x0 - 1 + pix % HC;
-      const bool v = i < HALO && yy >= 0 && yy < H && xx >= 0 && xx < W;
-      const int off = (((yy >> sh) * ws + (xx >> sh)) * cs + 8 * cb) * (int)sizeof(bf16_t);
-      hv[k] = __builtin_bit_cast(
-          uint4, __builtin_amdgcn_raw_buffer_load_b128(xr, v ? off + soff : -1, 0, 0));
+  for (int k = 0; k < HIT; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    const int yy = y0 - 1 + i / HC, xx = x0 - 1 + i % HC;
+    const bool v = i < HALO && yy >= 0 && yy < H && xx >= 0 && xx < W;
+    const int off = (yy * W + xx) * CC * (int)sizeof(bf16_t);
+    hv[k] = __builtin_bit_cast(uint4,
+                               __builtin_amdgcn_raw_buffer_load_b128(xr, v ? off : -1, 0, 0));
+  }
+#pragma unroll
+  for (int k = 0; k < WIT; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    const int tap = i % KB, col = i / KB, c = cobase + col;
+    const bool v = i < WGT && c < Cout;
+    const int off = (c * KB + tap) * CC * (int)sizeof(bf16_t);
+    wv[k] = __builtin_bit_cast(uint4,
+                               __builtin_amdgcn_raw_buffer_load_b128(wr, v ? off : -1, 0, 0));
+  }
+#pragma unroll
+  for (int k = 0; k < HIT; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    if (i < HALO) *reinterpret_cast<uint4*>(tile + i * PS) = hv[k];
+  }
+#pragma unroll
+  for (int k = 0; k < WIT; ++k) {
+    const int i = threadIdx.x + 256 * k;
+    if (i < WGT) *reinterpret_cast<uint4*>(wts + (i / KB) * WS + CC * (i % KB)) = wv[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) {
+    const int kb = 2 * s + half;
+    const bool kv = kb < KB;
+    const int tap = kv ? kb : 0;
+    const int dy = tap / 3, dx = tap % 3;
+    bf16x8 bw[BN];
+#pragma unroll
+    for (int bn = 0; bn < BN; ++bn) {
+      const bf16x8 w = ld8(wts + (32 * bn + li) * WS + CC * tap);
+      bw[bn] = kv ? w : zero8();
     }
 #pragma unroll
-    for (int k = 0; k < WIT; ++k) {
-      const int i = threadIdx.x + 256 * k;
-      const int kb = i % KBC, col = i / KBC;  // kb = tap * CB + cb
-      const int tap = kb / CB, cb = kb % CB, c = cobase + col;
-      const bool v = i < WGT && c < Cout;
-      const int off = ((c * 9 + tap) * Cin + c0 + 8 * cb) * (int)sizeof(bf16_t);
-      wv[k] = __builtin_bit_cast(uint4,
-                                 __builtin_amdgcn_raw_buffer_load_b128(wr, v ? off : -1, 0, 0));
-    }
-    __syncthreads();  // the previous chunk has been consumed
+    for (int bm = 0; bm < BM; ++bm) {
+      const bf16x8 a0 = ld8(tile + ((py0 + bm + dy) * HC + px + dx) * PS);
+      const bf16x8 a = kv ? a0 : zero8();
 #pragma unroll
-    for (int k = 0; k < HIT; ++k) {
-      const int i = threadIdx.x + 256 * k;
-      if (i < HALO) *reinterpret_cast<uint4*>(tile + (i / CB) * PS + 8 * (i % CB)) = hv[k];
-    }
-#pragma unroll
-    for (int k = 0; k < WIT; ++k) {
-      const int i = threadIdx.x + 256 * k;
-      if (i < WGT) *reinterpret_cast<uint4*>(wts + (i / KBC) * WS + 8 * (i % KBC)) = wv[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < STEPS; ++s) {
-      const int kb = 2 * s + half;
-      const bool kv = kb < KBC;
-      const int tap = kv ? kb / CB : 0, cb = kv ? kb % CB : 0;
-      const int dy = tap / 3, dx = tap % 3;
-      bf16x8 bw[BN];
-#pragma unroll
-      for (int bn = 0; bn < BN; ++bn) {
-        const bf16x8 w = ld8(wts + (32 * bn + li) * WS + 8 * (kv ? kb : 0));
-        bw[bn] = kv ? w : zero8();
-      }
-#pragma unroll
-      for (int bm = 0; bm < BM; ++bm) {
-        const bf16x8 a0 = ld8(tile + ((py0 + bm + dy) * HC + px + dx) * PS + 8 * cb);
-        const bf16x8 a = kv ? a0 : zero8();
-#pragma unroll
-        for (int bn = 0; bn < BN; ++bn)
-          acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bw[bn], acc[bm][bn], 0, 0, 0);
-      }
+      for (int bn = 0; bn < BN; ++bn)
+        acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bw[bn], acc[bm][bn], 0, 0, 0);
     }
   }
   __syncthreads();  // the tile has been read by every wave
@@ -313,31 +296,7 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd_lds(ConvIn in, int N, int H
     const int g = i % G8, q = i / G8, c = cobase + 8 * g;
     if (c >= Cout) continue;
     const size_t at = (((size_t)n * H + y0 + q / TW) * W + x0 + q % TW) * Cout + c;
-    B8 v;
-    v.u = *reinterpret_cast<const uint4*>(tile + q * OS + 8 * g);
-    if (mask) {
-      B8 y;
-      y.u = *reinterpret_cast<const uint4*>(mask + at);
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (bf2f(y.h[e]) <= 0.f) v.h[e] = 0;
-    }
-    *reinterpret_cast<uint4*>(Y + at) = v.u;
-  }
-  if (!pool) return;
-  for (int i = threadIdx.x; i < TH * TW / 4 * G8; i += 256) {
-    const int g = i % G8, q = i / G8, c = cobase + 8 * g;
-    if (c >= Cout) continue;
-    const int yo = q / (TW / 2), xo = q % (TW / 2);
-    const bf16_t* b = tile + (2 * yo * TW + 2 * xo) * OS + 8 * g;
-    B8 v0, v1, v2, v3;
-    v0.u = *reinterpret_cast<const uint4*>(b);
-    v1.u = *reinterpret_cast<const uint4*>(b + OS);
-    v2.u = *reinterpret_cast<const uint4*>(b + TW * OS);
-    v3.u = *reinterpret_cast<const uint4*>(b + (TW + 1) * OS);
-    *reinterpret_cast<uint4*>(
-        pool + (((size_t)n * (H / 2) + y0 / 2 + yo) * (W / 2) + x0 / 2 + xo) * Cout + c) =
-        max4(v0, v1, v2, v3).u;
+    *reinterpret_cast<uint4*>(Y + at) = *reinterpret_cast<const uint4*>(tile + q * OS + 8 * g);
   }
 }
 
@@ -1310,14 +1269,15 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
 #undef HUV_CONV_ROWS
     return hipGetLastError();
   }
-  if (chunk == 8 && W % 64 == 0 && H % 4 == 0 && (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) &&
-      (int64_t)H * W * in.C < (1ll << 30)) {
+  // the first layer's form: neither mask nor pool nor a second source
+  if (chunk == 8 && in.Cu == 0 && !mask && !pool && W % 64 == 0 && H % 4 == 0 &&
+      (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) && (int64_t)H * W * in.C < (1ll << 30)) {
     // tiles of 4 rows x 64 columns: BM = 2 pixel blocks per wave
     dim3 grid((unsigned)((int64_t)N * (H / 4) * (W / 64)),
               (unsigned)((Cout + (Cout <= 32 ? 31 : 63)) / (Cout <= 32 ? 32 : 64)));
-#define HUV_CONV_LDS(BN_)                                                                          \
-  hipLaunchKernelGGL((k_conv3x3_fwd_lds<2, BN_, 8>), grid, dim3(256), 0, s, in, N, H, W, Wt, bias, \
-                     Cout, relu, mask, Y, pool)
+#define HUV_CONV_LDS(BN_)                                                                     \
+  hipLaunchKernelGGL((k_conv3x3_fwd_lds<2, BN_>), grid, dim3(256), 0, s, in.X, H, W, Wt, bias, \
+                     Cout, relu, Y)
     if (Cout <= 32) HUV_CONV_LDS(1);
     else HUV_CONV_LDS(2);
 #undef HUV_CONV_LDS
