@@ -40,9 +40,13 @@ struct huv_ilt {
 namespace {
 
 constexpr int kBpi = 64;  // reduction blocks per image
-// Batch size the field kernel's split of the kernel sum is chosen for (m = 128,
-// three conditions, 32 kernels: 16 partial images instead of 32 for one target;
-// 5 targets then take 960 field work-groups of two kernels, not 1920 of one).
+// Batch size the field kernel's split of the kernel sum is chosen for, the same for
+// every batch (ilt_eval).  Fewer targets would want more splits, more targets fewer:
+// chosen for 1, 2 and 4, a gradient takes (us; annular source, three conditions of
+// distinct images, at 256^2 and 512^2 the same within 1 % up to 5 targets)
+//   1024^2, 1 target 243, 236, 239;  5 targets 321, 313, 314
+//   512^2, 24 targets 279, 279, 270;  64 targets, one condition 249, 247, 249
+// so 2 is the best or within 4 % of it over that range.
 constexpr int kSplitBatch = 2;
 
 struct IltBuffers {
