@@ -21,8 +21,8 @@ namespace huv {
 
 namespace {
 
-// Two doubles at the 8-byte alignment of any element.
-typedef double v2 __attribute__((vector_size(16), aligned(8)));
+// Two doubles of a row, at the 8-byte alignment of any element.
+typedef double v2 __attribute__((vector_size(16), aligned(8), may_alias));
 
 // Hermitian functions on the (2B+1)^2 box as real vectors of the same length:
 // the Gram products sum over both f and -f, so the half box carries sqrt(2).
