@@ -188,8 +188,13 @@ huvk::ConvIn decoder_input(huv_unet* u, int l) {
 huv_status conv_fwd(huv_unet* u, const Conv& c, const huvk::ConvIn& x, int l,
                     const huvk::ConvOut& y) {
   const Acts& a = u->a;
-  HCHK(huvk::launch_conv3x3_fwd(x, a.N, a.H >> l, a.W >> l, wbf(u, c), u->p + c.b_off, c.cout, 1, y,
-                                S(u)),
+  const int H = a.H >> l, W = a.W >> l;
+  huvk::ConvIn in = x;
+  if (x.Cu > 0 && !huvk::conv3x3_by_rows(x, a.N, H, W, c.cout)) {
+    HCHK(huvk::launch_upcat_fwd(x.U, x.Cu, x.X, x.C, a.N, H, W, a.tmp, S(u)), "U-Net upsample");
+    in = input(a.tmp, c.cin);
+  }
+  HCHK(huvk::launch_conv3x3_fwd(in, a.N, H, W, wbf(u, c), u->p + c.b_off, c.cout, 1, y, S(u)),
        "U-Net conv forward");
   return HUV_OK;
 }

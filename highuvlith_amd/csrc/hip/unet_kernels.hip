@@ -83,15 +83,18 @@ __device__ __forceinline__ B8 sum4_masked(const B8& a0, const B8& a1, const B8& 
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution.  Work-group = 4 waves along pixels; each wave
 // computes BM x BN blocks of 32 pixels x 32 output channels.  The operands
-// of step s + 1 are loaded before the products of step s are issued.
+// of step s + 1 are loaded before the products of step s are issued.  One source: a
+// choice between two at every load cost all layers a tenth of their time, and the
+// concatenation a third of its own, where writing it once takes 5 us (the 11
+// convolutions of a gradient of 2 fields of 96 x 32, base 64: 541 -> 506 us).
 // ---------------------------------------------------------------------------
 template <int BM, int BN>
-__global__ __launch_bounds__(256) void k_conv3x3_fwd(ConvIn in, int N, int H, int W,
+__global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ X, int N, int H,
+                                                     int W, int Cin,
                                                      const bf16_t* __restrict__ Wt,
                                                      const float* __restrict__ bias, int Cout,
                                                      int relu, const bf16_t* __restrict__ mask,
                                                      bf16_t* __restrict__ Y) {
-  const int Cin = in.Cu + in.C;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int half = lane >> 5, li = lane & 31;
   const int64_t NP = (int64_t)N * H * W;
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(ConvIn in, int N, int H, in
     for (int bm = 0; bm < BM; ++bm) {
       const int yy = py[bm] + dy, xx = px[bm] + dx;
       const bool v = kv && pv[bm] && yy >= 0 && yy < H && xx >= 0 && xx < W;
-      a[bm] = v ? ld8(in.at(pn[bm], yy, xx, H, W, cb * 8)) : zero8();
+      a[bm] = v ? ld8(X + (((int64_t)pn[bm] * H + yy) * W + xx) * Cin + cb * 8) : zero8();
     }
 #pragma unroll
     for (int bn = 0; bn < BN; ++bn) {
@@ -1244,7 +1247,7 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
   bf16_t *Y = out.Y, *pool = out.pool;
   const bool rows = conv3x3_by_rows(in, N, H, W, Cout);
   if (in.C % 8 != 0 || in.Cu % 8 != 0 || Cout % 8 != 0 || Cout < 8 || N < 1 || H < 1 || W < 1 ||
-      (pool && (H % 2 != 0 || W % 2 != 0)) ||
+      (pool && (H % 2 != 0 || W % 2 != 0)) || (in.Cu > 0 && !rows) ||
       (out.head && (!rows || Cout > 64 || !out.head_w || !out.head_b)) || (!Y && !out.head) ||
       (out.Cu > 0 && (!rows || pool || mask || out.Cu % 8 != 0 || out.Cu > Cout)))
     return hipErrorInvalidValue;
@@ -1269,8 +1272,8 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
 #undef HUV_CONV_ROWS
     return hipGetLastError();
   }
-  // the first layer's form: neither mask nor pool nor a second source
-  if (chunk == 8 && in.Cu == 0 && !mask && !pool && W % 64 == 0 && H % 4 == 0 &&
+  // the first layer's form: neither mask nor pool
+  if (chunk == 8 && !mask && !pool && W % 64 == 0 && H % 4 == 0 &&
       (int64_t)N * (H / 4) * (W / 64) < (1ll << 31) && (int64_t)H * W * in.C < (1ll << 30)) {
     // tiles of 4 rows x 64 columns: BM = 2 pixel blocks per wave
     dim3 grid((unsigned)((int64_t)N * (H / 4) * (W / 64)),
@@ -1286,12 +1289,12 @@ hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_
   constexpr int BM = 2;
   if (Cout <= 32) {
     dim3 grid((unsigned)((NP + 4 * 32 * BM - 1) / (4 * 32 * BM)), (unsigned)((Cout + 31) / 32));
-    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 1>), grid, dim3(256), 0, s, in, N, H, W, Wt, bias, Cout,
-                       relu, mask, Y);
+    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 1>), grid, dim3(256), 0, s, in.X, N, H, W, Cin, Wt, bias,
+                       Cout, relu, mask, Y);
   } else {
     dim3 grid((unsigned)((NP + 4 * 32 * BM - 1) / (4 * 32 * BM)), (unsigned)((Cout + 63) / 64));
-    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 2>), grid, dim3(256), 0, s, in, N, H, W, Wt, bias, Cout,
-                       relu, mask, Y);
+    hipLaunchKernelGGL((k_conv3x3_fwd<BM, 2>), grid, dim3(256), 0, s, in.X, N, H, W, Cin, Wt, bias,
+                       Cout, relu, mask, Y);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || !pool) return e;

@@ -13,7 +13,8 @@ typedef uint16_t bf16_t;  // raw BF16 bits
 
 // A convolution's input: C channels of X (N, H, W), after Cu channels of the
 // half-resolution U (N, H/2, W/2) read by nearest 2x upsampling when Cu > 0 (the
-// decoder's concatenation, which is never written out).  C, Cu multiples of 8.
+// decoder's concatenation, which is not written out where conv3x3_by_rows).  C, Cu
+// multiples of 8.
 struct ConvIn {
   const bf16_t* X = nullptr;
   int C = 0;
@@ -42,7 +43,7 @@ struct ConvOut {
   const float *head_w = nullptr, *head_b = nullptr;
 };
 // out = act(conv3x3(in) + bias), pad 1, stride 1, Cout channels (a multiple of 8).
-// relu: 0/1.  bias may be NULL.
+// relu: 0/1.  bias may be NULL.  Cu > 0 only where conv3x3_by_rows.
 hipError_t launch_conv3x3_fwd(const ConvIn& in, int N, int H, int W, const bf16_t* Wt,
                               const float* bias, int Cout, int relu, const ConvOut& out,
                               hipStream_t s);
