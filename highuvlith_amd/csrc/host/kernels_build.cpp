@@ -314,10 +314,10 @@ void interval_coverage(std::vector<double>& cov, double a, double b, int n, doub
 
 void dedup(std::vector<double>& e, double eps) {
   std::sort(e.begin(), e.end());
-  std::vector<double> o;
+  size_t n = 0;
   for (double v : e)
-    if (o.empty() || v - o.back() > eps) o.push_back(v);
-  e.swap(o);
+    if (n == 0 || v - e[n - 1] > eps) e[n++] = v;
+  e.resize(n);
 }
 
 // First edge >= v - eps (partition point).
@@ -403,26 +403,29 @@ struct PaintRect {
   int cls;  // index of its value; 0 is the background
 };
 
-// Cells of the rectangles g (painter order) on their own merged edges.
-void resolve_group(const std::vector<PaintRect>& g, const std::vector<cd>& values, double eps,
-                   std::vector<RectCell>& out) {
-  const cd bg = values[0];
-  if (g.size() == 1) {
-    if (g[0].cls) out.push_back({g[0].x0, g[0].x1, g[0].y0, g[0].y1, values[g[0].cls] - bg});
-    return;
-  }
-  std::vector<double> xe, ye;
-  xe.reserve(2 * g.size());
-  ye.reserve(2 * g.size());
-  for (const auto& r : g) {
-    xe.push_back(r.x0); xe.push_back(r.x1);
-    ye.push_back(r.y0); ye.push_back(r.y1);
+// The edges of the first `count` rectangles, merged.
+void own_edges(const std::vector<PaintRect>& g, size_t count, double eps, std::vector<double>& xe,
+               std::vector<double>& ye) {
+  xe.clear();
+  ye.clear();
+  xe.reserve(2 * count);
+  ye.reserve(2 * count);
+  for (size_t i = 0; i < count; ++i) {
+    xe.push_back(g[i].x0); xe.push_back(g[i].x1);
+    ye.push_back(g[i].y0); ye.push_back(g[i].y1);
   }
   dedup(xe, eps);
   dedup(ye, eps);
+}
+
+// Cells of the rectangles g (painter order) on the edges xe, ye.
+void resolve_on(const std::vector<PaintRect>& g, const std::vector<cd>& values, double eps,
+                const std::vector<double>& xe, const std::vector<double>& ye,
+                std::vector<int>& cells, std::vector<RectCell>& out) {
+  const cd bg = values[0];
   const int64_t nx = (int64_t)xe.size() - 1, ny = (int64_t)ye.size() - 1;
   if (nx < 1 || ny < 1) return;
-  std::vector<int> cells((size_t)(nx * ny), 0);
+  cells.assign((size_t)(nx * ny), 0);
   for (const auto& r : g) {
     const int64_t i0 = edge_index(ye, r.y0, eps), i1 = std::min(edge_index(ye, r.y1, eps), ny);
     const int64_t j0 = edge_index(xe, r.x0, eps), j1 = std::min(edge_index(xe, r.x1, eps), nx);
@@ -445,6 +448,51 @@ void resolve_group(const std::vector<PaintRect>& g, const std::vector<cd>& value
     }
     i = k;
   }
+}
+
+// Edges and cells of the group at hand, kept over a clip's groups.
+struct GroupScratch {
+  std::vector<double> xe, ye;
+  std::vector<int> cells;
+};
+
+// Cells of the rectangles g (painter order) on their own merged edges.
+void resolve_group(const std::vector<PaintRect>& g, const std::vector<cd>& values, double eps,
+                   GroupScratch& s, std::vector<RectCell>& out) {
+  if (g.size() == 1) {
+    if (g[0].cls)
+      out.push_back({g[0].x0, g[0].x1, g[0].y0, g[0].y1, values[g[0].cls] - values[0]});
+    return;
+  }
+  own_edges(g, g.size(), eps, s.xe, s.ye);
+  resolve_on(g, values, eps, s.xe, s.ye, s.cells, out);
+}
+
+// Layouts whose rectangles share their edges (tilings, bricks, aligned arrays: at most
+// four grid cells a rectangle) are resolved on one grid, with no groups to find, if
+// that cuts nothing: the cells are then at most as many as the rectangles.  64
+// rectangles tell most other layouts.  s: all edges if they are known, or empty.
+// 32 x 32 touching squares: 0.15 ms against 0.45 by groups, 40 x 20 bricks 0.13 against
+// 0.32.
+bool resolve_common_edges(const std::vector<PaintRect>& rs, const std::vector<cd>& values,
+                          double eps, GroupScratch& s, std::vector<RectCell>& out) {
+  std::vector<double>&xe = s.xe, &ye = s.ye;
+  const size_t R = rs.size();
+  auto many = [&] {
+    return xe.size() < 2 || ye.size() < 2 || (xe.size() - 1) * (ye.size() - 1) > 4 * R;
+  };
+  if (xe.empty()) {
+    if (R > 128) {
+      own_edges(rs, 64, eps, xe, ye);
+      if (many()) return false;
+    }
+    own_edges(rs, R, eps, xe, ye);
+  }
+  if (many()) return false;
+  resolve_on(rs, values, eps, xe, ye, s.cells, out);
+  if (out.size() <= R) return true;
+  out.clear();
+  return false;
 }
 
 // Disjoint sets of rectangles; a set's name is its first rectangle.
@@ -569,9 +617,11 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
   }
   if (rs.empty()) return true;
   const size_t R = rs.size();
+  GroupScratch scratch;
+  std::vector<double>&xe = scratch.xe, &ye = scratch.ye;
   if ((double)(2 * R + 1) * (double)(2 * R + 1) > (double)max_cells) {
     // the clip's whole edge grid, field edges included, against the limit
-    std::vector<double> xe{-half, half}, ye{-half, half};
+    xe = ye = {-half, half};
     for (const auto& r : rs) {
       xe.push_back(r.x0); xe.push_back(r.x1);
       ye.push_back(r.y0); ye.push_back(r.y1);
@@ -583,8 +633,12 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
   }
   std::vector<PaintRect> g;
   std::vector<RectCell> joined;
+  if (R > 1 && resolve_common_edges(rs, values, eps, scratch, out)) {
+    if (grid_cells) *grid_cells = (int64_t)out.size();
+    return true;
+  }
   if (grid_cells) {
-    resolve_group(rs, values, eps, joined);
+    resolve_group(rs, values, eps, scratch, joined);
     *grid_cells = (int64_t)joined.size();
   }
   // overlapping rectangles, and those that touch along an edge as well
@@ -611,7 +665,7 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
       g.clear();
       const int part = order[i].over;
       for (; i < R && order[i].over == part; ++i) g.push_back(rs[order[i].i]);
-      resolve_group(g, values, eps, out);
+      resolve_group(g, values, eps, scratch, out);
       ++count;
     }
     if (count < 2) continue;
@@ -620,7 +674,7 @@ bool resolve_rect_cells(const std::vector<RectFeature>& rects, cd bg, int n, dou
     g.clear();
     for (size_t k = first; k < i; ++k) g.push_back(rs[order[k].i]);
     joined.clear();
-    resolve_group(g, values, eps, joined);
+    resolve_group(g, values, eps, scratch, joined);
     if (joined.size() >= out.size() - before) continue;
     out.resize(before);
     out.insert(out.end(), joined.begin(), joined.end());

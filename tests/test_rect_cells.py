@@ -108,6 +108,34 @@ static int check(const List& l, cd bg) {
 """
 
 BODIES = {
+    # layouts with common edges take one grid's time: far less than groups would
+    "common": r"""
+int main() {
+  for (cd bg : {cd(0, 0), cd(1, 0)})
+    for (const List& l : {tiles(32, 32, 16, 16, 1, 0, 1.0), tiles(20, 40, 40, 20, 1, 20, 1.0),
+                          tiles(12, 11, 40, 30, 1, 0, 1.0), tiles(9, 1, 20, 800, 0.5, 0, 1.0),
+                          tiles(2, 1, 20, 40, 1, 0, 1.0), tiles(50, 45, 16, 16, 0.5, 0, 1.0),
+                          tiles(13, 10, 40, 40, 1.2, 0, 0.5)})
+      if (int e = check(l, bg)) return e;
+  const List tiling = tiles(32, 32, 16, 16, 1, 0, 1.0);
+  List apart = tiles(32, 32, 16, 16, 0.5, 0, 1.0);  // as many, none alike
+  for (auto& r : apart) {
+    r.x += uni(0, 4);
+    r.y += uni(0, 4);
+    r.w += uni(0, 3);
+  }
+  std::vector<RectCell> cells;
+  double cost[2] = {1e9, 1e9};
+  for (int k = 0; k < 30; ++k)
+    for (int c = 0; c < 2; ++c) {
+      const auto t0 = std::chrono::steady_clock::now();
+      resolve_rect_cells(c ? apart : tiling, cd(0, 0), N, PX, 1 << 30, cells);
+      cost[c] = std::min(cost[c], std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+    }
+  std::printf("%.3f ms, apart %.3f ms\n", 1e3 * cost[0], 1e3 * cost[1]);
+  return cost[0] <= 2.0 * cost[1] ? 0 : 7;
+}
+""",
     # a call's limit counts one grid's cells, whatever the clip is cut into; the bound
     # that spares the count holds, and lets 512 clips of 200 scattered contacts pass
     "limit": r"""
