@@ -54,6 +54,12 @@ union B8 {
   bf16_t h[8];
 };
 
+// Four as one 8-byte word.
+union B4 {
+  uint2 u;
+  bf16_t h[4];
+};
+
 // The maximum of four, channel by channel, keeping the winner's bits.
 __device__ __forceinline__ B8 max4(const B8& v0, const B8& v1, const B8& v2, const B8& v3) {
   B8 o;
@@ -83,10 +89,14 @@ __device__ __forceinline__ B8 sum4_masked(const B8& a0, const B8& a1, const B8& 
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution.  Work-group = 4 waves along pixels; each wave
 // computes BM x BN blocks of 32 pixels x 32 output channels.  The operands
-// of step s + 1 are loaded before the products of step s are issued.  One source: a
-// choice between two at every load cost all layers a tenth of their time, and the
-// concatenation a third of its own, where writing it once takes 5 us (the 11
-// convolutions of a gradient of 2 fields of 96 x 32, base 64: 541 -> 506 us).
+// of step s + 1 are loaded before the products of step s are issued.  The products are
+// weights x pixels: a lane has four consecutive channels of its pixel at a time, so the
+// output and the ReLU mask (which two-byte accesses made a third of a masked layer's
+// epilogue) go in 8-byte words.  One source: a choice between two at every load cost all
+// layers a tenth of their time, and the concatenation a third of its own, where writing
+// it once takes 5 us.  Bound by the latency of its loads, each operand read anew for
+// every tap: a gradient of 2 fields of 96 x 32, base 64, takes 766 us (with pixels x
+// weights 821, and the choice of sources 854), of 8 of 96 x 96, base 32, 603 (651).
 // ---------------------------------------------------------------------------
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ X, int N, int H,
@@ -152,30 +162,42 @@ __global__ __launch_bounds__(256) void k_conv3x3_fwd(const bf16_t* __restrict__ 
     for (int bm = 0; bm < BM; ++bm)
 #pragma unroll
       for (int bn = 0; bn < BN; ++bn)
-        acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bm], b[bn], acc[bm][bn], 0, 0, 0);
+        acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bn], a[bm], acc[bm][bn], 0, 0, 0);
 #pragma unroll
     for (int bm = 0; bm < BM; ++bm) a[bm] = an[bm];
 #pragma unroll
     for (int bn = 0; bn < BN; ++bn) b[bn] = bnx[bn];
   }
+  // a lane's pixel of block bm, four channels of block bn at a time
 #pragma unroll
-  for (int bn = 0; bn < BN; ++bn) {
-    if (co[bn] >= Cout) continue;
-    const float bv = bias ? bias[co[bn]] : 0.f;
+  for (int bn = 0; bn < BN; ++bn)
 #pragma unroll
-    for (int bm = 0; bm < BM; ++bm)
+    for (int q = 0; q < 4; ++q) {
+      const int c = cobase + 32 * bn + 8 * q + 4 * half;
+      if (c >= Cout) continue;
+      float bv[4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = 8 * (r / 4) + 4 * half + (r % 4);
-        const int64_t p = pbase + 32 * bm + i;
-        if (p < NP) {
-          float v = acc[bm][bn][r] + bv;
-          if (relu) v = fmaxf(v, 0.f);
-          const bool off = mask && bf2f(mask[p * Cout + co[bn]]) <= 0.f;
-          Y[p * Cout + co[bn]] = off ? (bf16_t)0 : f2bf(v);
+      for (int e = 0; e < 4; ++e) bv[e] = bias ? bias[c + e] : 0.f;
+#pragma unroll
+      for (int bm = 0; bm < BM; ++bm) {
+        const int64_t p = pbase + 32 * bm + li;
+        if (p >= NP) continue;
+        B4 v, m;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float f = acc[bm][bn][4 * q + e] + bv[e];
+          if (relu) f = fmaxf(f, 0.f);
+          v.h[e] = f2bf(f);
         }
+        if (mask) {
+          m.u = *reinterpret_cast<const uint2*>(mask + p * Cout + c);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (bf2f(m.h[e]) <= 0.f) v.h[e] = 0;
+        }
+        *reinterpret_cast<uint2*>(Y + p * Cout + c) = v.u;
       }
-  }
+    }
 }
 
 // ---------------------------------------------------------------------------
