@@ -688,7 +688,7 @@ huv_status rect_band_stage(Ctx* c, int nclips, int n, int B, int BB, const RectB
   if (e != hipSuccess) return hip_fail(e, "rect_tables launch");
   c->stage_end(ST_RECT_TABLES, ev);
   c->stage_begin(ST_RECT_BAND, &ev);
-  e = huvk::launch_rect_band(X, Y, d_coff, d_bg, nclips, n, B, BB, Mq, Mp, c->stream());
+  e = huvk::launch_rect_band(X, Y, d_coff, ncells, d_bg, nclips, n, B, BB, Mq, Mp, c->stream());
   if (e != hipSuccess) return hip_fail(e, "rect_band launch");
   c->stage_end(ST_RECT_BAND, ev);
   if (nedges > 0) {

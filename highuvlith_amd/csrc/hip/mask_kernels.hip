@@ -530,8 +530,8 @@ hipError_t launch_rect_tables(const double* cells, int64_t ncells, int n, double
 }
 
 hipError_t launch_rect_band(const double2* X, const double2* Y, const int64_t* coff,
-                            const double* bg, int nclips, int n, int B, int BB, float2* Mq,
-                            float2* Mp, hipStream_t s) {
+                            int64_t ncells, const double* bg, int nclips, int n, int B, int BB,
+                            float2* Mq, float2* Mp, hipStream_t s) {
   if (nclips <= 0) return hipSuccess;
   if (B < 0 || BB < B || BB > 1024) return hipErrorInvalidValue;
   const int W = 2 * BB + 1;
@@ -539,9 +539,11 @@ hipError_t launch_rect_band(const double2* X, const double2* Y, const int64_t* c
   const int gpc = (G * G + 63) / 64;
   if ((int64_t)gpc * nclips >= (1ll << 31)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(gpc * nclips));
-  // Up to two work-groups per CU: eight waves each, else two (512 clips of 64
-  // cells, B = 47: 4608 work-groups fill the chip without more).
-  if (gpc * nclips <= 512)
+  // Eight waves where there is at most one work-group per CU and each wave has a cell or
+  // two, else two.  Band 47, us with two and eight waves: 24 clips (216 work-groups) of 8
+  // cells 8.1 and 8.8, of 16 10.0 and 9.4, of 43 16.0 and 12.3; 56 clips (504) of 43 18.3
+  // and 19.6, of none 6.8 and 10.3.
+  if (gpc * nclips <= 256 && ncells >= 12 * (int64_t)nclips)
     hipLaunchKernelGGL(k_rect_band<8>, grid, dim3(512), 0, s, X, Y, coff, bg, n, B, BB, gpc, Mq,
                        Mp);
   else

@@ -15,8 +15,8 @@ hipError_t launch_rect_tables(const double* cells, int64_t ncells, int n, double
 // coff: nclips + 1 cell offsets; bg: nclips x (re, im).  Writes the (2BB+1)^2
 // box Mq of every clip (and its column-paired copy Mp when non-null).
 hipError_t launch_rect_band(const double2* X, const double2* Y, const int64_t* coff,
-                            const double* bg, int nclips, int n, int B, int BB, float2* Mq,
-                            float2* Mp, hipStream_t s);
+                            int64_t ncells, const double* bg, int nclips, int n, int B, int BB,
+                            float2* Mq, float2* Mp, hipStream_t s);
 
 // Largest band half-width of the polygon pass: one edge's two order tables
 // (2 x (2B + 1) entries of 32 bytes) must fit 64 KiB of LDS.
