@@ -1353,9 +1353,10 @@ __global__ __launch_bounds__(256, TMIN == -2 && MODE == 0 ? 5 : 1) void k_band_i
     // Rows y = P (2 pr) + p and y + P, columns x = c + C i: vector buffer
     // stores with the column offset C i in an SGPR, marked non-temporal (cache
     // policy bit 1): the images stream out without evicting the next step's
-    // inputs from L2 and the MALL.  Up to n = 512 a store covers half a line or
-    // less, which must meet its other part in L2: 63 planes of 512^2 24.5 -> 19.8 us
-    // without the mark, while the images of a batch up to 2048^2 lose 4%.
+    // inputs from L2 and the MALL.  At n = 512 a store covers half a line, which
+    // must meet its other part in L2: 63 planes of 512^2 24.5 -> 19.8 us, 300 92 -> 72
+    // without the mark, while the images of a batch up to 2048^2 lose 4 %, and those of
+    // 256^2 11 % (64 planes 12.6 -> 14.3 us, 300 27.8 -> 29.8).
     const int va = ((P * (2 * pr) + p) * n + c) * (int)sizeof(float);
     const int vb = va + P * n * (int)sizeof(float);
     if constexpr (CHAIN) {
@@ -1363,7 +1364,7 @@ __global__ __launch_bounds__(256, TMIN == -2 && MODE == 0 ? 5 : 1) void k_band_i
       else chain_task<false>(ch.beta, d, C, va, vb, mrc, rrc, orc);
     } else if constexpr (!FID) {
       auto store = [&](__amdgpu_buffer_rsrc_t rc) {
-        if (n <= 512) store_task<0>(d, C, va, vb, rc);
+        if (n == 512) store_task<0>(d, C, va, vb, rc);
         else store_task<2>(d, C, va, vb, rc);
       };
       if (!map.src) {
