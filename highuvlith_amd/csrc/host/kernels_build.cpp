@@ -470,8 +470,11 @@ void resolve_group(const std::vector<PaintRect>& g, const std::vector<cd>& value
 
 // Layouts whose rectangles share their edges (tilings, bricks, aligned arrays: at most
 // four grid cells a rectangle) are resolved on one grid, with no groups to find, if
-// that cuts nothing: the cells are then at most as many as the rectangles.  64
-// rectangles tell most other layouts.  s: all edges if they are known, or empty.
+// that cuts nothing: the cells are then at most as many as the rectangles.  Other
+// layouts are mostly told by their first sqrt(R) + 1 rectangles: k of them with no
+// common edge cut (2 k - 1)^2 cells, more than 4 R (96 clips of 43 jittered contacts:
+// 0.24 ms, with all their edges sorted first 0.61).  s: all edges if they are known, or
+// empty.
 // 32 x 32 touching squares: 0.15 ms against 0.45 by groups, 40 x 20 bricks 0.13 against
 // 0.32.
 bool resolve_common_edges(const std::vector<PaintRect>& rs, const std::vector<cd>& values,
@@ -482,8 +485,9 @@ bool resolve_common_edges(const std::vector<PaintRect>& rs, const std::vector<cd
     return xe.size() < 2 || ye.size() < 2 || (xe.size() - 1) * (ye.size() - 1) > 4 * R;
   };
   if (xe.empty()) {
-    if (R > 128) {
-      own_edges(rs, 64, eps, xe, ye);
+    const size_t few = (size_t)std::ceil(std::sqrt((double)R)) + 1;
+    if (few < R) {
+      own_edges(rs, few, eps, xe, ye);
       if (many()) return false;
     }
     own_edges(rs, R, eps, xe, ye);

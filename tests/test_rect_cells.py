@@ -138,6 +138,73 @@ int main() {
 """,
     # a call's limit counts one grid's cells, whatever the clip is cut into; the bound
     # that spares the count holds, and lets 512 clips of 200 scattered contacts pass
+    "apart": r"""
+// A plan that compares all pairs and gives each rectangle a list of its own.
+static size_t all_pairs(const List& l) {
+  struct Box { double x0, x1, y0, y1; };
+  std::vector<Box> b;
+  for (auto& r : l) b.push_back({r.x - r.w / 2, r.x + r.w / 2, r.y - r.h / 2, r.y + r.h / 2});
+  std::vector<int> root(b.size());
+  for (size_t i = 0; i < b.size(); ++i) {
+    root[i] = (int)i;
+    for (size_t j = 0; j < i; ++j)
+      if (b[i].x0 < b[j].x1 && b[j].x0 < b[i].x1 && b[i].y0 < b[j].y1 && b[j].y0 < b[i].y1)
+        root[i] = root[j];
+  }
+  std::vector<std::vector<int>> members(b.size());
+  for (size_t i = 0; i < b.size(); ++i) members[root[i]].push_back((int)i);
+  std::vector<RectCell> cells;
+  for (auto& m : members)
+    for (int i : m) cells.push_back({b[i].x0, b[i].x1, b[i].y0, b[i].y1, l[i].value});
+  return cells.size();
+}
+static List apart(int n) {  // an array with no common edges
+  List l = tiles(8, (n + 7) / 8, 128, 60, 0.4, 0, 1.0);
+  l.resize(n);
+  for (auto& r : l) {
+    r.x += uni(-6, 6);
+    r.y += uni(-6, 6);
+    r.w += uni(0, 30);
+  }
+  return l;
+}
+int main() {
+  // the first rectangles of a list are like its others, or are not
+  for (int n : {2, 3, 4, 5, 6, 9, 10, 16, 17, 43, 128, 129})
+    for (int k = 1; k <= n; k += std::max(1, n / 6)) {
+      const List a = apart(n);
+      List t = tiles(8, (n + 7) / 8, 60, 50, 1, 0, 1.0);
+      t.resize(n);
+      List at(a.begin(), a.begin() + k), ta(t.begin(), t.begin() + k);
+      at.insert(at.end(), t.begin() + k, t.end());
+      ta.insert(ta.end(), a.begin() + k, a.end());
+      for (const List& l : {a, t, at, ta})
+        if (int e = check(l, cd(0, 0))) return e;
+    }
+  std::vector<List> clips;
+  for (int i = 0; i < 24; ++i) clips.push_back(apart(64));
+  double cost[2] = {1e9, 1e9};
+  size_t cells = 0, other = 0;
+  std::vector<RectCell> out;
+  for (int k = 0; k < 200; ++k)
+    for (int c = 0; c < 2; ++c) {
+      cells = c ? cells : 0;
+      other = c ? 0 : other;
+      const auto t0 = std::chrono::steady_clock::now();
+      for (auto& l : clips) {
+        if (c) {
+          other += all_pairs(l);
+        } else {
+          resolve_rect_cells(l, cd(0, 0), N, PX, 1 << 30, out);
+          cells += out.size();
+        }
+      }
+      cost[c] = std::min(cost[c], std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+    }
+  std::printf("%.1f us, all pairs %.1f us, %zu %zu cells\n", 1e6 * cost[0], 1e6 * cost[1], cells, other);
+  return cost[0] <= 1.1 * cost[1] ? 0 : 8;
+}
+""",
     "limit": r"""
 int main() {
   std::vector<RectCell> with, without;
